@@ -115,6 +115,7 @@ void* ch_run(const pl_config* pc, const uint8_t* ref, int64_t ref_len, const cha
   int64_t G = 0;
   std::vector<JobDev> jobs((size_t)n_jobs);
   std::vector<JobStat> st((size_t)n_jobs);
+  std::vector<uint32_t> hist((size_t)n_jobs * PL_HIST, 0);
   for (int32_t j = 0; j < n_jobs; j++) {
     JobDev& J = jobs[j];
     std::memset(&J, 0, sizeof J);
@@ -237,12 +238,12 @@ void* ch_run(const pl_config* pc, const uint8_t* ref, int64_t ref_len, const cha
             int64_t dep = 0;
             for (int b = 0; b < 4; b++) dep += (uint32_t)o.f[PL_F_COUNT_A + b];
             dep += o.f[PL_F_DELETIONS];
-            S.hist[dep > 255 ? 255 : dep]++;
+            hist[(size_t)j * PL_HIST + (dep > 255 ? 255 : dep)]++;
           } else if (d == PL_D_SNP || d == PL_D_AMB) {
             int64_t dep = 0;
             for (int b = 0; b < 4; b++) dep += (uint32_t)o.f[PL_F_COUNT_A + b];
             dep += o.f[PL_F_DELETIONS];
-            cands.push_back({(uint32_t)g, (int32_t)dep, d, 0, -1});
+            cands.push_back({(uint32_t)g, (int32_t)dep, d, 0, -1, 0, 0, 0});
           }
         }
       }
@@ -271,8 +272,8 @@ void* ch_run(const pl_config* pc, const uint8_t* ref, int64_t ref_len, const cha
     calls[g] = cl;
     const int d = call_disp(cl);
     const int64_t dep = c.depth();
-    if (d == PL_D_CONFIRMED) st[j].hist[dep > 255 ? 255 : dep]++;
-    else if (d != PL_D_NONE) cands.push_back({g, (int32_t)dep, d, ilen, wrec});
+    if (d == PL_D_CONFIRMED) hist[(size_t)j * PL_HIST + (dep > 255 ? 255 : dep)]++;
+    else if (d != PL_D_NONE) cands.push_back({g, (int32_t)dep, d, ilen, (int32_t)wrec, 0, 0, 0});
   }
   std::stable_sort(cands.begin(), cands.end(), [](const Cand& a, const Cand& b) { return a.gpos < b.gpos; });
   std::vector<uint32_t> mutated((size_t)G + 1);
@@ -286,7 +287,7 @@ void* ch_run(const pl_config* pc, const uint8_t* ref, int64_t ref_len, const cha
     b = a;
     while (b < (int64_t)cands.size() && cands[b].gpos < (uint64_t)(J.out + J.size)) b++;
     uint32_t m0 = mut_n;
-    finalize_job(cf, J, st[j], pile, G, calls, cands.data(), a, b, mutated.data(), &mut_n, (uint32_t)mutated.size(), &ovf);
+    finalize_job(cf, J, st[j], &hist[(size_t)j * PL_HIST], pile, G, calls, cands.data(), a, b, mutated.data(), &mut_n, (uint32_t)mutated.size(), &ovf);
     for (uint32_t k = m0; k < mut_n; k++) {
       const uint32_t g = mutated[k];
       Col c = load_col(pile, G, g);

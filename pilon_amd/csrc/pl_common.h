@@ -25,6 +25,7 @@
 #define RI_SEG_SHIFT    27           // complex reads: number of segments (RMeta.op0 = first)
 #define RI_SEG_MASK     0xf8000000u
 #define RI_SEG_MAX      31           // more segments, or a long read: the read is walked instead
+#define PL_COST_BINS    256         // cost classes of the work queue's order
 #define PL_LR_NANOPORE  1
 #define PL_LR_PACBIO    2
 
@@ -126,8 +127,8 @@ struct JobStat {             // device-written per job
   int32_t n_confirmed;
   int32_t cand_lo, cand_hi;  // range in the sorted candidate list
   int32_t pad;
-  uint32_t hist[256];        // confirmed candidates by depth (255 = 255+)
 };
+#define PL_HIST 256          // per job: confirmed candidates by depth (255 = 255+), beside its JobStat
 
 // one piece of insertion/deletion evidence (PileUp.addInsertion/addDeletion)
 struct IndelRec {
@@ -141,13 +142,15 @@ struct IndelRec {
   int64_t src;               // insertion: first base (2-bit or nibble index); deletion: contig offset
 };
 
-// a change candidate (SNP/AMB from the window kernel, INS/DEL from the indel pass)
+// a change candidate (a column whose disposition before Pass 1 is a change)
 struct Cand {
   uint32_t gpos;
   int32_t depth;             // count + deletions before any Pass-1 mutation
   int32_t kind;              // pl_disposition
   int32_t len;               // indel length
-  int64_t rec;               // winning IndelRec index (INS/DEL)
+  int32_t rec;               // winning IndelRec index (INS/DEL)
+  uint8_t base, alt;         // BaseCall.base, altBase
+  uint16_t pad;
 };
 
 struct KConf {               // the knobs kernels read (Pilon.scala:52-73)
@@ -165,16 +168,22 @@ struct EngineArgs {
   int32_t n_wins;
   int32_t W;                 // window size (positions)
   int32_t* queue;            // persistent work queue head
-  const int32_t* worder;     // window processing order
+  uint8_t* cost;             // [n_wins] cost bin of each window (0 = most reads)
+  uint32_t* bins;            // [2 * PL_COST_BINS]: windows per cost bin, then queue slots taken per bin
   const WinHead* heads;      // [n_wins] window heads in processing order
   int32_t* pile;             // [PL_NFIELDS][G]
   pl_call* calls;            // [G]
   int64_t G;
   JobStat* st;
+  uint32_t* hist;            // [n_jobs][PL_HIST]
   IndelRec* rec; uint32_t* rec_n; uint32_t rec_cap;
-  Cand* cand; uint32_t* cand_n; uint32_t cand_cap;
+  uint32_t* win_rec;         // [2 * n_wins]: each window's first record and count
+  IndelRec* spill; uint32_t* spill_win; uint32_t* spill_n; uint32_t spill_cap;   // records beyond a window's LDS buffer
+  uint32_t* win_cur;         // [n_wins] records placed from the spill
+  uint64_t* cmask;           // [n_wins][W / 64] candidate columns of each window, a bit per position
+  int32_t* prec;             // [G] winning record of the columns the indel pass called (-1: none)
+  Cand* cand; uint32_t* cand_n; uint32_t cand_cap;   // candidates in position order
   uint32_t* defer; uint32_t* defer_n; uint32_t defer_cap;
-  uint32_t* rkey; uint32_t* rval;   // sorted record keys/indices
   uint32_t* mutated; uint32_t* mutated_n; uint32_t mutated_cap;
   int32_t* overflow;                // capacity overflow flag
   struct WideCol* wide; uint32_t* wide_n; uint32_t wide_cap;   // exact sums of wide columns

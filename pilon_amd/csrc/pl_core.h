@@ -374,9 +374,12 @@ PL_HD FragTail frag_tail(const RMeta& m) {
 // which frag_tail holds.  read_in_query reduces to the kept/valid flags when
 // every such read has pos - 1 >= qs (spanEnd >= pos - 1) and pos < L0 <= qe;
 // otherwise the window takes every read through the full path.
+PL_HD bool fragment_all(const JobDev& J, int32_t L0, int32_t back, int32_t back_fp) {
+  return (int64_t)L0 - back - 1 < (int64_t)J.qs || back_fp >= back;
+}
 PL_HD int64_t fragment_only_end(const int32_t* pos, int64_t lo, int64_t hi, const JobDev& J, int32_t L0,
                                 int32_t back, int32_t back_fp) {
-  if ((int64_t)L0 - back - 1 < (int64_t)J.qs || back_fp >= back) return lo;
+  if (fragment_all(J, L0, back, back_fp)) return lo;
   const int64_t x = (int64_t)L0 - back_fp;
   while (lo < hi) {
     const int64_t m = (lo + hi) >> 1;
@@ -1054,7 +1057,7 @@ PL_HD pl_call full_call(const RSDev* rsets, const JobDev& J, const Col& c, uint8
 // deleted(i+j) and adds pu.deletions into those pileups (:259-264).
 // cand[c_lo..c_hi) are the region's SNP/AMB/INS/DEL candidates sorted by
 // position; kind is set to 0 for those that do not become changes.
-PL_HD void finalize_job(const KConf& cf, const JobDev& J, JobStat& st, int32_t* pile, int64_t G,
+PL_HD void finalize_job(const KConf& cf, const JobDev& J, JobStat& st, const uint32_t* hist, int32_t* pile, int64_t G,
                         pl_call* calls, Cand* cand, int64_t c_lo, int64_t c_hi,
                         uint32_t* mutated, uint32_t* mut_n, uint32_t mut_cap, int32_t* overflow) {
   const int32_t md = min_depth_of(cf, st.base_count, J.size);
@@ -1062,7 +1065,7 @@ PL_HD void finalize_job(const KConf& cf, const JobDev& J, JobStat& st, int32_t* 
   // confirmed positions by depth, from the histogram when minDepth falls
   // inside it; otherwise counted exactly after the pass (confirmed_exact)
   int64_t nconf = 0;
-  if (md <= PL_CONF_HIST_MAX) for (int d = md; d < 256; d++) nconf += st.hist[d];
+  if (md <= PL_CONF_HIST_MAX) for (int d = md; d < PL_HIST; d++) nconf += hist[d];
   int64_t delEnd = -1;
   for (int64_t k = c_lo; k < c_hi; k++) {
     Cand& c = cand[k];

@@ -5,7 +5,9 @@
 //   pile   int32 [PL_NFIELDS][G]   field-major PileUp counters
 //   calls  pl_call [G]             BaseCall + disposition, 8 B
 //   rec    IndelRec [cap]          insertion/deletion evidence, 32 B each
-//   cand   Cand [cap]              change candidates (sparse)
+//   prec   int32 [G]               winning evidence record (called columns)
+//   cmask  bit [G]                 candidate columns, per window
+//   cand   Cand [cap]              change candidates (sparse), in order
 // Resident per contig: the raw reference bytes; per read set: the packed
 // reads plus 24 B/read of derived facts (span, alignment end, info word) and
 // a 4 B/read prefix count of kept reads.
@@ -135,21 +137,24 @@ struct HostReads {
 
 }  // namespace
 
+// the batch's device counters (EngineArgs points into them)
+enum { PL_N_REC = 0, PL_N_CAND, PL_N_DEFER, PL_N_MUTATED, PL_N_OVERFLOW, PL_N_QUEUE, PL_N_WIDE, PL_N_DEEP, PL_N_SPILL,
+       PL_COUNTERS = 16 };
+
 // One independent batch pipeline: its stream, events, device buffers and
 // host-side tables.  A context has one (the plain and batched forms); a
 // server has one per concurrent batch.
 struct Lane {
   hipStream_t stream = nullptr;
   hipEvent_t ev[4] = {};
-  DBuf rsarr, kparr, jobs, wins, worder, costk, costv, costtk, costtv, pile, calls, st, rec, rkey, rval, rtk, rtv,
-      cand, cands, ckey, cval, ctk, ctv, defer, mutated, counters, hist, tiles, strpool, stridx, stroff, gath,
-      wide, winwide, heads;
-  uint32_t rec_cap = 0, cand_cap = 0, defer_cap = 0, mut_cap = 0, wide_cap = 0;
+  DBuf rsarr, kparr, jobs, wins, cost, bins, pile, calls, prec, cmask, csums, st, dhist, rec, winrec, wincur, spill,
+      spillwin, cand, defer, mutated, counters, strpool, stridx, stroff, wide, winwide, heads;
+  DBuf hist, tiles;                // sort and scan scratch (uploads, K-mers)
+  uint32_t rec_cap = 0, spill_cap = 0, cand_cap = 0, defer_cap = 0, mut_cap = 0, wide_cap = 0;
   std::vector<JobDev> hjobs;
   std::vector<WinDev> hwins;
   std::vector<JobStat> hst;
   std::vector<Cand> hcand;
-  std::vector<pl_call> hccall;     // calls of the candidate columns
   std::vector<int64_t> hins_off;   // insertion string of candidate k in hins_pool (-1: none)
   std::string hins_pool;
   int64_t G = 0;
@@ -157,13 +162,11 @@ struct Lane {
   int32_t n_wins = 0;
   bool exported_flags = false;
   double last_ms = 0, last_win_ms = 0;
-  uint32_t last_counts[8] = {0};
+  uint32_t last_counts[PL_COUNTERS] = {0};
   int32_t last_persistent = 0;
   int32_t last_block = 0;
   bool last_graph = false;
   EngineArgs args;
-  uint32_t* rkey_sorted = nullptr;
-  uint32_t* rval_sorted = nullptr;
   // job/window tables on the device describe last_reqs at window W
   std::vector<JobReq> last_reqs;
   bool tables_valid = false;
@@ -185,27 +188,24 @@ struct Lane {
   DBuf jdepth;
   bool has_jdepth = false;
 
-  size_t device_bytes() const {
-    const DBuf* b[] = {&rsarr, &kparr, &jobs, &wins, &worder, &costk, &costv, &costtk, &costtv, &pile, &calls, &st,
-                       &rec, &rkey, &rval, &rtk, &rtv, &cand, &cands, &ckey, &cval, &ctk, &ctv, &defer, &mutated,
-                       &counters, &hist, &tiles, &strpool, &stridx, &stroff, &gath, &wide, &winwide, &heads};
-    size_t t = 0;
-    for (const DBuf* x : b) t += x->cap;
-    return t;
+  template <class F> void for_each_buffer(F&& f) {
+    DBuf* b[] = {&rsarr, &kparr, &jobs, &wins, &cost, &bins, &pile, &calls, &prec, &cmask, &csums, &st, &dhist, &rec,
+                 &winrec, &wincur, &spill, &spillwin, &cand, &defer, &mutated, &counters, &strpool, &stridx, &stroff,
+                 &wide, &winwide, &heads, &hist, &tiles, &jdepth};
+    for (DBuf* x : b) f(*x);
   }
-  void for_each_buffer(void (*f)(DBuf&, Arena*), Arena* a) {
-    DBuf* b[] = {&rsarr, &kparr, &jobs, &wins, &worder, &costk, &costv, &costtk, &costtv, &pile, &calls, &st, &rec,
-                 &rkey, &rval, &rtk, &rtv, &cand, &cands, &ckey, &cval, &ctk, &ctv, &defer, &mutated, &counters,
-                 &hist, &tiles, &strpool, &stridx, &stroff, &gath, &wide, &winwide, &heads, &jdepth};
-    for (DBuf* x : b) f(*x, a);
+  size_t device_bytes() {
+    size_t t = 0;
+    for_each_buffer([&](DBuf& d) { t += d.cap; });
+    return t - jdepth.cap;
   }
   // every device buffer of the lane carved from a (no allocation, no free)
-  void use_arena(Arena* a) { for_each_buffer([](DBuf& d, Arena* x) { d.release(); d.arena = x; }, a); }
+  void use_arena(Arena* a) { for_each_buffer([a](DBuf& d) { d.release(); d.arena = a; }); }
   void free_buffers() {
-    for_each_buffer([](DBuf& d, Arena*) { d.release(); }, nullptr);
+    for_each_buffer([](DBuf& d) { d.release(); });
     tables_valid = false;
     rs_seen = 0;
-    rec_cap = cand_cap = defer_cap = mut_cap = wide_cap = 0;
+    rec_cap = spill_cap = cand_cap = defer_cap = mut_cap = wide_cap = 0;
   }
 };
 
@@ -832,7 +832,7 @@ struct GraphKey {
   EngineArgs A;
   int32_t W, block, persistent, grid;
   uint64_t lds;
-  const void* bufs[8];
+  const void* bufs[2];
 };
 
 void drop_graph(Lane* L) {
@@ -870,26 +870,18 @@ void lane_destroy(Lane* L) {
 // timed set, events bracket the window kernel (not while capturing)
 pl_status enqueue_batch(Lane* L, EngineArgs& A, int persistent, int block, int grid, size_t lds, bool timed) {
   hipStream_t st = L->stream;
-  uint32_t* cnt = L->counters.as<uint32_t>();
   const int32_t n_jobs = A.n_jobs, n_wins = A.n_wins;
-  const int64_t G = A.G;
-  const int64_t words = (int64_t)n_jobs * (sizeof(JobStat) / 4);
-  k_init_stats<<<dim3((unsigned)std::min<int64_t>(4096, std::max<int64_t>(1, (words + 255) / 256))), dim3(256), 0, st>>>(A.st, n_jobs, cnt, 16);
-  k_init_stats2<<<dim3((n_jobs + 255) / 256), dim3(256), 0, st>>>(A.st, n_jobs);
-  k_plan<<<dim3((n_wins + 255) / 256), dim3(256), 0, st>>>(A.rs, A.jobs, L->wins.as<WinDev>(), n_wins, L->costk.as<uint32_t>());
-  HIPCHK(hipGetLastError());
-  A.worder = L->worder.as<int32_t>();
-  if (persistent) {
-    k_iota<<<dim3((unsigned)std::min<int64_t>(1024, (n_wins + 255) / 256)), dim3(256), 0, st>>>(L->costv.as<uint32_t>(), n_wins, cnt + 8);
-    uint32_t *sk, *sv;
-    pl_status s = radix_sort(L, L->costk.as<uint32_t>(), L->costv.as<uint32_t>(), L->costtk.as<uint32_t>(),
-                             L->costtv.as<uint32_t>(), cnt + 8, (uint32_t)n_wins, 16, &sk, &sv);
-    if (s) return s;
-    A.worder = (const int32_t*)sv;
+  const unsigned jb = (unsigned)(n_jobs + 3) / 4, pb = (unsigned)(n_wins + 15) / 16;
+  WinDev* wins = L->wins.as<WinDev>();
+  const uint32_t* const* kp = (const uint32_t* const*)L->kparr.p;
+  uint32_t* cnt = L->counters.as<uint32_t>();
+  // windows in their own order need no cost order: one launch prepares everything
+  const bool ordered = persistent && n_wins > grid;
+  k_begin<<<dim3(1 + jb + (ordered ? 0 : pb)), dim3(256), 0, st>>>(A, kp, cnt, PL_COUNTERS, wins, ordered ? 0 : 1);
+  if (ordered) {
+    k_plan<<<dim3(pb), dim3(256), 0, st>>>(A, wins);
+    k_heads<<<dim3((unsigned)(n_wins + 255) / 256), dim3(256), 0, st>>>(A);
   }
-  k_win_heads<<<dim3((n_wins + 255) / 256), dim3(256), 0, st>>>(A.jobs, A.wins, persistent ? A.worder : nullptr, n_wins,
-                                                                 (WinHead*)A.heads);
-  k_jobprep<<<dim3(n_jobs), dim3(64), 0, st>>>(A.rs, (const uint32_t* const*)L->kparr.p, A.jobs, A.st);
   HIPCHK(hipGetLastError());
   if (timed) HIPCHK(hipEventRecord(L->ev[2], st));
   if (block == 256) k_window<256><<<dim3(grid), dim3(256), lds, st>>>(A, persistent);
@@ -897,30 +889,16 @@ pl_status enqueue_batch(Lane* L, EngineArgs& A, int persistent, int block, int g
   else k_window<1024><<<dim3(grid), dim3(1024), lds, st>>>(A, persistent);
   HIPCHK(hipGetLastError());
   if (timed) HIPCHK(hipEventRecord(L->ev[3], st));
-  // evidence records: sort by (position, kind), then the deferred columns
-  const uint32_t gb = (uint32_t)std::min<int64_t>(4096, std::max<int64_t>(1, ((int64_t)A.rec_cap + 255) / 256));
-  k_rec_keys<<<dim3(gb), dim3(256), 0, st>>>(A.rec, A.rec_n, A.rec_cap, L->rkey.as<uint32_t>(), L->rval.as<uint32_t>());
-  uint32_t *rk, *rv;
-  pl_status s = radix_sort(L, L->rkey.as<uint32_t>(), L->rval.as<uint32_t>(), L->rtk.as<uint32_t>(), L->rtv.as<uint32_t>(),
-                           A.rec_n, A.rec_cap, bits_for(2 * (uint64_t)G), &rk, &rv);
-  if (s) return s;
-  A.rkey = rk; A.rval = rv;
-  L->rkey_sorted = rk; L->rval_sorted = rv;
-  const uint32_t gd = (uint32_t)std::min<int64_t>(2048, std::max<int64_t>(1, ((int64_t)A.defer_cap + 3) / 4));
-  k_indel_pass<<<dim3(gd), dim3(256), 0, st>>>(A, A.defer, A.defer_n, A.defer_cap, 0);
-  HIPCHK(hipGetLastError());
-  // candidates by position, then Pass 1 per region
-  const uint32_t gc = (uint32_t)std::min<int64_t>(1024, std::max<int64_t>(1, ((int64_t)A.cand_cap + 255) / 256));
-  k_cand_keys<<<dim3(gc), dim3(256), 0, st>>>(A.cand, A.cand_n, A.cand_cap, L->ckey.as<uint32_t>(), L->cval.as<uint32_t>());
-  uint32_t *ck, *cv;
-  s = radix_sort(L, L->ckey.as<uint32_t>(), L->cval.as<uint32_t>(), L->ctk.as<uint32_t>(), L->ctv.as<uint32_t>(),
-                 A.cand_n, A.cand_cap, bits_for((uint64_t)G), &ck, &cv);
-  if (s) return s;
-  k_cand_gather<<<dim3(gc), dim3(256), 0, st>>>(A.cand, A.cand_n, A.cand_cap, cv, L->cands.as<Cand>());
-  k_finalize<<<dim3(n_jobs), dim3(64), 0, st>>>(A, L->cands.as<Cand>(), A.cand_n, A.cand_cap, L->cands.as<Cand>());
-  k_confirm_exact<<<dim3((unsigned)std::min<int32_t>(n_wins, 1024)), dim3(256), 0, st>>>(A);
-  const uint32_t gm = (uint32_t)std::min<int64_t>(2048, std::max<int64_t>(1, ((int64_t)A.mutated_cap + 3) / 4));
-  k_indel_pass<<<dim3(gm), dim3(256), 0, st>>>(A, A.mutated, A.mutated_n, A.mutated_cap, 1);
+  // the deferred columns, the candidates in order, Pass 1 per region
+  const int64_t words = (int64_t)n_wins * (A.W / 64);
+  const unsigned cb = (unsigned)((words + PL_CAND_WORDS - 1) / PL_CAND_WORDS);
+  const unsigned gd = (unsigned)std::min<int64_t>(2048, std::max<int64_t>(1, ((int64_t)std::min<int64_t>(A.defer_cap, A.G) + 3) / 4));
+  k_spill_place<<<dim3(256), dim3(256), 0, st>>>(A);
+  k_indel_pass<<<dim3(gd), dim3(256), 0, st>>>(A);
+  if (cb > 1) k_cand_sums<<<dim3(cb), dim3(256), 0, st>>>(A, words, L->csums.as<uint32_t>());
+  k_cand_list<<<dim3(cb), dim3(256), 0, st>>>(A, words, L->csums.as<uint32_t>());
+  k_finalize<<<dim3(n_jobs), dim3(64), 0, st>>>(A);
+  k_after<<<dim3((unsigned)(PL_AFTER_BLOCKS + std::min<int32_t>(n_wins, 1024))), dim3(256), 0, st>>>(A);
   HIPCHK(hipGetLastError());
   return PL_OK;
 }
@@ -993,6 +971,7 @@ pl_status run_jobs(pl_ctx* c, Lane* L, const std::vector<JobReq>& reqs, int32_t 
   }
   // ---- capacities (grown and re-run on overflow)
   if (!L->rec_cap) { L->rec_cap = 1u << 18; L->cand_cap = 1u << 16; L->defer_cap = 1u << 16; L->mut_cap = 1u << 16; }
+  if (!L->spill_cap) L->spill_cap = 1u << 14;
   if (!L->wide_cap) L->wide_cap = 1u << 12;
   L->rec_cap = std::max<uint32_t>(L->rec_cap, (uint32_t)std::min<int64_t>(G / 16 + 65536, 1ll << 30));
   L->cand_cap = std::max<uint32_t>(L->cand_cap, (uint32_t)std::min<int64_t>(G / 256 + 16384, 1ll << 30));
@@ -1000,17 +979,20 @@ pl_status run_jobs(pl_ctx* c, Lane* L, const std::vector<JobReq>& reqs, int32_t 
   L->mut_cap = std::max<uint32_t>(L->mut_cap, (uint32_t)std::min<int64_t>(G / 256 + 16384, 1ll << 30));
   HIPCHK(L->jobs.ensure(sizeof(JobDev) * n_jobs));
   HIPCHK(L->wins.ensure(sizeof(WinDev) * n_wins));
-  HIPCHK(L->worder.ensure(4 * (size_t)n_wins));
   HIPCHK(L->winwide.ensure(8 * (size_t)n_wins));
+  HIPCHK(L->winrec.ensure(8 * (size_t)n_wins));
+  HIPCHK(L->wincur.ensure(4 * (size_t)n_wins));
   HIPCHK(L->heads.ensure(sizeof(WinHead) * (size_t)n_wins));
-  HIPCHK(L->costk.ensure(4 * (size_t)n_wins));
-  HIPCHK(L->costv.ensure(4 * (size_t)n_wins));
-  HIPCHK(L->costtk.ensure(4 * (size_t)n_wins));
-  HIPCHK(L->costtv.ensure(4 * (size_t)n_wins));
+  HIPCHK(L->cost.ensure((size_t)n_wins));
+  HIPCHK(L->bins.ensure(8 * PL_COST_BINS));
+  HIPCHK(L->cmask.ensure(8 * (size_t)n_wins * (size_t)(W / 64)));
+  HIPCHK(L->csums.ensure(4 * (((size_t)n_wins * (size_t)(W / 64) + PL_CAND_WORDS - 1) / PL_CAND_WORDS)));
+  HIPCHK(L->prec.ensure(4 * (size_t)G));
+  HIPCHK(L->dhist.ensure(4 * (size_t)PL_HIST * (size_t)n_jobs));
   HIPCHK(L->pile.ensure(4 * (size_t)PL_NFIELDS * G));
   HIPCHK(L->calls.ensure(sizeof(pl_call) * (size_t)G));
   HIPCHK(L->st.ensure(sizeof(JobStat) * n_jobs));
-  HIPCHK(L->counters.ensure(64));
+  HIPCHK(L->counters.ensure(4 * PL_COUNTERS));
   if (!same) {
     HIPCHK(hipMemcpyAsync(L->jobs.p, L->hjobs.data(), sizeof(JobDev) * n_jobs, hipMemcpyHostToDevice, st));
     HIPCHK(hipMemcpyAsync(L->wins.p, L->hwins.data(), sizeof(WinDev) * n_wins, hipMemcpyHostToDevice, st));
@@ -1032,22 +1014,12 @@ pl_status run_jobs(pl_ctx* c, Lane* L, const std::vector<JobReq>& reqs, int32_t 
   }
   for (int attempt = 0; attempt < 6; attempt++) {
     HIPCHK(L->rec.ensure(sizeof(IndelRec) * (size_t)L->rec_cap));
-    HIPCHK(L->rkey.ensure(4 * (size_t)L->rec_cap)); HIPCHK(L->rval.ensure(4 * (size_t)L->rec_cap));
-    HIPCHK(L->rtk.ensure(4 * (size_t)L->rec_cap)); HIPCHK(L->rtv.ensure(4 * (size_t)L->rec_cap));
+    HIPCHK(L->spill.ensure(sizeof(IndelRec) * (size_t)L->spill_cap));
+    HIPCHK(L->spillwin.ensure(4 * (size_t)L->spill_cap));
     HIPCHK(L->cand.ensure(sizeof(Cand) * (size_t)L->cand_cap));
-    HIPCHK(L->cands.ensure(sizeof(Cand) * (size_t)L->cand_cap));
-    HIPCHK(L->ckey.ensure(4 * (size_t)L->cand_cap)); HIPCHK(L->cval.ensure(4 * (size_t)L->cand_cap));
-    HIPCHK(L->ctk.ensure(4 * (size_t)L->cand_cap)); HIPCHK(L->ctv.ensure(4 * (size_t)L->cand_cap));
     HIPCHK(L->defer.ensure(4 * (size_t)L->defer_cap));
     HIPCHK(L->mutated.ensure(4 * (size_t)L->mut_cap));
     HIPCHK(L->wide.ensure(sizeof(WideCol) * (size_t)L->wide_cap));
-    // sort scratch for the largest sort, allocated before any capture
-    {
-      const uint32_t mx = std::max<uint32_t>(std::max<uint32_t>(L->rec_cap, L->cand_cap), (uint32_t)n_wins);
-      const int64_t nb = std::max<int64_t>(1, ((int64_t)mx + RS_TILE - 1) / RS_TILE);
-      HIPCHK(L->hist.ensure(sizeof(uint32_t) * ((size_t)256 * nb + 1)));
-      HIPCHK(L->tiles.ensure(sizeof(uint32_t) * (size_t)std::max<int64_t>(1, (256 * nb + SCAN_TILE - 1) / SCAN_TILE)));
-    }
     uint32_t* cnt = L->counters.as<uint32_t>();
     EngineArgs& A = L->args;
     std::memset(&A, 0, sizeof A);
@@ -1058,20 +1030,27 @@ pl_status run_jobs(pl_ctx* c, Lane* L, const std::vector<JobReq>& reqs, int32_t 
     A.wins = L->wins.as<WinDev>();
     A.n_wins = n_wins;
     A.W = W;
-    A.queue = (int32_t*)(cnt + 5);
-    A.deep = cnt + 7;
-    A.worder = L->worder.as<int32_t>();
+    A.queue = (int32_t*)(cnt + PL_N_QUEUE);
+    A.deep = cnt + PL_N_DEEP;
+    A.cost = L->cost.as<uint8_t>();
+    A.bins = L->bins.as<uint32_t>();
     A.heads = L->heads.as<WinHead>();
     A.pile = L->pile.as<int32_t>();
     A.calls = L->calls.as<pl_call>();
     A.G = G;
     A.st = L->st.as<JobStat>();
-    A.rec = L->rec.as<IndelRec>(); A.rec_n = cnt + 0; A.rec_cap = L->rec_cap;
-    A.cand = L->cand.as<Cand>(); A.cand_n = cnt + 1; A.cand_cap = L->cand_cap;
-    A.defer = L->defer.as<uint32_t>(); A.defer_n = cnt + 2; A.defer_cap = L->defer_cap;
-    A.mutated = L->mutated.as<uint32_t>(); A.mutated_n = cnt + 3; A.mutated_cap = L->mut_cap;
-    A.overflow = (int32_t*)(cnt + 4);
-    A.wide = L->wide.as<WideCol>(); A.wide_n = cnt + 6; A.wide_cap = L->wide_cap;
+    A.hist = L->dhist.as<uint32_t>();
+    A.rec = L->rec.as<IndelRec>(); A.rec_n = cnt + PL_N_REC; A.rec_cap = L->rec_cap;
+    A.win_rec = L->winrec.as<uint32_t>(); A.win_cur = L->wincur.as<uint32_t>();
+    A.spill = L->spill.as<IndelRec>(); A.spill_win = L->spillwin.as<uint32_t>();
+    A.spill_n = cnt + PL_N_SPILL; A.spill_cap = L->spill_cap;
+    A.cmask = L->cmask.as<uint64_t>();
+    A.prec = L->prec.as<int32_t>();
+    A.cand = L->cand.as<Cand>(); A.cand_n = cnt + PL_N_CAND; A.cand_cap = L->cand_cap;
+    A.defer = L->defer.as<uint32_t>(); A.defer_n = cnt + PL_N_DEFER; A.defer_cap = L->defer_cap;
+    A.mutated = L->mutated.as<uint32_t>(); A.mutated_n = cnt + PL_N_MUTATED; A.mutated_cap = L->mut_cap;
+    A.overflow = (int32_t*)(cnt + PL_N_OVERFLOW);
+    A.wide = L->wide.as<WideCol>(); A.wide_n = cnt + PL_N_WIDE; A.wide_cap = L->wide_cap;
     A.win_wide = L->winwide.as<int32_t>();
 
     if (use_graph) {
@@ -1079,8 +1058,7 @@ pl_status run_jobs(pl_ctx* c, Lane* L, const std::vector<JobReq>& reqs, int32_t 
       std::memset(&key, 0, sizeof key);
       key.A = A;
       key.W = W; key.block = block; key.persistent = persistent; key.grid = grid; key.lds = lds;
-      key.bufs[0] = L->hist.p; key.bufs[1] = L->tiles.p; key.bufs[2] = L->rsarr.p; key.bufs[3] = L->kparr.p;
-      key.bufs[4] = L->cands.p; key.bufs[5] = L->costtk.p; key.bufs[6] = L->rtk.p; key.bufs[7] = L->ctk.p;
+      key.bufs[0] = L->csums.p; key.bufs[1] = L->kparr.p;
       if (!L->gexec || L->gkey.size() != sizeof key || std::memcmp(L->gkey.data(), &key, sizeof key) != 0) {
         drop_graph(L);
         HIPCHK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
@@ -1105,9 +1083,8 @@ pl_status run_jobs(pl_ctx* c, Lane* L, const std::vector<JobReq>& reqs, int32_t 
       if (s) return s;
       HIPCHK(hipEventRecord(L->ev[1], st));
     }
-    L->rkey_sorted = A.rkey; L->rval_sorted = A.rval;
-    uint32_t hc[8];
-    HIPCHK(hipMemcpyAsync(hc, cnt, 32, hipMemcpyDeviceToHost, st));
+    uint32_t hc[PL_COUNTERS];
+    HIPCHK(hipMemcpyAsync(hc, cnt, sizeof hc, hipMemcpyDeviceToHost, st));
     HIPCHK(hipStreamSynchronize(st));
     float ms = 0, wms = -1.0f;
     HIPCHK(hipEventElapsedTime(&ms, L->ev[0], L->ev[1]));
@@ -1119,13 +1096,17 @@ pl_status run_jobs(pl_ctx* c, Lane* L, const std::vector<JobReq>& reqs, int32_t 
     L->last_persistent = persistent;
     L->last_block = block;
     bool grow = false;
-    if (hc[0] > L->rec_cap) { L->rec_cap = (uint32_t)std::min<uint64_t>(2ull * hc[0], 1u << 30); grow = true; }
-    if (hc[1] > L->cand_cap) { L->cand_cap = (uint32_t)std::min<uint64_t>(2ull * hc[1], 1u << 30); grow = true; }
-    if (hc[2] > L->defer_cap) { L->defer_cap = (uint32_t)std::min<uint64_t>(2ull * hc[2], 1u << 30); grow = true; }
-    if (hc[3] > L->mut_cap) { L->mut_cap = (uint32_t)std::min<uint64_t>(2ull * hc[3], 1u << 30); grow = true; }
-    if (hc[6] > L->wide_cap) { L->wide_cap = (uint32_t)std::min<uint64_t>(2ull * hc[6], 1u << 30); grow = true; }
+    auto fit = [&](uint32_t n, uint32_t* cap) {
+      if (n > *cap) { *cap = (uint32_t)std::min<uint64_t>(2ull * n, 1u << 30); grow = true; }
+    };
+    fit(hc[PL_N_REC], &L->rec_cap);
+    fit(hc[PL_N_SPILL], &L->spill_cap);
+    fit(hc[PL_N_CAND], &L->cand_cap);
+    fit(hc[PL_N_DEFER], &L->defer_cap);
+    fit(hc[PL_N_MUTATED], &L->mut_cap);
+    fit(hc[PL_N_WIDE], &L->wide_cap);
     if (!grow) {
-      if (hc[4]) return fail(PL_E_DEVICE, "capacity overflow flag set without an overfull counter");
+      if (hc[PL_N_OVERFLOW]) return fail(PL_E_DEVICE, "capacity overflow flag set without an overfull counter");
       return PL_OK;
     }
   }
@@ -1186,22 +1167,14 @@ pl_status fetch_batch_meta(Lane* L) {
   const size_t nj = L->hjobs.size();
   L->hst.resize(nj);
   HIPCHK(hipMemcpyAsync(L->hst.data(), L->st.p, sizeof(JobStat) * nj, hipMemcpyDeviceToHost, L->stream));
-  uint32_t cn = 0;
-  HIPCHK(hipMemcpyAsync(&cn, L->counters.as<uint32_t>() + 1, 4, hipMemcpyDeviceToHost, L->stream));
-  HIPCHK(hipStreamSynchronize(L->stream));
-  cn = std::min(cn, L->cand_cap);
+  // (the batch's counters came back with the run)
+  const uint32_t cn = std::min(L->last_counts[PL_N_CAND], L->cand_cap);
   L->hcand.resize(cn);
-  L->hccall.resize(cn);
   L->hins_off.assign(cn, -1);
   L->hins_pool.clear();
+  if (cn) HIPCHK(hipMemcpyAsync(L->hcand.data(), L->cand.p, sizeof(Cand) * cn, hipMemcpyDeviceToHost, L->stream));
+  HIPCHK(hipStreamSynchronize(L->stream));
   if (cn) {
-    HIPCHK(hipMemcpyAsync(L->hcand.data(), L->cands.p, sizeof(Cand) * cn, hipMemcpyDeviceToHost, L->stream));
-    HIPCHK(L->gath.ensure(sizeof(pl_call) * cn));
-    k_cand_calls<<<dim3((unsigned)std::min<uint32_t>(1024, (cn + 255) / 256)), dim3(256), 0, L->stream>>>(
-        L->cands.as<Cand>(), cn, L->calls.as<pl_call>(), L->gath.as<pl_call>());
-    HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(L->hccall.data(), L->gath.p, sizeof(pl_call) * cn, hipMemcpyDeviceToHost, L->stream));
-    HIPCHK(hipStreamSynchronize(L->stream));
     // insertion strings of every INS candidate, decoded on the device at once
     std::vector<int64_t> idx, off(1, 0);
     for (uint32_t k = 0; k < cn; k++)
@@ -1217,7 +1190,7 @@ pl_status fetch_batch_meta(Lane* L) {
       HIPCHK(hipMemcpyAsync(L->stridx.p, idx.data(), 8 * idx.size(), hipMemcpyHostToDevice, L->stream));
       HIPCHK(hipMemcpyAsync(L->stroff.p, off.data(), 8 * off.size(), hipMemcpyHostToDevice, L->stream));
       k_ins_strings<<<dim3((unsigned)((idx.size() + 63) / 64)), dim3(64), 0, L->stream>>>(
-          L->args, L->cands.as<Cand>(), L->stridx.as<int64_t>(), L->stroff.as<int64_t>(), (int32_t)idx.size(),
+          L->args, L->cand.as<Cand>(), L->stridx.as<int64_t>(), L->stroff.as<int64_t>(), (int32_t)idx.size(),
           L->strpool.as<uint8_t>());
       HIPCHK(hipGetLastError());
       L->hins_pool.resize((size_t)off.back());
@@ -1252,8 +1225,8 @@ pl_status job_changes(pl_ctx* c, Lane* L, size_t j, pl_region_stats* out, std::v
     x.loc = J.start + (int32_t)(cd.gpos - J.out);
     x.kind = cd.kind;
     x.ref = to_upper(ct.host[x.loc - 1]);
-    x.base = L->hccall[k].base;
-    x.alt = L->hccall[k].alt;
+    x.base = cd.base;
+    x.alt = cd.alt;
     if (cd.kind == PL_D_DEL) x.indel.assign((const char*)ct.host.data() + x.loc - 1, (size_t)cd.len);
     if (cd.kind == PL_D_INS) x.indel = L->hins_pool.substr((size_t)L->hins_off[k], (size_t)cd.len);
     ch.push_back(x);
@@ -1709,7 +1682,7 @@ pl_status pl_batch_repeat(pl_ctx* c, int32_t n_passes) {
   constexpr int kSlots = 64;   // passes in flight between two checks
   if (!L->rep_hc) {
     void* p = nullptr;
-    if (hipHostMalloc(&p, sizeof(uint32_t) * 8 * kSlots, hipHostMallocDefault) != hipSuccess) {
+    if (hipHostMalloc(&p, sizeof(uint32_t) * PL_COUNTERS * kSlots, hipHostMallocDefault) != hipSuccess) {
       (void)hipGetLastError();
       return fail(PL_E_OOM, "pinned host allocation failed");
     }
@@ -1722,18 +1695,19 @@ pl_status pl_batch_repeat(pl_ctx* c, int32_t n_passes) {
     HIPCHK(hipEventRecord(L->ev[0], st));
     for (int32_t i = 0; i < m; i++) {
       HIPCHK(hipGraphLaunch(L->gexec, st));
-      HIPCHK(hipMemcpyAsync(L->rep_hc + 8 * i, cnt, 32, hipMemcpyDeviceToHost, st));
+      HIPCHK(hipMemcpyAsync(L->rep_hc + PL_COUNTERS * i, cnt, 4 * PL_COUNTERS, hipMemcpyDeviceToHost, st));
     }
     HIPCHK(hipEventRecord(L->ev[1], st));
     HIPCHK(hipStreamSynchronize(st));
     for (int32_t i = 0; i < m; i++) {
-      const uint32_t* hc = L->rep_hc + 8 * i;
-      if (hc[0] > L->rec_cap || hc[1] > L->cand_cap || hc[2] > L->defer_cap || hc[3] > L->mut_cap ||
-          hc[6] > L->wide_cap || hc[4])
+      const uint32_t* hc = L->rep_hc + PL_COUNTERS * i;
+      if (hc[PL_N_REC] > L->rec_cap || hc[PL_N_SPILL] > L->spill_cap || hc[PL_N_CAND] > L->cand_cap ||
+          hc[PL_N_DEFER] > L->defer_cap || hc[PL_N_MUTATED] > L->mut_cap || hc[PL_N_WIDE] > L->wide_cap ||
+          hc[PL_N_OVERFLOW])
         return fail(PL_E_OOM, "pass %d of the repeated batch overflowed its buffers: run it with pl_batch_run",
                     done + i);
     }
-    std::memcpy(L->last_counts, L->rep_hc + 8 * (m - 1), sizeof L->last_counts);
+    std::memcpy(L->last_counts, L->rep_hc + PL_COUNTERS * (m - 1), sizeof L->last_counts);
     float ms = 0;
     HIPCHK(hipEventElapsedTime(&ms, L->ev[0], L->ev[1]));
     L->last_ms = ms / (float)m;
@@ -1749,9 +1723,9 @@ pl_status pl_last_batch_info(pl_ctx* c, pl_batch_info* o) {
   o->positions = L->G;
   o->n_regions = (int32_t)L->hjobs.size();
   o->n_windows = L->n_wins;
-  o->n_records = L->last_counts[0];
-  o->n_candidates = L->last_counts[1];
-  o->n_deferred = L->last_counts[2];
+  o->n_records = L->last_counts[PL_N_REC];
+  o->n_candidates = L->last_counts[PL_N_CAND];
+  o->n_deferred = L->last_counts[PL_N_DEFER];
   o->window = L->W;
   o->persistent = L->last_persistent;
   o->block = L->last_block;
@@ -1765,7 +1739,7 @@ pl_status pl_last_wide_columns(pl_ctx* c, pl_wide_col* out, int64_t cap, int64_t
   Lane* L = c ? &c->main : nullptr;
   if (!c || !n) return fail(PL_E_INVAL, "null argument");
   if (!L->tables_valid) return fail(PL_E_INVAL, "no batch on the device");
-  const uint32_t nw = std::min(L->last_counts[6], L->wide_cap);
+  const uint32_t nw = std::min(L->last_counts[PL_N_WIDE], L->wide_cap);
   *n = nw;
   if (!out || !nw) return PL_OK;
   if (cap < (int64_t)nw) return fail(PL_E_INVAL, "%u wide columns, room for %lld", nw, (long long)cap);

@@ -3,16 +3,22 @@
 //   k_prep           per read, once per resident read set: alignment end,
 //                    validity/adjMq, touched span, fragment, outliers
 //   k_scan_*         exclusive scans (keep-read prefix, radix histograms)
+//   k_begin          the batch's counters; per region: readCount
+//                    (BamFile.process), P ops, errors
 //   k_plan           per window: the sorted read range it must scan
-//   k_jobprep        per region: readCount (BamFile.process), P ops, errors
+//   k_heads          the windows in cost order, for the work queue
 //   k_window         the hot kernel: one workgroup owns a window of W
 //                    positions, accumulates every counter in LDS, scans
 //                    physCov, and writes counters + BaseCall once
-//   k_rs_*           LSD radix sort (evidence records, change candidates)
+//   k_spill_place    evidence records beyond a window's LDS buffer, put with
+//                    the window's others
 //   k_indel_pass     BaseCall of columns whose indel strings matter
+//   k_cand_*         the change candidates in position order
 //   k_finalize       Pass 1 per region: minDepth, deletion pass
-//   k_recompute      BaseCall of columns changed by the deletion pass
+//   k_after          columns changed by the deletion pass called again;
+//                    exact confirmed counts of very deep regions
 //   k_final_flags    final dispositions for export
+//   k_rs_*           LSD radix sort (the assembler's K-mers)
 //
 // Reference: broadinstitute/pilon v1.24, src/main/scala/org/broadinstitute/pilon/
 #include <hip/hip_runtime.h>
@@ -20,14 +26,6 @@
 #include "pl_kernels.h"
 
 namespace {
-
-__device__ __forceinline__ int64_t lower_pos_dev(const int32_t* pos, int64_t lo, int64_t hi, int64_t x) {
-  while (lo < hi) {
-    int64_t m = (lo + hi) >> 1;
-    if ((int64_t)pos[m] < x) lo = m + 1; else hi = m;
-  }
-  return lo;
-}
 
 __device__ __forceinline__ uint64_t lanemask_lt() {
   const int lane = threadIdx.x & 63;
@@ -316,54 +314,90 @@ __global__ void __launch_bounds__(256) k_scan_apply(const uint32_t* in, int64_t 
 }
 
 // ------------------------------------------------------------------ plan
-__global__ void k_plan(const RSDev* rsets, const JobDev* jobs, WinDev* wins, int32_t n_wins, uint32_t* cost) {
-  const int32_t w = blockIdx.x * blockDim.x + threadIdx.x;
-  if (w >= n_wins) return;
-  WinDev& win = wins[w];
-  const JobDev& J = jobs[win.job];
-  const RSDev& R = rsets[J.rs];
-  const int64_t L0 = (int64_t)J.start + win.p0, L1 = (int64_t)J.start + win.p1;
-  const int32_t back = R.scal[0], lead = R.scal[1];
-  win.lo = lower_pos_dev(R.pos, 0, R.n, L0 - back);
-  win.hi = lower_pos_dev(R.pos, win.lo, R.n, L1 + lead);
-  win.plo = fragment_only_end(R.pos, win.lo, win.hi, J, L0, back, R.scal[6]);
-  // descending-cost order key for the work queue (largest windows first):
-  // 16 bits, so the sort takes two passes; windows beyond 65,535 cost units
-  // share the front of the queue
-  const int64_t c = (win.hi - win.plo) + (win.plo - win.lo) / 8 + (int64_t)(win.p1 - win.p0) / 16;
-  cost[w] = 0xffffu - (uint32_t)(c > 0xffffll ? 0xffffll : c);
+namespace {
+
+// first index in pos[lo, hi) whose position is >= x, by an aligned group of
+// GL lanes (all 64 lanes of the wave active): GL probes a round cut the
+// range GL+1-fold, so 16 lanes take 5 dependent loads for a million reads
+// where one lane takes 20.
+template <int GL>
+__device__ __forceinline__ int64_t group_lower_pos(const int32_t* pos, int64_t lo, int64_t hi, int64_t x) {
+  const int lane = threadIdx.x & 63, gl = lane & (GL - 1), g0 = lane & ~(GL - 1);
+  const uint64_t gm = GL == 64 ? ~0ull : (1ull << (GL & 63)) - 1ull;
+  while (__ballot(hi - lo > GL)) {
+    const int64_t m = hi - lo;
+    const bool more = m > GL;
+    const bool less = more && (int64_t)pos[lo + (gl + 1) * m / (GL + 1)] < x;
+    const int k = __popcll((__ballot(less) >> g0) & gm);      // probes ascend: a prefix of the group
+    if (more) {
+      const int64_t a = lo;
+      if (k > 0) lo = a + k * m / (GL + 1) + 1;
+      if (k < GL) hi = a + (k + 1) * m / (GL + 1);
+    }
+  }
+  const bool less = lo + gl < hi && (int64_t)pos[lo + gl] < x;
+  return lo + __popcll((__ballot(less) >> g0) & gm);
 }
 
-// the window heads in processing order (worder null: window order)
-__global__ void k_win_heads(const JobDev* jobs, const WinDev* wins, const int32_t* worder, int32_t n_wins,
-                            WinHead* heads) {
-  const int32_t q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= n_wins) return;
-  const int32_t wi = worder ? worder[q] : q;
-  const WinDev w = wins[wi];
-  const JobDev& J = jobs[w.job];
+// cost bin of a window: 0 for the most work, four mantissa bits above 16
+// units (windows of one bin differ by at most 6%, what the queue's order is for)
+__device__ __forceinline__ uint32_t cost_bin(int64_t c) {
+  const uint32_t v = (uint32_t)(c > 0xffffll ? 0xffffll : c);
+  const uint32_t lg = 31u - (uint32_t)__clz((int)(v | 1u));
+  const uint32_t b = v < 16u ? v : (lg - 3u) * 16u + ((v >> (lg - 4u)) & 15u);
+  return PL_COST_BINS - 1u - b;
+}
+
+__device__ __forceinline__ void put_head(WinHead* heads, int32_t slot, int32_t wi, const WinDev& w, const JobDev& J) {
   WinHead h;
   h.wi = wi; h.job = w.job; h.p0 = w.p0; h.p1 = w.p1;
   h.lo = w.lo; h.hi = w.hi; h.plo = w.plo; h.out = J.out;
   h.rs = J.rs; h.start = J.start; h.stop = J.stop; h.qs = J.qs; h.qe = J.qe;
   h.pad[0] = h.pad[1] = h.pad[2] = 0;
-  heads[q] = h;
+  heads[slot] = h;
 }
 
-// ------------------------------------------------------------------ jobprep
+// The read ranges of 16 windows, one per group of 16 lanes of a 256-thread
+// block; returns this lane's window's cost bin (-1: past the last window).
+// Windows are few and short, so the three searches are all latency: a lane
+// per window took 27 us for 47,000 windows and 14 us for 400.
+__device__ int plan_windows(const EngineArgs& A, int32_t blk, WinDev* wins, bool heads) {
+  const int32_t w0 = blk * 16 + (int32_t)(threadIdx.x >> 4);
+  const bool in = w0 < A.n_wins;
+  const int32_t w = in ? w0 : A.n_wins - 1;                 // idle groups repeat the last window
+  WinDev win = wins[w];
+  const JobDev& J = A.jobs[win.job];
+  const RSDev& R = A.rs[J.rs];
+  const int64_t L0 = (int64_t)J.start + win.p0, L1 = (int64_t)J.start + win.p1;
+  const int32_t back = R.scal[0], lead = R.scal[1], fp = R.scal[6];
+  win.lo = group_lower_pos<16>(R.pos, 0, R.n, L0 - back);
+  win.hi = group_lower_pos<16>(R.pos, win.lo, R.n, L1 + lead);
+  // the end of the fragment-only reads: fragment_only_end with the group's search
+  const bool all = fragment_all(J, (int32_t)L0, back, fp);
+  const int64_t plo = group_lower_pos<16>(R.pos, win.lo, win.hi, L0 - fp);
+  win.plo = all ? win.lo : plo;
+  const int bin = (int)cost_bin((win.hi - win.plo) + (win.plo - win.lo) / 8 + (int64_t)(win.p1 - win.p0) / 16);
+  if (in && (threadIdx.x & 15) == 0) {
+    wins[w] = win;
+    A.cost[w] = (uint8_t)bin;
+    if (heads) put_head((WinHead*)A.heads, w, w, win, J);
+  }
+  return in ? bin : -1;
+}
+
 // readCount of BamFile.process (BamFile.scala:118-139): kept reads whose span
-// overlaps [qs, qe], from the keep-prefix plus the reads straddling qs.
-__global__ void __launch_bounds__(64) k_jobprep(const RSDev* rsets, const uint32_t* const* keep_prefix,
-                                                const JobDev* jobs, JobStat* st) {
-  const JobDev& J = jobs[blockIdx.x];
-  const RSDev& R = rsets[J.rs];
+// overlaps [qs, qe], from the keep-prefix plus the reads straddling qs.  One
+// wave per region, which also clears the region's counters.
+__device__ void job_begin(const EngineArgs& A, const uint32_t* const* keep_prefix, int32_t j) {
+  const JobDev& J = A.jobs[j];
+  const RSDev& R = A.rs[J.rs];
   const uint32_t* kp = keep_prefix[J.rs];
-  JobStat& S = st[blockIdx.x];
-  const int lane = threadIdx.x;
-  const int64_t a = lower_pos_dev(R.pos, 0, R.n, J.qs);
-  const int64_t b = lower_pos_dev(R.pos, a, R.n, (int64_t)J.qe + 1);
-  const int64_t a1 = lower_pos_dev(R.pos, a, b, (int64_t)J.qs + 1);
-  const int64_t a2 = lower_pos_dev(R.pos, 0, a, (int64_t)J.qs - R.scal[2]);
+  const int lane = threadIdx.x & 63;
+  for (int d = lane; d < PL_HIST; d += 64) A.hist[(int64_t)j * PL_HIST + d] = 0;
+  const int64_t a = group_lower_pos<64>(R.pos, 0, R.n, J.qs);
+  const int64_t b = group_lower_pos<64>(R.pos, a, R.n, (int64_t)J.qe + 1);
+  const int64_t a1 = group_lower_pos<64>(R.pos, a, b, (int64_t)J.qs + 1);
+  const int64_t a2 = group_lower_pos<64>(R.pos, 0, a, (int64_t)J.qs - R.scal[2]);
   int64_t adj = 0;
   // reads at pos == qs whose span ends before it (no reference-consuming op)
   for (int64_t r = a + lane; r < a1; r += 64) {
@@ -397,29 +431,79 @@ __global__ void __launch_bounds__(64) k_jobprep(const RSDev* rsets, const uint32
     }
   }
   if (lane == 0) {
+    JobStat S;
     S.read_count = (int64_t)kp[b] - (int64_t)kp[a] + adj;
+    S.base_count = 0;
+    S.aligned = 0;
     S.unknown_ops = unk;
-    if (bad_r != INT64_MAX) atomicMin((unsigned long long*)&S.err_read_inval, (unsigned long long)bad_r);
-    if (edge_r != INT64_MAX) atomicMin((unsigned long long*)&S.err_read_edge, (unsigned long long)edge_r);
+    S.err_read_edge = edge_r;
+    S.err_read_inval = bad_r;
+    S.overflow = S.min_depth = S.n_confirmed = S.cand_lo = S.cand_hi = S.pad = 0;
+    A.st[j] = S;
   }
 }
 
-__global__ void k_init_stats(JobStat* st, int32_t n_jobs, uint32_t* counters, int n_counters) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n_counters) counters[i] = 0;
-  const int64_t words = (int64_t)n_jobs * (sizeof(JobStat) / 4);
-  for (int64_t k = i; k < words; k += (int64_t)gridDim.x * blockDim.x) ((uint32_t*)st)[k] = 0;
+}  // namespace
+
+// Block 0 clears the batch's counters, the next blocks take four regions
+// each (job_begin).  With plan set (windows taken in their own order, so no
+// cost order is needed) the blocks after them plan the windows and write
+// their heads: the whole preparation of a plain launch is this kernel.
+__global__ void __launch_bounds__(256) k_begin(EngineArgs A, const uint32_t* const* keep_prefix, uint32_t* counters,
+                                               int n_counters, WinDev* wins, int plan) {
+  const int32_t jb = (A.n_jobs + 3) / 4;
+  int32_t b = (int32_t)blockIdx.x;
+  if (b == 0) {
+    if ((int)threadIdx.x < n_counters) counters[threadIdx.x] = 0;
+    if (!plan) for (int k = threadIdx.x; k < 2 * PL_COST_BINS; k += 256) A.bins[k] = 0;
+    return;
+  }
+  b -= 1;
+  if (b < jb) {
+    const int32_t j = b * 4 + (int32_t)(threadIdx.x >> 6);
+    if (j < A.n_jobs) job_begin(A, keep_prefix, j);
+    return;
+  }
+  if (plan) plan_windows(A, b - jb, wins, true);
 }
-// identity permutation + its length, for the window cost sort (a kernel,
-// not a host copy, so the whole batch pipeline can be captured in a graph)
+
+// the windows' read ranges and cost bins (persistent form)
+__global__ void __launch_bounds__(256) k_plan(EngineArgs A, WinDev* wins) {
+  const int bin = plan_windows(A, blockIdx.x, wins, false);
+  if (bin >= 0 && (threadIdx.x & 15) == 0) atomicAdd(&A.bins[bin], 1u);
+}
+
+// The window heads in cost order, most work first: a window's queue slot is
+// its bin's first slot, plus the slots its bin has handed out (one atomic per
+// bin and block), plus its rank in its block.  The order inside a bin is of
+// no consequence.  (A radix sort of exact keys took ten launches.)
+__global__ void __launch_bounds__(256) k_heads(EngineArgs A) {
+  static_assert(PL_COST_BINS == 256, "one bin per thread");
+  __shared__ uint32_t start[PL_COST_BINS], cnt[PL_COST_BINS];
+  __shared__ uint32_t ws[4];
+  const int tid = threadIdx.x;
+  const uint32_t v = A.bins[tid];
+  const uint32_t inc = wave_scan_dpp(v);
+  if ((tid & 63) == 63) ws[tid >> 6] = inc;
+  cnt[tid] = 0;
+  __syncthreads();
+  uint32_t s = inc - v;
+  for (int w = 0; w < (tid >> 6); w++) s += ws[w];
+  start[tid] = s;
+  const int32_t w = (int32_t)blockIdx.x * 256 + tid;
+  uint32_t bin = 0, rank = 0;
+  if (w < A.n_wins) { bin = A.cost[w]; rank = atomicAdd(&cnt[bin], 1u); }
+  __syncthreads();
+  if (cnt[tid]) start[tid] += atomicAdd(&A.bins[PL_COST_BINS + tid], cnt[tid]);
+  __syncthreads();
+  if (w < A.n_wins) put_head((WinHead*)A.heads, (int32_t)(start[bin] + rank), w, A.wins[w], A.jobs[A.wins[w].job]);
+}
+
+// identity permutation + its length, for a sort whose count is in device memory
 __global__ void k_iota(uint32_t* v, int32_t n, uint32_t* n_out) {
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
     v[i] = (uint32_t)i;
   if (blockIdx.x == 0 && threadIdx.x == 0) *n_out = (uint32_t)n;
-}
-__global__ void k_init_stats2(JobStat* st, int32_t n_jobs) {
-  const int32_t j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j < n_jobs) { st[j].err_read_edge = INT64_MAX; st[j].err_read_inval = INT64_MAX; }
 }
 
 // ------------------------------------------------------------------ window
@@ -430,9 +514,11 @@ struct LdsSink {
   unsigned long long *bs, *mqq, *ins_, *del_;
   uint32_t *bad_, *clp_;
   int32_t *pc, *is;
-  IndelRec* rec;
-  uint32_t* rec_n;
-  uint32_t rec_cap;
+  IndelRec* spill;
+  uint32_t* spill_win;
+  uint32_t* spill_n;
+  uint32_t spill_cap;
+  int32_t wi;
   IndelRec* lrec;        // the window's record buffer in LDS (PL_WIN_RECS)
   uint32_t* lrec_n;
   int32_t* overflow;
@@ -447,13 +533,13 @@ struct LdsSink {
   __device__ void count_base() { bcount++; }
   __device__ void bad(int p, int n) { atomicAdd(&bad_[p], (uint32_t)n); }
   __device__ void clip(int p) { atomicAdd(&clp_[p], 1u); }
-  // records collect in LDS and reach HBM with one atomic per window; a
-  // window with more than PL_WIN_RECS writes the rest directly
+  // records collect in LDS and reach HBM together at the window's end; a
+  // window with more than PL_WIN_RECS spills the rest (k_spill_place)
   __device__ void emit(const IndelRec& e) {
     const uint32_t j = atomicAdd(lrec_n, 1u);
     if (j < PL_WIN_RECS) { lrec[j] = e; return; }
-    uint32_t i = atomicAdd(rec_n, 1u);
-    if (i < rec_cap) rec[i] = e;
+    const uint32_t i = atomicAdd(spill_n, 1u);
+    if (i < spill_cap) { spill[i] = e; spill_win[i] = (uint32_t)wi; }
     else *overflow = 1;
   }
   __device__ void ins(int p, int32_t q, int32_t mq1, const IndelRec& e) {
@@ -515,7 +601,7 @@ __global__ void __launch_bounds__(BLOCK, PL_WIN_WAVES_EU) k_window(EngineArgs A,
   int32_t* pcA = (int32_t*)(clpA + W);
   int32_t* isA = pcA + W;
   int32_t* bdA = isA + W;   // badPair differences of bad runs (clips, invalid reads' M bases)
-  uint32_t* hist = (uint32_t*)(bdA + W);
+  uint32_t* hist = (uint32_t*)(bdA + W);   // PL_HIST entries
   __shared__ RunL s_run[NW * (2 * 64 + 1)];
   __shared__ int32_t s_w;
   __shared__ int32_t ws_a[NW], ws_b[NW], ws_c[NW];
@@ -574,7 +660,8 @@ __global__ void __launch_bounds__(BLOCK, PL_WIN_WAVES_EU) k_window(EngineArgs A,
 
     LdsSink sk;
     sk.W = W; sk.bs = bs; sk.mqq = mqq; sk.ins_ = insA; sk.del_ = delA; sk.bad_ = badA; sk.clp_ = clpA;
-    sk.pc = pcA; sk.is = isA; sk.rec = A.rec; sk.rec_n = A.rec_n; sk.rec_cap = A.rec_cap;
+    sk.pc = pcA; sk.is = isA; sk.spill = A.spill; sk.spill_win = A.spill_win; sk.spill_n = A.spill_n;
+    sk.spill_cap = A.spill_cap; sk.wi = wi;
     sk.lrec = s_rec; sk.lrec_n = &s_nrec;
     sk.overflow = A.overflow; sk.st = &A.st[win.job]; sk.bcount = 0; sk.aligned_n = 0;
 
@@ -873,43 +960,56 @@ __global__ void __launch_bounds__(BLOCK, PL_WIN_WAVES_EU) k_window(EngineArgs A,
     }
     __syncthreads();
 
-    // the window's evidence records: one atomic, coalesced 32-byte stores
+    // the window's evidence records, in one segment of the batch's: one
+    // atomic, coalesced 32-byte stores (room for the spilled ones at its end)
     {
-      const uint32_t nl = s_nrec < PL_WIN_RECS ? s_nrec : PL_WIN_RECS;
-      if (tid == 0 && nl) s_recbase = atomicAdd(A.rec_n, nl);
+      const uint32_t nt = s_nrec, nl = nt < PL_WIN_RECS ? nt : PL_WIN_RECS;
+      if (tid == 0) {
+        const uint32_t base = nt ? atomicAdd(A.rec_n, nt) : 0u;
+        s_recbase = base;
+        A.win_rec[2 * wi] = base;
+        A.win_rec[2 * wi + 1] = nt;
+        A.win_cur[wi] = 0;
+        if (nt && base + nt > A.rec_cap) *A.overflow = 1;
+      }
       __syncthreads();
       for (uint32_t t = tid; t < nl; t += BLOCK) {
         const uint32_t k = s_recbase + t;
         if (k < A.rec_cap) A.rec[k] = s_rec[t];
-        else *A.overflow = 1;
       }
     }
     const int64_t G = A.G;
     uint32_t wmask = 0;   // bit i: position tid + i*BLOCK is wide
-    for (int p = tid, it = 0; p < nW; p += BLOCK, it++) {
-      const uint64_t b4[4] = {bs[p], bs[W + p], bs[2 * W + p], bs[3 * W + p]};
-      PosOut o;
-      finalize_position(b4, mqq[p], insA[p], delA[p], badA[p], clpA[p], pcA[p], isA[p], R.ref[L0 + p - 1], cf, o);
-      const int64_t g = J.out + win.p0 + p;
+    for (int q0 = 64 * wave, it = 0; q0 < W; q0 += BLOCK, it++) {
+      const int p = q0 + lane;
+      const bool act = p < nW;
+      bool is_cand = false, defer = false;
+      if (act) {
+        const uint64_t b4[4] = {bs[p], bs[W + p], bs[2 * W + p], bs[3 * W + p]};
+        PosOut o;
+        finalize_position(b4, mqq[p], insA[p], delA[p], badA[p], clpA[p], pcA[p], isA[p], R.ref[L0 + p - 1], cf, o);
+        const int64_t g = J.out + win.p0 + p;
 #pragma unroll
-      for (int f = 0; f < PL_NFIELDS; f++) A.pile[(int64_t)f * G + g] = o.f[f];
-      if (o.wide) { o.call.flags |= PL_CF_WIDE; wmask |= 1u << it; }
-      A.calls[g] = o.call;
-      if (o.overflow) s_ovf = 1;
-      const int d = call_disp(o.call);
-      const int64_t dep = (int64_t)(uint32_t)o.f[0] + (uint32_t)o.f[1] + (uint32_t)o.f[2] + (uint32_t)o.f[3] +
-                          o.f[PL_F_DELETIONS];
-      const bool is_cand = !o.defer && (d == PL_D_SNP || d == PL_D_AMB);
-      if (!o.defer && d == PL_D_CONFIRMED) atomicAdd(&hist[dep > 255 ? 255 : (dep < 0 ? 0 : dep)], 1u);
-      // one global atomic per wave for each list
-      const uint32_t kd = wave_append(A.defer_n, o.defer);
-      const uint32_t kc = wave_append(A.cand_n, is_cand);
-      if (o.defer) {
-        if (kd < A.defer_cap) A.defer[kd] = (uint32_t)g;
-        else *A.overflow = 1;
+        for (int f = 0; f < PL_NFIELDS; f++) A.pile[(int64_t)f * G + g] = o.f[f];
+        if (o.wide) { o.call.flags |= PL_CF_WIDE; wmask |= 1u << it; }
+        A.calls[g] = o.call;
+        if (o.overflow) s_ovf = 1;
+        const int d = call_disp(o.call);
+        defer = o.defer;
+        is_cand = !o.defer && (d == PL_D_SNP || d == PL_D_AMB);
+        if (!o.defer && d == PL_D_CONFIRMED) {
+          const int64_t dep = (int64_t)(uint32_t)o.f[0] + (uint32_t)o.f[1] + (uint32_t)o.f[2] + (uint32_t)o.f[3] +
+                              o.f[PL_F_DELETIONS];
+          atomicAdd(&hist[dep > 255 ? 255 : (dep < 0 ? 0 : dep)], 1u);
+        }
       }
-      if (is_cand) {
-        if (kc < A.cand_cap) { Cand c; c.gpos = (uint32_t)g; c.depth = (int32_t)dep; c.kind = d; c.len = 0; c.rec = -1; A.cand[kc] = c; }
+      // the candidates as a bit per position, in order without a sort; the
+      // deferred columns as a list (their order is of no consequence)
+      const uint64_t cm = __ballot(is_cand);
+      if (lane == 0) A.cmask[(int64_t)wi * (W >> 6) + (q0 >> 6)] = cm;
+      const uint32_t kd = wave_append(A.defer_n, defer);
+      if (defer) {
+        if (kd < A.defer_cap) A.defer[kd] = (uint32_t)(J.out + win.p0 + p);
         else *A.overflow = 1;
       }
     }
@@ -958,8 +1058,8 @@ __global__ void __launch_bounds__(BLOCK, PL_WIN_WAVES_EU) k_window(EngineArgs A,
       if (t1s) atomicAdd((unsigned long long*)&S.aligned, t1s);
       if (s_ovf) atomicOr(&S.overflow, 1);
     }
-    for (int d = tid; d < 256; d += BLOCK)
-      if (hist[d]) atomicAdd((uint32_t*)&S.hist[d], hist[d]);
+    for (int d = tid; d < PL_HIST; d += BLOCK)
+      if (hist[d]) atomicAdd(&A.hist[(int64_t)win.job * PL_HIST + d], hist[d]);
     __syncthreads();
   }
 }
@@ -969,23 +1069,15 @@ template __global__ void k_window<512>(EngineArgs, int);
 template __global__ void k_window<1024>(EngineArgs, int);
 
 // ------------------------------------------------------------------ records
-__global__ void k_rec_keys(const IndelRec* rec, const uint32_t* rec_n, uint32_t cap, uint32_t* key, uint32_t* val) {
-  const uint32_t n = *rec_n < cap ? *rec_n : cap;
+// Spilled records into their windows' segments: behind the ones the window
+// kept in LDS, in any order (a column's records are counted, never ordered).
+__global__ void __launch_bounds__(256) k_spill_place(EngineArgs A) {
+  const uint32_t n = *A.spill_n < A.spill_cap ? *A.spill_n : A.spill_cap;
   for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-    key[i] = rec[i].key;
-    val[i] = i;
+    const uint32_t w = A.spill_win[i];
+    const uint32_t k = A.win_rec[2 * w] + PL_WIN_RECS + atomicAdd(&A.win_cur[w], 1u);
+    if (k < A.rec_cap) A.rec[k] = A.spill[i];
   }
-}
-__global__ void k_cand_keys(const Cand* c, const uint32_t* cand_n, uint32_t cap, uint32_t* key, uint32_t* val) {
-  const uint32_t n = *cand_n < cap ? *cand_n : cap;
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-    key[i] = c[i].gpos;
-    val[i] = i;
-  }
-}
-__global__ void k_cand_gather(const Cand* in, const uint32_t* cand_n, uint32_t cap, const uint32_t* val, Cand* out) {
-  const uint32_t n = *cand_n < cap ? *cand_n : cap;
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) out[i] = in[val[i]];
 }
 
 // ------------------------------------------------------------------ radix sort
@@ -1058,48 +1150,59 @@ __device__ __forceinline__ int32_t job_of(const JobDev* jobs, int32_t n_jobs, in
 
 namespace {
 
-// first index in keys[0, n) whose key is >= x, by the whole wave: 64 probes
-// per round cut the range 65-fold (4 dependent loads for a million keys)
-__device__ int64_t wave_lower_bound(const uint32_t* keys, int64_t n, uint32_t x, int lane) {
-  int64_t lo = 0, hi = n;
-  while (hi - lo > 64) {
-    const int64_t m = hi - lo;
-    const int64_t probe = lo + ((int64_t)(lane + 1) * m) / 65;
-    const int k = __popcll(__ballot(keys[probe] < x));   // probes ascend: a prefix of lanes
-    const int64_t plo = lo + ((int64_t)k * m) / 65;       // probe of lane k-1 (lo when k = 0)
-    const int64_t phi = lo + ((int64_t)(k + 1) * m) / 65; // probe of lane k (hi when k = 64)
-    if (k > 0) lo = plo + 1;
-    hi = k < 64 ? phi : hi;
+// a column's records among its window's
+struct ColRecs {
+  const IndelRec* recs;
+  int64_t a, b;              // the window's segment
+  uint32_t key;              // (gpos << 1) | kind
+};
+
+// the strict majority of a column's records by one lane in record order:
+// the exact form group_majority, over the records of one key
+__device__ Majority col_majority_serial(const RSDev& R, const ColRecs& C) {
+  Majority m;
+  m.n = m.win = 0;
+  m.rec = -1;
+  int32_t cnt = 0;
+  for (int64_t i = C.a; i < C.b; i++) {
+    if (C.recs[i].key != C.key) continue;
+    m.n++;
+    if (cnt == 0) { m.rec = i; cnt = 1; }
+    else if (rec_same(R, C.recs[i], C.recs[m.rec])) cnt++;
+    else cnt--;
   }
-  const int64_t i = lo + lane;
-  return lo + __popcll(__ballot(i < hi && keys[i] < x));
+  for (int64_t i = C.a; i < C.b; i++)
+    if (C.recs[i].key == C.key && rec_same(R, C.recs[i], C.recs[m.rec])) m.win++;
+  return m;
 }
 
-// strict majority over one (position, kind) group of sorted records, by the
-// whole wave.  Each lane runs a Boyer-Moore vote over its strided share of
-// the records, comparing (length, hash) classes; the 64 partial votes are
-// merged pairwise (a merge keeps a majority class if there is one), and the
-// winning class's string is counted exactly.  A class with a strict
-// majority whose representative string falls short (a hash collision) is
-// resolved by the serial scan.  Same result as group_majority.
-__device__ Majority wave_majority(const RSDev& R, const IndelRec* recs, const uint32_t* idx, int64_t a, int64_t b,
-                                  int lane) {
+// The strict majority over a column's records, by the whole wave.  The
+// window's records are not sorted: a window holds a handful, and the wave
+// tests 64 keys at a time, which costs less than sorting every record of
+// the batch did (four radix passes, 20 launches).  Each lane runs a
+// Boyer-Moore vote over the matching records of its strided share,
+// comparing (length, hash) classes; the 64 partial votes are merged pairwise
+// (a merge keeps a majority class if there is one), and the winning class's
+// string is counted exactly.  A class with a strict majority whose
+// representative string falls short (a hash collision) is resolved by the
+// serial scan.  Same result as group_majority.
+__device__ Majority wave_majority(const RSDev& R, const ColRecs& C, int lane) {
   Majority m;
-  m.n = (int32_t)(b - a);
-  m.win = 0;
+  m.n = m.win = 0;
   m.rec = -1;
-  if (b <= a) return m;
-  int32_t vl = -1, vc = 0;
+  int32_t vl = -1, vc = 0, n = 0;
   uint32_t vh = 0;
   int64_t vr = -1;
-  for (int64_t i = a + lane; i < b; i += 64) {
-    const int64_t r = idx[i];
-    const int32_t len = recs[r].len;
-    const uint32_t h = recs[r].hash;
-    if (vc == 0) { vl = len; vh = h; vr = r; vc = 1; }
-    else if (len == vl && h == vh) vc++;
+  for (int64_t i = C.a + lane; i < C.b; i += 64) {
+    const IndelRec& e = C.recs[i];
+    if (e.key != C.key) continue;
+    n++;
+    if (vc == 0) { vl = e.len; vh = e.hash; vr = i; vc = 1; }
+    else if (e.len == vl && e.hash == vh) vc++;
     else vc--;
   }
+  m.n = wave_sum(n);
+  if (m.n == 0) return m;
   for (int d = 1; d < 64; d <<= 1) {
     const int32_t ol = __shfl_xor(vl, d, 64), oc = __shfl_xor(vc, d, 64);
     const uint32_t oh = (uint32_t)__shfl_xor((int)vh, d, 64);
@@ -1110,11 +1213,11 @@ __device__ Majority wave_majority(const RSDev& R, const IndelRec* recs, const ui
   }
   const int64_t cr = __shfl((long long)vr, 0, 64);
   if (cr < 0) return m;
-  const IndelRec c = recs[cr];
+  const IndelRec c = C.recs[cr];
   int32_t cls = 0, same = 0;
-  for (int64_t i = a + lane; i < b; i += 64) {
-    const IndelRec& e = recs[idx[i]];
-    if (e.len == c.len && e.hash == c.hash) {
+  for (int64_t i = C.a + lane; i < C.b; i += 64) {
+    const IndelRec& e = C.recs[i];
+    if (e.key == C.key && e.len == c.len && e.hash == c.hash) {
       cls++;
       if (rec_same(R, e, c)) same++;
     }
@@ -1122,13 +1225,13 @@ __device__ Majority wave_majority(const RSDev& R, const IndelRec* recs, const ui
   cls = wave_sum(cls);
   same = wave_sum(same);
   if (2 * same > m.n) { m.win = same; m.rec = cr; return m; }
-  if (2 * cls > m.n) return group_majority(R, recs, idx, a, b);   // collision inside the majority class
+  if (2 * cls > m.n) return col_majority_serial(R, C);             // collision inside the majority class
   m.win = same;                                                     // no strict majority
   return m;
 }
 
 // the region (job) holding batch position g: the last job whose first
-// position is <= g, by the whole wave as in wave_lower_bound
+// position is <= g, by the whole wave: 64 probes a round
 __device__ int32_t wave_job_of(const JobDev* jobs, int32_t n_jobs, int64_t g, int lane) {
   int32_t lo = 0, hi = n_jobs;                          // first job with out > g lies in [lo, hi]
   while (hi - lo > 64) {
@@ -1148,19 +1251,18 @@ __device__ int32_t wave_job_of(const JobDev* jobs, int32_t n_jobs, int64_t g, in
 
 // One wave per listed column: the full BaseCall with the column's evidence
 // records (hetIndelCall), lane 0 writing the results.
-// mode 0: deferred columns (writes call, appends candidates, counts confirmed)
+// mode 0: deferred columns (writes call, marks candidates, counts confirmed)
 // mode 1: columns changed by the deletion pass (keeps disposition bits)
-__global__ void __launch_bounds__(256) k_indel_pass(EngineArgs A, const uint32_t* list, const uint32_t* list_n,
-                                                     uint32_t cap, int mode) {
-  const uint32_t n = *list_n < cap ? *list_n : cap;
-  const uint32_t nrec = *A.rec_n < A.rec_cap ? *A.rec_n : A.rec_cap;
+// Both leave the column's winning record in A.prec.
+__device__ void indel_columns(const EngineArgs& A, const uint32_t* list, uint32_t n, int mode, uint32_t first,
+                              uint32_t nw) {
   const int lane = threadIdx.x & 63;
-  const uint32_t nw = (gridDim.x * blockDim.x) >> 6;
-  for (uint32_t i = (blockIdx.x * blockDim.x + threadIdx.x) >> 6; i < n; i += nw) {
+  for (uint32_t i = first; i < n; i += nw) {
     const uint32_t g = list[i];
     const int32_t j = wave_job_of(A.jobs, A.n_jobs, g, lane);
     const JobDev& J = A.jobs[j];
     const RSDev& R = A.rs[J.rs];
+    const int32_t w = J.win0 + (int32_t)((g - J.out) / A.W);
     Col c = load_col(A.pile, A.G, g);
     const uint16_t wflag = A.calls[g].flags & PL_CF_WIDE;
     if (wflag) wide_patch(c, A.wide, A.wide_cap, A.win_wide, J, A.W, g);
@@ -1170,43 +1272,128 @@ __global__ void __launch_bounds__(256) k_indel_pass(EngineArgs A, const uint32_t
     const int need = indel_kind_needed(c, A.cf, &pct);
     int indel = 0;
     bool homo = true;
-    int32_t ilen = 0;
     int64_t wrec = -1;
     if (need) {
-      const uint32_t key = (g << 1) | (uint32_t)(need - 1);
-      const int64_t a = wave_lower_bound(A.rkey, nrec, key, lane);
-      int64_t b = a;
-      for (;;) {
-        const int64_t t = b + lane;
-        const int cnt = __popcll(__ballot(t < (int64_t)nrec && A.rkey[t] == key));
-        b += cnt;
-        if (cnt < 64) break;
-      }
-      const Majority mj = wave_majority(R, A.rec, A.rval, a, b, lane);
+      ColRecs C;
+      C.recs = A.rec;
+      C.key = (g << 1) | (uint32_t)(need - 1);
+      C.a = A.win_rec[2 * w];
+      C.b = C.a + A.win_rec[2 * w + 1];
+      if (C.b > (int64_t)A.rec_cap) C.b = A.rec_cap;              // an overfull buffer: the batch runs again
+      const Majority mj = wave_majority(R, C, lane);
       if (mj.rec >= 0) {
         const IndelRec& e = A.rec[mj.rec];
         const int d = het_indel_decide(mj.n, mj.win, e.len, (e.flags & 2u) != 0, pct, A.cf);
-        if (d) { indel = need; homo = d == 2; ilen = e.len; wrec = mj.rec; }
+        if (d) { indel = need; homo = d == 2; wrec = mj.rec; }
       }
     }
     if (lane != 0) continue;
     pl_call cl = make_call(bf, indel, homo, refb, A.cf);
     cl.flags |= wflag;
+    A.prec[g] = (int32_t)wrec;
     if (mode == 0) {
       A.calls[g] = cl;
       const int d = call_disp(cl);
       const int64_t dep = c.depth();
-      if (d == PL_D_CONFIRMED) atomicAdd((uint32_t*)&A.st[j].hist[dep > 255 ? 255 : (dep < 0 ? 0 : dep)], 1u);
+      if (d == PL_D_CONFIRMED) atomicAdd(&A.hist[(int64_t)j * PL_HIST + (dep > 255 ? 255 : (dep < 0 ? 0 : dep))], 1u);
       else if (d != PL_D_NONE) {
-        uint32_t k = atomicAdd(A.cand_n, 1u);
-        if (k < A.cand_cap) { Cand cd; cd.gpos = g; cd.depth = (int32_t)dep; cd.kind = d; cd.len = ilen; cd.rec = wrec; A.cand[k] = cd; }
-        else *A.overflow = 1;
+        const int32_t p = (int32_t)((g - J.out) % A.W);
+        atomicOr((unsigned long long*)&A.cmask[(int64_t)w * (A.W >> 6) + (p >> 6)], 1ull << (p & 63));
       }
     } else {
       pl_call& o = A.calls[g];
       o.base = cl.base; o.alt = cl.alt; o.q = cl.q;
       o.flags = (uint16_t)((cl.flags & ~PL_CF_DISP_MASK) | (o.flags & PL_CF_DISP_MASK) | PL_CF_DELETED);
     }
+  }
+}
+
+__global__ void __launch_bounds__(256) k_indel_pass(EngineArgs A) {
+  const uint32_t n = *A.defer_n < A.defer_cap ? *A.defer_n : A.defer_cap;
+  indel_columns(A, A.defer, n, 0, (blockIdx.x * blockDim.x + threadIdx.x) >> 6, (gridDim.x * blockDim.x) >> 6);
+}
+
+// ------------------------------------------------------------------ candidates
+// The change candidates in position order, from the windows' candidate
+// masks: windows follow each other in position order, so a candidate's place
+// is the number of mask bits before its own.  A block takes PL_CAND_WORDS
+// mask words; k_cand_sums gives each block's bits (launched when there is
+// more than one block), k_cand_list adds those of the blocks before it.  The
+// masks are an eighth of a byte per position, so both passes cost their
+// launch; sorting a candidate list took 17 launches.
+#define PL_CAND_WORDS 2048
+#define PL_CAND_PER (PL_CAND_WORDS / 256)
+__global__ void __launch_bounds__(256) k_cand_sums(EngineArgs A, int64_t n_words, uint32_t* sums) {
+  const int64_t x0 = (int64_t)blockIdx.x * PL_CAND_WORDS + threadIdx.x;
+  uint32_t n = 0;
+#pragma unroll
+  for (int k = 0; k < PL_CAND_PER; k++) {
+    const int64_t x = x0 + 256 * k;
+    if (x < n_words) n += (uint32_t)__popcll(A.cmask[x]);
+  }
+  n = wave_sum(n);
+  __shared__ uint32_t ws[4];
+  if ((threadIdx.x & 63) == 0) ws[threadIdx.x >> 6] = n;
+  __syncthreads();
+  if (threadIdx.x == 0) sums[blockIdx.x] = ws[0] + ws[1] + ws[2] + ws[3];
+}
+
+__global__ void __launch_bounds__(256) k_cand_list(EngineArgs A, int64_t n_words, const uint32_t* sums) {
+  __shared__ uint32_t ws[4], wp[4];
+  const int tid = threadIdx.x;
+  const int32_t MW = A.W >> 6;
+  uint32_t pre = 0;
+  for (int64_t b = tid; b < (int64_t)blockIdx.x; b += 256) pre += sums[b];
+  pre = wave_sum(pre);
+  if ((tid & 63) == 0) wp[tid >> 6] = pre;
+  const int64_t x0 = (int64_t)blockIdx.x * PL_CAND_WORDS + (int64_t)tid * PL_CAND_PER;
+  uint64_t m[PL_CAND_PER];
+  uint32_t n = 0;
+#pragma unroll
+  for (int k = 0; k < PL_CAND_PER; k++) {
+    m[k] = x0 + k < n_words ? A.cmask[x0 + k] : 0ull;
+    n += (uint32_t)__popcll(m[k]);
+  }
+  const uint32_t inc = wave_scan_dpp(n);
+  if ((tid & 63) == 63) ws[tid >> 6] = inc;
+  __syncthreads();
+  uint32_t at = wp[0] + wp[1] + wp[2] + wp[3] + inc - n;
+  for (int w = 0; w < (tid >> 6); w++) at += ws[w];
+#pragma unroll
+  for (int k = 0; k < PL_CAND_PER; k++) {
+    const int64_t x = x0 + k;
+    if (x >= n_words) break;
+    const int32_t wi = (int32_t)(x / MW), word = (int32_t)(x - (int64_t)wi * MW);
+    const bool edge = word == 0 || word == MW - 1;
+    if (!m[k] && !edge) continue;
+    const WinDev win = A.wins[wi];
+    const JobDev& J = A.jobs[win.job];
+    if (word == 0 && win.p0 == 0) A.st[win.job].cand_lo = (int32_t)at;
+    for (uint64_t b = m[k]; b; b &= b - 1) {
+      const int64_t g = J.out + win.p0 + 64 * word + (__ffsll((unsigned long long)b) - 1);
+      if (at < A.cand_cap) {
+        const pl_call cl = A.calls[g];
+        int64_t dep = 0;
+        for (int f = 0; f < 4; f++) dep += (int64_t)(uint32_t)A.pile[(int64_t)(PL_F_COUNT_A + f) * A.G + g];
+        dep += A.pile[(int64_t)PL_F_DELETIONS * A.G + g];
+        Cand c;
+        c.gpos = (uint32_t)g;
+        c.depth = (int32_t)dep;
+        c.kind = call_disp(cl);
+        c.len = 0;
+        c.rec = -1;
+        if (c.kind == PL_D_INS || c.kind == PL_D_DEL) { c.rec = A.prec[g]; c.len = A.rec[c.rec].len; }
+        c.base = cl.base;
+        c.alt = cl.alt;
+        c.pad = 0;
+        A.cand[at] = c;
+      } else {
+        *A.overflow = 1;
+      }
+      at++;
+    }
+    if (word == MW - 1 && win.p1 == J.size) A.st[win.job].cand_hi = (int32_t)at;
+    if (x == n_words - 1) *A.cand_n = at;
   }
 }
 
@@ -1219,39 +1406,18 @@ __global__ void __launch_bounds__(256) k_indel_pass(EngineArgs A, const uint32_t
 // deletion; each active deletion's positions are then mutated by the lanes.
 // Same result as finalize_job, which a region with more than PL_FIN_DELS
 // active deletions runs serially.
-__global__ void __launch_bounds__(64) k_finalize(EngineArgs A, const Cand* sorted, const uint32_t* cand_n, uint32_t cap,
-                                                 Cand* cand) {
+__global__ void __launch_bounds__(64) k_finalize(EngineArgs A) {
   __shared__ int64_t s_dg[PL_FIN_DELS];
   __shared__ int32_t s_dl[PL_FIN_DELS];
   const int32_t j = blockIdx.x;
   if (j >= A.n_jobs) return;
   const int lane = threadIdx.x;
-  const uint32_t n = *cand_n < cap ? *cand_n : cap;
   const JobDev& J = A.jobs[j];
   JobStat& st = A.st[j];
-  // candidates of this region: gpos in [out, out + size)
-  int64_t a, b;
-  {
-    int64_t lo = 0, hi = n;
-    while (hi - lo > 64) {
-      const int64_t m = hi - lo, pr = lo + ((int64_t)(lane + 1) * m) / 65;
-      const int k = __popcll(__ballot((int64_t)sorted[pr].gpos < J.out));
-      const int64_t plo = lo + ((int64_t)k * m) / 65, phi = lo + ((int64_t)(k + 1) * m) / 65;
-      if (k > 0) lo = plo + 1;
-      if (k < 64) hi = phi;
-    }
-    a = lo + __popcll(__ballot(lo + lane < hi && (int64_t)sorted[lo + lane].gpos < J.out));
-    lo = a; hi = n;
-    while (hi - lo > 64) {
-      const int64_t m = hi - lo, pr = lo + ((int64_t)(lane + 1) * m) / 65;
-      const int k = __popcll(__ballot((int64_t)sorted[pr].gpos < J.out + J.size));
-      const int64_t plo = lo + ((int64_t)k * m) / 65, phi = lo + ((int64_t)(k + 1) * m) / 65;
-      if (k > 0) lo = plo + 1;
-      if (k < 64) hi = phi;
-    }
-    b = lo + __popcll(__ballot(lo + lane < hi && (int64_t)sorted[lo + lane].gpos < J.out + J.size));
-  }
-  if (lane == 0) { st.cand_lo = (int32_t)a; st.cand_hi = (int32_t)b; }
+  const uint32_t* hist = A.hist + (int64_t)j * PL_HIST;
+  Cand* cand = A.cand;
+  const int64_t a = st.cand_lo;
+  const int64_t b = st.cand_hi < (int64_t)A.cand_cap ? st.cand_hi : (int64_t)A.cand_cap;
   const int32_t md = min_depth_of(A.cf, st.base_count, J.size);
   const bool none = st.read_count == 0;
   // active deletions, in order
@@ -1275,7 +1441,8 @@ __global__ void __launch_bounds__(64) k_finalize(EngineArgs A, const Cand* sorte
   __syncthreads();
   if (serial) {
     if (lane == 0)
-      finalize_job(A.cf, J, st, A.pile, A.G, A.calls, cand, a, b, A.mutated, A.mutated_n, A.mutated_cap, A.overflow);
+      finalize_job(A.cf, J, st, hist, A.pile, A.G, A.calls, cand, a, b, A.mutated, A.mutated_n, A.mutated_cap,
+                   A.overflow);
     return;
   }
   // every candidate at once: shallow, or under an active deletion (not its own)
@@ -1309,25 +1476,34 @@ __global__ void __launch_bounds__(64) k_finalize(EngineArgs A, const Cand* sorte
     }
   }
   dropped = wave_sum(dropped);
+  int64_t nconf = 0;     // minDepth above the histogram: counted by k_after
+  if (md <= PL_CONF_HIST_MAX) for (int d = md + lane; d < PL_HIST; d += 64) nconf += hist[d];
+  nconf = wave_sum(nconf);
   if (lane == 0) {
     st.min_depth = md;
-    int64_t nconf = 0;   // minDepth above the histogram: counted by k_confirm_exact
-    if (md <= PL_CONF_HIST_MAX) for (int d = md; d < 256; d++) nconf += st.hist[d];
-    else if (st.read_count != 0) atomicOr(A.deep, 1u);
+    if (md > PL_CONF_HIST_MAX && st.read_count != 0) atomicOr(A.deep, 1u);
     if (nconf > 0) nconf = nconf - dropped > 0 ? nconf - dropped : 0;   // the serial scan stops decrementing at 0
     st.n_confirmed = (int32_t)nconf;
   }
 }
 
-// Exact confirmed count of the regions whose minDepth lies above the depth
-// histogram (a --mindepth of 256 or more, or a region averaging more than
-// about 2,555x): every position of their windows is tested after the
-// deletion pass.  Other regions' windows are skipped after one load, so the
-// launch costs a few microseconds when no region needs it.
-__global__ void __launch_bounds__(256) k_confirm_exact(EngineArgs A) {
+// After the deletion pass: the first PL_AFTER_BLOCKS blocks call the columns
+// it changed again, the rest give the exact confirmed count of the regions
+// whose minDepth lies above the depth histogram (a --mindepth of 256 or more,
+// or a region averaging more than about 2,555x), whose every position is
+// tested.  The two write different things of a position and the count looks
+// at no deleted one, so one launch does both; it is short when no region
+// needs the count and no deletion was called.
+#define PL_AFTER_BLOCKS 256
+__global__ void __launch_bounds__(256) k_after(EngineArgs A) {
   __shared__ uint32_t s_n;
+  if (blockIdx.x < PL_AFTER_BLOCKS) {
+    const uint32_t n = *A.mutated_n < A.mutated_cap ? *A.mutated_n : A.mutated_cap;
+    indel_columns(A, A.mutated, n, 1, (blockIdx.x * blockDim.x + threadIdx.x) >> 6, (PL_AFTER_BLOCKS * blockDim.x) >> 6);
+    return;
+  }
   if (*(volatile uint32_t*)A.deep == 0) return;   // no region needs the exact count
-  for (int32_t w = blockIdx.x; w < A.n_wins; w += gridDim.x) {
+  for (int32_t w = (int32_t)blockIdx.x - PL_AFTER_BLOCKS; w < A.n_wins; w += (int32_t)gridDim.x - PL_AFTER_BLOCKS) {
     const WinDev win = A.wins[w];
     JobStat& S = A.st[win.job];
     const int32_t md = S.min_depth;
@@ -1371,11 +1547,6 @@ __global__ void k_final_flags(EngineArgs A) {
 }
 
 // insertion strings of INS changes into a byte pool
-// the calls of the candidate columns, in candidate order (one copy to the host)
-__global__ void k_cand_calls(const Cand* c, uint32_t n, const pl_call* calls, pl_call* out) {
-  for (uint32_t k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) out[k] = calls[c[k].gpos];
-}
-
 __global__ void k_ins_strings(EngineArgs A, const Cand* sorted, const int64_t* idx, const int64_t* off, int32_t n, uint8_t* pool) {
   const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;

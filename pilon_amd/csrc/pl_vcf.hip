@@ -321,31 +321,12 @@ pl_status vcf_format(pl_ctx* c, Lane* L, const std::vector<std::string>& rnames,
     HIPCHK(hipMemcpyAsync(emb + L->hjobs[0].out, fr->embed.data(), fr->embed.size(), hipMemcpyHostToDevice, st));
     V.embed = emb;
   }
-  if ((s = B.get(&V.ilist_n, 4)) || (s = B.get(&V.imap, 4 * (size_t)G)) || (s = B.get(&V.len, 4 * (size_t)G)))
-    return s;
   uint64_t* off;
-  if ((s = B.get(&off, 8 * (size_t)(G + 1)))) return s;
+  if ((s = B.get(&V.len, 4 * (size_t)G)) || (s = B.get(&off, 8 * (size_t)(G + 1)))) return s;
   V.off = off;
   EventPair ev;
   HIPCHK(ev.create());
   HIPCHK(hipEventRecord(ev.e0, st));
-  // indel-call columns, grown once if the first capacity was short
-  uint32_t icap = (uint32_t)std::min<int64_t>(G, 1 << 20) + 64, ni = 0;
-  for (int attempt = 0; attempt < 2; attempt++) {
-    if ((s = B.get(&V.ilist, 4 * (size_t)icap)) || (s = B.get(&V.irec, 8 * (size_t)icap))) return s;
-    V.icap = icap;
-    HIPCHK(hipMemsetAsync(V.ilist_n, 0, 4, st));
-    k_vcf_mark<<<dim3((unsigned)L->n_wins), dim3(256), 0, st>>>(V);
-    HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(&ni, V.ilist_n, 4, hipMemcpyDeviceToHost, st));
-    HIPCHK(hipStreamSynchronize(st));
-    if (ni <= icap) break;
-    icap = ni + 64;
-  }
-  if (ni) {
-    k_vcf_indel<<<dim3((unsigned)std::min<uint32_t>(4096, (ni + 3) / 4)), dim3(256), 0, st>>>(V);
-    HIPCHK(hipGetLastError());
-  }
   k_vcf_lines<false><<<dim3((unsigned)L->n_wins), dim3(256), 0, st>>>(V);
   HIPCHK(hipGetLastError());
   const int64_t tiles = std::max<int64_t>(1, (G + SCAN_TILE - 1) / SCAN_TILE);

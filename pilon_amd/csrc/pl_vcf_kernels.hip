@@ -3,13 +3,9 @@
 // Vcf.writeRecord, Vcf.scala:74-163).  Included at the end of
 // pl_kernels.hip: it uses that file's wave helpers.
 //
-// Three passes over the windows of the last batch, all reading the final
-// pileup, calls and sorted indel evidence the batch left in HBM:
-//   k_vcf_mark    lists the columns whose call is an insertion or deletion
-//                 (and not at region index 0, where writeRecord never
-//                 prints the indel allele);
-//   k_vcf_indel   finds each listed column's winning evidence record again
-//                 (the strict majority of the indel pass);
+// Two passes over the windows of the last batch, both reading the final
+// pileup, calls and indel evidence (each called column's winning record, left
+// by the indel pass) the batch left in HBM:
 //   k_vcf_lines   measures every locus's record lines; an exclusive
 //                 64-bit scan of the lengths gives each locus its offset;
 //   k_vcf_write   formats them again, staged in LDS, and stores them.
@@ -19,11 +15,6 @@ struct VcfArgs {
   const char* names;          // region names, concatenated
   const int64_t* name_off;    // [n_jobs + 1]
   uint32_t flags;             // PL_VCF_* (include/pilon_hip.h)
-  uint32_t* ilist;            // indel-call columns
-  uint32_t* ilist_n;
-  uint32_t icap;
-  int32_t* imap;              // column -> its index in ilist (listed columns only)
-  int64_t* irec;              // [icap] winning record of each listed column
   uint32_t* len;              // [G] bytes of the column's lines
   const uint64_t* off;        // [G + 1] their offsets
   char* text;
@@ -241,7 +232,7 @@ __device__ __forceinline__ uint32_t vcf_locus(char* out, const VcfArgs& V, const
   if (f & PL_CF_WIDE) wide_patch(v.c, V.A.wide, V.A.wide_cap, V.A.win_wide, J, V.A.W, g);
   const bool deleted = (f & PL_CF_DELETED) != 0 || (V.embed && V.embed[g]);
   int64_t rec = -1;
-  if (i > 0 && (f & (PL_CF_INSERTION | PL_CF_DELETION))) rec = V.irec[V.imap[g]];
+  if (i > 0 && (f & (PL_CF_INSERTION | PL_CF_DELETION))) rec = V.A.prec[g];
   vcf_record<WRITE>(o, V, J, R, name, name_len, minDepth, v, f, rec, i, deleted, true);
   if (i > 0 && (f & PL_CF_INDEL) && !deleted)
     vcf_record<WRITE>(o, V, J, R, name, name_len, minDepth, v, f, rec, i,
@@ -250,49 +241,6 @@ __device__ __forceinline__ uint32_t vcf_locus(char* out, const VcfArgs& V, const
 }
 
 }  // namespace
-
-__global__ void __launch_bounds__(256) k_vcf_mark(VcfArgs V) {
-  const WinDev win = V.A.wins[blockIdx.x];
-  const JobDev& J = V.A.jobs[win.job];
-  for (int p = win.p0 + threadIdx.x; p - threadIdx.x < win.p1; p += blockDim.x) {
-    const bool act = p < win.p1;
-    const int64_t g = J.out + p;
-    const bool want = act && p > 0 && (V.A.calls[g].flags & (PL_CF_INSERTION | PL_CF_DELETION));
-    const uint32_t k = wave_append(V.ilist_n, want);
-    if (want && k < V.icap) { V.ilist[k] = (uint32_t)g; V.imap[g] = (int32_t)k; }   // the host re-runs when k >= icap
-  }
-}
-
-// one wave per listed column: the winning record, as the indel pass found it
-__global__ void __launch_bounds__(256) k_vcf_indel(VcfArgs V) {
-  const EngineArgs& A = V.A;
-  const uint32_t n = *V.ilist_n < V.icap ? *V.ilist_n : V.icap;
-  const uint32_t nrec = *A.rec_n < A.rec_cap ? *A.rec_n : A.rec_cap;
-  const int lane = threadIdx.x & 63;
-  const uint32_t nw = (gridDim.x * blockDim.x) >> 6;
-  for (uint32_t k = (blockIdx.x * blockDim.x + threadIdx.x) >> 6; k < n; k += nw) {
-    const uint32_t g = V.ilist[k];
-    const int32_t j = wave_job_of(A.jobs, A.n_jobs, g, lane);
-    const RSDev& R = A.rs[A.jobs[j].rs];
-    const Col c = load_col(A.pile, A.G, g);
-    int32_t pct = 0;
-    const int need = indel_kind_needed(c, A.cf, &pct);
-    int64_t win = -1;
-    if (need) {
-      const uint32_t key = (g << 1) | (uint32_t)(need - 1);
-      const int64_t a = wave_lower_bound(A.rkey, nrec, key, lane);
-      int64_t b = a;
-      for (;;) {
-        const int64_t t = b + lane;
-        const int cnt = __popcll(__ballot(t < (int64_t)nrec && A.rkey[t] == key));
-        b += cnt;
-        if (cnt < 64) break;
-      }
-      win = wave_majority(R, A.rec, A.rval, a, b, lane).rec;
-    }
-    if (lane == 0) V.irec[k] = win;
-  }
-}
 
 // the length pass (WRITE false); the write pass is k_vcf_write
 template <bool WRITE>

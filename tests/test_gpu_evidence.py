@@ -1,0 +1,92 @@
+"""Indel evidence and candidate order of a batch against the oracle: windows
+whose records just fit their LDS buffer (128) and spill beyond it, at one
+column and over many, with the windows taken in their own order and, when
+more than the launch holds at once, in cost order."""
+import numpy as np
+import pytest
+
+from pilon_amd.abi import default_config
+from pilon_amd.reads import pack_reads
+from tests.helpers import assert_same_region, assert_same_stats
+
+pytestmark = pytest.mark.gpu
+
+
+def indel_reads(ref, sites, seed):
+    """60-base reads, `n` per (locus, op, length) site carrying the indel 30
+    bases in (two insertion strings, so that majorities differ)."""
+    rng = np.random.default_rng(seed)
+    out = []
+    for locus, op, ln, n in sites:
+        a = locus - 31
+        for k in range(n):
+            q = [int(x) for x in rng.integers(20, 41, 60 + (ln if op == "I" else 0))]
+            if op == "I":
+                ins = ("GATC" if k % 4 else "GTTC")[:ln]
+                out.append(dict(pos=a + 1, cigar=f"30M{ln}I30M", seq=ref[a:a + 30] + ins + ref[a + 30:a + 60], qual=q))
+            else:
+                out.append(dict(pos=a + 1, cigar=f"30M{ln}D30M", seq=ref[a:a + 30] + ref[a + 30 + ln:a + 60 + ln],
+                                qual=q[:60]))
+    return out
+
+
+@pytest.mark.parametrize("n", [127, 128, 129, 700])
+@pytest.mark.parametrize("window,persistent", [(64, 1), (512, 0)])
+def test_window_record_buffer(n, window, persistent):
+    from oracle import oracle as O
+    from pilon_amd.engine import Context
+    print(f"case: {n} records in one column, window {window}", flush=True)
+    rng = np.random.default_rng(n)
+    ref = "".join("ACGT"[x] for x in rng.integers(0, 4, 4000))
+    sites = [(1100, "I", 4, n), (1900, "D", 3, n // 2), (1920, "I", 2, n - n // 2)]
+    sites += [(2600 + 9 * k, "I" if k % 2 else "D", 1 + k % 4, 1 + k % 9) for k in range(60)]
+    b = pack_reads(indel_reads(ref, sites, n))
+    cfg = default_config()
+    ctx = Context(cfg, device=0)
+    try:
+        ctx.ref_upload(0, "ctg", ref)
+        rid = ctx.readset_upload(0, b)
+        pile, calls, stats = ctx.batch_run([(0, 1, 4000, rid)], window=window, block=256, persistent=persistent)
+        changes, _ = ctx.batch_fix()
+        text, _ = ctx.batch_vcf()
+    finally:
+        ctx.close()
+    want = O.run_region(cfg, ref.encode(), 1, 4000, [b], name="ctg", vcf=O.VCF_ON)
+    assert want["status"] == 0
+    assert_same_region(pile, calls, want, f"{n} records")
+    assert_same_stats(stats[0], want["stats"], f"{n} records")
+    assert changes == want["changes"]
+    assert text == want["vcf"]
+
+
+def test_candidates_over_many_blocks():
+    """Contigs whose candidate masks fill several list blocks, more windows
+    than the launch holds at once (cost order), regions of a single locus
+    among them: every region's changes in order."""
+    from oracle import oracle as O
+    from pilon_amd.engine import Context
+    from pilon_amd.synth import SynthData, preset
+    p = preset("c3", scale=0.01)
+    p.update(coverage=25, snv_rate=0.01, indel_rate=0.002, lens=p["lens"] + [300_001])
+    print("case: candidates over many blocks", flush=True)
+    d = SynthData(p)
+    cfg = default_config()
+    ctx = Context(cfg, device=0)
+    try:
+        ids = []
+        for i in range(d.n):
+            ctx.ref_upload(i, d.names[i], d.draft(i))
+            ids.append(ctx.readset_upload(i, d.batch(i)))
+        regions = [(i, 1, len(d.draft(i)), ids[i]) for i in range(d.n)] + [(0, 500, 500, ids[0])]
+        _, _, stats = ctx.batch_run(regions, window=64, block=256, persistent=1, copy_out=False)
+        changes, fasta = ctx.batch_fix(element=list(range(len(regions))))
+    finally:
+        ctx.close()
+    want_c = ""
+    for (i, s, e, _), st in zip(regions, stats):
+        w = O.run_region(cfg, d.draft(i), s, e, [d.batch(i)], name=d.names[i])
+        assert w["status"] == 0
+        assert_same_stats(st, w["stats"], f"{i}:{s}-{e}")
+        want_c += w["changes"]
+    assert changes == want_c
+    assert changes.count("\n") > 2000
