@@ -80,6 +80,7 @@ void* ch_run(const pl_config* pc, const uint8_t* ref, int64_t ref_len, const cha
   R.bases2 = s->bases2; R.quals = s->quals; R.n_exotic = s->n_exotic;
   R.exo_read = s->exo_read; R.exo_off = s->exo_off; R.nib = s->nib; R.lrt = lrt;
   R.meta = meta.data(); R.ref = ref; R.ref_len = ref_len;
+  R.all_long = lrt && n > 0 && std::all_of(lrt, lrt + n, [](uint8_t x) { return x != 0; });
   // ---- read-set prep (k_readset_prep)
   int32_t max_back = 0, max_lead = 0, max_back_fp = 0;
   std::vector<int64_t> outliers;
@@ -88,13 +89,12 @@ void* ch_run(const pl_config* pc, const uint8_t* ref, int64_t ref_len, const cha
   std::vector<Seg> segs;
   for (int64_t r = 0; r < n; r++) {
     RMeta& m = meta[r];
-    if (!((m.info & RI_KEEP) && !(m.info & (RI_SIMPLE | RI_EXOTIC | RI_BAD | RI_LR_MASK)))) continue;
-    const int c = build_segs(R, r, m.info, cf, nullptr);
+    if (!wants_segs(m.info)) continue;
+    const uint32_t c = seg_slots(R, r, m.info, cf);
     const size_t o = segs.size();
     segs.resize(o + (size_t)c);
-    if (c) build_segs(R, r, m.info, cf, segs.data() + o);
+    m.info = seg_fill(R, r, m.info, cf, segs.data(), (uint32_t)o, c);
     m.op0 = (uint32_t)o;
-    m.info = (m.info & ~RI_SEG_MASK) | ((uint32_t)(c < RI_SEG_MAX ? c : RI_SEG_MAX) << RI_SEG_SHIFT);
   }
   segs.emplace_back();
   R.segs = segs.data();
@@ -106,7 +106,7 @@ void* ch_run(const pl_config* pc, const uint8_t* ref, int64_t ref_len, const cha
     if (m.fr_lo < m.fr_hi) { lo = std::min<int64_t>(lo, m.fr_lo); hi = std::max<int64_t>(hi, (int64_t)m.fr_hi - 1); }
     if (lo > hi) continue;
     int64_t lead = R.pos[r] - lo, back = hi - R.pos[r];
-    if (lead > PL_MAX_LEAD || back > PL_MAX_BACK || R.seq_off[r + 1] - R.seq_off[r] >= PL_MAX_SEQ) { outliers.push_back(r); meta[r].info |= RI_OUTLIER; continue; }
+    if (lead > PL_MAX_LEAD || back > (R.all_long ? PL_MAX_BACK_LONG : PL_MAX_BACK) || R.seq_off[r + 1] - R.seq_off[r] >= PL_MAX_SEQ) { outliers.push_back(r); meta[r].info |= RI_OUTLIER; continue; }
     max_back = std::max<int32_t>(max_back, (int32_t)std::max<int64_t>(back, 0));
     max_lead = std::max<int32_t>(max_lead, (int32_t)std::max<int64_t>(lead, 0));
     if (m.fp_lo <= m.fp_hi && m.fp_hi > m.pos) max_back_fp = std::max<int32_t>(max_back_fp, m.fp_hi - m.pos);
@@ -180,6 +180,7 @@ void* ch_run(const pl_config* pc, const uint8_t* ref, int64_t ref_len, const cha
       // one-wave walks for the rest
       std::vector<Run> runs;
       std::vector<int64_t> cplx;
+      auto drop = [&](uint32_t lr, int32_t dl) { return lr_drops_deletion(R, J, lr, dl); };
       for (int64_t r = plo; r < hi; r++) {
         const RMeta m = meta[r];
         if ((m.info & RI_OUTLIER) || !read_in_query(m, J)) continue;
@@ -189,11 +190,20 @@ void* ch_run(const pl_config* pc, const uint8_t* ref, int64_t ref_len, const cha
         const int ns = (int)((m.info & RI_SEG_MASK) >> RI_SEG_SHIFT);
         if (m.info & RI_SIMPLE) {
           if (simple_run(m, R.seq_off[r], cf, L0, L1, rr, &sk.aligned_n, &sk.bcount)) runs.push_back(rr[0]);
+        } else if ((m.info & RI_LR_MASK) && ns == RI_SEG_LONG) {
+          // a long read: the segments that can touch the window
+          const Seg& h = R.segs[m.op0];
+          const Seg* sg = R.segs + m.op0 + 1;
+          const int32_t L = (int32_t)(R.seq_off[r + 1] - R.seq_off[r]);
+          int32_t i = (int32_t)(std::partition_point(sg, sg + h.len, [&](const Seg& g) { return seg_end(g) < L0; }) - sg);
+          for (; i < h.len && seg_key(sg[i]) < L1 + h.fin; i++)
+            if (seg_apply(R, J, cf, r, m.info, R.seq_off[r], L, L0, L1, sg[i], rr[0], &sk.aligned_n, &sk.bcount, sk, drop))
+              runs.push_back(rr[0]);
         } else if (!(m.info & RI_EXOTIC) && ns < RI_SEG_MAX) {
           // each segment on its own, as the kernel's lanes apply them
           const int32_t L = (int32_t)(R.seq_off[r + 1] - R.seq_off[r]);
           for (int i = 0; i < ns; i++)
-            if (seg_apply(J, cf, r, m.info, R.seq_off[r], L, L0, L1, R.segs[m.op0 + i], rr[0], &sk.aligned_n, &sk.bcount, sk))
+            if (seg_apply(R, J, cf, r, m.info, R.seq_off[r], L, L0, L1, R.segs[m.op0 + i], rr[0], &sk.aligned_n, &sk.bcount, sk, drop))
               runs.push_back(rr[0]);
         } else {
           cplx.push_back(r);
@@ -204,7 +214,8 @@ void* ch_run(const pl_config* pc, const uint8_t* ref, int64_t ref_len, const cha
           const int p = ru.p0 + i;
           if (ru.fl & EF_VALID) {
             const int64_t q = ru.q + i;
-            const int32_t qual = (ru.fl & EF_NOQUAL) ? cf.default_qual : (int32_t)R.quals[q];
+            const int32_t qual = (ru.fl & EF_NANO) && nanopore_exclude(R, J, (int64_t)L0 + p - J.start) ? 0
+                                 : (ru.fl & EF_NOQUAL) ? cf.default_qual : (int32_t)R.quals[q];
             const int b = (R.bases2[q >> 2] >> (2 * (q & 3))) & 3;
             if (qual >= cf.min_qual) sk.base(p, b, qual, (int32_t)((ru.fl >> 16) & 0x1ffu));
           } else {

@@ -24,7 +24,8 @@
 #define RI_LR_MASK      0x06000000u
 #define RI_SEG_SHIFT    27           // complex reads: number of segments (RMeta.op0 = first)
 #define RI_SEG_MASK     0xf8000000u
-#define RI_SEG_MAX      31           // more segments, or a long read: the read is walked instead
+#define RI_SEG_MAX      31           // more segments: the read is walked instead
+#define RI_SEG_LONG     1            // of a long read: its segments follow a header segment
 #define PL_COST_BINS    256         // cost classes of the work queue's order
 #define PL_LR_NANOPORE  1
 #define PL_LR_PACBIO    2
@@ -33,6 +34,14 @@
 // outlier list instead of the sorted scan.
 #define PL_MAX_LEAD 4096
 #define PL_MAX_BACK 8192
+// ... and in a set of long reads only, whose reads mostly reach further: each
+// window scans the headers this far back, but a read on the outlier list is
+// walked, every CIGAR op of it, by every window it touches and looked at by
+// all the others
+#define PL_MAX_BACK_LONG 65536
+// long reads a wave takes at a time, each with a run of segments: a window of
+// a set of long reads has fewer than a hundred reads
+#define PL_LONG_READS 4
 // a read with this much sequence or more is walked as an outlier, and a read
 // whose sequence starts this far past its tile's first read takes the
 // complex path: together they keep tile-relative sequence offsets in int32
@@ -83,6 +92,8 @@ struct RSDev {               // one resident read set (one contig, sorted by pos
   int32_t* scal;             // [0]=max_back [1]=max_lead [2]=max_qspan [3]=n_outlier(int)
                              // [6]=max_back of the pileup footprints alone
   FragTail* ftail;           // [n] per read
+  int32_t all_long;          // every read is a long read
+  int32_t nano;              // some read is a nanopore read
 };
 
 struct JobDev {              // one region of a batch
@@ -178,8 +189,8 @@ struct EngineArgs {
   uint32_t* hist;            // [n_jobs][PL_HIST]
   IndelRec* rec; uint32_t* rec_n; uint32_t rec_cap;
   uint32_t* win_rec;         // [2 * n_wins]: each window's first record and count
-  IndelRec* spill; uint32_t* spill_win; uint32_t* spill_n; uint32_t spill_cap;   // records beyond a window's LDS buffer
-  uint32_t* win_cur;         // [n_wins] records placed from the spill
+  // records beyond a window's LDS buffer, with their window and their place among its records
+  IndelRec* spill; uint2* spill_at; uint32_t* spill_n; uint32_t spill_cap;
   uint64_t* cmask;           // [n_wins][W / 64] candidate columns of each window, a bit per position
   int32_t* prec;             // [G] winning record of the columns the indel pass called (-1: none)
   Cand* cand; uint32_t* cand_n; uint32_t cand_cap;   // candidates in position order

@@ -263,6 +263,12 @@ PL_HD bool nanopore_exclude(const RSDev& R, const JobDev& J, int64_t i0) {
   return R.ref[i0 - 2] == 'C' && R.ref[i0 - 1] == 'C' && R.ref[i0 + 1] == 'G' && R.ref[i0 + 2] == 'G';
 }
 
+// A long read's deletion at locus dl is dropped (PileUpRegion.scala:180-182).
+PL_HD bool lr_drops_deletion(const RSDev& R, const JobDev& J, uint32_t lr, int32_t dl) {
+  const int64_t i0 = (int64_t)dl - J.start;
+  return homo_run4(R, i0) || (lr == PL_LR_NANOPORE && nanopore_exclude(R, J, i0));
+}
+
 // Insertion event of one I op (PileUpRegion.scala:150-162): gate, left
 // normalisation, then addInsertion at the final locus if it lies in the window.
 // A long read's insertion (lr > 0) is dropped where homoRun(iloc) >= 4, and
@@ -316,10 +322,7 @@ PL_HD void del_event(const RSDev& R, const JobDev& J, const KConf& cf, const Rea
     }
   }
   if (dl < J.start) { s.edge(r); return; }
-  if (lr) {
-    const int64_t i0 = (int64_t)dl - J.start;
-    if (homo_run4(R, i0) || (lr == PL_LR_NANOPORE && nanopore_exclude(R, J, i0))) return;
-  }
+  if (lr && lr_drops_deletion(R, J, lr, dl)) return;
   if (dl >= L0 && dl < L1) {
     uint32_t hasN;
     const uint32_t h = del_hash(R.ref, (int64_t)dl - 1, len, &hasN);
@@ -481,6 +484,7 @@ PL_HD void walk_read(const RSDev& R, const JobDev& J, const KConf& cf, int64_t r
 #define EF_VALID  (1u << 25)
 #define EF_NOQUAL (1u << 26)
 #define EF_BAD    (1u << 27)
+#define EF_NANO   (1u << 28)   // nanopore: quality 0 where nanopore_exclude
 struct Run {
   int32_t p0;        // window index of the first base
   int32_t n;
@@ -516,7 +520,12 @@ PL_HD int simple_run(const RMeta& m, int64_t seq0, const KConf& cf, int32_t L0, 
 // normalisation already applied (final locus, rotation, string hash) and,
 // for deletions, each slid-over base that addRead adds len bases later.
 // Region gates (inRegion) are applied at window time.
-enum { SEG_M = 0, SEG_S = 1, SEG_I = 2, SEG_D = 3, SEG_A = 4 };
+// A long read has hundreds of segments over many windows, so a window takes
+// only the ones that can touch it: its segments follow a header (SEG_H: len =
+// their count, fin = the furthest left of its op's locus one of them
+// reaches) in CIGAR order, in which the op's locus (seg_key) and the end of
+// its reference span (seg_end) both ascend.
+enum { SEG_M = 0, SEG_S = 1, SEG_I = 2, SEG_D = 3, SEG_A = 4, SEG_H = 5 };
 struct __attribute__((aligned(16))) Seg {
   int32_t kq;        // kind | quals(readOffset or rl) << 8
   int32_t locus;     // M: first locus; S: clipStart; I/D: locus before normalisation; A: slid dloc
@@ -529,9 +538,37 @@ struct __attribute__((aligned(16))) Seg {
 };
 PL_HD int seg_kind(const Seg& g) { return g.kq & 0xff; }
 PL_HD int32_t seg_qual(const Seg& g) { return g.kq >> 8; }
+PL_HD int32_t seg_key(const Seg& g) {
+  const int k = seg_kind(g);
+  return k == SEG_A ? g.pad : k == SEG_S && g.roff == 0 ? g.locus + g.len : g.locus;
+}
+PL_HD int32_t seg_end(const Seg& g) {
+  const int k = seg_kind(g);
+  return k == SEG_A ? g.pad + g.len : k == SEG_I ? g.locus : g.locus + g.len;
+}
+
+// Whether a long read's segments may be cut to a window's: clips only at its
+// ends (one between other ops would break the order of seg_end).
+PL_HD bool long_segs_ok(const RSDev& R, int64_t r) {
+  const int64_t c0 = R.cigar_off[r], c1 = R.cigar_off[r + 1];
+  int32_t done = 0;                                        // read bases before the op
+  bool last = false;
+  const int32_t L = (int32_t)(R.seq_off[r + 1] - R.seq_off[r]);
+  for (int64_t k = c0; k < c1; k++) {
+    const int op = (int)(R.cigar[k] & 15);
+    const int32_t len = (int32_t)(R.cigar[k] >> 4);
+    if (last && (consumes_read(op) || consumes_ref(op)) && len > 0) return false;
+    if (op == 4 && len > 0 && done > 0) last = true;
+    if (consumes_read(op)) done += len;
+    else if (consumes_ref(op) && len > 0 && done == 0) return false;   // a deletion before the first base
+  }
+  return L > 0;
+}
 
 // Writes the segments of read r into out (if non-null); returns their count.
+// lr: longReadType of the read (the insertions it drops have no segment).
 PL_HD int build_segs(const RSDev& R, int64_t r, uint32_t info, const KConf& cf, Seg* out) {
+  const uint32_t lr = (info & RI_LR_MASK) >> RI_LR_SHIFT;
   const int64_t c0 = R.cigar_off[r], c1 = R.cigar_off[r + 1];
   const int32_t L = (int32_t)(R.seq_off[r + 1] - R.seq_off[r]);
   const int32_t pos = R.pos[r];
@@ -557,9 +594,13 @@ PL_HD int build_segs(const RSDev& R, int64_t r, uint32_t info, const KConf& cf, 
       }
       n++;
     } else if (op == 1 && len > 0 && valid && tr && locus <= R.ref_len) {
+      int32_t rot = 0, il = 0;
+      if (out || lr) il = slide_insertion(R.ref, a, readOffset, len, locus, &rot);
+      if (lr && il < R.ref_len && homo_run4(R, il)) {      // dropped (PileUpRegion.scala:160)
+        readOffset += len;
+        continue;
+      }
       if (out) {
-        int32_t rot;
-        const int32_t il = slide_insertion(R.ref, a, readOffset, len, locus, &rot);
         uint32_t hasN;
         const uint32_t h = ins_hash(a, readOffset, len, rot, &hasN);
         Seg& g = out[n];
@@ -595,6 +636,44 @@ PL_HD int build_segs(const RSDev& R, int64_t r, uint32_t info, const KConf& cf, 
   return n;
 }
 
+// segments are built for multi-op reads (not RI_SIMPLE) that addRead processes
+PL_HD bool wants_segs(uint32_t info) {
+  return (info & RI_KEEP) && !(info & (RI_SIMPLE | RI_EXOTIC | RI_BAD));
+}
+// Table entries of read r: its segments, a header before a long read's.  0
+// for none and for a long read that is walked (odd clips, or deletions that
+// slide so far that the table would outgrow the CIGAR).
+PL_HD uint32_t seg_slots(const RSDev& R, int64_t r, uint32_t info, const KConf& cf) {
+  if (!wants_segs(info)) return 0u;
+  const bool lr = (info & RI_LR_MASK) != 0;
+  if (lr && !long_segs_ok(R, r)) return 0u;
+  const int64_t n = build_segs(R, r, info, cf, nullptr);
+  if (!lr) return (uint32_t)n;
+  return n > 0 && n <= 4 * (R.cigar_off[r + 1] - R.cigar_off[r]) + 64 ? (uint32_t)n + 1u : 0u;
+}
+// Fills read r's c entries from segs[o]; returns its info word (RMeta.op0 becomes o).
+PL_HD uint32_t seg_fill(const RSDev& R, int64_t r, uint32_t info, const KConf& cf, Seg* segs, uint32_t o, uint32_t c) {
+  uint32_t n = c < RI_SEG_MAX ? c : (uint32_t)RI_SEG_MAX;
+  if (!(info & RI_LR_MASK)) {
+    if (c) build_segs(R, r, info, cf, segs + o);
+  } else if (c == 0) {
+    n = RI_SEG_MAX;
+  } else {
+    n = RI_SEG_LONG;
+    build_segs(R, r, info, cf, segs + o + 1);
+    int32_t reach = 0;                                     // how far left of its op's locus a segment touches
+    for (uint32_t i = o + 1; i < o + c; i++) {
+      const Seg& g = segs[i];
+      const int kd = seg_kind(g);
+      const int32_t first = kd == SEG_I || kd == SEG_D ? g.fin : kd == SEG_A ? g.locus + g.len : g.locus;
+      reach = seg_key(g) - first > reach ? seg_key(g) - first : reach;
+    }
+    Seg& h = segs[o];
+    h.kq = SEG_H; h.locus = R.pos[r]; h.roff = 0; h.len = (int32_t)c - 1; h.fin = reach; h.hash = 0; h.rotn = 0; h.pad = 0;
+  }
+  return (info & ~RI_SEG_MASK) | (n << RI_SEG_SHIFT);
+}
+
 // One segment of a multi-op read at window time, applied on its own: every
 // segment carries what its gates need (a slide add carries its deletion's
 // locus), so the segments of a read can be applied in any order or in
@@ -602,11 +681,17 @@ PL_HD int build_segs(const RSDev& R, int64_t r, uint32_t info, const KConf& cf, 
 // region gates of PileUpRegion.addRead; an M segment with trusted in-window
 // bases, or an in-window clip, returns 1 and its run in ru (clip runs and
 // runs of invalid reads carry EF_BAD: badPair only).
-template <class Sink>
-PL_HD int seg_apply(const JobDev& J, const KConf& cf, int64_t r, uint32_t info, int64_t seq0, int32_t L,
-                    int32_t L0, int32_t L1, const Seg& g, Run& ru, int64_t* aligned, int64_t* bcount, Sink& s) {
+// A long read's indels carry indelMq (PileUpRegion.scala:142), and its
+// deletion at in-window locus d is dropped where lr_drop(lr, d) holds
+// (lr_drops_deletion, or the window's table of it).
+template <class Sink, class Drop>
+PL_HD int seg_apply(const RSDev& R, const JobDev& J, const KConf& cf, int64_t r, uint32_t info, int64_t seq0, int32_t L,
+                    int32_t L0, int32_t L1, const Seg& g, Run& ru, int64_t* aligned, int64_t* bcount, Sink& s,
+                    Drop&& lr_drop) {
   const bool valid = (info & RI_VALID) != 0;
   const int32_t mq1 = (int32_t)(info & RI_ADJMQ_MASK) + 1;
+  const uint32_t lr = (info & RI_LR_MASK) >> RI_LR_SHIFT;
+  const int32_t imq1 = lr && mq1 > 9 ? 9 : mq1;
   const int32_t flank = cf.flank;
   const int kd = seg_kind(g);
   if (kd == SEG_M) {                                       // (:184-193)
@@ -619,7 +704,9 @@ PL_HD int seg_apply(const JobDev& J, const KConf& cf, int64_t r, uint32_t info, 
     if (L - flank - g.roff < i1) i1 = L - flank - g.roff;
     if (i1 <= i0) return 0;
     ru.p0 = g.locus + i0 - L0; ru.n = i1 - i0; ru.q = seq0 + g.roff + i0;
-    ru.fl = valid ? (((uint32_t)mq1 << 16) | EF_VALID | ((info & RI_NOQUAL) ? EF_NOQUAL : 0u)) : EF_BAD;
+    ru.fl = valid ? (((uint32_t)mq1 << 16) | EF_VALID | ((info & RI_NOQUAL) ? EF_NOQUAL : 0u) |
+                     (lr == PL_LR_NANOPORE ? EF_NANO : 0u))
+                  : EF_BAD;
     if (valid) *bcount += i1 - i0;
     return 1;
   }
@@ -637,14 +724,14 @@ PL_HD int seg_apply(const JobDev& J, const KConf& cf, int64_t r, uint32_t info, 
   if (kd == SEG_I) {                                       // (:150-162)
     if (g.locus >= J.start && g.locus <= J.stop) {
       const int32_t il = g.fin;
-      if (il < J.start) s.edge(r);
+      if (il < J.start || (lr && (int64_t)il >= R.ref_len)) s.edge(r);
       else if (il >= L0 && il < L1) {
         IndelRec e;
         e.key = (uint32_t)(((uint64_t)(J.out + (il - J.start)) << 1) | 0u);
-        e.len = g.len; e.qual = (int16_t)seg_qual(g); e.mq1 = (uint16_t)mq1;
+        e.len = g.len; e.qual = (int16_t)seg_qual(g); e.mq1 = (uint16_t)imq1;
         e.hash = g.hash; e.rot = g.rotn & 0x3fffffff; e.flags = (g.rotn >> 30) & 1 ? 2u : 0u;
         e.src = seq0 + g.roff;
-        s.ins(il - L0, seg_qual(g), mq1, e);
+        s.ins(il - L0, seg_qual(g), imq1, e);
       }
     }
     return 0;
@@ -654,13 +741,13 @@ PL_HD int seg_apply(const JobDev& J, const KConf& cf, int64_t r, uint32_t info, 
     if (g.locus >= J.start && g.locus <= J.stop && e1 >= J.start && e1 <= J.stop) {
       const int32_t dl = g.fin;
       if (dl < J.start) s.edge(r);
-      else if (dl >= L0 && dl < L1) {
+      else if (dl >= L0 && dl < L1 && !(lr && lr_drop(lr, dl))) {
         IndelRec e;
         e.key = (uint32_t)(((uint64_t)(J.out + (dl - J.start)) << 1) | 1u);
-        e.len = g.len; e.qual = (int16_t)seg_qual(g); e.mq1 = (uint16_t)mq1;
+        e.len = g.len; e.qual = (int16_t)seg_qual(g); e.mq1 = (uint16_t)imq1;
         e.hash = g.hash; e.rot = 0; e.flags = (g.rotn >> 30) & 1 ? 2u : 0u;
         e.src = (int64_t)dl - 1;
-        s.del(dl - L0, seg_qual(g), mq1, e);
+        s.del(dl - L0, seg_qual(g), imq1, e);
       }
     }
     return 0;

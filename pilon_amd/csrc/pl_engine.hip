@@ -147,8 +147,8 @@ enum { PL_N_REC = 0, PL_N_CAND, PL_N_DEFER, PL_N_MUTATED, PL_N_OVERFLOW, PL_N_QU
 struct Lane {
   hipStream_t stream = nullptr;
   hipEvent_t ev[4] = {};
-  DBuf rsarr, kparr, jobs, wins, cost, bins, pile, calls, prec, cmask, csums, st, dhist, rec, winrec, wincur, spill,
-      spillwin, cand, defer, mutated, counters, strpool, stridx, stroff, wide, winwide, heads;
+  DBuf rsarr, kparr, jobs, wins, cost, bins, pile, calls, prec, cmask, csums, st, dhist, rec, winrec, spill,
+      spillat, cand, defer, mutated, counters, strpool, stridx, stroff, wide, winwide, heads;
   DBuf hist, tiles;                // sort and scan scratch (uploads, K-mers)
   uint32_t rec_cap = 0, spill_cap = 0, cand_cap = 0, defer_cap = 0, mut_cap = 0, wide_cap = 0;
   std::vector<JobDev> hjobs;
@@ -190,7 +190,7 @@ struct Lane {
 
   template <class F> void for_each_buffer(F&& f) {
     DBuf* b[] = {&rsarr, &kparr, &jobs, &wins, &cost, &bins, &pile, &calls, &prec, &cmask, &csums, &st, &dhist, &rec,
-                 &winrec, &wincur, &spill, &spillwin, &cand, &defer, &mutated, &counters, &strpool, &stridx, &stroff,
+                 &winrec, &spill, &spillat, &cand, &defer, &mutated, &counters, &strpool, &stridx, &stroff,
                  &wide, &winwide, &heads, &hist, &tiles, &jdepth};
     for (DBuf* x : b) f(*x);
   }
@@ -389,7 +389,11 @@ pl_status readset_upload(pl_ctx* c, int32_t contig_id, const pl_read_soa* s, int
   UP(d.exo_read, s->exo_read, 8 * s->n_exotic, 0);
   UP(d.exo_off, s->exo_off, 8 * s->n_exotic, 0);
   UP(d.nib, s->nib, s->n_exotic ? nib_bytes(s) : 0, 64);
-  if (lrt) { UP(d.lrt, lrt, n, 0); }
+  if (lrt) {
+    UP(d.lrt, lrt, n, 0);
+    d.all_long = n > 0 && std::memchr(lrt, 0, (size_t)n) == nullptr;
+    d.nano = n > 0 && std::memchr(lrt, PL_LR_NANOPORE, (size_t)n) != nullptr;
+  }
 #undef UP
   d.n_exotic = s->n_exotic;
   d.ref = it->second.dev;
@@ -817,7 +821,11 @@ pl_status readsets_upload_many(pl_ctx* c, int32_t n_sets, const int32_t* contig_
     d.seq_off = (const int64_t*)(U + q.f[6].at); d.bases2 = (const uint8_t*)(U + q.f[7].at);
     d.quals = (const int8_t*)(U + q.f[8].at); d.exo_read = (const int64_t*)(U + q.f[9].at);
     d.exo_off = (const int64_t*)(U + q.f[10].at); d.nib = (const uint8_t*)(U + q.f[11].at);
-    if (q.f.size() > 12) d.lrt = (const uint8_t*)(U + q.f[12].at);
+    if (q.f.size() > 12) {
+      d.lrt = (const uint8_t*)(U + q.f[12].at);
+      d.all_long = 1;
+      d.nano = bt == PL_BAM_NANOPORE;
+    }
     d.n_exotic = sets[i]->n_exotic;
     ncig[(size_t)i] = q.ncig;
     nb[(size_t)i] = q.nb;
@@ -833,6 +841,7 @@ struct GraphKey {
   int32_t W, block, persistent, grid;
   uint64_t lds;
   const void* bufs[2];
+  void (*wk)(EngineArgs, int);
 };
 
 void drop_graph(Lane* L) {
@@ -866,9 +875,16 @@ void lane_destroy(Lane* L) {
   for (int i = 0; i < 4; i++) L->ev[i] = nullptr;
 }
 
+typedef void (*WindowKernel)(EngineArgs, int);
+WindowKernel window_kernel(int block, bool lng) {
+  if (lng) return block == 256 ? k_window<256, true> : block == 512 ? k_window<512, true> : k_window<1024, true>;
+  return block == 256 ? k_window<256, false> : block == 512 ? k_window<512, false> : k_window<1024, false>;
+}
+
 // the device pipeline of one batch, enqueued on the lane's stream; with
 // timed set, events bracket the window kernel (not while capturing)
-pl_status enqueue_batch(Lane* L, EngineArgs& A, int persistent, int block, int grid, size_t lds, bool timed) {
+pl_status enqueue_batch(Lane* L, EngineArgs& A, WindowKernel wk, int persistent, int block, int grid, size_t lds,
+                        bool timed) {
   hipStream_t st = L->stream;
   const int32_t n_jobs = A.n_jobs, n_wins = A.n_wins;
   const unsigned jb = (unsigned)(n_jobs + 3) / 4, pb = (unsigned)(n_wins + 15) / 16;
@@ -884,9 +900,7 @@ pl_status enqueue_batch(Lane* L, EngineArgs& A, int persistent, int block, int g
   }
   HIPCHK(hipGetLastError());
   if (timed) HIPCHK(hipEventRecord(L->ev[2], st));
-  if (block == 256) k_window<256><<<dim3(grid), dim3(256), lds, st>>>(A, persistent);
-  else if (block == 512) k_window<512><<<dim3(grid), dim3(512), lds, st>>>(A, persistent);
-  else k_window<1024><<<dim3(grid), dim3(1024), lds, st>>>(A, persistent);
+  wk<<<dim3(grid), dim3(block), lds, st>>>(A, persistent);
   HIPCHK(hipGetLastError());
   if (timed) HIPCHK(hipEventRecord(L->ev[3], st));
   // the deferred columns, the candidates in order, Pass 1 per region
@@ -912,7 +926,7 @@ size_t window_lds_total(int32_t W, int block) {
 
 pl_status run_jobs(pl_ctx* c, Lane* L, const std::vector<JobReq>& reqs, int32_t W, int persistent, int block, bool use_graph) {
   if (reqs.empty()) return fail(PL_E_INVAL, "empty batch");
-  if (W < 64 || W % 64 || W > 2048) return fail(PL_E_INVAL, "window %d must be a multiple of 64 in [64, 2048]", W);
+  if (W < 64 || W % 64 || W > PL_MAX_WINDOW) return fail(PL_E_INVAL, "window %d must be a multiple of 64 in [64, 2048]", W);
   if (block != 256 && block != 512 && block != 1024) return fail(PL_E_INVAL, "block %d must be 256, 512 or 1024", block);
   if (window_lds_total(W, block) > 160 * 1024)
     return fail(PL_E_INVAL, "window %d with block %d needs more than the 160 KB of LDS of a CU", W, block);
@@ -981,7 +995,6 @@ pl_status run_jobs(pl_ctx* c, Lane* L, const std::vector<JobReq>& reqs, int32_t 
   HIPCHK(L->wins.ensure(sizeof(WinDev) * n_wins));
   HIPCHK(L->winwide.ensure(8 * (size_t)n_wins));
   HIPCHK(L->winrec.ensure(8 * (size_t)n_wins));
-  HIPCHK(L->wincur.ensure(4 * (size_t)n_wins));
   HIPCHK(L->heads.ensure(sizeof(WinHead) * (size_t)n_wins));
   HIPCHK(L->cost.ensure((size_t)n_wins));
   HIPCHK(L->bins.ensure(8 * PL_COST_BINS));
@@ -1001,9 +1014,10 @@ pl_status run_jobs(pl_ctx* c, Lane* L, const std::vector<JobReq>& reqs, int32_t 
     L->tables_valid = true;
   }
   const size_t lds = window_lds(W);
-  const void* kfn = block == 256 ? (const void*)k_window<256> : block == 512 ? (const void*)k_window<512>
-                                                                             : (const void*)k_window<1024>;
-  HIPCHK(hipFuncSetAttribute(kfn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  bool lng = false;
+  for (const JobReq& q : reqs) lng = lng || (c->rsets[q.rs] && c->rsets[q.rs]->d.lrt);
+  const WindowKernel wk = window_kernel(block, lng);
+  HIPCHK(hipFuncSetAttribute((const void*)wk, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   int grid = n_wins;
   if (persistent) {
     // workgroups per CU: LDS (dynamic + static run tables) and 32 waves
@@ -1015,7 +1029,7 @@ pl_status run_jobs(pl_ctx* c, Lane* L, const std::vector<JobReq>& reqs, int32_t 
   for (int attempt = 0; attempt < 6; attempt++) {
     HIPCHK(L->rec.ensure(sizeof(IndelRec) * (size_t)L->rec_cap));
     HIPCHK(L->spill.ensure(sizeof(IndelRec) * (size_t)L->spill_cap));
-    HIPCHK(L->spillwin.ensure(4 * (size_t)L->spill_cap));
+    HIPCHK(L->spillat.ensure(8 * (size_t)L->spill_cap));
     HIPCHK(L->cand.ensure(sizeof(Cand) * (size_t)L->cand_cap));
     HIPCHK(L->defer.ensure(4 * (size_t)L->defer_cap));
     HIPCHK(L->mutated.ensure(4 * (size_t)L->mut_cap));
@@ -1041,8 +1055,8 @@ pl_status run_jobs(pl_ctx* c, Lane* L, const std::vector<JobReq>& reqs, int32_t 
     A.st = L->st.as<JobStat>();
     A.hist = L->dhist.as<uint32_t>();
     A.rec = L->rec.as<IndelRec>(); A.rec_n = cnt + PL_N_REC; A.rec_cap = L->rec_cap;
-    A.win_rec = L->winrec.as<uint32_t>(); A.win_cur = L->wincur.as<uint32_t>();
-    A.spill = L->spill.as<IndelRec>(); A.spill_win = L->spillwin.as<uint32_t>();
+    A.win_rec = L->winrec.as<uint32_t>();
+    A.spill = L->spill.as<IndelRec>(); A.spill_at = L->spillat.as<uint2>();
     A.spill_n = cnt + PL_N_SPILL; A.spill_cap = L->spill_cap;
     A.cmask = L->cmask.as<uint64_t>();
     A.prec = L->prec.as<int32_t>();
@@ -1059,11 +1073,12 @@ pl_status run_jobs(pl_ctx* c, Lane* L, const std::vector<JobReq>& reqs, int32_t 
       key.A = A;
       key.W = W; key.block = block; key.persistent = persistent; key.grid = grid; key.lds = lds;
       key.bufs[0] = L->csums.p; key.bufs[1] = L->kparr.p;
+      key.wk = wk;
       if (!L->gexec || L->gkey.size() != sizeof key || std::memcmp(L->gkey.data(), &key, sizeof key) != 0) {
         drop_graph(L);
         HIPCHK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
         EngineArgs Acap = A;
-        pl_status s = enqueue_batch(L, Acap, persistent, block, grid, lds, false);
+        pl_status s = enqueue_batch(L, Acap, wk, persistent, block, grid, lds, false);
         hipGraph_t g = nullptr;
         const hipError_t e = hipStreamEndCapture(st, &g);
         if (s) { if (g) (void)hipGraphDestroy(g); return s; }
@@ -1079,7 +1094,7 @@ pl_status run_jobs(pl_ctx* c, Lane* L, const std::vector<JobReq>& reqs, int32_t 
       HIPCHK(hipEventRecord(L->ev[1], st));
     } else {
       HIPCHK(hipEventRecord(L->ev[0], st));
-      pl_status s = enqueue_batch(L, A, persistent, block, grid, lds, true);
+      pl_status s = enqueue_batch(L, A, wk, persistent, block, grid, lds, true);
       if (s) return s;
       HIPCHK(hipEventRecord(L->ev[1], st));
     }

@@ -114,11 +114,6 @@ __device__ __forceinline__ T wave_total_dpp(T v) { return lane63(wave_scan_dpp(v
 }  // namespace
 
 // ------------------------------------------------------------------ k_prep
-// segments are built for multi-op reads (not RI_SIMPLE) that addRead processes
-PL_HD bool wants_segs(uint32_t info) {
-  return (info & RI_KEEP) && !(info & (RI_SIMPLE | RI_EXOTIC | RI_BAD | RI_LR_MASK));
-}
-
 // the read set's scalars (scal[0], [1], [2], [6]: maxima, -1 = none;
 // flags: scal[4], scal[5]) gathered over a thread's reads, then over its
 // wave, so one wave gives one atomic per scalar
@@ -157,7 +152,7 @@ __device__ __forceinline__ void prep_one(const RSDev& R, int64_t r, const KConf&
     const int64_t L = R.seq_off[r + 1] - R.seq_off[r];
     for (int64_t k = 0; k < L; k++) qd[k] = (int8_t)cf.default_qual;
   }
-  segcount[r] = wants_segs(m.info) ? (uint32_t)build_segs(R, r, m.info, cf, nullptr) : 0u;
+  segcount[r] = seg_slots(R, r, m.info, cf);
   const bool keep = (m.info & RI_KEEP) != 0;
   if (keep) {
     int64_t lo = INT64_MAX, hi = INT64_MIN;
@@ -168,7 +163,7 @@ __device__ __forceinline__ void prep_one(const RSDev& R, int64_t r, const KConf&
     }
     if (lo <= hi) {
       const int64_t lead = m.pos - lo, back = hi - m.pos;
-      if (lead > PL_MAX_LEAD || back > PL_MAX_BACK || R.seq_off[r + 1] - R.seq_off[r] >= PL_MAX_SEQ) {
+      if (lead > PL_MAX_LEAD || back > (R.all_long ? PL_MAX_BACK_LONG : PL_MAX_BACK) || R.seq_off[r + 1] - R.seq_off[r] >= PL_MAX_SEQ) {
         m.info |= RI_OUTLIER;
         int k = atomicAdd(&scal[3], 1);
         if (k < out_cap) outliers[k] = r;
@@ -222,15 +217,14 @@ __global__ void k_prep_sets(const RSDev* sets, const int64_t* blk, int32_t n_set
 }
 
 // fills the segment table; RMeta.op0 of a multi-op read becomes its first
-// segment and the info word carries the count (RI_SEG_MAX = too many: walked)
+// entry and the info word carries the count (RI_SEG_MAX = too many: walked)
 __device__ __forceinline__ void segfill_one(const RSDev& R, int64_t r, const KConf& cf, const uint32_t* segoff,
                                             Seg* segs) {
   RMeta m = R.meta[r];
   if (!wants_segs(m.info)) return;
   const uint32_t o = segoff[r], c = segoff[r + 1] - o;
-  if (c) build_segs(R, r, m.info, cf, segs + o);
+  m.info = seg_fill(R, r, m.info, cf, segs, o, c);
   m.op0 = o;
-  m.info = (m.info & ~RI_SEG_MASK) | ((c < RI_SEG_MAX ? c : (uint32_t)RI_SEG_MAX) << RI_SEG_SHIFT);
   R.meta[r] = m;
 }
 
@@ -515,11 +509,12 @@ struct LdsSink {
   uint32_t *bad_, *clp_;
   int32_t *pc, *is;
   IndelRec* spill;
-  uint32_t* spill_win;
+  uint2* spill_at;
   uint32_t* spill_n;
   uint32_t spill_cap;
   int32_t wi;
-  IndelRec* lrec;        // the window's record buffer in LDS (PL_WIN_RECS)
+  IndelRec* lrec;        // the window's record buffer in LDS
+  uint32_t lrec_cap;
   uint32_t* lrec_n;
   int32_t* overflow;
   JobStat* st;
@@ -534,12 +529,12 @@ struct LdsSink {
   __device__ void bad(int p, int n) { atomicAdd(&bad_[p], (uint32_t)n); }
   __device__ void clip(int p) { atomicAdd(&clp_[p], 1u); }
   // records collect in LDS and reach HBM together at the window's end; a
-  // window with more than PL_WIN_RECS spills the rest (k_spill_place)
+  // window with more than fit spills the rest (k_spill_place)
   __device__ void emit(const IndelRec& e) {
     const uint32_t j = atomicAdd(lrec_n, 1u);
-    if (j < PL_WIN_RECS) { lrec[j] = e; return; }
+    if (j < lrec_cap) { lrec[j] = e; return; }
     const uint32_t i = atomicAdd(spill_n, 1u);
-    if (i < spill_cap) { spill[i] = e; spill_win[i] = (uint32_t)wi; }
+    if (i < spill_cap) { spill[i] = e; spill_at[i] = make_uint2((uint32_t)wi, j); }
     else *overflow = 1;
   }
   __device__ void ins(int p, int32_t q, int32_t mq1, const IndelRec& e) {
@@ -577,6 +572,51 @@ __device__ __forceinline__ int64_t uniform64(int64_t v) {
 
 }  // namespace
 
+// The segments of a long read (n from sg) that can touch a window: the first
+// whose reference span ends at or after L0 in *first, and how many follow
+// with their locus below x (both ascend).  An aligned group of 16 lanes a
+// read, all 64 lanes of the wave active; both searches probe together.
+__device__ __forceinline__ int32_t long_seg_range(const Seg* sg, uint32_t n, int32_t L0, int64_t x, int lane,
+                                                  uint32_t* first) {
+  static_assert(PL_LONG_READS == 4, "16 lanes a read");
+  const int gl = lane & 15, g0 = lane & 48;
+  uint32_t lo[2] = {0, 0}, hi[2] = {n, n};
+  while (__ballot(hi[0] - lo[0] > 16u || hi[1] - lo[1] > 16u)) {
+    bool less[2];
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+      const uint32_t m = hi[k] - lo[k];
+      less[k] = false;
+      if (m > 16u) {
+        const Seg& g = sg[lo[k] + (uint32_t)((uint64_t)(gl + 1) * m / 17)];
+        less[k] = k == 0 ? seg_end(g) < L0 : (int64_t)seg_key(g) < x;
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+      const uint64_t m = hi[k] - lo[k];
+      const int c = __popcll((__ballot(less[k]) >> g0) & 0xffffull);
+      const uint32_t a = lo[k];
+      if (m > 16u) {
+        if (c > 0) lo[k] = a + (uint32_t)(c * m / 17) + 1;
+        if (c < 16) hi[k] = a + (uint32_t)((c + 1) * m / 17);
+      }
+    }
+  }
+  uint32_t at[2];
+#pragma unroll
+  for (int k = 0; k < 2; k++) {
+    bool less = false;
+    if (lo[k] + gl < hi[k]) {
+      const Seg& g = sg[lo[k] + gl];
+      less = k == 0 ? seg_end(g) < L0 : (int64_t)seg_key(g) < x;
+    }
+    at[k] = lo[k] + (uint32_t)__popcll((__ballot(less) >> g0) & 0xffffull);
+  }
+  *first = at[0];
+  return at[1] > at[0] ? (int32_t)(at[1] - at[0]) : 0;
+}
+
 // One workgroup owns a window of W positions; every counter of those
 // positions lives in LDS until the window is done.  Reads are taken in tiles
 // of BLOCK (one per thread): the headers of a tile are loaded in parallel,
@@ -587,7 +627,9 @@ __device__ __forceinline__ int64_t uniform64(int64_t v) {
 // through walk_read, one wave per read.
 static_assert(PL_CHUNK % 2 == 1 && PL_CHUNK <= 31, "an odd chunk of at most 31 bases (two 16-base words)");
 
-template <int BLOCK>
+// LONG: the batch's read sets hold long reads (their segments and the
+// nanopore base rule cost the other batches' kernel seven spilled registers).
+template <int BLOCK, bool LONG>
 __global__ void __launch_bounds__(BLOCK, PL_WIN_WAVES_EU) k_window(EngineArgs A, int persistent) {
   constexpr int NW = BLOCK / 64;
   extern __shared__ __align__(16) unsigned long long lds[];
@@ -607,8 +649,12 @@ __global__ void __launch_bounds__(BLOCK, PL_WIN_WAVES_EU) k_window(EngineArgs A,
   __shared__ int32_t ws_a[NW], ws_b[NW], ws_c[NW];
   __shared__ unsigned long long red[2][NW];
   __shared__ int32_t s_ovf;
-  __shared__ IndelRec s_rec[PL_WIN_RECS];
+  // (the bit tables of a long-read window take the room of 24 records)
+  constexpr uint32_t RECS = LONG ? PL_WIN_RECS - 24 : PL_WIN_RECS;
+  __shared__ IndelRec s_rec[RECS];
   __shared__ uint32_t s_nrec, s_recbase;
+  // a bit per position: nanopore_exclude, and homo_run4 at its region index
+  __shared__ uint64_t s_nx[LONG ? PL_MAX_WINDOW / 64 + 1 : 1], s_hx[LONG ? PL_MAX_WINDOW / 64 : 1];
   // the current window's head and the next one's, fetched while the
   // current window is piled (persistent form), with their queue slots
   __shared__ WinHead s_head[2];
@@ -656,33 +702,51 @@ __global__ void __launch_bounds__(BLOCK, PL_WIN_WAVES_EU) k_window(EngineArgs A,
       if ((lds_words & 1) && tid == 0) lds[lds_words - 1] = 0ull;
     }
     if (tid == 0) { s_ovf = 0; s_nrec = 0; }
+    const bool nano = LONG && R.nano != 0;
+    if constexpr (LONG) {
+      for (int q0 = 64 * wave; q0 < W; q0 += BLOCK) {
+        const bool in = q0 + lane < nW;
+        const uint64_t xm = __ballot(in && nano && nanopore_exclude(R, J, (int64_t)win.p0 + q0 + lane));
+        const uint64_t hm = __ballot(in && homo_run4(R, (int64_t)win.p0 + q0 + lane));
+        if (lane == 0) { s_nx[q0 >> 6] = xm; s_hx[q0 >> 6] = hm; }
+      }
+      if (tid == 0) s_nx[W >> 6] = 0;
+    }
+    auto lr_drop = [&](uint32_t lr, int32_t dl) {
+      const int d = dl - L0;
+      return ((s_hx[d >> 6] | (lr == PL_LR_NANOPORE ? s_nx[d >> 6] : 0ull)) >> (d & 63) & 1ull) != 0;
+    };
     __syncthreads();
 
     LdsSink sk;
     sk.W = W; sk.bs = bs; sk.mqq = mqq; sk.ins_ = insA; sk.del_ = delA; sk.bad_ = badA; sk.clp_ = clpA;
-    sk.pc = pcA; sk.is = isA; sk.spill = A.spill; sk.spill_win = A.spill_win; sk.spill_n = A.spill_n;
+    sk.pc = pcA; sk.is = isA; sk.spill = A.spill; sk.spill_at = A.spill_at; sk.spill_n = A.spill_n;
     sk.spill_cap = A.spill_cap; sk.wi = wi;
-    sk.lrec = s_rec; sk.lrec_n = &s_nrec;
+    sk.lrec = s_rec; sk.lrec_cap = RECS; sk.lrec_n = &s_nrec;
     sk.overflow = A.overflow; sk.st = &A.st[win.job]; sk.bcount = 0; sk.aligned_n = 0;
 
     // Each wave takes its own chunks of 64 reads (wave-strided over the
     // window's read range): staging, the run scan and the base loop are
-    // wave-local, so the read loop has no workgroup barrier.
+    // wave-local, so the read loop has no workgroup barrier.  In a set of
+    // long reads a chunk is PL_LONG_READS reads: a window has about a hundred
+    // of them, and 64 to a wave left three of four waves idle.
     RunL* wrun = s_run + wave * (2 * 64 + 1);
+    const int CR = LONG && R.all_long ? PL_LONG_READS : 64;
+    const bool stager = lane < CR;
     // the next chunk's read facts are loaded while the current one is piled
-    int64_t t0 = win.plo + 64 * wave;
+    int64_t t0 = win.plo + CR * wave;
     RMeta mN;
     int64_t sN = 0, eN = 0, qN = 0;
     mN.info = 0;
-    if (t0 + lane < win.hi) { mN = gm[t0 + lane]; sN = gso[t0 + lane]; eN = gso[t0 + lane + 1]; }
+    if (stager && t0 + lane < win.hi) { mN = gm[t0 + lane]; sN = gso[t0 + lane]; eN = gso[t0 + lane + 1]; }
     if (t0 < win.hi) qN = gso[t0];
-    for (; t0 < win.hi; t0 += BLOCK) {
+    for (; t0 < win.hi; t0 += CR * NW) {
       const int64_t qbase = qN;
       const RMeta m = mN;
       const int64_t seq0 = sN, seqE = eN;
       {
-        const int64_t tn = t0 + BLOCK;
-        if (tn + lane < win.hi) { mN = gm[tn + lane]; sN = gso[tn + lane]; eN = gso[tn + lane + 1]; }
+        const int64_t tn = t0 + CR * NW;
+        if (stager && tn + lane < win.hi) { mN = gm[tn + lane]; sN = gso[tn + lane]; eN = gso[tn + lane + 1]; }
         if (tn < win.hi) qN = gso[tn];
       }
       // ---- stage: one read per lane.  A simple read gives at most one run;
@@ -693,17 +757,18 @@ __global__ void __launch_bounds__(BLOCK, PL_WIN_WAVES_EU) k_window(EngineArgs A,
       Run ru0;
       ru0.n = 0;
       int nrun = 0;
-      bool cplx = false, segr = false;
+      bool cplx = false, segr = false, lng = false;
       uint32_t rinfo = 0, rop0 = 0;   // facts of a segmented read, for the lanes that apply its segments
       int64_t rseq0 = 0;
-      if (r < win.hi) {
+      if (stager && r < win.hi) {
         if (!(m.info & RI_OUTLIER) && read_in_query(m, J)) {
           frag_event(m, J, L0, L1, sk);
           if (m.fp_hi >= L0 && m.fp_lo < L1) {
             if (seq0 - qbase >= PL_TILE_SPAN) cplx = true;
             else if (m.info & RI_SIMPLE) nrun = simple_run(m, seq0, cf, L0, L1, &ru0, &sk.aligned_n, &sk.bcount);
             else if (!(m.info & RI_EXOTIC) && ((m.info & RI_SEG_MASK) >> RI_SEG_SHIFT) < RI_SEG_MAX) {
-              segr = true;
+              lng = LONG && (m.info & RI_LR_MASK) != 0;
+              segr = !lng;
               rinfo = m.info; rop0 = m.op0; rseq0 = seq0;
             } else {
               cplx = true;
@@ -711,7 +776,7 @@ __global__ void __launch_bounds__(BLOCK, PL_WIN_WAVES_EU) k_window(EngineArgs A,
           }
         }
       }
-      const int32_t rlen = segr ? (int32_t)(seqE - rseq0) : 0;
+      const int32_t rlen = segr || lng ? (int32_t)(seqE - rseq0) : 0;
       // a run that only adds badPair over a range (M bases of an invalid
       // read) goes to the difference array, not to the base loop
       if (nrun > 0 && (ru0.fl & EF_BAD)) {
@@ -757,7 +822,7 @@ __global__ void __launch_bounds__(BLOCK, PL_WIN_WAVES_EU) k_window(EngineArgs A,
           continue;
         }
         Run ru;
-        int got = has ? seg_apply(J, cf, t0 + own, info, s0, Lc, L0, L1, g, ru, &sk.aligned_n, &sk.bcount, sk) : 0;
+        int got = has ? seg_apply(R, J, cf, t0 + own, info, s0, Lc, L0, L1, g, ru, &sk.aligned_n, &sk.bcount, sk, lr_drop) : 0;
         if (got && (ru.fl & EF_BAD)) {
           atomicAdd(&bdA[ru.p0], 1);
           if (ru.p0 + ru.n < nW) atomicAdd(&bdA[ru.p0 + ru.n], -1);
@@ -792,8 +857,16 @@ __global__ void __launch_bounds__(BLOCK, PL_WIN_WAVES_EU) k_window(EngineArgs A,
         Cc = lane63(ci);
         if (lane < ncr) wrun[Es + lane] = RunL{Cs + ci - cn, cr.pi, cr.q0, cr.off};
       }
-      const int32_t E = Es + ncr;
-      const int32_t CT = Cs + Cc;
+      int32_t E = Es + ncr;
+      int32_t CT = Cs + Cc;
+      // The chunk's long reads follow, PL_LONG_READS at a time and 64 of
+      // their segments a round: the runs of each round are a run table of
+      // their own for the base loop below.  16 lanes hold one read's facts.
+      uint64_t pendl = __ballot(lng);
+      int lsrc = 0;
+      uint32_t linfo = 0, lfirst = 0;
+      int32_t lat = 0, ltot = 0, lp1 = 0, lp2 = 0, lp3 = 0;
+      for (;;) {
       if (lane == 0) wrun[E] = RunL{CT, 0u, 0, 0};
       // LDS operations of one wave complete in order: the table written
       // above is what the loop below reads
@@ -862,6 +935,14 @@ __global__ void __launch_bounds__(BLOCK, PL_WIN_WAVES_EU) k_window(EngineArgs A,
           uint32_t x[PL_CHUNK / 16 + 1];
 #pragma unroll
           for (int k = 0; k < PL_CHUNK / 16 + 1; k++) x[k] = __builtin_amdgcn_alignbit(bw[k + 1], bw[k], 2u * (qq & 15u));
+          if (nano) {
+            // nanopore bases inside CC_GG pile with quality 0: four mask bits to four bytes at a time
+            const uint32_t* nx = (const uint32_t*)s_nx + (p >> 5);
+            const uint32_t xb = (ru.pi & EF_NANO) && act ? __builtin_amdgcn_alignbit(nx[1], nx[0], (uint32_t)p & 31u) : 0u;
+#pragma unroll
+            for (int k = 0; k < PL_CHUNK / 4 + 1; k++)
+              w[k] &= ~((((xb >> (4 * k)) & 15u) * 0x00204081u & 0x01010101u) * 255u);
+          }
           // the next batch: its runs, and its loads
           int rrn = rr;
           uint32_t qn = 0u;
@@ -897,6 +978,65 @@ __global__ void __launch_bounds__(BLOCK, PL_WIN_WAVES_EU) k_window(EngineArgs A,
           cur = lane63(rr);
           rr = rrn;
         }
+      }
+      if constexpr (!LONG) break;
+      // ---- the next round of a long read's segments
+      E = CT = 0;
+      bool more = true;
+      while (more && E == 0) {
+        if (lat >= ltot) {
+          if (!pendl) { more = false; break; }
+          int own = -1;
+#pragma unroll
+          for (int j = 0; j < PL_LONG_READS; j++) {
+            const int l = pendl ? __ffsll((unsigned long long)pendl) - 1 : -1;
+            if ((lane >> 4) == j) own = l;
+            pendl &= pendl - 1;
+          }
+          lsrc = own < 0 ? 0 : own;
+          linfo = (uint32_t)__shfl((int)rinfo, lsrc, 64);
+          const uint32_t o = (uint32_t)__shfl((int)rop0, lsrc, 64);
+          uint32_t lo = 0, n = 0;
+          int32_t reach = 0;
+          if (own >= 0) { const Seg h = R.segs[o]; n = (uint32_t)h.len; reach = h.fin; }
+          lfirst = o + 1;
+          const int32_t cnt = long_seg_range(R.segs + lfirst, n, L0, (int64_t)L1 + reach, lane, &lo);
+          lfirst += lo;
+          const int32_t c0 = __builtin_amdgcn_readlane(cnt, 0), c1 = __builtin_amdgcn_readlane(cnt, 16),
+                        c2 = __builtin_amdgcn_readlane(cnt, 32), c3 = __builtin_amdgcn_readlane(cnt, 48);
+          lat = 0;
+          lp1 = c0; lp2 = lp1 + c1; lp3 = lp2 + c2; ltot = lp3 + c3;
+          continue;
+        }
+        const int32_t t = lat + lane;
+        const bool has = t < ltot;
+        const int j = (t >= lp1) + (t >= lp2) + (t >= lp3);
+        const int from = 16 * j;
+        const int src = __shfl(lsrc, from, 64);
+        const uint32_t info = (uint32_t)__shfl((int)linfo, from, 64);
+        const uint32_t at = (uint32_t)__shfl((int)lfirst, from, 64) + (uint32_t)(t - (j == 0 ? 0 : j == 1 ? lp1 : j == 2 ? lp2 : lp3));
+        const int64_t s0 = ((int64_t)__shfl((int)(rseq0 >> 32), src, 64) << 32) |
+                           (uint32_t)__shfl((int)(uint32_t)rseq0, src, 64);
+        const int32_t Lc = __shfl(rlen, src, 64);
+        lat += 64;
+        Seg g;
+        if (has) g = R.segs[at];
+        Run ru;
+        ru.n = 0;
+        int got = has ? seg_apply(R, J, cf, t0 + src, info, s0, Lc, L0, L1, g, ru, &sk.aligned_n, &sk.bcount, sk, lr_drop) : 0;
+        if (got && (ru.fl & EF_BAD)) {
+          atomicAdd(&bdA[ru.p0], 1);
+          if (ru.p0 + ru.n < nW) atomicAdd(&bdA[ru.p0 + ru.n], -1);
+          got = 0;
+        }
+        const uint64_t lv = got ? (1ull << 32) + (uint64_t)((ru.n + PL_CHUNK - 1) / PL_CHUNK) : 0ull;
+        const uint64_t li = wave_scan_dpp(lv), lt = lane63(li);
+        if (got) wrun[(int32_t)((li - lv) >> 32)] =
+            RunL{(int32_t)(uint32_t)(li - lv), (uint32_t)ru.p0 | ru.fl, (int32_t)(ru.q - qbase) + qsh, ru.n};
+        E = (int32_t)(lt >> 32);
+        CT = (int32_t)(uint32_t)lt;
+      }
+      if (!more) break;
       }
       // ---- everything else about the chunk's complex reads, one at a time
       for (uint64_t cm = __ballot(cplx); cm; cm &= cm - 1) {
@@ -963,13 +1103,12 @@ __global__ void __launch_bounds__(BLOCK, PL_WIN_WAVES_EU) k_window(EngineArgs A,
     // the window's evidence records, in one segment of the batch's: one
     // atomic, coalesced 32-byte stores (room for the spilled ones at its end)
     {
-      const uint32_t nt = s_nrec, nl = nt < PL_WIN_RECS ? nt : PL_WIN_RECS;
+      const uint32_t nt = s_nrec, nl = nt < RECS ? nt : RECS;
       if (tid == 0) {
         const uint32_t base = nt ? atomicAdd(A.rec_n, nt) : 0u;
         s_recbase = base;
         A.win_rec[2 * wi] = base;
         A.win_rec[2 * wi + 1] = nt;
-        A.win_cur[wi] = 0;
         if (nt && base + nt > A.rec_cap) *A.overflow = 1;
       }
       __syncthreads();
@@ -1064,18 +1203,21 @@ __global__ void __launch_bounds__(BLOCK, PL_WIN_WAVES_EU) k_window(EngineArgs A,
   }
 }
 
-template __global__ void k_window<256>(EngineArgs, int);
-template __global__ void k_window<512>(EngineArgs, int);
-template __global__ void k_window<1024>(EngineArgs, int);
+template __global__ void k_window<256, false>(EngineArgs, int);
+template __global__ void k_window<512, false>(EngineArgs, int);
+template __global__ void k_window<1024, false>(EngineArgs, int);
+template __global__ void k_window<256, true>(EngineArgs, int);
+template __global__ void k_window<512, true>(EngineArgs, int);
+template __global__ void k_window<1024, true>(EngineArgs, int);
 
 // ------------------------------------------------------------------ records
-// Spilled records into their windows' segments: behind the ones the window
-// kept in LDS, in any order (a column's records are counted, never ordered).
+// Spilled records into their windows' segments, each at the place it took
+// among the window's records when it was found.
 __global__ void __launch_bounds__(256) k_spill_place(EngineArgs A) {
   const uint32_t n = *A.spill_n < A.spill_cap ? *A.spill_n : A.spill_cap;
   for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-    const uint32_t w = A.spill_win[i];
-    const uint32_t k = A.win_rec[2 * w] + PL_WIN_RECS + atomicAdd(&A.win_cur[w], 1u);
+    const uint2 at = A.spill_at[i];
+    const uint32_t k = A.win_rec[2 * at.x] + at.y;
     if (k < A.rec_cap) A.rec[k] = A.spill[i];
   }
 }

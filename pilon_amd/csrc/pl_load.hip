@@ -452,7 +452,11 @@ pl_status loader_finish(pl_loader* ld, int32_t nref, const int32_t* contig_ids, 
     d.exo_off = (const int64_t*)(U + o_exo) + T(r, 2);
     d.nib = U + o_nib + T(r, 3);
     d.n_exotic = (int64_t)(T(r + 1, 2) - T(r, 2));
-    if (lr) d.lrt = U + o_lrt + f;
+    if (lr) {
+      d.lrt = U + o_lrt + f;
+      d.all_long = 1;
+      d.nano = bam_type == PL_BAM_NANOPORE;
+    }
     rs.push_back(std::move(R));
     ncig.push_back((int64_t)(T(r + 1, 0) - T(r, 0)));
     nb.push_back((int64_t)(T(r + 1, 1) - T(r, 1)));

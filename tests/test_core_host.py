@@ -102,3 +102,24 @@ def test_edge_detected_by_core_host():
     case = K.case_insertion_rotation(start=14)
     got = CH.run(default_config(), case["ref"].encode(), K.batch_of(case), [(14, 40)], W=64)[0]
     assert got["status"] == 4
+
+
+@pytest.mark.parametrize("read_len", [700, 9500])
+@pytest.mark.parametrize("lr,W", [("nanopore", 64), ("pacbio", 512)])
+def test_long_reads_by_segments_core_host(read_len, lr, W):
+    """Reads of many windows piled by the segments each window can touch."""
+    from pilon_amd.abi import BAM_TYPES
+    from tests.test_gpu_longread import long_data
+    name, draft, b = long_data(read_len, 7 + read_len)
+    cfg = default_config(longread=1, min_qual=3)
+    lrt = np.full(b.n, K.LR_TYPE[lr], np.uint8)
+    regions = [(1, len(draft)), (1001, 9000)]
+    got = CH.run(cfg, draft, b, regions, W=W, name=name, lrt=lrt, set_kinds=2 if lr == "nanopore" else 0)
+    assert any(g["status"] == 0 for g in got)
+    for (s, e), g in zip(regions, got):
+        ref = oracle().run_region(cfg, draft, s, e, [b], name=name, set_types=[BAM_TYPES[lr]])
+        assert g["status"] == ref["status"]
+        if g["status"] == 0:
+            assert_same_region(g["pile"], g["calls"], ref, f"{lr} {s}-{e}")
+            assert_same_stats(g["stats"], ref["stats"])
+            assert g["changes"] == ref["changes"] and g["bases"] == ref["bases"]

@@ -81,3 +81,58 @@ def test_frags_and_nanopore_region():
             assert changes == ref["changes"] and bases == ref["bases"]
     finally:
         ctx.close()
+
+
+def long_data(read_len, seed):
+    """A contig with homopolymer and tandem runs (indels slide far) under
+    unpaired reads of read_len, an indel every 30 bases, some clipped, some
+    with N (walked)."""
+    from pilon_amd.reads import ReadBatch
+    from pilon_amd.synth import SynthData, preset
+    p = preset("c1", scale=0.4, seed=seed)
+    p.update(read_len=read_len, insert_mean=read_len, insert_sd=0, coverage=15, err_indel_rate=0.03, err_indel_max=3,
+             sub_rate=0.02, clip_frac=0.3, clip_min=5, clip_max=400, n_rate=2e-5, qual_lo=0, qual_hi=25, repeat_copies=3,
+             repeat_len=2000)
+    d = SynthData(p)
+    b = d.batch(0)
+    b = ReadBatch(b.pos, np.zeros_like(b.tlen), b.flag & 0xA010, b.mapq, b.cigar_off, b.cigar, b.seq_off, b.bases2,
+                  b.quals, b.exo_read, b.exo_off, b.nib)
+    draft = bytearray(d.draft(0))
+    for k in range(40):                       # runs the reads' indels are normalised along
+        a = 500 + 900 * k
+        draft[a:a + 70] = (b"A" * 70 if k % 3 == 0 else b"CAG" * 23 + b"C" if k % 3 == 1 else b"CCAGG" * 14)
+    return d.names[0], bytes(draft), b
+
+
+@pytest.mark.parametrize("read_len", [700, 3001, 9500])
+@pytest.mark.parametrize("lr,window,block", [("nanopore", 512, 256), ("pacbio", 64, 512), ("nanopore", 1024, 1024)])
+def test_long_reads_by_segments(read_len, lr, window, block):
+    """Reads of many windows, whose segments each window takes its own part
+    of: read lengths below and above the short sets' scan margin, windows of
+    one and several chunks of reads."""
+    from oracle import oracle as O
+    from pilon_amd.engine import Context, contig_regions
+    print(f"case: {lr} reads of {read_len}, window {window}", flush=True)
+    name, draft, b = long_data(read_len, 7 + read_len)
+    cfg = default_config(longread=1, min_qual=3)
+    ctx = Context(cfg, device=0)
+    try:
+        ctx.ref_upload(0, name, draft)
+        rid = ctx.readset_upload(0, b, bam_type=lr)
+        rid2 = ctx.readset_upload_many([(0, b, lr)])[0]
+        regions = [(1, len(draft)), (1001, 9000)]
+        want = [O.run_region(cfg, draft, s, e, [b], name=name, set_types=[BAM_TYPES[lr]]) for s, e in regions]
+        regions = [x for x, w in zip(regions, want) if w["status"] == 0]
+        want = [w for w in want if w["status"] == 0]
+        assert want
+        for ids in (rid, rid2):
+            pile, calls, stats = ctx.batch_run([(0, s, e, ids) for s, e in regions], window=window, block=block,
+                                               persistent=1)
+            off = 0
+            for (s, e), st, w in zip(regions, stats, want):
+                n = e - s + 1
+                assert_same_region(pile[:, off:off + n], calls[off:off + n], w, f"{lr} {s}-{e}")
+                assert_same_stats(st, w["stats"], f"{lr} {s}-{e}")
+                off += n
+    finally:
+        ctx.close()
