@@ -437,7 +437,7 @@ plh::Outcome log_fix(const std::string& name, int32_t rs, int32_t re, const AsmF
 // The issue regions of a finished region (gaps, possible breaks).
 pl_status region_issue_lists(pl_region* r, std::vector<std::pair<int32_t, int32_t>> lists[7]) {
   return on_region_lane(r, [&](pl_ctx* c, Lane* L, const std::vector<std::string>&, const std::vector<int32_t>& contigs) {
-    VcfBufs B;
+    ScratchBufs B(L);
     TrackArgs T;
     double ms = 0;
     if (pl_status s = tracks_of_lane(c, L, contigs, B, T, &ms, true)) return s;

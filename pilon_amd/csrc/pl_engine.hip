@@ -87,6 +87,48 @@ struct DBuf {
   template <class T> T* as() const { return (T*)p; }
 };
 
+// Device memory of passes that need scratch for one call (VCF, tracks,
+// K-mers): blocks handed out by bumping an offset and taken back when the
+// call ends (ScratchBufs), kept for the lane's next call up to
+// PL_SCRATCH_KEEP.  A call's hipMalloc and hipFree of its dozen buffers took
+// longer than its kernels on small batches.
+#define PL_SCRATCH_KEEP ((size_t)2 << 30)
+struct Scratch {
+  struct Block { uint8_t* p; size_t n; };
+  std::vector<Block> blocks;
+  size_t at = 0, used = 0;         // the block in use and how much of it
+  size_t want = 0;                 // size of the next first block
+  void* top = nullptr;             // the innermost ScratchBufs alive
+  hipError_t get(size_t bytes, void** out) {
+    bytes = (std::max<size_t>(bytes, 1) + 255) & ~(size_t)255;
+    while (at < blocks.size() && bytes > blocks[at].n - used) { at++; used = 0; }
+    if (at == blocks.size()) {
+      Block b{nullptr, std::max(bytes, blocks.empty() && want ? want : (size_t)1 << 20)};
+      const hipError_t e = hipMalloc((void**)&b.p, b.n);
+      if (e != hipSuccess) return e;
+      blocks.push_back(b);
+      used = 0;
+    }
+    *out = blocks[at].p + used;
+    used += bytes;
+    return hipSuccess;
+  }
+  void release() {
+    for (Block& b : blocks) (void)hipFree(b.p);
+    blocks.clear();
+    at = used = 0;
+  }
+  // nothing in use any more: many blocks become one next time, and none is
+  // kept above the bound
+  void settle() {
+    size_t t = 0;
+    for (const Block& b : blocks) t += b.n;
+    at = used = 0;
+    if (t > PL_SCRATCH_KEEP) { want = 0; release(); }
+    else if (blocks.size() > 16) { want = t; release(); }
+  }
+};
+
 struct Contig {
   std::string name;
   std::vector<uint8_t> host;
@@ -183,6 +225,7 @@ struct Lane {
   hipEvent_t stage_ev[2] = {nullptr, nullptr};
   // pinned slots for the counters of repeated passes (pl_batch_repeat)
   uint32_t* rep_hc = nullptr;
+  Scratch scratch;
   // depth of the batch's "jumps" reads before Pass 1, per position, which
   // fragment coverage leaves out (valid for the last batch when set)
   DBuf jdepth;
@@ -303,32 +346,23 @@ pl_status scan_u32(Lane* L, const uint32_t* in, uint32_t* out, int64_t n) {
   return PL_OK;
 }
 
-// LSD radix sort of (key, val) pairs whose count is in device memory;
-// returns in *rk/*rv the buffers holding the sorted result.
-pl_status radix_sort(Lane* L, uint32_t* k, uint32_t* v, uint32_t* tk, uint32_t* tv, const uint32_t* n_dev,
-                     uint32_t cap, int bits, uint32_t** rk, uint32_t** rv) {
-  const int32_t nb = (int32_t)std::max<int64_t>(1, ((int64_t)cap + RS_TILE - 1) / RS_TILE);
-  HIPCHK(L->hist.ensure(sizeof(uint32_t) * ((size_t)256 * nb + 1)));
-  uint32_t *ik = k, *iv = v, *ok = tk, *ov = tv;
-  const int passes = std::max(1, (bits + 7) / 8);
-  for (int p = 0; p < passes; p++) {
-    k_rs_hist<<<dim3(nb), dim3(256), 0, L->stream>>>(ik, n_dev, cap, 8 * p, L->hist.as<uint32_t>(), nb);
-    pl_status s = scan_u32(L, L->hist.as<uint32_t>(), L->hist.as<uint32_t>(), (int64_t)256 * nb);
-    if (s) return s;
-    k_rs_scatter<<<dim3(nb), dim3(256), 0, L->stream>>>(ik, iv, ok, ov, n_dev, cap, 8 * p, L->hist.as<uint32_t>(), nb);
-    HIPCHK(hipGetLastError());
-    std::swap(ik, ok);
-    std::swap(iv, ov);
-  }
-  *rk = ik;
-  *rv = iv;
-  return PL_OK;
-}
+// records of a radix sort: a 64-bit key and a value, as three arrays
+struct SortRecs { uint32_t *lo, *hi, *v; };
 
-int bits_for(uint64_t maxkey) {
-  int b = 0;
-  while (b < 32 && (maxkey >> b)) b++;
-  return std::max(b, 1);
+// Stable LSD radix sort of n records by the low `bits` bits of their keys;
+// a is where they are, b room for as many; a holds the result.
+pl_status radix_sort(Lane* L, SortRecs& a, SortRecs& b, uint32_t n, int bits) {
+  const int32_t nb = (int32_t)std::max<int64_t>(1, ((int64_t)n + RS_TILE - 1) / RS_TILE);
+  HIPCHK(L->hist.ensure(sizeof(uint32_t) * ((size_t)256 * nb + 1)));
+  uint32_t* h = L->hist.as<uint32_t>();
+  for (int shift = 0; shift < bits; shift += 8) {
+    k_rs_hist<<<dim3(nb), dim3(256), 0, L->stream>>>(a.lo, a.hi, n, shift, h, nb);
+    if (pl_status s = scan_u32(L, h, h, (int64_t)256 * nb)) return s;
+    k_rs_scatter<<<dim3(nb), dim3(256), 0, L->stream>>>(a.lo, a.hi, a.v, b.lo, b.hi, b.v, n, shift, h, nb);
+    HIPCHK(hipGetLastError());
+    std::swap(a, b);
+  }
+  return PL_OK;
 }
 
 void to_kconf(const pl_config& p, KConf& k) {
@@ -861,6 +895,7 @@ void lane_destroy(Lane* L) {
   if (L->stream) (void)hipStreamSynchronize(L->stream);
   drop_graph(L);
   L->free_buffers();
+  L->scratch.release();
   for (int k = 0; k < 2; k++) {
     if (L->stage_ev[k]) (void)hipEventDestroy(L->stage_ev[k]);
     if (L->stage[k]) (void)hipHostFree(L->stage[k]);

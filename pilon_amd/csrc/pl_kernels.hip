@@ -1223,58 +1223,106 @@ __global__ void __launch_bounds__(256) k_spill_place(EngineArgs A) {
 }
 
 // ------------------------------------------------------------------ radix sort
-__global__ void __launch_bounds__(256) k_rs_hist(const uint32_t* keys, const uint32_t* n_ptr, uint32_t cap, int shift,
+// One stable 8-bit pass of an LSD sort of (hi:lo, v) records held as three
+// arrays: digits per tile (k_rs_hist), the scan of digit-major counts, and
+// the scatter.  A digit comes from lo for shift < 32, else from hi.
+__device__ __forceinline__ uint32_t rs_digit(const uint32_t* lo, const uint32_t* hi, uint32_t i, int shift) {
+  return (shift < 32 ? lo[i] >> shift : hi[i] >> (shift - 32)) & 255u;
+}
+__global__ void __launch_bounds__(256) k_rs_hist(const uint32_t* lo, const uint32_t* hi, uint32_t n, int shift,
                                                  uint32_t* hist, int32_t nblocks) {
   __shared__ uint32_t h[256];
   h[threadIdx.x] = 0;
   __syncthreads();
-  const uint32_t n = *n_ptr < cap ? *n_ptr : cap;
-  const int64_t base = (int64_t)blockIdx.x * RS_TILE;
+  const uint32_t base = blockIdx.x * RS_TILE;
+#pragma unroll
   for (int i = 0; i < RS_ITEMS; i++) {
-    const int64_t idx = base + (int64_t)i * 256 + threadIdx.x;
-    if (idx < n) atomicAdd(&h[(keys[idx] >> shift) & 255u], 1u);
+    const uint32_t idx = base + i * 256 + threadIdx.x;
+    if (idx < n) atomicAdd(&h[rs_digit(lo, hi, idx, shift)], 1u);
   }
   __syncthreads();
   hist[(int64_t)threadIdx.x * nblocks + blockIdx.x] = h[threadIdx.x];
 }
 
-__global__ void __launch_bounds__(256) k_rs_scatter(const uint32_t* kin, const uint32_t* vin, uint32_t* kout, uint32_t* vout,
-                                                    const uint32_t* n_ptr, uint32_t cap, int shift,
+// A tile's records are ranked wave by wave (each wave a quarter of the tile,
+// 64 records a round, no workgroup barrier between rounds), put in digit
+// order in LDS and stored from there, so that consecutive lanes store
+// consecutive records of a digit.  12 M records, 12 bytes each, 8 bits: see
+// kmer_graph for what the pass takes.
+__global__ void __launch_bounds__(256) k_rs_scatter(const uint32_t* lo, const uint32_t* hi, const uint32_t* v,
+                                                    uint32_t* lo2, uint32_t* hi2, uint32_t* v2, uint32_t n, int shift,
                                                     const uint32_t* off, int32_t nblocks) {
-  __shared__ uint32_t run[256];
-  __shared__ uint32_t wc[4][256];
-  const int tid = threadIdx.x, wave = tid >> 6;
-  run[tid] = off[(int64_t)tid * nblocks + blockIdx.x];
-  for (int w = 0; w < 4; w++) wc[w][tid] = 0;
+  __shared__ uint32_t cnt[4][256];
+  __shared__ uint32_t dst[256];                              // a digit's place in the output, less its place in the tile
+  __shared__ uint32_t ws[4];
+  __shared__ uint32_t slo[RS_TILE], shi[RS_TILE], sv[RS_TILE];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  for (int w = 0; w < 4; w++) cnt[w][tid] = 0;
   __syncthreads();
-  const uint32_t n = *n_ptr < cap ? *n_ptr : cap;
-  const int64_t base = (int64_t)blockIdx.x * RS_TILE;
-  for (int round = 0; round < RS_ITEMS; round++) {
-    const int64_t idx = base + (int64_t)round * 256 + tid;
-    const bool valid = idx < n;
-    const uint32_t k = valid ? kin[idx] : 0u;
-    const uint32_t v = valid ? vin[idx] : 0u;
-    const uint32_t d = (k >> shift) & 255u;
-    uint64_t m = __ballot(valid);
+  const uint32_t base = blockIdx.x * RS_TILE, wbase = base + (uint32_t)wave * (RS_TILE / 4);
+  const uint32_t have = n - base < RS_TILE ? n - base : RS_TILE;
+  uint32_t kl[RS_ITEMS], kh[RS_ITEMS], kv[RS_ITEMS], at[RS_ITEMS];
+#pragma unroll
+  for (int r = 0; r < RS_ITEMS; r++) {
+    const uint32_t i = wbase + 64 * r + lane;
+    const bool in = i < n;
+    kl[r] = in ? lo[i] : 0u;
+    kh[r] = in ? hi[i] : 0u;
+    kv[r] = in ? v[i] : 0u;
+  }
+#pragma unroll
+  for (int r = 0; r < RS_ITEMS; r++) {
+    const bool in = wbase + 64 * r + lane < n;
+    const uint32_t d = (shift < 32 ? kl[r] >> shift : kh[r] >> (shift - 32)) & 255u;
+    uint64_t m = __ballot(in);
 #pragma unroll
     for (int b = 0; b < 8; b++) {
       const bool bit = ((d >> b) & 1u) != 0;
-      const uint64_t bb = __ballot(valid && bit);
+      const uint64_t bb = __ballot(in && bit);
       m &= bit ? bb : ~bb;
     }
     const uint32_t rank = (uint32_t)__popcll(m & lanemask_lt());
-    if (valid && rank == 0) wc[wave][d] = (uint32_t)__popcll(m);
+    // one wave's LDS operations complete in order: every lane reads the
+    // count before its digit's first lane raises it
+    at[r] = cnt[wave][d] + rank;
+    __builtin_amdgcn_wave_barrier();
+    if (in && rank == 0) cnt[wave][d] += (uint32_t)__popcll(m);
+    __builtin_amdgcn_wave_barrier();
+  }
+  __syncthreads();
+  {
+    uint32_t c[4], t = 0;
+    for (int w = 0; w < 4; w++) { c[w] = cnt[w][tid]; t += c[w]; }
+    const uint32_t inc = wave_scan_dpp(t);
+    if (lane == 63) ws[wave] = inc;
     __syncthreads();
-    if (valid) {
-      uint32_t pre = run[d];
-      for (int w = 0; w < wave; w++) pre += wc[w][d];
-      kout[pre + rank] = k;
-      vout[pre + rank] = v;
+    uint32_t s = inc - t;
+    for (int w = 0; w < wave; w++) s += ws[w];
+    dst[tid] = off[(int64_t)tid * nblocks + blockIdx.x] - s;
+    for (int w = 0; w < 4; w++) { cnt[w][tid] = s; s += c[w]; }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < RS_ITEMS; r++) {
+    if (wbase + 64 * r + lane < n) {
+      const uint32_t d = (shift < 32 ? kl[r] >> shift : kh[r] >> (shift - 32)) & 255u;
+      const uint32_t p = cnt[wave][d] + at[r];
+      slo[p] = kl[r];
+      shi[p] = kh[r];
+      sv[p] = kv[r];
     }
-    __syncthreads();
-    run[tid] += wc[0][tid] + wc[1][tid] + wc[2][tid] + wc[3][tid];
-    for (int w = 0; w < 4; w++) wc[w][tid] = 0;
-    __syncthreads();
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < RS_ITEMS; r++) {
+    const uint32_t p = 256 * r + tid;
+    if (p < have) {
+      const uint32_t a = slo[p], b = shi[p];
+      const uint32_t o = dst[(shift < 32 ? a >> shift : b >> (shift - 32)) & 255u] + p;
+      lo2[o] = a;
+      hi2[o] = b;
+      v2[o] = sv[p];
+    }
   }
 }
 

@@ -1,11 +1,19 @@
 // pl_kmer.hip — the host side of the assembler's K-mer graph (included at
 // the end of pl_engine.hip): the reads go to the device, the occurrences
-// are emitted and grouped by K-mer (an LSD radix sort by a 64-bit hash of
-// the K-mer; should two distinct K-mers share a hash, six stable 32-bit
+// are emitted and grouped by K-mer (an LSD radix sort by some bits of a
+// 64-bit hash of the K-mer; should two distinct K-mers share them, stable
 // sorts by the K-mer's own words, last word first), summed and called per
-// K-mer by the k_kmer_* kernels; the kept K-mers come back in byte order.
+// K-mer, and the kept K-mers put in byte order and written as text, by the
+// k_kmer_* kernels.
 
 namespace {
+
+// bits of x's binary form
+int bits_of(int64_t x) {
+  int b = 0;
+  for (; x; x >>= 1) b++;
+  return b;
+}
 
 pl_status kmer_graph(pl_ctx* c, const pl_read_soa* R, int32_t K, int32_t min_depth, char** kmers, uint8_t** next,
                      uint8_t** alt, int64_t* n_out, double* device_ms) {
@@ -17,11 +25,12 @@ pl_status kmer_graph(pl_ctx* c, const pl_read_soa* R, int32_t K, int32_t min_dep
   // occurrences per read (both strands of every offset 0 .. L-K-1), the
   // nibble offset of each non-ACGT read, and the stream sizes
   std::vector<int64_t> occ((size_t)n + 1, 0), exo((size_t)n, -1);
-  int64_t nreads = 0, nib_bytes = 1;
+  int64_t nreads = 0, nib_bytes = 1, longest = 0;
   for (int64_t i = 0; i < n; i++) {
     const int64_t L = R->seq_off[i + 1] - R->seq_off[i];
     occ[(size_t)i + 1] = occ[(size_t)i] + (L > K ? 2 * (L - K) : 0);
     if (L > K) nreads++;
+    longest = std::max(longest, L);
   }
   for (int64_t k = 0; k < R->n_exotic; k++) {
     const int64_t r = R->exo_read[k];
@@ -40,7 +49,7 @@ pl_status kmer_graph(pl_ctx* c, const pl_read_soa* R, int32_t K, int32_t min_dep
   HIPCHK(hipSetDevice(c->device));
   Lane* L = &c->main;
   hipStream_t st = L->stream;
-  VcfBufs B;
+  ScratchBufs B(L);
   KmerArgs A;
   std::memset(&A, 0, sizeof A);
   A.n_reads = n;
@@ -70,100 +79,114 @@ pl_status kmer_graph(pl_ctx* c, const pl_read_soa* R, int32_t K, int32_t min_dep
   A.seq_off = dso; A.bases2 = db2; A.quals = dq; A.flag = dfl; A.mapq = dmq; A.exo_of = dexo; A.nib = dnib;
   A.occ_off = docc;
   const uint32_t nocc = (uint32_t)N;
-  uint32_t *perm, *keys, *tk, *tv, *ncount, *head, *seg;
-  if ((s = B.get(&A.kw, 4 * (size_t)PL_KMER_STRIDE * (size_t)N)) || (s = B.get(&A.val, 4 * (size_t)N)) ||
-      (s = B.get(&A.hw, 8 * (size_t)N)) || (s = B.get(&A.collide, 4)) ||
-      (s = B.get(&perm, 4 * (size_t)N)) || (s = B.get(&keys, 4 * (size_t)N)) || (s = B.get(&tk, 4 * (size_t)N)) ||
-      (s = B.get(&tv, 4 * (size_t)N)) || (s = B.get(&ncount, 4)) || (s = B.get(&head, 4 * (size_t)N)) ||
-      (s = B.get(&seg, 4 * ((size_t)N + 1))))                // the scan also writes the total at [N]
+  // Hash bits the order is by: twice those of N, so that of N distinct
+  // K-mers two share them in about half the calls at worst and, of the third
+  // or less that are distinct in reads with errors, in a few of a hundred.
+  const int bits = std::min(64, (2 * bits_of(N) + 7) / 8 * 8);
+  A.hmask = bits >= 64 ? ~0u : bits > 32 ? (1u << (bits - 32)) - 1u : 0u;
+  A.cap = (uint32_t)(N / std::max(min_depth, 1)) + 1;
+  SortRecs a, b;
+  uint32_t* counts;                                          // list_n, out_n, flags[2]
+  if ((s = B.get(&A.kw, 4 * (size_t)PL_KMER_STRIDE * (size_t)N)) || (s = B.get(&a.lo, 4 * (size_t)N)) || (s = B.get(&a.hi, 4 * (size_t)N)) || (s = B.get(&a.v, 4 * (size_t)N)) ||
+      (s = B.get(&b.lo, 4 * (size_t)N)) || (s = B.get(&b.hi, 4 * (size_t)N)) || (s = B.get(&b.v, 4 * (size_t)N)) ||
+      (s = B.get(&A.list, 4 * (size_t)A.cap)) || (s = B.get(&counts, 16)) ||
+      (s = B.get(&A.out_kw, 4 * (size_t)A.words * (size_t)A.cap)) || (s = B.get(&A.out_next, (size_t)A.cap)) ||
+      (s = B.get(&A.out_alt, (size_t)A.cap)))
     return s;
+  A.list_n = counts;
+  A.out_n = counts + 1;
+  A.flags = counts + 2;
   EventPair ev;
   HIPCHK(ev.create());
   HIPCHK(hipEventRecord(ev.e0, st));
   const unsigned gb = (unsigned)((N + 255) / 256);
-  k_kmer_emit<<<dim3((unsigned)n), dim3(256), 0, st>>>(A);
+  A.hlo = a.lo; A.hhi = a.hi; A.perm = a.v;
+  if (longest <= PL_KMER_WAVE_BASES) k_kmer_emit<true><<<dim3((unsigned)((n + 3) / 4)), dim3(256), 0, st>>>(A);
+  else k_kmer_emit<false><<<dim3((unsigned)n), dim3(256), 0, st>>>(A);
   HIPCHK(hipGetLastError());
-  // sort the occurrences (perm) by the 32-bit keys src[0..nw) of each, the
-  // least significant first: each stable sort keeps the order of the later keys
-  auto sort_by = [&](const uint32_t* const* src, uint32_t stride, int nw) -> pl_status {
-    k_iota<<<dim3(std::min<unsigned>(gb, 4096)), dim3(256), 0, st>>>(perm, (int32_t)N, ncount);
-    for (int w = 0; w < nw; w++) {
-      k_kmer_gather<<<dim3(gb), dim3(256), 0, st>>>(src[w], stride, perm, nocc, keys);
-      uint32_t *rk, *rv;
-      if (pl_status e = radix_sort(L, keys, perm, tk, tv, ncount, nocc, 32, &rk, &rv)) return e;
-      if (rv != perm) HIPCHK(hipMemcpyAsync(perm, rv, 4 * (size_t)N, hipMemcpyDeviceToDevice, st));
+  if ((s = radix_sort(L, a, b, nocc, bits))) return s;
+  // m records in word order (src[w] + record * stride: word w), last word first
+  auto sort_by_words = [&](uint32_t* const* src, uint32_t stride, uint32_t m) -> pl_status {
+    const unsigned g = (m + 255) / 256;
+    k_iota<<<dim3(std::min<unsigned>(g, 4096)), dim3(256), 0, st>>>(a.v, (int32_t)m, counts);
+    for (int w = A.words - 1; w >= 0; w--) {
+      k_kmer_gather<<<dim3(g), dim3(256), 0, st>>>(src[w], stride, a.v, m, a.lo);
+      if (pl_status e = radix_sort(L, a, b, m, 32)) return e;
     }
     return PL_OK;
   };
-  A.perm = perm;
-  A.head = head;
-  const uint32_t* by_hash[2] = {A.hw, A.hw + (size_t)N};
-  if ((s = sort_by(by_hash, 1, 2))) return s;
-  A.by_hash = 1;
-  HIPCHK(hipMemsetAsync(A.collide, 0, 4, st));
-  k_kmer_heads<<<dim3(gb), dim3(256), 0, st>>>(A);
-  uint32_t collide = 0;
-  HIPCHK(hipMemcpyAsync(&collide, A.collide, 4, hipMemcpyDeviceToHost, st));
-  HIPCHK(hipStreamSynchronize(st));
-  // PILON_HIP_KMER_WORD_SORT in the environment takes this path without a
-  // collision (tests compare it with the hash order's graph)
-  if (collide || std::getenv("PILON_HIP_KMER_WORD_SORT")) {
-    // two K-mers share a hash: order by the words themselves instead
-    const uint32_t* by_words[PL_KMER_WORDS];
-    for (int w = 0; w < A.words; w++) by_words[w] = A.kw + (size_t)(A.words - 1 - w);
-    if ((s = sort_by(by_words, PL_KMER_STRIDE, A.words))) return s;
-    A.by_hash = 0;
-    k_kmer_heads<<<dim3(gb), dim3(256), 0, st>>>(A);
+  uint32_t hc[4] = {0, 0, 0, 0};
+  auto counted = [&]() -> pl_status {
+    HIPCHK(hipMemcpyAsync(hc, counts, 16, hipMemcpyDeviceToHost, st));
+    HIPCHK(hipStreamSynchronize(st));
+    return PL_OK;
+  };
+  // PILON_HIP_KMER_WORD_SORT in the environment takes the word order without
+  // a collision (tests compare it with the hash order's graph)
+  bool by_words = std::getenv("PILON_HIP_KMER_WORD_SORT") != nullptr;
+  for (;; by_words = true) {
+    if (by_words) {
+      uint32_t* src[PL_KMER_WORDS];
+      uint32_t *head, *seg;
+      for (int w = 0; w < A.words; w++) src[w] = A.kw + w;
+      if ((s = B.get(&head, 4 * (size_t)N)) || (s = B.get(&seg, 4 * ((size_t)N + 1)))) return s;
+      if ((s = sort_by_words(src, PL_KMER_STRIDE, nocc))) return s;
+      A.hlo = a.lo; A.hhi = a.hi; A.perm = a.v;
+      k_kmer_heads<<<dim3(gb), dim3(256), 0, st>>>(A, head);
+      if ((s = scan_u32(L, head, seg, N))) return s;
+      k_kmer_number<<<dim3(gb), dim3(256), 0, st>>>(A, head, seg);
+    }
+    A.hlo = a.lo; A.hhi = a.hi; A.perm = a.v;
+    HIPCHK(hipMemsetAsync(counts, 0, 16, st));
+    k_kmer_list<<<dim3((unsigned)((N + 256 * PL_KMER_LIST_PER - 1) / (256 * PL_KMER_LIST_PER))), dim3(256), 0, st>>>(A);
+    HIPCHK(hipGetLastError());
+    if ((s = counted())) return s;
+    if (hc[0]) k_kmer_call<<<dim3((unsigned)(((int64_t)hc[0] * 16 + 255) / 256)), dim3(256), 0, st>>>(A);
+    HIPCHK(hipGetLastError());
+    if ((s = counted())) return s;
+    if (!hc[2] || by_words) break;                            // else two K-mers share the hash bits
   }
-  if ((s = scan_u32(L, head, seg, N))) return s;
-  uint32_t ns = 0;                                          // distinct K-mers
-  HIPCHK(hipMemcpyAsync(&ns, seg + N, 4, hipMemcpyDeviceToHost, st));
-  HIPCHK(hipStreamSynchronize(st));
-  A.seg = seg;
-  A.n_seg = ns;
-  if ((s = B.get(&A.starts, 4 * ((size_t)ns + 1))) || (s = B.get(&A.out_n, 4)) ||
-      (s = B.get(&A.out_kw, 4 * (size_t)A.words * (size_t)ns)) || (s = B.get(&A.out_next, (size_t)ns)) ||
-      (s = B.get(&A.out_alt, (size_t)ns)))
-    return s;
-  HIPCHK(hipMemsetAsync(A.out_n, 0, 4, st));
-  HIPCHK(hipMemcpyAsync(A.starts + ns, &nocc, 4, hipMemcpyHostToDevice, st));
-  k_kmer_starts<<<dim3(gb), dim3(256), 0, st>>>(A);
-  k_kmer_call<<<dim3((ns + 255) / 256), dim3(256), 0, st>>>(A);
-  HIPCHK(hipGetLastError());
-  HIPCHK(hipEventRecord(ev.e1, st));
-  uint32_t nk = 0;
-  HIPCHK(hipMemcpyAsync(&nk, A.out_n, 4, hipMemcpyDeviceToHost, st));
-  HIPCHK(hipStreamSynchronize(st));
-  std::vector<uint32_t> kw((size_t)A.words * ns);
-  std::vector<uint8_t> nx(nk), al(nk);
-  HIPCHK(hipMemcpyAsync(kw.data(), A.out_kw, 4 * (size_t)A.words * ns, hipMemcpyDeviceToHost, st));
+  const uint32_t nk = hc[1];
+  uint8_t* dtext = nullptr;
+  const size_t tb = ((size_t)K * nk + 255) & ~(size_t)255, nb = ((size_t)nk + 255) & ~(size_t)255;
   if (nk) {
-    HIPCHK(hipMemcpyAsync(nx.data(), A.out_next, nk, hipMemcpyDeviceToHost, st));
-    HIPCHK(hipMemcpyAsync(al.data(), A.out_alt, nk, hipMemcpyDeviceToHost, st));
+    const unsigned gk = (nk + 255) / 256;
+    if (nk <= PL_KMER_RANK_MAX) {
+      HIPCHK(hipMemsetAsync(a.lo, 0, 4 * (size_t)nk, st));
+      k_kmer_rank<<<dim3(gk, (nk + PL_KMER_RANK_TILE - 1) / PL_KMER_RANK_TILE), dim3(256), 0, st>>>(A, nk, a.lo);
+      k_kmer_place<<<dim3(gk), dim3(256), 0, st>>>(a.lo, nk, a.v);
+    } else {
+      k_kmer_keys<<<dim3(gk), dim3(256), 0, st>>>(A, nk, a.lo, a.hi, a.v);
+      if ((s = radix_sort(L, a, b, nk, 64))) return s;
+      if (A.words > 2) {
+        k_kmer_ties<<<dim3(gk), dim3(256), 0, st>>>(A, nk, a.lo, a.hi, a.v);
+        HIPCHK(hipGetLastError());
+        if ((s = counted())) return s;
+        if (hc[3]) {
+          uint32_t* src[PL_KMER_WORDS];
+          for (int w = 0; w < A.words; w++) src[w] = A.out_kw + (size_t)w * A.cap;
+          if ((s = sort_by_words(src, 1, nk))) return s;
+        }
+      }
+    }
+    HIPCHK(hipGetLastError());
+    if ((s = B.get(&dtext, tb + 2 * nb))) return s;
+    const size_t threads = std::max<size_t>(((size_t)K * nk + 3) / 4, nk);
+    k_kmer_text<<<dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st>>>(A, nk, a.v, dtext, dtext + tb,
+                                                                              dtext + tb + nb);
+    HIPCHK(hipGetLastError());
   }
-  HIPCHK(hipStreamSynchronize(st));
-  float t = 0.f;
-  HIPCHK(hipEventElapsedTime(&t, ev.e0, ev.e1));
-  // the K-mers as text, in byte order
-  static const char NIB[] = "=ACMGRSVTWYHKDBN";
-  std::string text((size_t)K * nk, ' ');
-  for (uint32_t k = 0; k < nk; k++)
-    for (int j = 0; j < K; j++)
-      text[(size_t)K * k + j] = NIB[(kw[(size_t)(j >> 3) * ns + k] >> (28 - 4 * (j & 7))) & 15u];
-  std::vector<uint32_t> ord(nk);
-  for (uint32_t k = 0; k < nk; k++) ord[k] = k;
-  std::sort(ord.begin(), ord.end(), [&](uint32_t a, uint32_t b) {
-    return std::memcmp(text.data() + (size_t)K * a, text.data() + (size_t)K * b, (size_t)K) < 0;
-  });
+  HIPCHK(hipEventRecord(ev.e1, st));
   char* ko = (char*)malloc((size_t)K * nk + 1);
   uint8_t* no = (uint8_t*)malloc((size_t)nk + 1);
   uint8_t* ao = (uint8_t*)malloc((size_t)nk + 1);
-  if (!ko || !no || !ao) { free(ko); free(no); free(ao); return fail(PL_E_OOM, "host allocation failed"); }
-  for (uint32_t i = 0; i < nk; i++) {
-    std::memcpy(ko + (size_t)K * i, text.data() + (size_t)K * ord[i], (size_t)K);
-    no[i] = nx[ord[i]];
-    ao[i] = al[ord[i]];
-  }
+  s = ko && no && ao ? PL_OK : fail(PL_E_OOM, "host allocation failed");
+  if (!s && nk && !(s = copy_to_host(L, ko, dtext, (size_t)K * nk)) && !(s = copy_to_host(L, no, dtext + tb, nk)))
+    s = copy_to_host(L, ao, dtext + tb + nb, nk);
+  float t = 0.f;
+  if (!s && (hipEventSynchronize(ev.e1) != hipSuccess || hipEventElapsedTime(&t, ev.e0, ev.e1) != hipSuccess))
+    s = fail(PL_E_DEVICE, "K-mer graph events");
+  if (s) { free(ko); free(no); free(ao); return s; }
   *kmers = ko; *next = no; *alt = ao; *n_out = nk;
   if (device_ms) *device_ms = t;
   return PL_OK;

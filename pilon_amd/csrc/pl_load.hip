@@ -257,7 +257,7 @@ __global__ void __launch_bounds__(256) k_ld_table(LoadArgs A, uint64_t* tab) {
 inline unsigned ld_grid(int64_t n) { return (unsigned)std::max<int64_t>(1, std::min<int64_t>((n + 255) / 256, 1 << 16)); }
 
 // 64-bit exclusive prefix sums of a u32 array (out[n] = the total)
-pl_status scan_u32_to_u64(Lane* L, const uint32_t* in, int64_t n, uint64_t* out, VcfBufs& B) {
+pl_status scan_u32_to_u64(Lane* L, const uint32_t* in, int64_t n, uint64_t* out, ScratchBufs& B) {
   const int64_t tiles = std::max<int64_t>(1, (n + SCAN_TILE - 1) / SCAN_TILE);
   uint64_t* tsum;
   if (pl_status s = B.get(&tsum, 8 * (size_t)tiles)) return s;
@@ -300,7 +300,7 @@ pl_status loader_finish(pl_loader* ld, int32_t nref, const int32_t* contig_ids, 
   hipStream_t st = L->stream;
   const int64_t N = ld->n_rec;
   HIPCHK(hipStreamSynchronize(st));
-  VcfBufs B;
+  ScratchBufs B(L);
   LoadArgs A;
   std::memset(&A, 0, sizeof A);
   A.R = ld->bytes;

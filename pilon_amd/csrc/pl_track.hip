@@ -11,7 +11,8 @@ const char* const kTrackNames[PL_NTRACKS] = {
 
 // computeGc's buffer values of the listed contigs that have none yet, built
 // together in one device block
-pl_status build_gcv(pl_ctx* c, const std::vector<int32_t>& ids, hipStream_t st) {
+pl_status build_gcv(pl_ctx* c, const std::vector<int32_t>& ids, Lane* L) {
+  hipStream_t st = L->stream;
   std::vector<int32_t> miss;
   for (int32_t id : ids)
     if (!c->contigs.at(id).gcv) miss.push_back(id);
@@ -42,7 +43,7 @@ pl_status build_gcv(pl_ctx* c, const std::vector<int32_t>& ids, hipStream_t st) 
     return fail(PL_E_OOM, "device allocation of %zu bytes failed", bytes);
   std::shared_ptr<uint8_t> mem(block, [](uint8_t* p) { (void)hipFree(p); });
   for (size_t i = 0; i < jobs.size(); i++) jobs[i].gcv = block + off[i];
-  VcfBufs B;
+  ScratchBufs B(L);
   uint8_t* carry;
   GcvJob* dj;
   pl_status s;
@@ -65,7 +66,7 @@ pl_status build_gcv(pl_ctx* c, const std::vector<int32_t>& ids, hipStream_t st) 
 
 // The track values of the lane's last batch into T.vals (device), in B's
 // buffers; contigs[j] is region j's contig.  ms accumulates the device time.
-pl_status tracks_of_lane(pl_ctx* c, Lane* L, const std::vector<int32_t>& contigs, VcfBufs& B, TrackArgs& T,
+pl_status tracks_of_lane(pl_ctx* c, Lane* L, const std::vector<int32_t>& contigs, ScratchBufs& B, TrackArgs& T,
                          double* ms, bool issues = false) {
   HIPCHK(hipSetDevice(c->device));
   hipStream_t st = L->stream;
@@ -75,7 +76,7 @@ pl_status tracks_of_lane(pl_ctx* c, Lane* L, const std::vector<int32_t>& contigs
   T.A = L->args;
   // the contigs' GC buffers (once per contig) and each region's pointer
   if ((int32_t)contigs.size() != nj) return fail(PL_E_INVAL, "%d contigs for %d regions", (int)contigs.size(), nj);
-  if (pl_status s = build_gcv(c, contigs, st)) return s;
+  if (pl_status s = build_gcv(c, contigs, L)) return s;
   std::vector<const uint8_t*> gp((size_t)nj);
   for (int32_t j = 0; j < nj; j++) gp[(size_t)j] = c->contigs.at(contigs[(size_t)j]).gcv;
   const uint8_t** dgp;
@@ -113,7 +114,7 @@ pl_status tracks_copy(pl_ctx* c, Lane* L, const std::vector<int32_t>& contigs, i
   if (values && n_values < (int64_t)PL_NTRACKS * G)
     return fail(PL_E_INVAL, "values holds %lld entries, the batch needs %lld", (long long)n_values,
                 (long long)PL_NTRACKS * G);
-  VcfBufs B;
+  ScratchBufs B(L);
   TrackArgs T;
   double ms = 0;
   if (pl_status s = tracks_of_lane(c, L, contigs, B, T, &ms)) return s;
@@ -131,7 +132,7 @@ pl_status wig_of_lane(pl_ctx* c, Lane* L, const std::vector<std::string>& rnames
   const int64_t G = L->G;
   const int32_t nj = (int32_t)L->hjobs.size();
   hipStream_t st = L->stream;
-  VcfBufs B;
+  ScratchBufs B(L);
   TrackArgs T;
   double ms = 0;
   if (pl_status s = tracks_of_lane(c, L, contigs, B, T, &ms)) return s;
@@ -282,7 +283,7 @@ pl_status bed_of_lane(pl_ctx* c, Lane* L, const std::vector<std::string>& rnames
   *len = 0;
   const int64_t G = L->G;
   const int32_t nj = (int32_t)L->hjobs.size();
-  VcfBufs B;
+  ScratchBufs B(L);
   TrackArgs T;
   double ms = 0;
   if (pl_status s = tracks_of_lane(c, L, contigs, B, T, &ms, true)) return s;
@@ -343,7 +344,7 @@ pl_status region_jump_depth(pl_region* r) {
   pl_status s = run_jobs(c, X, q, PL_DEFAULT_WINDOW, 0, PL_DEFAULT_BLOCK, false);
   if (!s) s = fetch_batch_meta(X);
   if (!s) {
-    VcfBufs B;
+    ScratchBufs B(X);
     TrackArgs T;
     std::memset(&T, 0, sizeof T);
     T.A = X->args;

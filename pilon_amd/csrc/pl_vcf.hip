@@ -5,17 +5,34 @@
 
 namespace {
 
-// device buffers of one VCF pass, freed on every exit
-struct VcfBufs {
-  std::vector<void*> p;
-  ~VcfBufs() { for (void* x : p) (void)hipFree(x); }
+// Device buffers of one call, given back on every exit: to the lane's
+// scratch (calls nest, so the last one begun is the first to end), or freed
+// when they were allocated while a call begun later was still using it.
+struct ScratchBufs {
+  explicit ScratchBufs(Lane* lane) : s(lane->scratch), at(s.at), used(s.used), outer(s.top) { s.top = this; }
+  ~ScratchBufs() {
+    for (void* x : own) (void)hipFree(x);
+    s.top = outer;
+    s.at = at;
+    s.used = used;
+    if (!outer) s.settle();
+  }
+  ScratchBufs(const ScratchBufs&) = delete;
+  ScratchBufs& operator=(const ScratchBufs&) = delete;
   template <class T> pl_status get(T** out, size_t n) {
     void* q = nullptr;
-    if (hipMalloc(&q, n ? n : 1) != hipSuccess) return fail(PL_E_OOM, "device allocation of %zu bytes failed", n);
-    p.push_back(q);
+    const hipError_t e = s.top == this ? s.get(n, &q) : hipMalloc(&q, n ? n : 1);
+    if (e != hipSuccess) return fail(PL_E_OOM, "device allocation of %zu bytes failed", n);
+    if (s.top != this) own.push_back(q);
     *out = (T*)q;
     return PL_OK;
   }
+
+ private:
+  Scratch& s;
+  size_t at, used;
+  void* outer;
+  std::vector<void*> own;
 };
 
 void add_line(std::string& s, const std::string& l) { s += l; s += '\n'; }
@@ -216,7 +233,7 @@ pl_status pl_vcf_header(const char* const* names, const int64_t* lengths, int32_
 
 namespace {
 
-pl_status tracks_of_lane(pl_ctx* c, Lane* L, const std::vector<int32_t>& contigs, VcfBufs& B, TrackArgs& T,
+pl_status tracks_of_lane(pl_ctx* c, Lane* L, const std::vector<int32_t>& contigs, ScratchBufs& B, TrackArgs& T,
                          double* ms, bool issues);
 
 // GenomeRegion.duplicationEvents (GenomeRegion.scala:731-737) of one region
@@ -245,7 +262,8 @@ std::vector<std::pair<int32_t, int32_t>> dup_runs(const uint8_t* m, int32_t star
 // the host puts between them (Vcf.writeDup before a duplication event's
 // first locus) at their byte offsets in the device text.
 struct VcfText {
-  VcfBufs B;
+  explicit VcfText(Lane* L) : B(L) {}
+  ScratchBufs B;
   const char* dtext = nullptr;
   uint64_t total = 0;
   std::vector<std::pair<uint64_t, std::string>> inserts;   // ascending offsets
@@ -299,7 +317,7 @@ pl_status vcf_format(pl_ctx* c, Lane* L, const std::vector<std::string>& rnames,
     names += rnames[(size_t)j];
     noff.push_back((int64_t)names.size());
   }
-  VcfBufs& B = out.B;
+  ScratchBufs& B = out.B;
   VcfArgs V;
   std::memset(&V, 0, sizeof V);
   V.A = L->args;
@@ -355,7 +373,7 @@ pl_status vcf_format(pl_ctx* c, Lane* L, const std::vector<std::string>& rnames,
   // a writeDup line (Vcf.scala:194-202) before the records of the first
   // locus of each, at that locus's offset in the device text
   {
-    VcfBufs B2;
+    ScratchBufs B2(L);
     TrackArgs T;
     double tms = 0;
     if ((s = tracks_of_lane(c, L, contigs, B2, T, &tms, true))) return s;
@@ -400,7 +418,7 @@ pl_status vcf_of_lane(pl_ctx* c, Lane* L, const std::vector<std::string>& rnames
                       uint32_t flags, char** text, int64_t* len, double* device_ms, const FixRecords* fr = nullptr) {
   *text = nullptr;
   *len = 0;
-  VcfText V;
+  VcfText V(L);
   if (pl_status s = vcf_format(c, L, rnames, contigs, flags, V, fr)) return s;
   const uint64_t n = V.bytes();
   char* out = (char*)malloc((size_t)n + 1);
@@ -516,7 +534,7 @@ pl_status pl_batch_vcf_stream(pl_ctx* c, uint32_t flags, pl_text_sink sink, void
   std::vector<std::string> names;
   std::vector<int32_t> contigs;
   if (pl_status s = batch_names(c, &c->main, &names, &contigs)) return s;
-  VcfText V;
+  VcfText V(&c->main);
   if (pl_status s = vcf_format(c, &c->main, names, contigs, flags, V)) return s;
   if (pl_status s = vcf_emit(&c->main, V, [&](const char* p, size_t n) { return sink(user, p, (int64_t)n) == 0; }))
     return s;

@@ -1,0 +1,53 @@
+"""The K-mer graph's byte order and grouping on the device against the
+oracle's: counts of kept K-mers about the limit of the counted order (8,192)
+and above it, K-mers that agree in their first 16 bases (a handful, and more
+than one thread orders), codes other than A, C, G, T among them."""
+import numpy as np
+import pytest
+
+from pilon_amd.abi import default_config
+from pilon_amd.reads import pack_reads
+
+pytestmark = pytest.mark.gpu
+
+
+def reads_of(kind, n, K, rng):
+    """Reads of K + 1 bases, each K-mer in `depth` of them."""
+    out = []
+    for i in range(n):
+        seq = "".join(rng.choice(list("ACGT"), K + 1))
+        if kind == "prefix":                     # 8 to a 16-base prefix
+            seq = "".join("ACGT"[(i // 8 >> (2 * b)) & 3] for b in range(16)) + seq[16:]
+        elif kind == "one_prefix":
+            seq = "ACGTTGCATTGACCAG" + seq[16:]
+        elif kind == "codes" and i % 3 == 0:
+            seq = seq[:K // 2] + "RYMN"[i % 4] + seq[K // 2 + 1:]
+        out.append(seq)
+    return out
+
+
+@pytest.mark.parametrize("kind,n,K", [("plain", 4095, 47), ("plain", 4097, 47), ("plain", 9000, 16), ("plain", 300, 7),
+                                      ("prefix", 6000, 47), ("one_prefix", 200, 47), ("one_prefix", 5000, 33),
+                                      ("codes", 3000, 48), ("codes", 5000, 31)])
+def test_kmer_byte_order(kind, n, K):
+    from oracle import oracle as O
+    from pilon_amd.engine import Context
+    print(f"case: kmer order {kind} n={n} K={K}", flush=True)
+    rng = np.random.default_rng(n + K)
+    depth = 3
+    reads = []
+    for seq in reads_of(kind, n, K, rng):
+        for _ in range(depth):
+            reads.append(dict(pos=1, cigar=f"{K + 1}M", seq=seq, qual=[int(x) for x in rng.integers(2, 41, K + 1)],
+                              mapq=int(rng.integers(0, 61))))
+    b = pack_reads(reads, sort=False)
+    cfg = default_config()
+    ctx = Context(cfg, device=0)
+    try:
+        for min_depth in (depth, 1):
+            got, _ = ctx.kmer_graph(b, K=K, min_depth=min_depth)
+            st, ref = O.kmer_graph(cfg, b, K=K, min_depth=min_depth)
+            assert st == 0 and len(ref) >= min(n, 200)
+            assert got == ref
+    finally:
+        ctx.close()
