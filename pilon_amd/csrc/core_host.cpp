@@ -254,7 +254,7 @@ void* ch_run(const pl_config* pc, const uint8_t* ref, int64_t ref_len, const cha
             int64_t dep = 0;
             for (int b = 0; b < 4; b++) dep += (uint32_t)o.f[PL_F_COUNT_A + b];
             dep += o.f[PL_F_DELETIONS];
-            cands.push_back({(uint32_t)g, (int32_t)dep, d, 0, -1, 0, 0, 0});
+            cands.push_back({(uint32_t)g, (int32_t)dep, d, 0, -1, 0, 0, 0, {}});
           }
         }
       }
@@ -284,7 +284,7 @@ void* ch_run(const pl_config* pc, const uint8_t* ref, int64_t ref_len, const cha
     const int d = call_disp(cl);
     const int64_t dep = c.depth();
     if (d == PL_D_CONFIRMED) hist[(size_t)j * PL_HIST + (dep > 255 ? 255 : dep)]++;
-    else if (d != PL_D_NONE) cands.push_back({g, (int32_t)dep, d, ilen, (int32_t)wrec, 0, 0, 0});
+    else if (d != PL_D_NONE) cands.push_back({g, (int32_t)dep, d, ilen, (int32_t)wrec, 0, 0, 0, {}});
   }
   std::stable_sort(cands.begin(), cands.end(), [](const Cand& a, const Cand& b) { return a.gpos < b.gpos; });
   std::vector<uint32_t> mutated((size_t)G + 1);

@@ -153,6 +153,7 @@ struct IndelRec {
   int64_t src;               // insertion: first base (2-bit or nibble index); deletion: contig offset
 };
 
+#define PL_CAND_INS 32
 // a change candidate (a column whose disposition before Pass 1 is a change)
 struct Cand {
   uint32_t gpos;
@@ -162,6 +163,7 @@ struct Cand {
   int32_t rec;               // winning IndelRec index (INS/DEL)
   uint8_t base, alt;         // BaseCall.base, altBase
   uint16_t pad;
+  uint8_t ins[PL_CAND_INS];  // an insertion's string when it fits (k_after)
 };
 
 struct KConf {               // the knobs kernels read (Pilon.scala:52-73)

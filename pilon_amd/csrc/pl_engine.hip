@@ -186,12 +186,26 @@ enum { PL_N_REC = 0, PL_N_CAND, PL_N_DEFER, PL_N_MUTATED, PL_N_OVERFLOW, PL_N_QU
 // One independent batch pipeline: its stream, events, device buffers and
 // host-side tables.  A context has one (the plain and batched forms); a
 // server has one per concurrent batch.
+#define PL_MAIL_BYTES ((size_t)1 << 20)
+#define PL_MAIL_CANDS 1024       // candidates brought back before their number is known
 struct Lane {
   hipStream_t stream = nullptr;
   hipEvent_t ev[4] = {};
-  DBuf rsarr, kparr, jobs, wins, cost, bins, pile, calls, prec, cmask, csums, st, dhist, rec, winrec, spill,
-      spillat, cand, defer, mutated, counters, strpool, stridx, stroff, wide, winwide, heads;
+  DBuf rsarr, kparr, jobs, wins, cost, bins, pile, calls, prec, cmask, csums, res, dhist, rec, winrec, spill,
+      spillat, defer, mutated, strpool, stridx, stroff, wide, winwide, heads;
   DBuf hist, tiles;                // sort and scan scratch (uploads, K-mers)
+  // res holds what the host needs of a batch, one copy's worth: the counters,
+  // the regions' JobStat, the candidates
+  uint32_t* counters() const { return res.as<uint32_t>(); }
+  JobStat* stats() const { return (JobStat*)(res.as<uint8_t>() + 4 * PL_COUNTERS); }
+  static size_t cand_at(size_t n_jobs) { return (4 * PL_COUNTERS + sizeof(JobStat) * n_jobs + 63) & ~(size_t)63; }
+  Cand* cands(size_t n_jobs) const { return (Cand*)(res.as<uint8_t>() + cand_at(n_jobs)); }
+  // pinned host memory a batch's results come back in (PL_MAIL_BYTES; the
+  // context's lanes, never in use together, share one)
+  uint8_t* mail = nullptr;
+  bool own_mail = false;
+  size_t mail_res = 0;             // bytes of res in it
+  size_t mail_pile = 0, mail_calls = 0;   // where the last batch's pileup and calls are in it (0: they are not)
   uint32_t rec_cap = 0, spill_cap = 0, cand_cap = 0, defer_cap = 0, mut_cap = 0, wide_cap = 0;
   std::vector<JobDev> hjobs;
   std::vector<WinDev> hwins;
@@ -232,8 +246,8 @@ struct Lane {
   bool has_jdepth = false;
 
   template <class F> void for_each_buffer(F&& f) {
-    DBuf* b[] = {&rsarr, &kparr, &jobs, &wins, &cost, &bins, &pile, &calls, &prec, &cmask, &csums, &st, &dhist, &rec,
-                 &winrec, &spill, &spillat, &cand, &defer, &mutated, &counters, &strpool, &stridx, &stroff,
+    DBuf* b[] = {&rsarr, &kparr, &jobs, &wins, &cost, &bins, &pile, &calls, &prec, &cmask, &csums, &res, &dhist, &rec,
+                 &winrec, &spill, &spillat, &defer, &mutated, &strpool, &stridx, &stroff,
                  &wide, &winwide, &heads, &hist, &tiles, &jdepth};
     for (DBuf* x : b) f(*x);
   }
@@ -885,7 +899,13 @@ void drop_graph(Lane* L) {
   L->graph = nullptr;
 }
 
-pl_status lane_init(Lane* L) {
+// mail: the lane's result memory (null: its own)
+pl_status lane_init(Lane* L, uint8_t* mail = nullptr) {
+  L->mail = mail;
+  if (!mail) {
+    HIPCHK(hipHostMalloc((void**)&L->mail, PL_MAIL_BYTES, hipHostMallocDefault));
+    L->own_mail = true;
+  }
   HIPCHK(hipStreamCreateWithFlags(&L->stream, hipStreamNonBlocking));
   for (int i = 0; i < 4; i++) HIPCHK(hipEventCreate(&L->ev[i]));
   return PL_OK;
@@ -902,6 +922,9 @@ void lane_destroy(Lane* L) {
     L->stage_ev[k] = nullptr;
     L->stage[k] = nullptr;
   }
+  if (L->own_mail) (void)hipHostFree(L->mail);
+  L->mail = nullptr;
+  L->own_mail = false;
   if (L->rep_hc) (void)hipHostFree(L->rep_hc);
   L->rep_hc = nullptr;
   for (int i = 0; i < 4; i++) if (L->ev[i]) (void)hipEventDestroy(L->ev[i]);
@@ -925,7 +948,7 @@ pl_status enqueue_batch(Lane* L, EngineArgs& A, WindowKernel wk, int persistent,
   const unsigned jb = (unsigned)(n_jobs + 3) / 4, pb = (unsigned)(n_wins + 15) / 16;
   WinDev* wins = L->wins.as<WinDev>();
   const uint32_t* const* kp = (const uint32_t* const*)L->kparr.p;
-  uint32_t* cnt = L->counters.as<uint32_t>();
+  uint32_t* cnt = L->counters();
   // windows in their own order need no cost order: one launch prepares everything
   const bool ordered = persistent && n_wins > grid;
   k_begin<<<dim3(1 + jb + (ordered ? 0 : pb)), dim3(256), 0, st>>>(A, kp, cnt, PL_COUNTERS, wins, ordered ? 0 : 1);
@@ -959,7 +982,10 @@ size_t window_lds_total(int32_t W, int block) {
   return window_lds(W) + 32 * (size_t)block + 1024 + sizeof(IndelRec) * PL_WIN_RECS;
 }
 
-pl_status run_jobs(pl_ctx* c, Lane* L, const std::vector<JobReq>& reqs, int32_t W, int persistent, int block, bool use_graph) {
+// bring: the caller wants the pileup and calls of a small batch (those that
+// fit the mail come back with the counters, export_all hands them out)
+pl_status run_jobs(pl_ctx* c, Lane* L, const std::vector<JobReq>& reqs, int32_t W, int persistent, int block, bool use_graph,
+                   bool bring = false) {
   if (reqs.empty()) return fail(PL_E_INVAL, "empty batch");
   if (W < 64 || W % 64 || W > PL_MAX_WINDOW) return fail(PL_E_INVAL, "window %d must be a multiple of 64 in [64, 2048]", W);
   if (block != 256 && block != 512 && block != 1024) return fail(PL_E_INVAL, "block %d must be 256, 512 or 1024", block);
@@ -1039,8 +1065,6 @@ pl_status run_jobs(pl_ctx* c, Lane* L, const std::vector<JobReq>& reqs, int32_t 
   HIPCHK(L->dhist.ensure(4 * (size_t)PL_HIST * (size_t)n_jobs));
   HIPCHK(L->pile.ensure(4 * (size_t)PL_NFIELDS * G));
   HIPCHK(L->calls.ensure(sizeof(pl_call) * (size_t)G));
-  HIPCHK(L->st.ensure(sizeof(JobStat) * n_jobs));
-  HIPCHK(L->counters.ensure(4 * PL_COUNTERS));
   if (!same) {
     HIPCHK(hipMemcpyAsync(L->jobs.p, L->hjobs.data(), sizeof(JobDev) * n_jobs, hipMemcpyHostToDevice, st));
     HIPCHK(hipMemcpyAsync(L->wins.p, L->hwins.data(), sizeof(WinDev) * n_wins, hipMemcpyHostToDevice, st));
@@ -1065,11 +1089,11 @@ pl_status run_jobs(pl_ctx* c, Lane* L, const std::vector<JobReq>& reqs, int32_t 
     HIPCHK(L->rec.ensure(sizeof(IndelRec) * (size_t)L->rec_cap));
     HIPCHK(L->spill.ensure(sizeof(IndelRec) * (size_t)L->spill_cap));
     HIPCHK(L->spillat.ensure(8 * (size_t)L->spill_cap));
-    HIPCHK(L->cand.ensure(sizeof(Cand) * (size_t)L->cand_cap));
+    HIPCHK(L->res.ensure(Lane::cand_at((size_t)n_jobs) + sizeof(Cand) * (size_t)L->cand_cap));
     HIPCHK(L->defer.ensure(4 * (size_t)L->defer_cap));
     HIPCHK(L->mutated.ensure(4 * (size_t)L->mut_cap));
     HIPCHK(L->wide.ensure(sizeof(WideCol) * (size_t)L->wide_cap));
-    uint32_t* cnt = L->counters.as<uint32_t>();
+    uint32_t* cnt = L->counters();
     EngineArgs& A = L->args;
     std::memset(&A, 0, sizeof A);
     A.cf = c->cf;
@@ -1087,7 +1111,7 @@ pl_status run_jobs(pl_ctx* c, Lane* L, const std::vector<JobReq>& reqs, int32_t 
     A.pile = L->pile.as<int32_t>();
     A.calls = L->calls.as<pl_call>();
     A.G = G;
-    A.st = L->st.as<JobStat>();
+    A.st = L->stats();
     A.hist = L->dhist.as<uint32_t>();
     A.rec = L->rec.as<IndelRec>(); A.rec_n = cnt + PL_N_REC; A.rec_cap = L->rec_cap;
     A.win_rec = L->winrec.as<uint32_t>();
@@ -1095,7 +1119,7 @@ pl_status run_jobs(pl_ctx* c, Lane* L, const std::vector<JobReq>& reqs, int32_t 
     A.spill_n = cnt + PL_N_SPILL; A.spill_cap = L->spill_cap;
     A.cmask = L->cmask.as<uint64_t>();
     A.prec = L->prec.as<int32_t>();
-    A.cand = L->cand.as<Cand>(); A.cand_n = cnt + PL_N_CAND; A.cand_cap = L->cand_cap;
+    A.cand = L->cands((size_t)n_jobs); A.cand_n = cnt + PL_N_CAND; A.cand_cap = L->cand_cap;
     A.defer = L->defer.as<uint32_t>(); A.defer_n = cnt + PL_N_DEFER; A.defer_cap = L->defer_cap;
     A.mutated = L->mutated.as<uint32_t>(); A.mutated_n = cnt + PL_N_MUTATED; A.mutated_cap = L->mut_cap;
     A.overflow = (int32_t*)(cnt + PL_N_OVERFLOW);
@@ -1133,9 +1157,24 @@ pl_status run_jobs(pl_ctx* c, Lane* L, const std::vector<JobReq>& reqs, int32_t 
       if (s) return s;
       HIPCHK(hipEventRecord(L->ev[1], st));
     }
-    uint32_t hc[PL_COUNTERS];
-    HIPCHK(hipMemcpyAsync(hc, cnt, sizeof hc, hipMemcpyDeviceToHost, st));
+    // results in one wait: counters, stats and the first candidates in one
+    // copy, a small batch's pileup and calls behind them
+    const size_t head = Lane::cand_at((size_t)n_jobs);
+    L->mail_res = head <= PL_MAIL_BYTES / 2 ? std::min(PL_MAIL_BYTES / 2, head + sizeof(Cand) * (size_t)std::min<uint32_t>(L->cand_cap, PL_MAIL_CANDS))
+                                            : 4 * PL_COUNTERS;
+    HIPCHK(hipMemcpyAsync(L->mail, L->res.p, L->mail_res, hipMemcpyDeviceToHost, st));
+    L->mail_pile = L->mail_calls = 0;
+    if (bring && (size_t)G * (4 * PL_NFIELDS + sizeof(pl_call)) <= PL_MAIL_BYTES / 2) {
+      k_final_flags<<<dim3(n_wins), dim3(256), 0, st>>>(A);
+      HIPCHK(hipGetLastError());
+      L->mail_pile = PL_MAIL_BYTES / 2;
+      L->mail_calls = L->mail_pile + 4 * (size_t)PL_NFIELDS * (size_t)G;
+      HIPCHK(hipMemcpyAsync(L->mail + L->mail_pile, L->pile.p, 4 * (size_t)PL_NFIELDS * (size_t)G, hipMemcpyDeviceToHost, st));
+      HIPCHK(hipMemcpyAsync(L->mail + L->mail_calls, L->calls.p, sizeof(pl_call) * (size_t)G, hipMemcpyDeviceToHost, st));
+    }
     HIPCHK(hipStreamSynchronize(st));
+    uint32_t hc[PL_COUNTERS];
+    std::memcpy(hc, L->mail, sizeof hc);
     float ms = 0, wms = -1.0f;
     HIPCHK(hipEventElapsedTime(&ms, L->ev[0], L->ev[1]));
     if (!use_graph) HIPCHK(hipEventElapsedTime(&wms, L->ev[2], L->ev[3]));
@@ -1156,6 +1195,7 @@ pl_status run_jobs(pl_ctx* c, Lane* L, const std::vector<JobReq>& reqs, int32_t 
     fit(hc[PL_N_MUTATED], &L->mut_cap);
     fit(hc[PL_N_WIDE], &L->wide_cap);
     if (!grow) {
+      L->exported_flags = L->mail_pile != 0;
       if (hc[PL_N_OVERFLOW]) return fail(PL_E_DEVICE, "capacity overflow flag set without an overfull counter");
       return PL_OK;
     }
@@ -1216,19 +1256,31 @@ pl_status autotune(pl_ctx* c, Lane* L, const std::vector<JobReq>& q, int persist
 pl_status fetch_batch_meta(Lane* L) {
   const size_t nj = L->hjobs.size();
   L->hst.resize(nj);
-  HIPCHK(hipMemcpyAsync(L->hst.data(), L->st.p, sizeof(JobStat) * nj, hipMemcpyDeviceToHost, L->stream));
-  // (the batch's counters came back with the run)
   const uint32_t cn = std::min(L->last_counts[PL_N_CAND], L->cand_cap);
   L->hcand.resize(cn);
   L->hins_off.assign(cn, -1);
   L->hins_pool.clear();
-  if (cn) HIPCHK(hipMemcpyAsync(L->hcand.data(), L->cand.p, sizeof(Cand) * cn, hipMemcpyDeviceToHost, L->stream));
-  HIPCHK(hipStreamSynchronize(L->stream));
+  // from the mail, and from the device what was not in it
+  const size_t st_end = 4 * PL_COUNTERS + sizeof(JobStat) * nj, c0 = Lane::cand_at(nj);
+  bool wait = false;
+  if (L->mail_res >= st_end) {
+    std::memcpy(L->hst.data(), L->mail + 4 * PL_COUNTERS, sizeof(JobStat) * nj);
+  } else {
+    HIPCHK(hipMemcpyAsync(L->hst.data(), L->stats(), sizeof(JobStat) * nj, hipMemcpyDeviceToHost, L->stream));
+    wait = true;
+  }
+  const uint32_t cm = L->mail_res > c0 ? (uint32_t)std::min<size_t>(cn, (L->mail_res - c0) / sizeof(Cand)) : 0;
+  if (cm) std::memcpy(L->hcand.data(), L->mail + c0, sizeof(Cand) * cm);
+  if (cn > cm) {
+    HIPCHK(hipMemcpyAsync(L->hcand.data() + cm, L->cands(nj) + cm, sizeof(Cand) * (cn - cm), hipMemcpyDeviceToHost, L->stream));
+    wait = true;
+  }
+  if (wait) HIPCHK(hipStreamSynchronize(L->stream));
   if (cn) {
-    // insertion strings of every INS candidate, decoded on the device at once
+    // the insertion strings too long for their candidates, decoded on the device at once
     std::vector<int64_t> idx, off(1, 0);
     for (uint32_t k = 0; k < cn; k++)
-      if (L->hcand[k].kind == PL_D_INS) {
+      if (L->hcand[k].kind == PL_D_INS && L->hcand[k].len > PL_CAND_INS) {
         L->hins_off[k] = off.back();
         idx.push_back(k);
         off.push_back(off.back() + L->hcand[k].len);
@@ -1240,7 +1292,7 @@ pl_status fetch_batch_meta(Lane* L) {
       HIPCHK(hipMemcpyAsync(L->stridx.p, idx.data(), 8 * idx.size(), hipMemcpyHostToDevice, L->stream));
       HIPCHK(hipMemcpyAsync(L->stroff.p, off.data(), 8 * off.size(), hipMemcpyHostToDevice, L->stream));
       k_ins_strings<<<dim3((unsigned)((idx.size() + 63) / 64)), dim3(64), 0, L->stream>>>(
-          L->args, L->cand.as<Cand>(), L->stridx.as<int64_t>(), L->stroff.as<int64_t>(), (int32_t)idx.size(),
+          L->args, L->cands(nj), L->stridx.as<int64_t>(), L->stroff.as<int64_t>(), (int32_t)idx.size(),
           L->strpool.as<uint8_t>());
       HIPCHK(hipGetLastError());
       L->hins_pool.resize((size_t)off.back());
@@ -1278,7 +1330,10 @@ pl_status job_changes(pl_ctx* c, Lane* L, size_t j, pl_region_stats* out, std::v
     x.base = cd.base;
     x.alt = cd.alt;
     if (cd.kind == PL_D_DEL) x.indel.assign((const char*)ct.host.data() + x.loc - 1, (size_t)cd.len);
-    if (cd.kind == PL_D_INS) x.indel = L->hins_pool.substr((size_t)L->hins_off[k], (size_t)cd.len);
+    if (cd.kind == PL_D_INS) {
+      if (cd.len <= PL_CAND_INS) x.indel.assign((const char*)cd.ins, (size_t)cd.len);
+      else x.indel = L->hins_pool.substr((size_t)L->hins_off[k], (size_t)cd.len);
+    }
     ch.push_back(x);
   }
   const ReadSet& rs = *c->rsets[J.rs];
@@ -1303,22 +1358,42 @@ pl_status job_changes(pl_ctx* c, Lane* L, size_t j, pl_region_stats* out, std::v
   return PL_OK;
 }
 
+pl_status final_flags(Lane* L) {
+  if (L->exported_flags) return PL_OK;
+  k_final_flags<<<dim3(L->n_wins), dim3(256), 0, L->stream>>>(L->args);
+  HIPCHK(hipGetLastError());
+  L->exported_flags = true;
+  return PL_OK;
+}
+
 // pileup / final calls of job j of the last batch into host buffers
 pl_status job_export(Lane* L, size_t j, int32_t* pile, pl_call* calls) {
   const JobDev& J = L->hjobs[j];
-  if (calls && !L->exported_flags) {
-    k_final_flags<<<dim3(L->n_wins), dim3(256), 0, L->stream>>>(L->args);
-    HIPCHK(hipGetLastError());
-    L->exported_flags = true;
-  }
+  if (calls) if (pl_status s = final_flags(L)) return s;
   if (pile)
-    for (int f = 0; f < PL_NFIELDS; f++)
-      HIPCHK(hipMemcpyAsync(pile + (size_t)f * J.size, L->pile.as<int32_t>() + (size_t)f * L->G + J.out,
-                            4 * (size_t)J.size, hipMemcpyDeviceToHost, L->stream));
+    HIPCHK(hipMemcpy2DAsync(pile, 4 * (size_t)J.size, L->pile.as<int32_t>() + J.out, 4 * (size_t)L->G, 4 * (size_t)J.size,
+                            PL_NFIELDS, hipMemcpyDeviceToHost, L->stream));
   if (calls)
     HIPCHK(hipMemcpyAsync(calls, L->calls.as<pl_call>() + J.out, sizeof(pl_call) * (size_t)J.size,
                           hipMemcpyDeviceToHost, L->stream));
   HIPCHK(hipStreamSynchronize(L->stream));
+  return PL_OK;
+}
+
+pl_status copy_to_host(Lane* L, void* dst, const void* src, size_t bytes);   // pl_vcf.hip
+
+// pileup / final calls of the whole last batch: its layout is the caller's,
+// so each is one copy
+pl_status export_all(Lane* L, int32_t* pile, pl_call* calls) {
+  const size_t pb = 4 * (size_t)PL_NFIELDS * (size_t)L->G, cb = sizeof(pl_call) * (size_t)L->G;
+  if (L->mail_pile) {
+    if (pile) std::memcpy(pile, L->mail + L->mail_pile, pb);
+    if (calls) std::memcpy(calls, L->mail + L->mail_calls, cb);
+    return PL_OK;
+  }
+  if (calls) if (pl_status s = final_flags(L)) return s;
+  if (pile) if (pl_status s = copy_to_host(L, pile, L->pile.p, pb)) return s;
+  if (calls) if (pl_status s = copy_to_host(L, calls, L->calls.p, cb)) return s;
   return PL_OK;
 }
 
@@ -1434,10 +1509,10 @@ pl_status pl_ctx_create(const pl_config* cfg, int device, pl_ctx** out) {
   c->device = device;
   c->n_cu = prop.multiProcessorCount;
   pl_status st = lane_init(&c->main);
-  if (!st) st = lane_init(&c->aux);
-  if (!st) st = lane_init(&c->na);
+  if (!st) st = lane_init(&c->aux, c->main.mail);
+  if (!st) st = lane_init(&c->na, c->main.mail);
   if (!st) st = scratch_address(device, &c->na_arena.base);
-  if (st) { lane_destroy(&c->main); lane_destroy(&c->aux); lane_destroy(&c->na); return st; }
+  if (st) { lane_destroy(&c->aux); lane_destroy(&c->na); lane_destroy(&c->main); return st; }
   c->na_arena.size = PL_NOALLOC_SCRATCH_BYTES;
   c->na.use_arena(&c->na_arena);
   *out = c.release();
@@ -1447,9 +1522,9 @@ pl_status pl_ctx_create(const pl_config* cfg, int device, pl_ctx** out) {
 void pl_ctx_destroy(pl_ctx* c) {
   if (!c) return;
   (void)hipSetDevice(c->device);
-  lane_destroy(&c->main);
   lane_destroy(&c->aux);
   lane_destroy(&c->na);
+  lane_destroy(&c->main);
   c->rsets.clear();
   for (auto& kv : c->contigs) if (kv.second.dev) (void)hipFree(kv.second.dev);
   c->contigs.clear();
@@ -1589,11 +1664,11 @@ pl_status pl_region_finish(pl_region* r, int32_t* pile, pl_call* calls, pl_regio
     r->batches.clear();
   }
   std::vector<JobReq> q{{id, r->start, r->stop}};
-  pl_status s = run_jobs(c, L, q, PL_DEFAULT_WINDOW, 0, PL_DEFAULT_BLOCK, false);
+  pl_status s = run_jobs(c, L, q, PL_DEFAULT_WINDOW, 0, PL_DEFAULT_BLOCK, false, pile || calls);
   if (!s) s = fetch_batch_meta(L);
   if (!s) s = job_status(L, 0);
   if (!s) s = job_changes(c, L, 0, &r->stats, &r->changes);
-  if (!s) s = job_export(L, 0, pile, calls);
+  if (!s) s = export_all(L, pile, calls);
   if (temp) {
     r->temp = std::move(c->rsets[id]);
     r->temp_id = id;
@@ -1654,20 +1729,7 @@ pl_status batch_outputs(pl_ctx* c, Lane* L, int32_t n, int32_t* pile, pl_call* c
   for (int32_t i = 0; i < n; i++) if ((s = job_status(L, i))) return s;
   if (stats)
     for (int32_t i = 0; i < n; i++) if ((s = job_changes(c, L, i, &stats[i], nullptr))) return s;
-  if (pile || calls) {
-    int64_t off = 0;
-    for (int32_t i = 0; i < n; i++) {
-      const int64_t sz = L->hjobs[i].size;
-      std::vector<int32_t> tmp;
-      if (pile) tmp.resize((size_t)PL_NFIELDS * sz);
-      if ((s = job_export(L, i, pile ? tmp.data() : nullptr, calls ? calls + off : nullptr))) return s;
-      if (pile)
-        for (int f = 0; f < PL_NFIELDS; f++)
-          std::memcpy(pile + (size_t)f * L->G + off, tmp.data() + (size_t)f * sz, 4 * (size_t)sz);
-      off += sz;
-    }
-  }
-  return PL_OK;
+  return export_all(L, pile, calls);
 }
 
 }  // namespace
@@ -1689,7 +1751,7 @@ pl_status pl_batch_run(pl_ctx* c, const pl_region_desc* regions, int32_t n, cons
   if (W == 0 || block == 0) {
     if ((s = autotune(c, L, q, persistent, &W, &block))) return s;
   }
-  if ((s = run_jobs(c, L, q, W, persistent, block, use_graph))) return s;
+  if ((s = run_jobs(c, L, q, W, persistent, block, use_graph, pile || calls))) return s;
   return batch_outputs(c, L, n, pile, calls, stats);
 }
 
@@ -1715,7 +1777,7 @@ pl_status pl_batch_run_noalloc(pl_ctx* c, const pl_region_desc* regions, int32_t
   L->free_buffers();
   c->na_arena.used = 0;
   c->na_arena.exhausted = false;
-  s = run_jobs(c, L, q, W, persistent, block, false);
+  s = run_jobs(c, L, q, W, persistent, block, false, pile || calls);
   if (!s) s = batch_outputs(c, L, n, pile, calls, stats);
   if (s && c->na_arena.exhausted)
     return fail(PL_E_OOM, "the batch's device buffers exceed the %zu-byte scratch array", PL_NOALLOC_SCRATCH_BYTES);
@@ -1739,7 +1801,7 @@ pl_status pl_batch_repeat(pl_ctx* c, int32_t n_passes) {
     L->rep_hc = (uint32_t*)p;
   }
   hipStream_t st = L->stream;
-  const uint32_t* cnt = L->counters.as<uint32_t>();
+  const uint32_t* cnt = L->counters();
   for (int32_t done = 0; done < n_passes;) {
     const int32_t m = std::min<int32_t>(kSlots, n_passes - done);
     HIPCHK(hipEventRecord(L->ev[0], st));

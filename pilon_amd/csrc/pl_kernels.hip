@@ -1678,7 +1678,7 @@ __global__ void __launch_bounds__(64) k_finalize(EngineArgs A) {
 }
 
 // After the deletion pass: the first PL_AFTER_BLOCKS blocks call the columns
-// it changed again, the rest give the exact confirmed count of the regions
+// it changed again and spell the insertions, the rest give the exact confirmed count of the regions
 // whose minDepth lies above the depth histogram (a --mindepth of 256 or more,
 // or a region averaging more than about 2,555x), whose every position is
 // tested.  The two write different things of a position and the count looks
@@ -1690,6 +1690,15 @@ __global__ void __launch_bounds__(256) k_after(EngineArgs A) {
   if (blockIdx.x < PL_AFTER_BLOCKS) {
     const uint32_t n = *A.mutated_n < A.mutated_cap ? *A.mutated_n : A.mutated_cap;
     indel_columns(A, A.mutated, n, 1, (blockIdx.x * blockDim.x + threadIdx.x) >> 6, (PL_AFTER_BLOCKS * blockDim.x) >> 6);
+    // the strings of the insertions that became changes
+    const uint32_t nc = *A.cand_n < A.cand_cap ? *A.cand_n : A.cand_cap;
+    for (uint32_t k = blockIdx.x * blockDim.x + threadIdx.x; k < nc; k += PL_AFTER_BLOCKS * blockDim.x) {
+      Cand& c = A.cand[k];
+      if (c.kind != PL_D_INS || c.len > PL_CAND_INS) continue;
+      const RSDev& R = A.rs[A.jobs[job_of(A.jobs, A.n_jobs, c.gpos)].rs];
+      const IndelRec& e = A.rec[c.rec];
+      for (int32_t q = 0; q < c.len; q++) c.ins[q] = rec_char(R, e, q);
+    }
     return;
   }
   if (*(volatile uint32_t*)A.deep == 0) return;   // no region needs the exact count
@@ -1736,7 +1745,7 @@ __global__ void k_final_flags(EngineArgs A) {
   }
 }
 
-// insertion strings of INS changes into a byte pool
+// the insertion strings too long for their candidate, into a byte pool
 __global__ void k_ins_strings(EngineArgs A, const Cand* sorted, const int64_t* idx, const int64_t* off, int32_t n, uint8_t* pool) {
   const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
