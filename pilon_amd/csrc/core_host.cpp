@@ -342,7 +342,7 @@ void* ch_run(const pl_config* pc, const uint8_t* ref, int64_t ref_len, const cha
     if (pc->longread && !(set_kinds & 1)) plh::exclude_motifs(ch, ref, J.start, J.stop, (set_kinds & 2) != 0);
     std::string nm(name);
     std::string rb((const char*)ref + J.start - 1, (size_t)J.size);
-    plh::FixResult fr = plh::fix_region(*pc, nm, J.start, rb, ch, nm + "_pilon", 0);
+    plh::FixResult fr = plh::fix_region(*pc, nm, J.start, &rb, ch, nm + "_pilon", 0);
     H->changes.push_back(fr.changes);
     H->bases.push_back(fr.bases);
     pl_region_stats& o = stats_out[j];

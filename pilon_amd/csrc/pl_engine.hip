@@ -171,10 +171,10 @@ struct HostReads {
   std::vector<int64_t> cigar_off{0};
   std::vector<uint32_t> cigar;
   std::vector<int64_t> seq_off{0};
-  std::vector<uint8_t> bases2;  // 2-bit codes, one per base here (packed on upload)
+  std::vector<uint8_t> bases2;
   std::vector<int8_t> quals;
   std::vector<int64_t> exo_read, exo_off;
-  std::vector<uint8_t> nibc;    // one nibble code per base of exotic reads
+  std::vector<uint8_t> nib;
 };
 
 }  // namespace
@@ -342,13 +342,35 @@ pl_status region_jump_depth(pl_region* r);   // pl_track.hip
 
 namespace {
 
-pl_status upload(void** dst, const void* src, size_t bytes, size_t pad, std::vector<void*>& mem, hipStream_t s) {
-  HIPCHK(hipMalloc(dst, bytes + pad + 16));
-  mem.push_back(*dst);
-  if (bytes) HIPCHK(hipMemcpyAsync(*dst, src, bytes, hipMemcpyHostToDevice, s));
-  if (pad + 16) HIPCHK(hipMemsetAsync((uint8_t*)*dst + bytes, 0, pad + 16, s));
-  return PL_OK;
-}
+// Device buffers of one call, given back on every exit: to the lane's
+// scratch (calls nest, so the last one begun is the first to end), or freed
+// when they were allocated while a call begun later was still using it.
+struct ScratchBufs {
+  explicit ScratchBufs(Lane* lane) : s(lane->scratch), at(s.at), used(s.used), outer(s.top) { s.top = this; }
+  ~ScratchBufs() {
+    for (void* x : own) (void)hipFree(x);
+    s.top = outer;
+    s.at = at;
+    s.used = used;
+    if (!outer) s.settle();
+  }
+  ScratchBufs(const ScratchBufs&) = delete;
+  ScratchBufs& operator=(const ScratchBufs&) = delete;
+  template <class T> pl_status get(T** out, size_t n) {
+    void* q = nullptr;
+    const hipError_t e = s.top == this ? s.get(n, &q) : hipMalloc(&q, n ? n : 1);
+    if (e != hipSuccess) return fail(PL_E_OOM, "device allocation of %zu bytes failed", n);
+    if (s.top != this) own.push_back(q);
+    *out = (T*)q;
+    return PL_OK;
+  }
+
+ private:
+  Scratch& s;
+  size_t at, used;
+  void* outer;
+  std::vector<void*> own;
+};
 
 pl_status scan_u32(Lane* L, const uint32_t* in, uint32_t* out, int64_t n) {
   const int64_t tiles = std::max<int64_t>(1, (n + SCAN_TILE - 1) / SCAN_TILE);
@@ -420,43 +442,53 @@ pl_status readset_upload(pl_ctx* c, int32_t contig_id, const pl_read_soa* s, int
   const int64_t ncig = s->cigar_off[n];
   const int64_t nb = s->seq_off[n];
   hipStream_t st = L->stream;
-  pl_status e;
+  // everything but the segment table in one allocation, zero where no read
+  // array lies; what only this call needs in the lane's scratch
+  struct Part { const void* src; size_t bytes, at; };
+  size_t size = 0;
+  auto part = [&](const void* src, int64_t bytes, size_t pad) {
+    const Part x{src, (size_t)bytes, size};
+    size = (size + (size_t)bytes + pad + 16 + 255) & ~(size_t)255;
+    return x;
+  };
+  const Part up[] = {part(s->pos, 4 * n, 0), part(s->tlen, 4 * n, 0), part(s->flag, 2 * n, 0), part(s->mapq, n, 0),
+                     part(s->cigar_off, 8 * (n + 1), 0), part(s->cigar, 4 * ncig, 0), part(s->seq_off, 8 * (n + 1), 0),
+                     part(s->bases2, (nb + 3) / 4, 64), part(s->quals, nb, 64), part(s->exo_read, 8 * s->n_exotic, 0),
+                     part(s->exo_off, 8 * s->n_exotic, 0), part(s->nib, s->n_exotic ? nib_bytes(s) : 0, 64),
+                     part(lrt, lrt ? n : 0, 0)};
+  const size_t copied = size;
+  int64_t ocap = 4096 + n / 256;
+  const Part meta = part(nullptr, (int64_t)sizeof(RMeta) * (n + 1), 0), ftail = part(nullptr, (int64_t)sizeof(FragTail) * (n + 1), 0),
+             kp = part(nullptr, 4 * (n + 1), 0), scal = part(nullptr, 64, 0), outs = part(nullptr, 8 * ocap, 0);
   void* p;
-#define UP(field, src, bytes, pad)                                  \
-  if ((e = upload(&p, (src), (size_t)(bytes), (pad), rs->mem, st))) return e; \
-  field = (decltype(field))p;
-  UP(d.pos, s->pos, 4 * n, 0);
-  UP(d.tlen, s->tlen, 4 * n, 0);
-  UP(d.flag, s->flag, 2 * n, 0);
-  UP(d.mapq, s->mapq, n, 0);
-  UP(d.cigar_off, s->cigar_off, 8 * (n + 1), 0);
-  UP(d.cigar, s->cigar, 4 * ncig, 0);
-  UP(d.seq_off, s->seq_off, 8 * (n + 1), 0);
-  UP(d.bases2, s->bases2, (nb + 3) / 4, 64);
-  UP(d.quals, s->quals, nb, 64);
-  UP(d.exo_read, s->exo_read, 8 * s->n_exotic, 0);
-  UP(d.exo_off, s->exo_off, 8 * s->n_exotic, 0);
-  UP(d.nib, s->nib, s->n_exotic ? nib_bytes(s) : 0, 64);
+  HIPCHK(hipMalloc(&p, size));
+  rs->mem.push_back(p);
+  uint8_t* D = (uint8_t*)p;
+  HIPCHK(hipMemsetAsync(D, 0, copied, st));
+  for (const Part& x : up)
+    if (x.bytes) HIPCHK(hipMemcpyAsync(D + x.at, x.src, x.bytes, hipMemcpyHostToDevice, st));
+  d.pos = (const int32_t*)(D + up[0].at); d.tlen = (const int32_t*)(D + up[1].at); d.flag = (const uint16_t*)(D + up[2].at);
+  d.mapq = D + up[3].at; d.cigar_off = (const int64_t*)(D + up[4].at); d.cigar = (const uint32_t*)(D + up[5].at);
+  d.seq_off = (const int64_t*)(D + up[6].at); d.bases2 = D + up[7].at; d.quals = (const int8_t*)(D + up[8].at);
+  d.exo_read = (const int64_t*)(D + up[9].at); d.exo_off = (const int64_t*)(D + up[10].at); d.nib = D + up[11].at;
   if (lrt) {
-    UP(d.lrt, lrt, n, 0);
+    d.lrt = D + up[12].at;
     d.all_long = n > 0 && std::memchr(lrt, 0, (size_t)n) == nullptr;
     d.nano = n > 0 && std::memchr(lrt, PL_LR_NANOPORE, (size_t)n) != nullptr;
   }
-#undef UP
   d.n_exotic = s->n_exotic;
   d.ref = it->second.dev;
   d.ref_len = it->second.len;
-  HIPCHK(hipMalloc(&p, sizeof(RMeta) * (size_t)(n + 1))); rs->mem.push_back(p); d.meta = (RMeta*)p;
-  HIPCHK(hipMalloc(&p, 64)); rs->mem.push_back(p); d.scal = (int32_t*)p;
-  HIPCHK(hipMalloc(&p, sizeof(FragTail) * (size_t)(n + 1))); rs->mem.push_back(p); d.ftail = (FragTail*)p;
+  d.meta = (RMeta*)(D + meta.at);
+  d.scal = (int32_t*)(D + scal.at);
+  d.ftail = (FragTail*)(D + ftail.at);
+  rs->kp = (uint32_t*)(D + kp.at);
+  int64_t* outl = (int64_t*)(D + outs.at);
+  ScratchBufs B(L);
   uint32_t *keepflag, *segcount, *segoff;
-  HIPCHK(hipMalloc(&p, 4 * (size_t)(n + 1))); keepflag = (uint32_t*)p;
-  HIPCHK(hipMalloc(&p, 4 * (size_t)(n + 1))); segcount = (uint32_t*)p;
-  HIPCHK(hipMalloc(&p, 4 * (size_t)(n + 1))); segoff = (uint32_t*)p;
-  HIPCHK(hipMalloc(&p, 4 * (size_t)(n + 1))); rs->mem.push_back(p); rs->kp = (uint32_t*)p;
-  int64_t ocap = 4096 + n / 256;
-  int64_t* outl;
-  HIPCHK(hipMalloc(&p, 8 * (size_t)ocap)); rs->mem.push_back(p); outl = (int64_t*)p;
+  if (pl_status e = B.get(&keepflag, 4 * (size_t)(n + 1))) return e;
+  if (pl_status e = B.get(&segcount, 4 * (size_t)(n + 1))) return e;
+  if (pl_status e = B.get(&segoff, 4 * (size_t)(n + 1))) return e;
   for (int attempt = 0; attempt < 2; attempt++) {
     HIPCHK(hipMemsetAsync(d.scal, 0, 64, st));
     const int64_t blocks = std::min<int64_t>(std::max<int64_t>(1, (n + 255) / 256), 8192);
@@ -495,9 +527,6 @@ pl_status readset_upload(pl_ctx* c, int32_t contig_id, const pl_read_soa* s, int
   d.outliers = outl;
   d.n_outlier = no;
   HIPCHK(hipStreamSynchronize(st));
-  (void)hipFree(keepflag);
-  (void)hipFree(segcount);
-  (void)hipFree(segoff);
   rs->bytes = 4 * n + 4 * n + 2 * n + n + 8 * (n + 1) + 4 * ncig + 8 * (n + 1) + (nb + 3) / 4 + nb + 32 * n + 8 * n + 8 * n;
   c->rsets.push_back(std::move(rs));
   c->rs_version++;
@@ -1397,38 +1426,49 @@ pl_status export_all(Lane* L, int32_t* pile, pl_call* calls) {
   return PL_OK;
 }
 
-void append_reads(HostReads& h, const pl_read_soa* s) {
-  const int64_t n = s->n_reads;
-  const int64_t r0 = (int64_t)h.pos.size();
-  h.pos.insert(h.pos.end(), s->pos, s->pos + n);
-  h.tlen.insert(h.tlen.end(), s->tlen, s->tlen + n);
-  h.flag.insert(h.flag.end(), s->flag, s->flag + n);
-  h.mapq.insert(h.mapq.end(), s->mapq, s->mapq + n);
-  const int64_t c0 = h.cigar_off.back(), s0 = h.seq_off.back();
-  for (int64_t i = 0; i < n; i++) {
-    h.cigar_off.push_back(c0 + s->cigar_off[i + 1]);
-    h.seq_off.push_back(s0 + s->seq_off[i + 1]);
-  }
-  h.cigar.insert(h.cigar.end(), s->cigar, s->cigar + s->cigar_off[n]);
-  const int64_t nb = s->seq_off[n];
-  h.quals.insert(h.quals.end(), s->quals, s->quals + nb);
-  for (int64_t q = 0; q < nb; q++) h.bases2.push_back((s->bases2[q >> 2] >> (2 * (q & 3))) & 3);
-  for (int64_t k = 0; k < s->n_exotic; k++) {
-    const int64_t r = s->exo_read[k];
-    const int64_t L = s->seq_off[r + 1] - s->seq_off[r];
-    h.exo_read.push_back(r0 + r);
-    h.exo_off.push_back((int64_t)h.nibc.size());
-    for (int64_t q = 0; q < L; q++) {
-      const int64_t x = s->exo_off[k] + q;
-      const uint8_t b = s->nib[x >> 1];
-      h.nibc.push_back((x & 1) ? (b & 15) : (b >> 4));
-    }
+// the caller's arrays into h (empty before)
+void copy_reads(HostReads& h, const pl_read_soa* s) {
+  const int64_t n = s->n_reads, nb = s->seq_off[n];
+  h.pos.assign(s->pos, s->pos + n);
+  h.tlen.assign(s->tlen, s->tlen + n);
+  h.flag.assign(s->flag, s->flag + n);
+  h.mapq.assign(s->mapq, s->mapq + n);
+  h.cigar_off.assign(s->cigar_off, s->cigar_off + n + 1);
+  h.seq_off.assign(s->seq_off, s->seq_off + n + 1);
+  h.cigar_off[0] = h.seq_off[0] = 0;
+  h.cigar.assign(s->cigar, s->cigar + s->cigar_off[n]);
+  h.quals.assign(s->quals, s->quals + nb);
+  h.bases2.assign(s->bases2, s->bases2 + (nb + 3) / 4);
+  if (s->n_exotic > 0) {
+    h.exo_read.assign(s->exo_read, s->exo_read + s->n_exotic);
+    h.exo_off.assign(s->exo_off, s->exo_off + s->n_exotic);
+    h.nib.assign(s->nib, s->nib + nib_bytes(s) - 1);
+    h.nib.push_back(0);
   }
 }
 
 // merge the plain-form batches (of PL_BAM_* types) into one coordinate-sorted set and upload it
 pl_status upload_host_batches(pl_ctx* c, int32_t contig, std::vector<HostReads>& bs, const std::vector<int32_t>& types,
                               int32_t* id) {
+  int kinds = 0;
+  for (int32_t t : types) kinds |= (t == PL_BAM_FRAGS ? RS_FRAGS : 0) | (t == PL_BAM_NANOPORE ? RS_NANO : 0);
+  auto long_type = [](int32_t t) { return (uint8_t)(t == PL_BAM_NANOPORE ? PL_LR_NANOPORE : t == PL_BAM_PACBIO ? PL_LR_PACBIO : 0); };
+  // one BAM with reads: its arrays are the set's
+  int32_t only = -1, filled = 0;
+  for (int32_t b = 0; b < (int32_t)bs.size(); b++) if (!bs[b].pos.empty()) { only = b; filled++; }
+  if (filled == 1 && std::adjacent_find(bs[only].exo_read.begin(), bs[only].exo_read.end(), std::greater_equal<int64_t>()) ==
+                         bs[only].exo_read.end()) {
+    const HostReads& h = bs[only];
+    pl_read_soa s;
+    std::memset(&s, 0, sizeof s);
+    s.n_reads = (int64_t)h.pos.size();
+    s.pos = h.pos.data(); s.tlen = h.tlen.data(); s.flag = h.flag.data(); s.mapq = h.mapq.data();
+    s.cigar_off = h.cigar_off.data(); s.cigar = h.cigar.data(); s.seq_off = h.seq_off.data();
+    s.bases2 = h.bases2.data(); s.quals = h.quals.data();
+    s.n_exotic = (int64_t)h.exo_read.size(); s.exo_read = h.exo_read.data(); s.exo_off = h.exo_off.data(); s.nib = h.nib.data();
+    const std::vector<uint8_t> lrt(long_type(types[only]) ? h.pos.size() : 0, long_type(types[only]));
+    return readset_upload(c, contig, &s, id, lrt.empty() ? nullptr : lrt.data(), kinds);
+  }
   struct Ref { int32_t b; int64_t r; };
   std::vector<Ref> order;
   for (int32_t b = 0; b < (int32_t)bs.size(); b++)
@@ -1443,18 +1483,15 @@ pl_status upload_host_batches(pl_ctx* c, int32_t contig, std::vector<HostReads>&
   std::vector<int8_t> quals;
   std::vector<uint8_t> codes, nibc, lrt(n);
   bool any_lr = false;
-  int kinds = 0;
-  for (int32_t t : types) kinds |= (t == PL_BAM_FRAGS ? RS_FRAGS : 0) | (t == PL_BAM_NANOPORE ? RS_NANO : 0);
   for (int64_t i = 0; i < n; i++) {
-    const int32_t t = types[order[i].b];
-    lrt[i] = t == PL_BAM_NANOPORE ? PL_LR_NANOPORE : t == PL_BAM_PACBIO ? PL_LR_PACBIO : 0;
+    lrt[i] = long_type(types[order[i].b]);
     any_lr = any_lr || lrt[i];
     const HostReads& h = bs[order[i].b];
     const int64_t r = order[i].r;
     pos[i] = h.pos[r]; tlen[i] = h.tlen[r]; flag[i] = h.flag[r]; mapq[i] = h.mapq[r];
     cigar.insert(cigar.end(), h.cigar.begin() + h.cigar_off[r], h.cigar.begin() + h.cigar_off[r + 1]);
     quals.insert(quals.end(), h.quals.begin() + h.seq_off[r], h.quals.begin() + h.seq_off[r + 1]);
-    codes.insert(codes.end(), h.bases2.begin() + h.seq_off[r], h.bases2.begin() + h.seq_off[r + 1]);
+    for (int64_t q = h.seq_off[r]; q < h.seq_off[r + 1]; q++) codes.push_back((h.bases2[q >> 2] >> (2 * (q & 3))) & 3);
     cigar_off[i + 1] = (int64_t)cigar.size();
     seq_off[i + 1] = (int64_t)quals.size();
     auto it = std::lower_bound(h.exo_read.begin(), h.exo_read.end(), r);
@@ -1462,7 +1499,8 @@ pl_status upload_host_batches(pl_ctx* c, int32_t contig, std::vector<HostReads>&
       const int64_t k = it - h.exo_read.begin();
       exo_read.push_back(i);
       exo_off.push_back((int64_t)nibc.size());
-      nibc.insert(nibc.end(), h.nibc.begin() + h.exo_off[k], h.nibc.begin() + h.exo_off[k] + (h.seq_off[r + 1] - h.seq_off[r]));
+      for (int64_t q = h.exo_off[k]; q < h.exo_off[k] + (h.seq_off[r + 1] - h.seq_off[r]); q++)
+        nibc.push_back((q & 1) ? (h.nib[q >> 1] & 15) : (h.nib[q >> 1] >> 4));
     }
   }
   std::vector<uint8_t> bases2((codes.size() + 3) / 4 + 8, 0), nib(nibc.size() / 2 + 8, 0);
@@ -1616,7 +1654,7 @@ pl_status pl_region_add_reads_typed(pl_region* r, const pl_read_soa* reads, int3
     if (reads->pos[i] < reads->pos[i - 1]) return fail(PL_E_INVAL, "reads must be coordinate-sorted within a call");
   r->batches.emplace_back();   // one batch per BAM; merged by position at finish
   r->types.push_back(bam_type);
-  if (reads->n_reads > 0) append_reads(r->batches.back(), reads);
+  if (reads->n_reads > 0) copy_reads(r->batches.back(), reads);
   return PL_OK;
 }
 
@@ -1689,7 +1727,7 @@ pl_status pl_region_fix(pl_region* r, const char* new_name, int64_t offset, char
   std::string nn = new_name ? new_name : plh::pilon_name(ct.name);
   // bigFixList holds the reassembly's fixes last found first
   const std::vector<plh::Fix> big(r->big.rbegin(), r->big.rend());
-  plh::FixResult fr = plh::fix_region(r->ctx->pc, ct.name, r->start, rb, r->changes, nn, offset, big);
+  plh::FixResult fr = plh::fix_region(r->ctx->pc, ct.name, r->start, &rb, r->changes, nn, offset, big);
   if (changes_text) {
     *changes_text = (char*)malloc(fr.changes.size() + 1);
     std::memcpy(*changes_text, fr.changes.c_str(), fr.changes.size() + 1);

@@ -89,13 +89,16 @@ inline bool match_target(const std::string& t, std::string* name, int64_t* start
 namespace {
 
 // .changes lines, fixed bases and counts of job j of the lane's last batch
-pl_status job_fix(pl_ctx* c, Lane* L, size_t j, const std::string& new_name, int64_t offset, plh::FixResult* out) {
+// (bases: false for the lines and the change in length alone)
+pl_status job_fix(pl_ctx* c, Lane* L, size_t j, const std::string& new_name, int64_t offset, bool bases,
+                  plh::FixResult* out) {
   std::vector<plh::Change> ch;
   if (pl_status s = job_changes(c, L, j, nullptr, &ch)) return s;
   const JobDev& J = L->hjobs[j];
   const Contig& ct = c->contigs.at(c->rsets[J.rs]->contig);
-  const std::string rb((const char*)ct.host.data() + J.start - 1, (size_t)J.size);
-  *out = plh::fix_region(c->pc, ct.name, J.start, rb, ch, new_name, offset);
+  std::string rb;
+  if (bases) rb.assign((const char*)ct.host.data() + J.start - 1, (size_t)J.size);
+  *out = plh::fix_region(c->pc, ct.name, J.start, bases ? &rb : nullptr, ch, new_name, offset);
   return PL_OK;
 }
 
@@ -132,6 +135,7 @@ pl_status pl_batch_fix(pl_ctx* c, const int32_t* element, int32_t n_element, cha
   const size_t ne = el0.size() - 1;
   // per element: offsets accumulate over its regions (GenomeFile.scala:149-153),
   // so an element's regions are fixed in order by one task; elements in parallel
+  const bool want_bases = fasta_text != nullptr;
   std::vector<std::vector<plh::FixResult>> res(ne);
   std::vector<pl_status> err(ne, PL_OK);
   std::vector<std::string> msg(ne);
@@ -142,13 +146,15 @@ pl_status pl_batch_fix(pl_ctx* c, const int32_t* element, int32_t n_element, cha
       int64_t offset = 0;
       for (size_t j = el0[e]; j < el0[e + 1]; j++) {
         plh::FixResult fr;
-        if (pl_status s = job_fix(c, L, j, nn, offset, &fr)) { err[e] = s; msg[e] = g_err; break; }
-        offset += (int64_t)fr.bases.size() - L->hjobs[j].size;
+        if (pl_status s = job_fix(c, L, j, nn, offset, want_bases, &fr)) { err[e] = s; msg[e] = g_err; break; }
+        offset += fr.delta;
         res[e].push_back(std::move(fr));
       }
     }
   };
-  const unsigned nth = (unsigned)std::min<size_t>(ne, std::max(1u, std::min(16u, std::thread::hardware_concurrency())));
+  // threads where there is work for them: bases to splice, or very many lines
+  const unsigned nth = !want_bases && L->hcand.size() < 20000 ? 1u
+      : (unsigned)std::min<size_t>(ne, std::max(1u, std::min(16u, std::thread::hardware_concurrency())));
   std::vector<std::thread> pool;
   for (unsigned t = 1; t < nth; t++) {
     try { pool.emplace_back(work); } catch (...) { break; }
@@ -162,7 +168,16 @@ pl_status pl_batch_fix(pl_ctx* c, const int32_t* element, int32_t n_element, cha
     if (changes_len) *changes_len = (int64_t)all.size();
     if (changes_text && !(*changes_text = dup_text(all))) return fail(PL_E_OOM, "host allocation failed");
   }
-  if (fasta_text || fasta_len) {
+  if (fasta_len && !fasta_text) {                 // the length fasta_element would give
+    int64_t len = 0;
+    for (size_t e = 0; e < ne; e++) {
+      int64_t nb = 0;
+      for (size_t j = el0[e]; j < el0[e + 1]; j++) nb += L->hjobs[j].size + res[e][j - el0[e]].delta;
+      len += 2 + (int64_t)plh::pilon_name(names[el0[e]]).size() + nb + (nb + 79) / 80;
+    }
+    *fasta_len = len;
+  }
+  if (fasta_text) {
     std::string fa;
     for (size_t e = 0; e < ne; e++) {
       std::string seq;
@@ -170,7 +185,7 @@ pl_status pl_batch_fix(pl_ctx* c, const int32_t* element, int32_t n_element, cha
       plh::fasta_element(fa, plh::pilon_name(names[el0[e]]), seq.data(), seq.size());
     }
     if (fasta_len) *fasta_len = (int64_t)fa.size();
-    if (fasta_text && !(*fasta_text = dup_text(fa))) {
+    if (!(*fasta_text = dup_text(fa))) {
       if (changes_text && *changes_text) { free(*changes_text); *changes_text = nullptr; }
       return fail(PL_E_OOM, "host allocation failed");
     }
@@ -290,7 +305,7 @@ pl_status pl_serve_fetch_fix(pl_server* S, int64_t ticket, const char* new_name,
   const Contig& ct = c->contigs.at(c->rsets[d.job.rs]->contig);
   const std::string rb((const char*)ct.host.data() + d.job.start - 1, (size_t)(d.job.stop - d.job.start + 1));
   const std::string nn = new_name ? std::string(new_name) : plh::pilon_name(ct.name);
-  const plh::FixResult fr = plh::fix_region(c->pc, ct.name, d.job.start, rb, d.changes, nn, offset);
+  const plh::FixResult fr = plh::fix_region(c->pc, ct.name, d.job.start, &rb, d.changes, nn, offset);
   if (changes_len) *changes_len = (int64_t)fr.changes.size();
   if (bases_len) *bases_len = (int64_t)fr.bases.size();
   if (changes_text && !(*changes_text = dup_text(fr.changes))) return fail(PL_E_OOM, "host allocation failed");

@@ -89,9 +89,13 @@ inline std::vector<Fix> fix_fix_list(std::vector<Fix> in) {
 // kept fixes right to left; they are sorted and no two overlap (each starts
 // after the last base its predecessor replaces), so one left-to-right splice
 // gives the same bases in time linear in the region.
-inline void apply_fixes(std::string& bases, int32_t region_start, const std::vector<Fix>& list) {
+// Returns the change in length; bases null: that alone.
+inline int64_t apply_fixes(std::string* bases_out, int32_t region_start, const std::vector<Fix>& list) {
   const std::vector<Fix> kept = fix_fix_list(list);
-  if (kept.empty()) return;
+  int64_t delta = 0;
+  for (const Fix& f : kept) delta += (int64_t)f.patch.size() - (int64_t)f.was.size();
+  if (kept.empty() || !bases_out) return delta;
+  std::string& bases = *bases_out;
   std::string out;
   out.reserve(bases.size() + 64);
   size_t at = 0;
@@ -103,6 +107,7 @@ inline void apply_fixes(std::string& bases, int32_t region_start, const std::vec
   }
   out.append(bases, at, std::string::npos);
   bases.swap(out);
+  return delta;
 }
 
 // GenomeFile.processRegions' newName (GenomeFile.scala:137-140): name + sep +
@@ -119,7 +124,7 @@ inline std::string region_string(const std::string& name, int64_t s, int64_t e) 
   return name + buf;
 }
 
-struct FixResult { std::string changes, bases; int snps = 0, amb = 0, ins = 0, ins_bases = 0, dels = 0, del_bases = 0; };
+struct FixResult { std::string changes, bases; int64_t delta = 0; int snps = 0, amb = 0, ins = 0, ins_bases = 0, dels = 0, del_bases = 0; };
 
 // identifyAndFixIssues' snpFixList and smallFixList (GenomeRegion.scala:
 // 307-355), each in List order (the last one prepended first), with the
@@ -165,25 +170,27 @@ inline std::string snp_fixed_bases(const pl_config& cf, int32_t start, const std
   FixResult R;
   fix_lists(cf, changes, snp, small, R);
   std::string b = region_bases;
-  apply_fixes(b, start, snp);
+  apply_fixes(&b, start, snp);
   return b;
 }
 
 // identifyAndFixIssues for one region (GenomeRegion.scala:307-413): the
 // snps/indels fixes, with big (bigFixList, in List order: the reassembly
 // fixes, the last one found first) applied after them, and writeChanges
-// (:645-657).  region_bases is contigBases[start-1 .. stop-1].
+// (:645-657).  region_bases is contigBases[start-1 .. stop-1] (null: only
+// the changes and the change in length are wanted).
 inline FixResult fix_region(const pl_config& cf, const std::string& name, int32_t start,
-                            const std::string& region_bases, const std::vector<Change>& changes,
+                            const std::string* region_bases, const std::vector<Change>& changes,
                             const std::string& new_name, int64_t offset, const std::vector<Fix>& big = {}) {
   FixResult R;
   std::vector<Fix> snp, small;
   fix_lists(cf, changes, snp, small, R);
-  R.bases = region_bases;
-  apply_fixes(R.bases, start, snp);
+  std::string* bases = region_bases ? &R.bases : nullptr;
+  if (bases) *bases = *region_bases;
+  R.delta = apply_fixes(bases, start, snp);
   std::vector<Fix> later = small;                  // fixIssues(smallFixList ++ bigFixList)
   later.insert(later.end(), big.begin(), big.end());
-  apply_fixes(R.bases, start, later);
+  R.delta += apply_fixes(bases, start, later);
   std::vector<Fix> all = snp;
   all.insert(all.end(), later.begin(), later.end());
   int64_t delta = 0;

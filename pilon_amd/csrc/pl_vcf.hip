@@ -5,36 +5,6 @@
 
 namespace {
 
-// Device buffers of one call, given back on every exit: to the lane's
-// scratch (calls nest, so the last one begun is the first to end), or freed
-// when they were allocated while a call begun later was still using it.
-struct ScratchBufs {
-  explicit ScratchBufs(Lane* lane) : s(lane->scratch), at(s.at), used(s.used), outer(s.top) { s.top = this; }
-  ~ScratchBufs() {
-    for (void* x : own) (void)hipFree(x);
-    s.top = outer;
-    s.at = at;
-    s.used = used;
-    if (!outer) s.settle();
-  }
-  ScratchBufs(const ScratchBufs&) = delete;
-  ScratchBufs& operator=(const ScratchBufs&) = delete;
-  template <class T> pl_status get(T** out, size_t n) {
-    void* q = nullptr;
-    const hipError_t e = s.top == this ? s.get(n, &q) : hipMalloc(&q, n ? n : 1);
-    if (e != hipSuccess) return fail(PL_E_OOM, "device allocation of %zu bytes failed", n);
-    if (s.top != this) own.push_back(q);
-    *out = (T*)q;
-    return PL_OK;
-  }
-
- private:
-  Scratch& s;
-  size_t at, used;
-  void* outer;
-  std::vector<void*> own;
-};
-
 void add_line(std::string& s, const std::string& l) { s += l; s += '\n'; }
 
 constexpr size_t kStageChunk = (size_t)32 << 20;

@@ -63,8 +63,9 @@ def test_candidates_over_many_blocks():
     """Contigs whose candidate masks fill several list blocks, more windows
     than the launch holds at once (cost order), regions of a single locus
     among them: every region's changes in order."""
+    import ctypes as C
     from oracle import oracle as O
-    from pilon_amd.engine import Context
+    from pilon_amd.engine import Context, lib
     from pilon_amd.synth import SynthData, preset
     p = preset("c3", scale=0.01)
     p.update(coverage=25, snv_rate=0.01, indel_rate=0.002, lens=p["lens"] + [300_001])
@@ -80,6 +81,11 @@ def test_candidates_over_many_blocks():
         regions = [(i, 1, len(d.draft(i)), ids[i]) for i in range(d.n)] + [(0, 500, 500, ids[0])]
         _, _, stats = ctx.batch_run(regions, window=64, block=256, persistent=1, copy_out=False)
         changes, fasta = ctx.batch_fix(element=list(range(len(regions))))
+        el = np.arange(len(regions), dtype=np.int32)
+        ptr, clen, flen = C.c_void_p(), C.c_int64(), C.c_int64()
+        assert lib().pl_batch_fix(ctx.h, el.ctypes.data, len(el), C.byref(ptr), C.byref(clen), None, C.byref(flen)) == 0
+        assert C.string_at(ptr, clen.value).decode() == changes and flen.value == len(fasta)
+        lib().pl_free(ptr)
     finally:
         ctx.close()
     want_c = ""
