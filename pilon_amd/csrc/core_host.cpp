@@ -28,6 +28,7 @@ struct HostSink {
   void frag(int p, int d, int32_t size) { pc[p] = j_add(pc[p], d); is[p] = j_add(is[p], size); }
   void aligned(int n) { aligned_n += n; }
   void base(int p, int b, int32_t q, int32_t mq1) { bs[b * W + p] += pack_base(q, mq1); mqq[p] += pack_mq_q(mq1, q); }
+  void slide(int p, int b, int32_t q, int32_t mq1) { base(p, b, q, mq1); }
   void count_base() { bcount++; }
   void bad(int p, int n) { bad_[p] += (uint32_t)n; }
   void clip(int p) { clp_[p] += 1; }
@@ -235,6 +236,32 @@ void* ch_run(const pl_config* pc, const uint8_t* ref, int64_t ref_len, const cha
         const int64_t g = J.out + p0 + p;
         PosOut o;
         finalize_position(b4, mqq[p], insA[p], delA[p], badA[p], clpA[p], apc, ais, ref[L0 + p - 1], cf, o);
+        // the same column through the narrow counters, when it fits them
+        if (cf.min_qual >= 0 && o.f[PL_F_INSERTIONS] <= PL_NARROW_MAX && o.f[PL_F_DELETIONS] <= PL_NARROW_MAX) {
+          NarrowCol N;
+          N.m0 = 1 + (int32_t)(g % 61);
+          N.mqcorr = o.f[PL_F_MQSUM] - o.f[PL_F_DELQUAL];
+          N.qsum = o.f[PL_F_QSUM];
+          bool fits = !o.wide && o.f[PL_F_INSQUAL] >= 0 && o.f[PL_F_DELQUAL] >= 0;
+          int64_t depth = 0;
+          for (int b = 0; b < 4; b++) {
+            const int64_t n1 = (uint32_t)o.f[PL_F_COUNT_A + b], sq = std::min<int64_t>(o.qs[b] / N.m0, n1 * 127);
+            fits = fits && sq >= 0;
+            depth += n1;
+            N.cell[b] = (uint32_t)(n1 << PL_NARROW_SHIFT) | (uint32_t)sq;
+            N.qcorr[b] = (int32_t)(o.qs[b] - N.m0 * sq);
+            N.mqcorr -= N.m0 * (int32_t)n1;
+            N.qsum -= (int32_t)sq;
+          }
+          N.ins = ((uint32_t)o.f[PL_F_INSERTIONS] << PL_NARROW_SHIFT) | (uint32_t)o.f[PL_F_INSQUAL];
+          N.del = ((uint32_t)o.f[PL_F_DELETIONS] << PL_NARROW_SHIFT) | (uint32_t)o.f[PL_F_DELQUAL];
+          N.clips = clpA[p]; N.bad = badA[p]; N.pc = apc; N.is = ais;
+          if (fits && depth + o.f[PL_F_INSERTIONS] + o.f[PL_F_DELETIONS] <= PL_NARROW_MAX) {
+            PosOut w = o;
+            finalize_narrow(N, ref[L0 + p - 1], cf, o);
+            std::memcpy(o.qs, w.qs, sizeof o.qs);
+          }
+        }
         if (o.overflow) S.overflow = 1;
         if (o.wide) {
           o.call.flags |= PL_CF_WIDE;

@@ -91,6 +91,7 @@ struct RSDev {               // one resident read set (one contig, sorted by pos
   int64_t* outliers;         // ascending read indices
   int32_t* scal;             // [0]=max_back [1]=max_lead [2]=max_qspan [3]=n_outlier(int)
                              // [6]=max_back of the pileup footprints alone
+                             // [7]=some read has more than two clips
   FragTail* ftail;           // [n] per read
   int32_t all_long;          // every read is a long read
   int32_t nano;              // some read is a nanopore read
@@ -112,7 +113,8 @@ struct WinDev {
   int32_t order;             // position in the work queue
   int64_t lo, hi;            // reads whose pos is in [locus(p0)-back, locus(p1)+lead)
   int64_t plo;               // reads in [lo, plo) reach the window only through their fragments
-  int64_t pad_;
+  int32_t m0;                // adjMq + 1 of most of a sample of the reads in [plo, hi)
+  int32_t pad_;
 };
 
 // What the window kernel needs about one window and its region, in the
@@ -123,7 +125,8 @@ struct __attribute__((aligned(16))) WinHead {
   int64_t lo, hi, plo;       // read ranges (WinDev)
   int64_t out;               // the region's first batch position
   int32_t rs, start, stop, qs, qe;   // read set and JobDev bounds
-  int32_t pad[3];
+  int32_t m0;                        // adjMq + 1 of most of a sample of its reads
+  int32_t pad[2];
 };
 
 struct JobStat {             // device-written per job
@@ -201,5 +204,6 @@ struct EngineArgs {
   int32_t* overflow;                // capacity overflow flag
   struct WideCol* wide; uint32_t* wide_n; uint32_t wide_cap;   // exact sums of wide columns
   int32_t* win_wide;                // [2 * n_wins]: each window's first wide entry and count
+  WinHead* wheads; uint32_t* wide_wins; int32_t* wqueue;   // windows beyond the narrow counters, and their queue
   uint32_t* deep;                   // set when some region's minDepth is above the confirmed histogram
 };

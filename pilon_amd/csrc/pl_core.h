@@ -151,7 +151,7 @@ PL_HD uint32_t del_hash(const uint8_t* ref, int64_t off, int32_t len, uint32_t* 
 // (PileUpRegion.scala:107,139-141), the span of positions the read can touch
 // (M bases, soft clips, slid indels) and its physical-coverage fragment
 // (physCovIncr, PileUpRegion.scala:62-73).
-struct PrepOut { RMeta m; int32_t events; };
+struct PrepOut { RMeta m; int32_t events; bool clips; };   // clips: more than two S ops
 
 PL_HD PrepOut prep_read(const RSDev& R, int64_t r, const KConf& cf) {
   PrepOut o;
@@ -162,7 +162,7 @@ PL_HD PrepOut prep_read(const RSDev& R, int64_t r, const KConf& cf) {
   const int64_t c0 = R.cigar_off[r], c1 = R.cigar_off[r + 1];
   const int32_t L = (int32_t)(R.seq_off[r + 1] - R.seq_off[r]);
   uint32_t info = 0;
-  int32_t refLen = 0, readLen = 0, clipped = 0, nP = 0;
+  int32_t refLen = 0, readLen = 0, clipped = 0, nP = 0, nS = 0;
   bool bad = false, hasS = false;
   for (int64_t k = c0; k < c1; k++) {
     uint32_t w = R.cigar[k];
@@ -171,7 +171,7 @@ PL_HD PrepOut prep_read(const RSDev& R, int64_t r, const KConf& cf) {
     if (op > 8) bad = true;
     if (consumes_ref(op)) refLen += ln;
     if (consumes_read(op)) readLen += ln;
-    if (op == 4) { clipped = j_add(clipped, ln); hasS = true; }
+    if (op == 4) { clipped = j_add(clipped, ln); hasS = true; nS++; }
     if (op == 6) nP++;
   }
   if (L > 0 && readLen != L) bad = true;
@@ -243,6 +243,7 @@ PL_HD PrepOut prep_read(const RSDev& R, int64_t r, const KConf& cf) {
   o.m.pos = pos; o.m.info = info; o.m.fp_lo = lo; o.m.fp_hi = hi;
   o.m.fr_lo = flo; o.m.fr_hi = fhi; o.m.aend = aend; o.m.op0 = op0;
   o.events = events;
+  o.clips = nS > 2;
   return o;
 }
 
@@ -316,7 +317,7 @@ PL_HD void del_event(const RSDev& R, const JobDev& J, const KConf& cf, const Rea
       if (t >= L0 && t < L1) {
         const int b = a.bi(rl);
         const int32_t q = a.qual(rl);
-        if (b >= 0 && q >= cf.min_qual) s.base(t - L0, b, q, mq1);
+        if (b >= 0 && q >= cf.min_qual) s.slide(t - L0, b, q, mq1);
         s.count_base();
       }
     }
@@ -758,7 +759,7 @@ PL_HD int seg_apply(const RSDev& R, const JobDev& J, const KConf& cf, int64_t r,
     const int32_t dl = g.locus, t = g.locus + g.len;
     if (dgate && dl >= J.start && dl <= J.stop && t >= J.start && t <= J.stop && t >= L0 && t < L1) {
       const int32_t q = seg_qual(g);
-      if (g.fin >= 0 && q >= cf.min_qual) s.base(t - L0, g.fin, q, mq1);
+      if (g.fin >= 0 && q >= cf.min_qual) s.slide(t - L0, g.fin, q, mq1);
       s.count_base();
     }
   }
@@ -1105,6 +1106,92 @@ PL_HD void finalize_position(const uint64_t bs[4], uint64_t mqq, uint64_t ins, u
   int need = indel_kind_needed(c, cf, &pct);
   o.defer = need != 0;
   o.call = make_call(bf, 0, true, refb, cf);
+}
+
+// ------------------------------------------------------- narrow counters
+// A window of at most PL_NARROW_MAX reads and events holds a column in 32-bit
+// words: per base count << 20 | sum of quals (quals 0..127), insertions and
+// deletions count << 20 | mqSum (adjMq + 1 at most 256 each).  Most reads of a
+// window share one adjMq + 1, m0: a base of theirs costs one 32-bit add, and
+// qualSum = m0 * (sum of quals); others add their difference from m0.
+#define PL_NARROW_MAX 4095
+#define PL_NARROW_SHIFT 20
+#define PL_NARROW_LOW ((1u << PL_NARROW_SHIFT) - 1u)
+struct NarrowCol {
+  uint32_t cell[4];
+  int32_t qcorr[4];          // sum over other reads' bases of (mq1 - m0) * qual
+  int32_t mqcorr;            // ... of mq1 - m0
+  int32_t qsum;              // quals of the column's insertions and deletions
+  uint32_t ins, del;
+  uint32_t clips, bad;
+  int32_t pc, is;
+  int32_t m0;
+};
+
+// finalize_position from narrow counters: the same column in 32-bit
+// arithmetic (qualSums are at most 4095 * 127 * 256, their sum four times that).
+PL_HD void finalize_narrow(const NarrowCol& N, uint8_t refb, const KConf& cf, PosOut& o) {
+  o.overflow = false;
+  o.wide = false;
+  int32_t n = 0, mqSum = N.mqcorr, qSum = N.qsum;
+  int32_t qs[4], bc[4];
+  for (int b = 0; b < 4; b++) {
+    bc[b] = (int32_t)(N.cell[b] >> PL_NARROW_SHIFT);
+    const int32_t sq = (int32_t)(N.cell[b] & PL_NARROW_LOW);
+    qs[b] = N.m0 * sq + N.qcorr[b];
+    n += bc[b];
+    qSum += sq;
+    o.f[PL_F_COUNT_A + b] = bc[b];
+    o.f[PL_F_QUAL_A + b] = qs[b];
+  }
+  const int32_t insertions = (int32_t)(N.ins >> PL_NARROW_SHIFT), insQual = (int32_t)(N.ins & PL_NARROW_LOW);
+  const int32_t deletions = (int32_t)(N.del >> PL_NARROW_SHIFT), delQual = (int32_t)(N.del & PL_NARROW_LOW);
+  mqSum += N.m0 * n + delQual;
+  o.f[PL_F_MQSUM] = mqSum;
+  o.f[PL_F_QSUM] = qSum;
+  o.f[PL_F_PHYSCOV] = N.pc;
+  o.f[PL_F_INSERTSIZE] = N.pc > 0 ? j_div(N.is, N.pc) : N.is;
+  o.f[PL_F_BADPAIR] = (int32_t)N.bad;
+  o.f[PL_F_DELETIONS] = deletions;
+  o.f[PL_F_DELQUAL] = delQual;
+  o.f[PL_F_INSERTIONS] = insertions;
+  o.f[PL_F_INSQUAL] = insQual;
+  o.f[PL_F_CLIPS] = (int32_t)N.clips;
+  // base_facts
+  const bool byq = qSum > 0;
+  const int32_t s0 = byq ? qs[0] : bc[0], s1 = byq ? qs[1] : bc[1], s2 = byq ? qs[2] : bc[2], s3 = byq ? qs[3] : bc[3];
+  const int r0 = (s1 > s0) + (s2 > s0) + (s3 > s0);
+  const int r1 = (s0 >= s1) + (s2 > s1) + (s3 > s1);
+  const int r2 = (s0 >= s2) + (s1 >= s2) + (s3 > s2);
+  const int o0 = r0 == 0 ? 0 : r1 == 0 ? 1 : r2 == 0 ? 2 : 3;
+  const int o1 = r0 == 1 ? 0 : r1 == 1 ? 1 : r2 == 1 ? 2 : 3;
+  const int32_t q0 = o0 == 0 ? qs[0] : o0 == 1 ? qs[1] : o0 == 2 ? qs[2] : qs[3];
+  const int32_t q1 = o1 == 0 ? qs[0] : o1 == 1 ? qs[1] : o1 == 2 ? qs[2] : qs[3];
+  const int32_t total = qs[0] + qs[1] + qs[2] + qs[3], half = total / 2;
+  const int32_t homoScore = q0 - (total - q0);
+  const int32_t d0 = half > q0 ? half - q0 : q0 - half, d1 = half > q1 ? half - q1 : q1 - half;
+  const int32_t heteroScore = total - d0 - d1;
+  const int32_t dd = homoScore > heteroScore ? homoScore - heteroScore : heteroScore - homoScore;
+  const uint64_t num = (uint64_t)(uint32_t)dd * (uint32_t)n;
+  BaseFacts f;
+  f.base = n > 0 ? o0 : 4;
+  f.alt = o1;
+  f.homo = homoScore >= heteroScore;
+  if (mqSum <= 0) f.score = 0;
+  else if (num <= 0xffffffffull) f.score = (int64_t)((uint32_t)num / (uint32_t)mqSum);
+  else f.score = (int64_t)(num / (uint64_t)mqSum);
+  // (score is below 2^31: num / mqSum <= dd as mqSum >= n)
+  f.q = n > 0 ? (int64_t)((uint32_t)f.score / (uint32_t)n) : 0;
+  o.defer = false;
+  if ((insertions > 2 && insertions > deletions) || (deletions > 2 && deletions > insertions)) {
+    Col c;
+    for (int b = 0; b < 4; b++) { c.bc[b] = bc[b]; c.qs[b] = qs[b]; }
+    c.mqSum = mqSum; c.qSum = qSum; c.deletions = deletions; c.insertions = insertions;
+    c.insQual = insQual; c.delQual = delQual;
+    int32_t pct;
+    o.defer = indel_kind_needed(c, cf, &pct) != 0;
+  }
+  o.call = make_call(f, 0, true, refb, cf);
 }
 
 // The full BaseCall of one position from the pileup and its sorted evidence

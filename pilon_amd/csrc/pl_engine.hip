@@ -181,6 +181,7 @@ struct HostReads {
 
 // the batch's device counters (EngineArgs points into them)
 enum { PL_N_REC = 0, PL_N_CAND, PL_N_DEFER, PL_N_MUTATED, PL_N_OVERFLOW, PL_N_QUEUE, PL_N_WIDE, PL_N_DEEP, PL_N_SPILL,
+       PL_N_WIDE_WINS, PL_N_WIDE_QUEUE,
        PL_COUNTERS = 16 };
 
 // One independent batch pipeline: its stream, events, device buffers and
@@ -192,7 +193,7 @@ struct Lane {
   hipStream_t stream = nullptr;
   hipEvent_t ev[4] = {};
   DBuf rsarr, kparr, jobs, wins, cost, bins, pile, calls, prec, cmask, csums, res, dhist, rec, winrec, spill,
-      spillat, defer, mutated, strpool, stridx, stroff, wide, winwide, heads;
+      spillat, defer, mutated, strpool, stridx, stroff, wide, winwide, heads, wheads;
   DBuf hist, tiles;                // sort and scan scratch (uploads, K-mers)
   // res holds what the host needs of a batch, one copy's worth: the counters,
   // the regions' JobStat, the candidates
@@ -248,7 +249,7 @@ struct Lane {
   template <class F> void for_each_buffer(F&& f) {
     DBuf* b[] = {&rsarr, &kparr, &jobs, &wins, &cost, &bins, &pile, &calls, &prec, &cmask, &csums, &res, &dhist, &rec,
                  &winrec, &spill, &spillat, &defer, &mutated, &strpool, &stridx, &stroff,
-                 &wide, &winwide, &heads, &hist, &tiles, &jdepth};
+                 &wide, &winwide, &heads, &wheads, &hist, &tiles, &jdepth};
     for (DBuf* x : b) f(*x);
   }
   size_t device_bytes() {
@@ -910,17 +911,6 @@ pl_status readsets_upload_many(pl_ctx* c, int32_t n_sets, const int32_t* contig_
   return prep_sets(c, rs, ncig, nb, out_ids);
 }
 
-// Everything a captured graph bakes in: the kernel arguments (buffer
-// pointers, capacities, sizes) and the launch shapes.  A replay is valid
-// only while all of it is unchanged.
-struct GraphKey {
-  EngineArgs A;
-  int32_t W, block, persistent, grid;
-  uint64_t lds;
-  const void* bufs[2];
-  void (*wk)(EngineArgs, int);
-};
-
 void drop_graph(Lane* L) {
   if (L->gexec) (void)hipGraphExecDestroy(L->gexec);
   if (L->graph) (void)hipGraphDestroy(L->graph);
@@ -963,15 +953,34 @@ void lane_destroy(Lane* L) {
 }
 
 typedef void (*WindowKernel)(EngineArgs, int);
-WindowKernel window_kernel(int block, bool lng) {
-  if (lng) return block == 256 ? k_window<256, true> : block == 512 ? k_window<512, true> : k_window<1024, true>;
-  return block == 256 ? k_window<256, false> : block == 512 ? k_window<512, false> : k_window<1024, false>;
+WindowKernel window_kernel(int block, bool lng, bool narrow) {
+  if (lng) return block == 256 ? k_window<256, true, false> : block == 512 ? k_window<512, true, false> : k_window<1024, true, false>;
+  if (narrow)
+    return block == 256 ? k_window<256, false, true> : block == 512 ? k_window<512, false, true> : k_window<1024, false, true>;
+  return block == 256 ? k_window<256, false, false> : block == 512 ? k_window<512, false, false> : k_window<1024, false, false>;
 }
+
+// How a batch's windows are piled: the kernel and its launch, and for the
+// narrow form the wide launch of the windows it leaves.
+struct WindowLaunch {
+  WindowKernel wk = nullptr, wide = nullptr;
+  int block = 0, grid = 0, wide_block = 0, wide_grid = 0;
+  size_t lds = 0, wide_lds = 0;
+};
+
+// Everything a captured graph bakes in: the kernel arguments (buffer
+// pointers, capacities, sizes) and the launch shapes.  A replay is valid
+// only while all of it is unchanged.
+struct GraphKey {
+  EngineArgs A;
+  int32_t W, persistent;
+  const void* bufs[2];
+  WindowLaunch wl;
+};
 
 // the device pipeline of one batch, enqueued on the lane's stream; with
 // timed set, events bracket the window kernel (not while capturing)
-pl_status enqueue_batch(Lane* L, EngineArgs& A, WindowKernel wk, int persistent, int block, int grid, size_t lds,
-                        bool timed) {
+pl_status enqueue_batch(Lane* L, EngineArgs& A, const WindowLaunch& wl, int persistent, bool timed) {
   hipStream_t st = L->stream;
   const int32_t n_jobs = A.n_jobs, n_wins = A.n_wins;
   const unsigned jb = (unsigned)(n_jobs + 3) / 4, pb = (unsigned)(n_wins + 15) / 16;
@@ -979,7 +988,7 @@ pl_status enqueue_batch(Lane* L, EngineArgs& A, WindowKernel wk, int persistent,
   const uint32_t* const* kp = (const uint32_t* const*)L->kparr.p;
   uint32_t* cnt = L->counters();
   // windows in their own order need no cost order: one launch prepares everything
-  const bool ordered = persistent && n_wins > grid;
+  const bool ordered = persistent && n_wins > wl.grid;
   k_begin<<<dim3(1 + jb + (ordered ? 0 : pb)), dim3(256), 0, st>>>(A, kp, cnt, PL_COUNTERS, wins, ordered ? 0 : 1);
   if (ordered) {
     k_plan<<<dim3(pb), dim3(256), 0, st>>>(A, wins);
@@ -987,7 +996,8 @@ pl_status enqueue_batch(Lane* L, EngineArgs& A, WindowKernel wk, int persistent,
   }
   HIPCHK(hipGetLastError());
   if (timed) HIPCHK(hipEventRecord(L->ev[2], st));
-  wk<<<dim3(grid), dim3(block), lds, st>>>(A, persistent);
+  wl.wk<<<dim3(wl.grid), dim3(wl.block), wl.lds, st>>>(A, persistent ? 1 : 0);
+  if (wl.wide) wl.wide<<<dim3(wl.wide_grid), dim3(wl.wide_block), wl.wide_lds, st>>>(A, 2);
   HIPCHK(hipGetLastError());
   if (timed) HIPCHK(hipEventRecord(L->ev[3], st));
   // the deferred columns, the candidates in order, Pass 1 per region
@@ -1005,10 +1015,12 @@ pl_status enqueue_batch(Lane* L, EngineArgs& A, WindowKernel wk, int persistent,
 }
 
 // LDS the window kernel needs for a window of W positions (dynamic part)
-size_t window_lds(int32_t W) { return PL_WIN_LDS_PER_POS * (size_t)W + 1024; }
+size_t window_lds(int32_t W, bool narrow = false) {
+  return (narrow ? PL_NARROW_LDS_PER_POS : PL_WIN_LDS_PER_POS) * (size_t)W + 4 * PL_HIST;
+}
 // ... and per workgroup in total, with the per-wave run tables
-size_t window_lds_total(int32_t W, int block) {
-  return window_lds(W) + 32 * (size_t)block + 1024 + sizeof(IndelRec) * PL_WIN_RECS;
+size_t window_lds_total(int32_t W, int block, bool narrow = false) {
+  return window_lds(W, narrow) + 32 * (size_t)block + 1024 + sizeof(IndelRec) * PL_WIN_RECS;
 }
 
 // bring: the caller wants the pileup and calls of a small batch (those that
@@ -1086,6 +1098,7 @@ pl_status run_jobs(pl_ctx* c, Lane* L, const std::vector<JobReq>& reqs, int32_t 
   HIPCHK(L->winwide.ensure(8 * (size_t)n_wins));
   HIPCHK(L->winrec.ensure(8 * (size_t)n_wins));
   HIPCHK(L->heads.ensure(sizeof(WinHead) * (size_t)n_wins));
+  HIPCHK(L->wheads.ensure(sizeof(WinHead) * (size_t)n_wins));
   HIPCHK(L->cost.ensure((size_t)n_wins));
   HIPCHK(L->bins.ensure(8 * PL_COST_BINS));
   HIPCHK(L->cmask.ensure(8 * (size_t)n_wins * (size_t)(W / 64)));
@@ -1101,18 +1114,27 @@ pl_status run_jobs(pl_ctx* c, Lane* L, const std::vector<JobReq>& reqs, int32_t 
     L->last_reqs = reqs;
     L->tables_valid = true;
   }
-  const size_t lds = window_lds(W);
   bool lng = false;
   for (const JobReq& q : reqs) lng = lng || (c->rsets[q.rs] && c->rsets[q.rs]->d.lrt);
-  const WindowKernel wk = window_kernel(block, lng);
-  HIPCHK(hipFuncSetAttribute((const void*)wk, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-  int grid = n_wins;
-  if (persistent) {
-    // workgroups per CU: LDS (dynamic + static run tables) and 32 waves
-    const int by_lds = (int)(160 * 1024 / window_lds_total(W, block));
-    const int by_waves = 32 / (block / 64);
-    const int per_cu = std::max(1, std::min(by_lds, by_waves));
-    grid = std::min(n_wins, c->n_cu * per_cu);
+  // 32-bit counters hold quals of 0 and more, which minQual >= 0 leaves
+  const bool narrow = !lng && c->cf.min_qual >= 0;
+  auto workgroups = [&](int blk, bool nar) {
+    // per CU: LDS (dynamic + static run tables) and 32 waves
+    return std::max(1, std::min((int)(160 * 1024 / window_lds_total(W, blk, nar)), 32 / (blk / 64)));
+  };
+  WindowLaunch wl;
+  wl.wk = window_kernel(block, lng, narrow);
+  wl.block = block;
+  wl.lds = window_lds(W, narrow);
+  wl.grid = persistent ? std::min(n_wins, c->n_cu * workgroups(block, narrow)) : n_wins;
+  HIPCHK(hipFuncSetAttribute((const void*)wl.wk, hipFuncAttributeMaxDynamicSharedMemorySize, (int)wl.lds));
+  if (narrow) {
+    // the windows left are few and deep: 16 waves each where the LDS allows
+    wl.wide_block = window_lds_total(W, 1024) <= 160 * 1024 ? 1024 : block;
+    wl.wide = window_kernel(wl.wide_block, false, false);
+    wl.wide_lds = window_lds(W);
+    wl.wide_grid = std::min(n_wins, c->n_cu * workgroups(wl.wide_block, false));
+    HIPCHK(hipFuncSetAttribute((const void*)wl.wide, hipFuncAttributeMaxDynamicSharedMemorySize, (int)wl.wide_lds));
   }
   for (int attempt = 0; attempt < 6; attempt++) {
     HIPCHK(L->rec.ensure(sizeof(IndelRec) * (size_t)L->rec_cap));
@@ -1134,6 +1156,9 @@ pl_status run_jobs(pl_ctx* c, Lane* L, const std::vector<JobReq>& reqs, int32_t 
     A.W = W;
     A.queue = (int32_t*)(cnt + PL_N_QUEUE);
     A.deep = cnt + PL_N_DEEP;
+    A.wheads = L->wheads.as<WinHead>();
+    A.wide_wins = cnt + PL_N_WIDE_WINS;
+    A.wqueue = (int32_t*)(cnt + PL_N_WIDE_QUEUE);
     A.cost = L->cost.as<uint8_t>();
     A.bins = L->bins.as<uint32_t>();
     A.heads = L->heads.as<WinHead>();
@@ -1159,14 +1184,13 @@ pl_status run_jobs(pl_ctx* c, Lane* L, const std::vector<JobReq>& reqs, int32_t 
       GraphKey key;
       std::memset(&key, 0, sizeof key);
       key.A = A;
-      key.W = W; key.block = block; key.persistent = persistent; key.grid = grid; key.lds = lds;
+      key.W = W; key.persistent = persistent; key.wl = wl;
       key.bufs[0] = L->csums.p; key.bufs[1] = L->kparr.p;
-      key.wk = wk;
       if (!L->gexec || L->gkey.size() != sizeof key || std::memcmp(L->gkey.data(), &key, sizeof key) != 0) {
         drop_graph(L);
         HIPCHK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
         EngineArgs Acap = A;
-        pl_status s = enqueue_batch(L, Acap, wk, persistent, block, grid, lds, false);
+        pl_status s = enqueue_batch(L, Acap, wl, persistent, false);
         hipGraph_t g = nullptr;
         const hipError_t e = hipStreamEndCapture(st, &g);
         if (s) { if (g) (void)hipGraphDestroy(g); return s; }
@@ -1182,7 +1206,7 @@ pl_status run_jobs(pl_ctx* c, Lane* L, const std::vector<JobReq>& reqs, int32_t 
       HIPCHK(hipEventRecord(L->ev[1], st));
     } else {
       HIPCHK(hipEventRecord(L->ev[0], st));
-      pl_status s = enqueue_batch(L, A, wk, persistent, block, grid, lds, true);
+      pl_status s = enqueue_batch(L, A, wl, persistent, true);
       if (s) return s;
       HIPCHK(hipEventRecord(L->ev[1], st));
     }

@@ -12,9 +12,14 @@
 #ifndef PL_WIN_WAVES_EU
 #define PL_WIN_WAVES_EU 3         // minimum waves per SIMD the window kernel is compiled for
 #endif
+#ifndef PL_NARROW_WAVES_EU
+#define PL_NARROW_WAVES_EU 3
+#endif
 #define PL_DEFAULT_WINDOW 512     // plain region form and autotuner fallback
 #define PL_DEFAULT_BLOCK 256
 #define PL_MAX_WINDOW 2048
 #define PL_WIN_LDS_PER_POS 76     // window LDS bytes per position (counters + difference arrays)
+#define PL_NARROW_LDS_PER_POS 60  // ... with 32-bit counters
+#define PL_WIN_WALKS 256          // reads a narrow window walks
 #define PL_WIN_RECS 128           // indel evidence records a window buffers in LDS
 #define PL_FIN_DELS 1024          // active deletion calls one region keeps in LDS in Pass 1

@@ -115,7 +115,7 @@ __device__ __forceinline__ T wave_total_dpp(T v) { return lane63(wave_scan_dpp(v
 
 // ------------------------------------------------------------------ k_prep
 // the read set's scalars (scal[0], [1], [2], [6]: maxima, -1 = none;
-// flags: scal[4], scal[5]) gathered over a thread's reads, then over its
+// flags: scal[4], scal[5], scal[7]) gathered over a thread's reads, then over its
 // wave, so one wave gives one atomic per scalar
 struct PrepAcc {
   int32_t back = -1, lead = -1, span = -1, fp = -1;
@@ -136,6 +136,7 @@ __device__ __forceinline__ void prep_flush(PrepAcc a, int32_t* scal) {
     if (a.fp >= 0) atomicMax(&scal[6], a.fp);
     if (a.flags & 1u) atomicOr(&scal[4], 1);
     if (a.flags & 2u) atomicOr(&scal[5], 1);
+    if (a.flags & 4u) atomicOr(&scal[7], 1);
   }
 }
 
@@ -177,6 +178,7 @@ __device__ __forceinline__ void prep_one(const RSDev& R, int64_t r, const KConf&
     acc.span = max(acc.span, spanEnd - m.pos > 0 ? spanEnd - m.pos : 0);
     if (m.info & RI_UNK_MASK) acc.flags |= 1u;
     if (m.info & (RI_BAD | RI_EDGE_CLIP)) acc.flags |= 2u;
+    if (o.clips) acc.flags |= 4u;
   }
   R.meta[r] = m;
   R.ftail[r] = frag_tail(m);
@@ -342,12 +344,14 @@ __device__ __forceinline__ uint32_t cost_bin(int64_t c) {
   return PL_COST_BINS - 1u - b;
 }
 
-__device__ __forceinline__ void put_head(WinHead* heads, int32_t slot, int32_t wi, const WinDev& w, const JobDev& J) {
+__device__ __forceinline__ void put_head(WinHead* heads, int32_t slot, int32_t wi, const WinDev& w, const JobDev& J,
+                                         int32_t m0) {
   WinHead h;
   h.wi = wi; h.job = w.job; h.p0 = w.p0; h.p1 = w.p1;
   h.lo = w.lo; h.hi = w.hi; h.plo = w.plo; h.out = J.out;
   h.rs = J.rs; h.start = J.start; h.stop = J.stop; h.qs = J.qs; h.qe = J.qe;
-  h.pad[0] = h.pad[1] = h.pad[2] = 0;
+  h.m0 = m0;
+  h.pad[0] = h.pad[1] = 0;
   heads[slot] = h;
 }
 
@@ -370,11 +374,27 @@ __device__ int plan_windows(const EngineArgs& A, int32_t blk, WinDev* wins, bool
   const bool all = fragment_all(J, (int32_t)L0, back, fp);
   const int64_t plo = group_lower_pos<16>(R.pos, win.lo, win.hi, L0 - fp);
   win.plo = all ? win.lo : plo;
+  // adjMq + 1 of most of 16 reads spread over the window's (1 when none is valid)
+  uint32_t mq1 = 0;
+  {
+    const int gl = threadIdx.x & 15, nr = (int)(win.hi - win.plo < 16 ? win.hi - win.plo : 16);
+    if (gl < nr) {
+      const uint32_t info = R.meta[win.plo + (win.hi - win.plo) * gl / nr].info;
+      if (info & RI_VALID) mq1 = (info & RI_ADJMQ_MASK) + 1u;
+    }
+    uint32_t same = 0;
+#pragma unroll
+    for (int d = 0; d < 16; d++) same += (uint32_t)__shfl_xor((int)mq1, d, 64) == mq1;
+    uint32_t best = mq1 ? same << 16 | mq1 : 1u;
+#pragma unroll
+    for (int d = 1; d < 16; d <<= 1) best = max(best, (uint32_t)__shfl_xor((int)best, d, 64));
+    win.m0 = (int32_t)(best & 0xffffu);
+  }
   const int bin = (int)cost_bin((win.hi - win.plo) + (win.plo - win.lo) / 8 + (int64_t)(win.p1 - win.p0) / 16);
   if (in && (threadIdx.x & 15) == 0) {
     wins[w] = win;
     A.cost[w] = (uint8_t)bin;
-    if (heads) put_head((WinHead*)A.heads, w, w, win, J);
+    if (heads) put_head((WinHead*)A.heads, w, w, win, J, win.m0);
   }
   return in ? bin : -1;
 }
@@ -490,7 +510,7 @@ __global__ void __launch_bounds__(256) k_heads(EngineArgs A) {
   __syncthreads();
   if (cnt[tid]) start[tid] += atomicAdd(&A.bins[PL_COST_BINS + tid], cnt[tid]);
   __syncthreads();
-  if (w < A.n_wins) put_head((WinHead*)A.heads, (int32_t)(start[bin] + rank), w, A.wins[w], A.jobs[A.wins[w].job]);
+  if (w < A.n_wins) put_head((WinHead*)A.heads, (int32_t)(start[bin] + rank), w, A.wins[w], A.jobs[A.wins[w].job], A.wins[w].m0);
 }
 
 // identity permutation + its length, for a sort whose count is in device memory
@@ -503,30 +523,48 @@ __global__ void k_iota(uint32_t* v, int32_t n, uint32_t* n_out) {
 // ------------------------------------------------------------------ window
 namespace {
 
-struct LdsSink {
+// What both forms of the window's counters share: the fragment differences,
+// the evidence records, errors.
+struct SinkBase {
+  int32_t *pc, *is;
+  IndelRec* lrec;        // the window's record buffer in LDS
+  uint32_t lrec_cap;
+  uint32_t* lrec_n;
+  JobStat* st;
+  int64_t bcount, aligned_n;
+  __device__ void frag(int p, int d, int32_t size) { atomicAdd(&pc[p], d); atomicAdd(&is[p], size); }
+  __device__ void aligned(int n) { aligned_n += n; }
+  __device__ void count_base() { bcount++; }
+  __device__ void edge(int64_t r) { atomicMin((unsigned long long*)&st->err_read_edge, (unsigned long long)r); }
+};
+
+// 64-bit counters for any depth: 76 bytes a position.
+struct WideLds : SinkBase {
+  static constexpr bool narrow = false;
   int W;
   unsigned long long *bs, *mqq, *ins_, *del_;
   uint32_t *bad_, *clp_;
-  int32_t *pc, *is;
+  int32_t* bd;           // badPair differences of bad runs (clips, invalid reads' M bases)
   IndelRec* spill;
   uint2* spill_at;
   uint32_t* spill_n;
   uint32_t spill_cap;
   int32_t wi;
-  IndelRec* lrec;        // the window's record buffer in LDS
-  uint32_t lrec_cap;
-  uint32_t* lrec_n;
   int32_t* overflow;
-  JobStat* st;
-  int64_t bcount, aligned_n;
-  __device__ void frag(int p, int d, int32_t size) { atomicAdd(&pc[p], d); atomicAdd(&is[p], size); }
-  __device__ void aligned(int n) { aligned_n += n; }
+  __device__ uint32_t* init(unsigned long long* lds, int w) {   // returns the depth histogram's place
+    W = w;
+    bs = lds; mqq = bs + 4 * W; ins_ = mqq + W; del_ = ins_ + W;
+    bad_ = (uint32_t*)(del_ + W); clp_ = bad_ + W;
+    pc = (int32_t*)(clp_ + W); is = pc + W; bd = is + W;
+    return (uint32_t*)(bd + W);
+  }
   __device__ void base(int p, int b, int32_t q, int32_t mq1) {
     atomicAdd(&bs[b * W + p], (unsigned long long)pack_base(q, mq1));
     atomicAdd(&mqq[p], (unsigned long long)pack_mq_q(mq1, q));
   }
-  __device__ void count_base() { bcount++; }
+  __device__ void slide(int p, int b, int32_t q, int32_t mq1) { base(p, b, q, mq1); }
   __device__ void bad(int p, int n) { atomicAdd(&bad_[p], (uint32_t)n); }
+  __device__ void bad_run(int p, int n, int nW) { atomicAdd(&bd[p], 1); if (p + n < nW) atomicAdd(&bd[p + n], -1); }
   __device__ void clip(int p) { atomicAdd(&clp_[p], 1u); }
   // records collect in LDS and reach HBM together at the window's end; a
   // window with more than fit spills the rest (k_spill_place)
@@ -547,7 +585,74 @@ struct LdsSink {
     atomicAdd(&mqq[p], (unsigned long long)pack_mq_q(mq1, q));
     emit(e);
   }
-  __device__ void edge(int64_t r) { atomicMin((unsigned long long*)&st->err_read_edge, (unsigned long long)r); }
+  __device__ int32_t bad_diff(int i) const { return bd[i]; }
+  __device__ void finish(int p, uint8_t refb, const KConf& cf, int32_t pcv, int32_t isv, int32_t bdv, PosOut& o) const {
+    const uint64_t b4[4] = {bs[p], bs[W + p], bs[2 * W + p], bs[3 * W + p]};
+    finalize_position(b4, mqq[p], ins_[p], del_[p], bad_[p] + (uint32_t)bdv, clp_[p], pcv, isv, refb, cf, o);
+  }
+};
+
+// 32-bit counters (NarrowCol), 60 bytes a position: a base of an m0 read is
+// one 32-bit LDS add where the 64-bit form takes two 64-bit ones.  A window
+// of more than PL_NARROW_MAX reads, slid bases and indels, of more records
+// than the LDS buffer holds, or of a set with reads of many clips is left to
+// the wide form (k_window): its quals and counts could leave their 20 and 12
+// bits.  512 positions, narrow for wide: 24 Mb at 60x 2.05 -> 1.80 ms, 2 Mb
+// at 250x 0.45 -> 0.30 ms (at 60x the window's own phases, not the bases,
+// take two thirds of the time).
+struct NarrowLds : SinkBase {
+  static constexpr bool narrow = true;
+  int W;
+  int32_t m0;
+  uint32_t* cell;        // [4][W]
+  int32_t *qc, *mc, *qs; // [4][W], [W], [W]
+  uint32_t *in_, *de_;
+  uint32_t* cb;          // clips << 16, plus the badPair difference (signed); then badPair
+  uint32_t* extra;       // slid bases and indels of the window
+  __device__ uint32_t* init(unsigned long long* lds, int w) {
+    W = w;
+    cell = (uint32_t*)lds;
+    qc = (int32_t*)(cell + 4 * W); mc = qc + 4 * W; qs = mc + W;
+    in_ = (uint32_t*)(qs + W); de_ = in_ + W; cb = de_ + W;
+    pc = (int32_t*)(cb + W); is = pc + W;
+    return (uint32_t*)(is + W);
+  }
+  __device__ void base(int p, int b, int32_t q, int32_t mq1) {
+    atomicAdd(&cell[b * W + p], (1u << PL_NARROW_SHIFT) + (uint32_t)q);
+    if (mq1 != m0) { atomicAdd(&qc[b * W + p], (mq1 - m0) * q); atomicAdd(&mc[p], mq1 - m0); }
+  }
+  __device__ void slide(int p, int b, int32_t q, int32_t mq1) { atomicAdd(extra, 1u); base(p, b, q, mq1); }
+  __device__ void bad(int p, int n) { atomicAdd(&cb[p], (uint32_t)n); if (p + 1 < W) atomicAdd(&cb[p + 1], 0u - (uint32_t)n); }
+  __device__ void bad_run(int p, int n, int nW) { atomicAdd(&cb[p], 1u); if (p + n < nW) atomicAdd(&cb[p + n], ~0u); }
+  __device__ void clip(int p) { atomicAdd(&cb[p], 1u << 16); }
+  __device__ void emit(const IndelRec& e) {
+    const uint32_t j = atomicAdd(lrec_n, 1u);
+    if (j < lrec_cap) lrec[j] = e;
+  }
+  __device__ void ins(int p, int32_t q, int32_t mq1, const IndelRec& e) {
+    atomicAdd(extra, 1u);
+    atomicAdd(&in_[p], (1u << PL_NARROW_SHIFT) + (uint32_t)mq1);
+    atomicAdd(&qs[p], q);
+    emit(e);
+  }
+  __device__ void del(int p, int32_t q, int32_t mq1, const IndelRec& e) {
+    atomicAdd(extra, 1u);
+    atomicAdd(&de_[p], (1u << PL_NARROW_SHIFT) + (uint32_t)mq1);
+    atomicAdd(&qs[p], q);
+    emit(e);
+  }
+  __device__ int32_t bad_diff(int i) const { return (int32_t)(int16_t)(cb[i] & 0xffffu); }
+  __device__ void finish(int p, uint8_t refb, const KConf& cf, int32_t pcv, int32_t isv, int32_t bdv, PosOut& o) const {
+    NarrowCol N;
+#pragma unroll
+    for (int b = 0; b < 4; b++) { N.cell[b] = cell[b * W + p]; N.qcorr[b] = qc[b * W + p]; }
+    N.mqcorr = mc[p]; N.qsum = qs[p];
+    N.ins = in_[p]; N.del = de_[p];
+    const uint32_t x = cb[p];
+    N.clips = (x - (uint32_t)(int32_t)(int16_t)(x & 0xffffu)) >> 16; N.bad = (uint32_t)bdv;
+    N.pc = pcv; N.is = isv; N.m0 = m0;
+    finalize_narrow(N, refb, cf, o);
+  }
 };
 
 // global-address-space views: loads through them compile to global_load_*
@@ -618,32 +723,44 @@ __device__ __forceinline__ int32_t long_seg_range(const Seg* sg, uint32_t n, int
 }
 
 // One workgroup owns a window of W positions; every counter of those
-// positions lives in LDS until the window is done.  Reads are taken in tiles
-// of BLOCK (one per thread): the headers of a tile are loaded in parallel,
-// each read is classified, and the trusted in-window bases of all "simple"
-// reads (one M/=/X op, 2-bit bases) are processed as one flattened stream in
-// which consecutive lanes take consecutive bases — coalesced loads and
-// conflict-free LDS atomics.  Reads with clips, indels or exotic bases go
-// through walk_read, one wave per read.
+// positions lives in LDS until the window is done.  Each wave takes chunks of
+// up to 64 reads, one read per lane: headers are loaded in parallel, each
+// read is classified, and the trusted in-window bases of its runs (the M ops
+// of 2-bit reads) are piled as one stream of PL_CHUNK-base pieces, one piece
+// per lane.  Clips and indels are applied one segment per lane; other reads
+// go through walk_read, one wave per read.
+//
+// What bounds it: latency.  At 60x a window is ~9 batches of pieces a wave
+// (a third of the time) and a dozen dependent phases (head, read facts,
+// segments, sums, columns, statistics) at 3 waves a SIMD; VALU issue is
+// half used, LDS a fifth, HBM 40%.  Measured on 24 Mb, 512 positions: the
+// facts of the first chunk asked for before the counters are cleared, the
+// segment of the evidence records and the reference before the sums, sums
+// scanned in registers, simple runs in their table before the segments are
+// applied (161 VGPRs for 168 and 2 spilled): 1.87 -> 1.80 ms.  Tried and
+// slower: 4 waves a SIMD (16 spills, 1.99), loads two batches ahead (13
+// spills, 2.09), 512 threads a window (3.86).
 static_assert(PL_CHUNK % 2 == 1 && PL_CHUNK <= 31, "an odd chunk of at most 31 bases (two 16-base words)");
 
 // LONG: the batch's read sets hold long reads (their segments and the
 // nanopore base rule cost the other batches' kernel seven spilled registers).
-template <int BLOCK, bool LONG>
-__global__ void __launch_bounds__(BLOCK, PL_WIN_WAVES_EU) k_window(EngineArgs A, int persistent) {
+// NARROW: the window's counters are 32-bit words (NarrowLds); a window they
+// do not hold is added to A.wheads, and a wide launch of mode 2 piles those.
+// mode: 0 a window per workgroup, 1 windows from the queue, 2 the windows of
+// A.wheads from their queue.
+template <int BLOCK, bool LONG, bool NARROW>
+__global__ void __launch_bounds__(BLOCK, NARROW ? PL_NARROW_WAVES_EU : PL_WIN_WAVES_EU) k_window(EngineArgs A, int mode) {
+  static_assert(!(LONG && NARROW), "long reads have an event every few bases");
   constexpr int NW = BLOCK / 64;
+  using Counters = typename std::conditional<NARROW, NarrowLds, WideLds>::type;
   extern __shared__ __align__(16) unsigned long long lds[];
   const int W = A.W;
-  unsigned long long* bs = lds;
-  unsigned long long* mqq = bs + 4 * W;
-  unsigned long long* insA = mqq + W;
-  unsigned long long* delA = insA + W;
-  uint32_t* badA = (uint32_t*)(delA + W);
-  uint32_t* clpA = badA + W;
-  int32_t* pcA = (int32_t*)(clpA + W);
-  int32_t* isA = pcA + W;
-  int32_t* bdA = isA + W;   // badPair differences of bad runs (clips, invalid reads' M bases)
-  uint32_t* hist = (uint32_t*)(bdA + W);   // PL_HIST entries
+  __shared__ uint32_t s_extra, s_ncx;
+  __shared__ uint16_t s_cx[NARROW ? PL_WIN_WALKS : 1];   // reads to walk, from win.plo
+  const bool persistent = mode != 0;
+  const WinHead* heads = mode == 2 ? A.wheads : A.heads;
+  int32_t* queue = mode == 2 ? A.wqueue : A.queue;
+  const int32_t n_heads = mode == 2 ? (int32_t)*A.wide_wins : A.n_wins;
   __shared__ RunL s_run[NW * (2 * 64 + 1)];
   __shared__ int32_t s_w;
   __shared__ int32_t ws_a[NW], ws_b[NW], ws_c[NW];
@@ -660,23 +777,23 @@ __global__ void __launch_bounds__(BLOCK, PL_WIN_WAVES_EU) k_window(EngineArgs A,
   __shared__ WinHead s_head[2];
   __shared__ int32_t s_slot[2];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int lds_words = (PL_WIN_LDS_PER_POS * W) / 8 + 256 / 2;
+  const int lds_words = ((NARROW ? PL_NARROW_LDS_PER_POS : PL_WIN_LDS_PER_POS) * W) / 8 + 256 / 2;
   const KConf& cf = A.cf;
   (void)s_w;
 
   if (tid == 0) {
-    const int32_t q = persistent ? atomicAdd(A.queue, 1) : (int32_t)blockIdx.x;
+    const int32_t q = persistent ? atomicAdd(queue, 1) : (int32_t)blockIdx.x;
     s_slot[0] = q;
-    if (q < A.n_wins) s_head[0] = A.heads[q];
+    if (q < n_heads) s_head[0] = heads[q];
   }
   __syncthreads();
   for (int iter = 0;; iter++) {
     const int cur = iter & 1;
-    if (__builtin_amdgcn_readfirstlane(s_slot[cur]) >= A.n_wins) break;
+    if (__builtin_amdgcn_readfirstlane(s_slot[cur]) >= n_heads) break;
     if (!persistent && iter > 0) break;
     // the next window's slot: taken now, its head loaded after the read loop
     int32_t next_slot = 0;
-    if (persistent && tid == 0) next_slot = atomicAdd(A.queue, 1);
+    if (persistent && tid == 0) next_slot = atomicAdd(queue, 1);
     // the head through LDS, made wave-uniform so every field is a scalar
     WinHead win;
     {
@@ -691,17 +808,47 @@ __global__ void __launch_bounds__(BLOCK, PL_WIN_WAVES_EU) k_window(EngineArgs A,
     J.size = win.stop - win.start + 1; J.win0 = 0; J.nwin = 0; J.out = win.out; J.rlo = 0; J.rhi = 0;
     const RSDev& R = A.rs[win.rs];
     const int32_t L0 = J.start + win.p0, L1 = J.start + win.p1, nW = win.p1 - win.p0;
+    auto next_window = [&]() {                 // by thread 0
+      s_slot[cur ^ 1] = persistent ? next_slot : n_heads;
+      if (persistent && next_slot < n_heads) s_head[cur ^ 1] = heads[next_slot];
+    };
+    auto to_wide = [&]() { A.wheads[atomicAdd(A.wide_wins, 1u)] = s_head[cur]; };
+    const int64_t reads_in = win.hi - win.plo + R.n_outlier;
+    if (NARROW && reads_in > PL_NARROW_MAX) {
+      if (tid == 0) { to_wide(); next_window(); }
+      __syncthreads();
+      continue;
+    }
     // hot streams of this read set, held in scalar registers for the window
     const int8_t* __restrict__ gq = R.quals;
     const uint8_t* __restrict__ gb = R.bases2;
     const int64_t* __restrict__ gso = R.seq_off;
     const RMeta* __restrict__ gm = R.meta;
+    // Each wave takes its own chunks of up to 64 reads (wave-strided over the
+    // window's read range): staging, the run scan and the base loop are
+    // wave-local, so the read loop has no workgroup barrier.  Where it takes
+    // at most a quarter more chunks they are cut to the same size, as many
+    // for each wave: 512-position windows of 530 reads 0.318 -> 0.306 ms a
+    // 2 Mb batch, but windows of 290 reads, 8 chunks of 37 for 5 of 64,
+    // 1.80 -> 1.94 ms a 24 Mb batch (staging is per chunk).  In a set of long
+    // reads a chunk is PL_LONG_READS reads: a window has about a hundred.
+    RunL* wrun = s_run + wave * (2 * 64 + 1);
+    int CR = PL_LONG_READS;
+    if (!(LONG && R.all_long)) {
+      const int32_t n = (int32_t)(win.hi - win.plo);
+      const int32_t ch = (n + 63) >> 6, even = (ch + NW - 1) / NW * NW;
+      CR = ch <= NW || 4 * even <= 5 * ch ? (n > even ? (n + even - 1) / even : 1) : 64;
+    }
+    const bool stager = lane < CR;
+    // the next chunk's read facts are loaded while the current one is piled,
+    // the first one's while the counters are cleared
+    int64_t t0 = win.plo + CR * wave;
     {
       uint4* l4 = (uint4*)lds;   // 16-byte stores: lds is 16-byte aligned
       for (int k = tid; k < lds_words / 2; k += BLOCK) l4[k] = make_uint4(0u, 0u, 0u, 0u);
       if ((lds_words & 1) && tid == 0) lds[lds_words - 1] = 0ull;
     }
-    if (tid == 0) { s_ovf = 0; s_nrec = 0; }
+    if (tid == 0) { s_ovf = 0; s_nrec = 0; s_extra = 0; s_ncx = 0; }
     const bool nano = LONG && R.nano != 0;
     if constexpr (LONG) {
       for (int q0 = 64 * wave; q0 < W; q0 += BLOCK) {
@@ -718,37 +865,25 @@ __global__ void __launch_bounds__(BLOCK, PL_WIN_WAVES_EU) k_window(EngineArgs A,
     };
     __syncthreads();
 
-    LdsSink sk;
-    sk.W = W; sk.bs = bs; sk.mqq = mqq; sk.ins_ = insA; sk.del_ = delA; sk.bad_ = badA; sk.clp_ = clpA;
-    sk.pc = pcA; sk.is = isA; sk.spill = A.spill; sk.spill_at = A.spill_at; sk.spill_n = A.spill_n;
-    sk.spill_cap = A.spill_cap; sk.wi = wi;
+    Counters sk;
+    uint32_t* hist = sk.init(lds, W);          // PL_HIST entries
     sk.lrec = s_rec; sk.lrec_cap = RECS; sk.lrec_n = &s_nrec;
-    sk.overflow = A.overflow; sk.st = &A.st[win.job]; sk.bcount = 0; sk.aligned_n = 0;
+    sk.st = &A.st[win.job]; sk.bcount = 0; sk.aligned_n = 0;
+    int32_t* const pcA = sk.pc;
+    int32_t* const isA = sk.is;
+    if constexpr (NARROW) {
+      sk.m0 = win.m0;
+      sk.extra = &s_extra;
+    } else {
+      sk.spill = A.spill; sk.spill_at = A.spill_at; sk.spill_n = A.spill_n; sk.spill_cap = A.spill_cap; sk.wi = wi;
+      sk.overflow = A.overflow;
+    }
 
-    // Each wave takes its own chunks of 64 reads (wave-strided over the
-    // window's read range): staging, the run scan and the base loop are
-    // wave-local, so the read loop has no workgroup barrier.  In a set of
-    // long reads a chunk is PL_LONG_READS reads: a window has about a hundred
-    // of them, and 64 to a wave left three of four waves idle.
-    RunL* wrun = s_run + wave * (2 * 64 + 1);
-    const int CR = LONG && R.all_long ? PL_LONG_READS : 64;
-    const bool stager = lane < CR;
-    // the next chunk's read facts are loaded while the current one is piled
-    int64_t t0 = win.plo + CR * wave;
-    RMeta mN;
-    int64_t sN = 0, eN = 0, qN = 0;
-    mN.info = 0;
-    if (stager && t0 + lane < win.hi) { mN = gm[t0 + lane]; sN = gso[t0 + lane]; eN = gso[t0 + lane + 1]; }
-    if (t0 < win.hi) qN = gso[t0];
     for (; t0 < win.hi; t0 += CR * NW) {
-      const int64_t qbase = qN;
-      const RMeta m = mN;
-      const int64_t seq0 = sN, seqE = eN;
-      {
-        const int64_t tn = t0 + CR * NW;
-        if (stager && tn + lane < win.hi) { mN = gm[tn + lane]; sN = gso[tn + lane]; eN = gso[tn + lane + 1]; }
-        if (tn < win.hi) qN = gso[tn];
-      }
+      RMeta m = RMeta(); int64_t seq0 = 0, seqE = 0;
+      m.info = 0;
+      if (stager && t0 + lane < win.hi) { m = gm[t0 + lane]; seq0 = gso[t0 + lane]; seqE = gso[t0 + lane + 1]; }
+      const int64_t qbase = gso[t0];
       // ---- stage: one read per lane.  A simple read gives at most one run;
       // a read with clips or indels is applied below one segment per lane;
       // the rest (non-ACGT bases, too many segments) are walked.
@@ -780,9 +915,22 @@ __global__ void __launch_bounds__(BLOCK, PL_WIN_WAVES_EU) k_window(EngineArgs A,
       // a run that only adds badPair over a range (M bases of an invalid
       // read) goes to the difference array, not to the base loop
       if (nrun > 0 && (ru0.fl & EF_BAD)) {
-        if (ru0.n > 0) { atomicAdd(&bdA[ru0.p0], 1); if (ru0.p0 + ru0.n < nW) atomicAdd(&bdA[ru0.p0 + ru0.n], -1); }
+        if (ru0.n > 0) sk.bad_run(ru0.p0, ru0.n, nW);
         nrun = 0;
       }
+      // ---- run table: simple runs (wave scan), then the segments' runs.  Runs
+      // are cut in chunks of PL_CHUNK bases; .off is the run's first chunk in
+      // the chunk stream, .n its length in bases.
+      const uint64_t v = nrun > 0 ? (1ull << 32) + (uint64_t)((ru0.n + PL_CHUNK - 1) / PL_CHUNK) : 0ull;
+      const uint64_t inc = wave_scan_dpp(v);
+      const uint64_t tot = lane63(inc);
+      if (nrun > 0) {
+        const uint64_t ex = inc - v;
+        wrun[(int32_t)(ex >> 32)] =
+            RunL{(int32_t)(uint32_t)ex, (uint32_t)ru0.p0 | ru0.fl, (int32_t)(ru0.q - qbase) + qsh, ru0.n};
+      }
+      const int32_t Es = (int32_t)(tot >> 32);
+      const int32_t Cs = (int32_t)(uint32_t)tot;
       // ---- reads with clips or indels, one lane per segment: each round
       // loads and applies the segments of as many pending reads as fit the
       // 64 lanes (usually all of the chunk's in one round).  Base-loop runs
@@ -824,8 +972,7 @@ __global__ void __launch_bounds__(BLOCK, PL_WIN_WAVES_EU) k_window(EngineArgs A,
         Run ru;
         int got = has ? seg_apply(R, J, cf, t0 + own, info, s0, Lc, L0, L1, g, ru, &sk.aligned_n, &sk.bcount, sk, lr_drop) : 0;
         if (got && (ru.fl & EF_BAD)) {
-          atomicAdd(&bdA[ru.p0], 1);
-          if (ru.p0 + ru.n < nW) atomicAdd(&bdA[ru.p0 + ru.n], -1);
+          sk.bad_run(ru.p0, ru.n, nW);
           got = 0;
         }
         const uint64_t gmask = __ballot(got != 0);
@@ -833,19 +980,6 @@ __global__ void __launch_bounds__(BLOCK, PL_WIN_WAVES_EU) k_window(EngineArgs A,
             RunL{ru.n, (uint32_t)ru.p0 | ru.fl, (int32_t)(ru.q - qbase) + qsh, 0};
         ncr += __popcll(gmask);
       }
-      // ---- run table: simple runs (wave scan), then the staged runs.  Runs
-      // are cut in chunks of PL_CHUNK bases; .off is the run's first chunk in
-      // the chunk stream, .n its length in bases.
-      const uint64_t v = nrun > 0 ? (1ull << 32) + (uint64_t)((ru0.n + PL_CHUNK - 1) / PL_CHUNK) : 0ull;
-      const uint64_t inc = wave_scan_dpp(v);
-      const uint64_t tot = lane63(inc);
-      if (nrun > 0) {
-        const uint64_t ex = inc - v;
-        wrun[(int32_t)(ex >> 32)] =
-            RunL{(int32_t)(uint32_t)ex, (uint32_t)ru0.p0 | ru0.fl, (int32_t)(ru0.q - qbase) + qsh, ru0.n};
-      }
-      const int32_t Es = (int32_t)(tot >> 32);
-      const int32_t Cs = (int32_t)(uint32_t)tot;
       int32_t Cc = 0;
       if (ncr > 0) {
         // every lane reads its staged run before any lane writes (one wave,
@@ -875,31 +1009,29 @@ __global__ void __launch_bounds__(BLOCK, PL_WIN_WAVES_EU) k_window(EngineArgs A,
       // one run per lane.  A chunk's quals come in as PL_CHUNK/4 + 2 dwords
       // and its 2-bit bases as PL_CHUNK/16 + 2, realigned with funnel shifts
       // (the loads of the next batch of chunks are in flight while the
-      // current batch does its atomics); each base then costs a
-      // byte and a 2-bit extract and two LDS atomics whose step offset is the
-      // instruction's immediate.  Lanes of one run are PL_CHUNK (odd)
-      // positions apart, so their 64-bit atomics spread over all LDS banks.
+      // current batch does its atomics); each base then costs its word and a
+      // 2-bit extract and one LDS atomic (two in the wide form) whose step
+      // offset is the instruction's immediate.  Lanes of one run are PL_CHUNK
+      // (odd) positions apart, so their atomics spread over all LDS banks.
       if (CT > 0) {
         const int32_t mq = cf.min_qual;
-        const uint32_t W8 = 8u * (uint32_t)W;
+        const uint32_t WB = (NARROW ? 4u : 8u) * (uint32_t)W;   // bytes of one base's counters
         const int64_t qb4 = qbase & ~(int64_t)3, qb16 = qbase & ~(int64_t)15;
         const gu32* tq32 = (const gu32*)(gq + qb4);
         const gu32* tb32 = (const gu32*)(gb + (qb16 >> 2));
         const uint32_t qd = (uint32_t)(qb4 - qb16);
-        // run of chunk cb + lane = the last run whose first chunk is <= it
+        // Run of chunk cb + lane = the last run whose first chunk is <= it,
+        // from the run of chunk cb - 1 (or of chunk 0) on: the first chunks
+        // of the runs that start in the batch, as a bit mask.
         auto run_of = [&](int32_t cb, int cur) -> int {
-          const int32_t C = cb + lane;
-          const int32_t lim = CT < cb + 64 ? CT : cb + 64;
-          int rr = cur;
-          for (int c = cur;;) {
-            const int ib = c + 1 + lane;
-            const int32_t bnd = ib <= E ? wrun[ib].off : INT32_MAX;
-            const int nb = __popcll(__ballot(bnd < lim));
-            for (int i = 0; i < nb; i++) rr += (C >= __builtin_amdgcn_readlane(bnd, i)) ? 1 : 0;
-            if (nb < 64) break;
-            c += 64;
-          }
-          return rr;
+          const int ib = cur + 1 + lane;
+          const int32_t bnd = ib <= E ? wrun[ib].off : INT32_MAX;
+          const int nb = __popcll(__ballot(bnd < CT && bnd < cb + 64));
+          uint64_t starts = 0;
+          for (int i = 0; i < nb; i++) starts |= 1ull << (__builtin_amdgcn_readlane(bnd, i) - cb);
+          const uint64_t before = starts >> 1;              // starts at or before a lane's chunk: before it, shifted by one
+          return cur + (int)(starts & 1ull) +
+                 (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(before >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)before, 0u));
         };
         // sequence offset of chunk C of run ru (0 for a lane past the end)
         auto chunk_q = [&](const RunL& ru, int32_t C) -> uint32_t {
@@ -915,13 +1047,12 @@ __global__ void __launch_bounds__(BLOCK, PL_WIN_WAVES_EU) k_window(EngineArgs A,
 #pragma unroll
           for (int k = 0; k < PL_CHUNK / 16 + 2; k++) bw[k] = tb32[(qq >> 4) + k];
         };
-        int cur = 0;
         int rr = run_of(0, 0);
-        load(chunk_q(wrun[lane < CT ? rr : 0], lane));
+        RunL ru = wrun[lane < CT ? rr : 0];
+        load(chunk_q(ru, lane));
         for (int32_t cb = 0; cb < CT; cb += 64) {
           const int32_t C = cb + lane;
           const bool act = C < CT;
-          const RunL ru = wrun[act ? rr : cur];
           const int32_t d = PL_CHUNK * (C - ru.off);
           int32_t cnt = ru.pad - d;
           cnt = act ? (cnt < PL_CHUNK ? cnt : PL_CHUNK) : 0;
@@ -944,39 +1075,95 @@ __global__ void __launch_bounds__(BLOCK, PL_WIN_WAVES_EU) k_window(EngineArgs A,
               w[k] &= ~((((xb >> (4 * k)) & 15u) * 0x00204081u & 0x01010101u) * 255u);
           }
           // the next batch: its runs, and its loads
-          int rrn = rr;
+          RunL run_n = ru;
           uint32_t qn = 0u;
           if (cb + 64 < CT) {
-            const int curn = lane63(rr);
-            rrn = run_of(cb + 64, curn);
-            qn = chunk_q(wrun[C + 64 < CT ? rrn : curn], C + 64);
+            const int cur = lane63(rr);
+            rr = run_of(cb + 64, cur);
+            run_n = wrun[C + 64 < CT ? rr : cur];
+            qn = chunk_q(run_n, C + 64);
           }
           load(qn);
-          unsigned long long* bsp = bs + p;
-          unsigned long long* mqp = mqq + p;
           // The base's counter array is b*W entries on: a 24-bit multiply-add
-          // (b < 4, 8*W < 2^24).  With minQual >= 0 every qual that passes is
-          // non-negative, so qual*mq1 >= 0 and the count part is the constant
-          // 1 << PL_BASE_SHIFT (pack_base without its sign extension).
-          auto pile = [&](auto nonneg) {
+          // (b < 4, 8*W < 2^24), the step an offset of the instruction.
+          if constexpr (NARROW) {
+            // Each base's word, its count bit and its qual, is one byte
+            // permute of the quals and a mask with 0x10 in the valid bases'
+            // bytes (bit 4 of byte 2 of the word: PL_NARROW_SHIFT); a lane's
+            // bases past its chunk, or below minQual, add 0, so the 13 adds
+            // need no execution mask: 3 VALU instructions a base where the
+            // masked form took 7.  (An add of 0 past the window's positions
+            // stays inside the counters.)
+            static_assert(PL_NARROW_SHIFT == 20, "bit 4 of byte 2");
+            uint32_t mm[PL_CHUNK / 4 + 1];
+            uint32_t hi = 0;
 #pragma unroll
-            for (int t = 0; t < PL_CHUNK; t++) {
-              const int32_t qual = (int32_t)(int8_t)(w[t >> 2] >> (8 * (t & 3)));
-              const uint32_t b = (x[t >> 4] >> (2 * (t & 15))) & 3u;
-              if (t < cnt && qual >= mq) {
-                unsigned long long* cell = (unsigned long long*)((char*)bsp + __umul24(b, W8)) + t;
-                const unsigned long long v = decltype(nonneg)::value
-                                                 ? ((1ull << PL_BASE_SHIFT) | (uint32_t)(qual * mq1))
-                                                 : (unsigned long long)pack_base(qual, mq1);
-                atomicAdd(cell, v);
-                atomicAdd(mqp + t, (unsigned long long)pack_mq_q(mq1, qual));
+            for (int k = 0; k < PL_CHUNK / 4 + 1; k++) {
+              const int32_t nb = cnt - 4 * k;                  // valid bytes of word k
+              const uint32_t vm = (uint32_t)((1ull << (8 * (nb < 0 ? 0 : nb > 4 ? 4 : nb))) - 1ull);
+              w[k] &= vm;
+              mm[k] = vm & 0x10101010u;
+              hi |= w[k];
+            }
+            if (mq > 0 || __ballot((hi & 0x80808080u) != 0u)) {
+              // quals below minQual (and negative ones): a byte of (qual | 128) -
+              // minQual keeps its top bit where qual >= minQual
+              const uint32_t mr = (uint32_t)(mq > 128 ? 128 : mq) * 0x01010101u;
+#pragma unroll
+              for (int k = 0; k < PL_CHUNK / 4 + 1; k++) {
+                const uint32_t ok = mq > 127 ? 0u : (((w[k] | 0x80808080u) - mr) & ~w[k] & 0x80808080u) >> 7;
+                w[k] &= ok * 255u;
+                mm[k] &= ok * 255u;
               }
             }
-          };
-          if (mq >= 0) pile(std::integral_constant<bool, true>{});
-          else pile(std::integral_constant<bool, false>{});
-          cur = lane63(rr);
-          rr = rrn;
+            char* const cellp = (char*)(sk.cell + p);
+            if (act) {
+#pragma unroll
+              for (int t = 0; t < PL_CHUNK; t++) {
+                const uint32_t v = __builtin_amdgcn_perm(mm[t >> 2], w[t >> 2],
+                                                         0x0c000c00u | (uint32_t)((4 + (t & 3)) << 16) | (uint32_t)(t & 3));
+                const uint32_t b = (x[t >> 4] >> (2 * (t & 15))) & 3u;
+                atomicAdd((uint32_t*)(cellp + __umul24(b, WB)) + t, v);
+              }
+            }
+            const int32_t dm = mq1 - sk.m0;
+            if (act && dm != 0) {                              // a read of another adjMq: its bases' differences
+              char* const qcp = (char*)(sk.qc + p);
+              int32_t* const mcp = sk.mc + p;
+#pragma unroll
+              for (int t = 0; t < PL_CHUNK; t++) {
+                const uint32_t b = (x[t >> 4] >> (2 * (t & 15))) & 3u;
+                if (t < cnt) {
+                  atomicAdd((int32_t*)(qcp + __umul24(b, WB)) + t, dm * (int32_t)((w[t >> 2] >> (8 * (t & 3))) & 255u));
+                  atomicAdd(mcp + t, (mm[t >> 2] >> (8 * (t & 3)) & 255u) ? dm : 0);
+                }
+              }
+            }
+          } else {
+            // With minQual >= 0 every qual that passes is non-negative, so
+            // qual*mq1 >= 0 and the count part is the constant
+            // 1 << PL_BASE_SHIFT (pack_base without its sign extension).
+            unsigned long long* bsp = sk.bs + p;
+            unsigned long long* mqp = sk.mqq + p;
+            auto pile = [&](auto nonneg) {
+#pragma unroll
+              for (int t = 0; t < PL_CHUNK; t++) {
+                const int32_t qual = (int32_t)(int8_t)(w[t >> 2] >> (8 * (t & 3)));
+                const uint32_t b = (x[t >> 4] >> (2 * (t & 15))) & 3u;
+                if (t < cnt && qual >= mq) {
+                  unsigned long long* cell = (unsigned long long*)((char*)bsp + __umul24(b, WB)) + t;
+                  const unsigned long long v = decltype(nonneg)::value
+                                                   ? ((1ull << PL_BASE_SHIFT) | (uint32_t)(qual * mq1))
+                                                   : (unsigned long long)pack_base(qual, mq1);
+                  atomicAdd(cell, v);
+                  atomicAdd(mqp + t, (unsigned long long)pack_mq_q(mq1, qual));
+                }
+              }
+            };
+            if (mq >= 0) pile(std::integral_constant<bool, true>{});
+            else pile(std::integral_constant<bool, false>{});
+          }
+          ru = run_n;
         }
       }
       if constexpr (!LONG) break;
@@ -1025,8 +1212,7 @@ __global__ void __launch_bounds__(BLOCK, PL_WIN_WAVES_EU) k_window(EngineArgs A,
         ru.n = 0;
         int got = has ? seg_apply(R, J, cf, t0 + src, info, s0, Lc, L0, L1, g, ru, &sk.aligned_n, &sk.bcount, sk, lr_drop) : 0;
         if (got && (ru.fl & EF_BAD)) {
-          atomicAdd(&bdA[ru.p0], 1);
-          if (ru.p0 + ru.n < nW) atomicAdd(&bdA[ru.p0 + ru.n], -1);
+          sk.bad_run(ru.p0, ru.n, nW);
           got = 0;
         }
         const uint64_t lv = got ? (1ull << 32) + (uint64_t)((ru.n + PL_CHUNK - 1) / PL_CHUNK) : 0ull;
@@ -1038,19 +1224,30 @@ __global__ void __launch_bounds__(BLOCK, PL_WIN_WAVES_EU) k_window(EngineArgs A,
       }
       if (!more) break;
       }
-      // ---- everything else about the chunk's complex reads, one at a time
-      for (uint64_t cm = __ballot(cplx); cm; cm &= cm - 1) {
-        const int l = __ffsll((unsigned long long)cm) - 1;
-        walk_read(R, J, cf, t0 + l, L0, L1, lane, 64, sk, false);
+      // ---- everything else about the chunk's complex reads: the wide form
+      // walks them here, the narrow one after the read loop, where the
+      // loop's registers are free
+      if constexpr (NARROW) {
+        if (cplx) {
+          const uint32_t k = atomicAdd(&s_ncx, 1u);
+          if (k < PL_WIN_WALKS) s_cx[k] = (uint16_t)(r - win.plo);
+        }
+      } else {
+        for (uint64_t cm = __ballot(cplx); cm; cm &= cm - 1) {
+          const int l = __ffsll((unsigned long long)cm) - 1;
+          walk_read(R, J, cf, t0 + l, L0, L1, lane, 64, sk, false);
+        }
       }
       __builtin_amdgcn_wave_barrier();
     }
+    bool many_clips = false;
     // reads that reach the window only through their fragments: 8 bytes
     // each, +1/+size at position 0 summed per wave
     {
       // read the descriptors again here rather than hold them through the read loop
       asm volatile("" ::: "memory");
       const FragTail* __restrict__ ft = R.ftail;
+      many_clips = NARROW && R.scal[7] != 0;
       const int64_t flo = win.lo, fhi = win.plo;
       uint32_t c0 = 0, s0 = 0;
       for (int64_t r = flo + tid; r < fhi; r += BLOCK) {
@@ -1061,72 +1258,83 @@ __global__ void __launch_bounds__(BLOCK, PL_WIN_WAVES_EU) k_window(EngineArgs A,
       s0 = wave_total_dpp(s0);
       if (lane == 0 && c0) sk.frag(0, (int32_t)c0, (int32_t)s0);
     }
-    for (int64_t k = wave; k < R.n_outlier; k += NW) {
-      const int64_t r = uniform64(R.outliers[k]);
-      walk_read(R, J, cf, r, L0, L1, lane, 64, sk, true);
+    if constexpr (!NARROW) {
+      for (int64_t k = wave; k < R.n_outlier; k += NW)
+        walk_read(R, J, cf, uniform64(R.outliers[k]), L0, L1, lane, 64, sk, true);
     }
-    if (tid == 0) {
-      s_slot[cur ^ 1] = persistent ? next_slot : A.n_wins;
-      if (persistent && next_slot < A.n_wins) s_head[cur ^ 1] = A.heads[next_slot];
-    }
+    if (tid == 0) next_window();
     __syncthreads();
-
-    // inclusive scan of the physCov / insertSize differences over the window
-    {
-      const int per = (W + BLOCK - 1) / BLOCK;
-      const int b0 = tid * per;
-      int32_t spc = 0, sis = 0, sbd = 0;
-      for (int i = 0; i < per; i++)
-        if (b0 + i < W) {
-          spc = j_add(spc, pcA[b0 + i]); sis = j_add(sis, isA[b0 + i]); sbd = j_add(sbd, bdA[b0 + i]);
-        }
-      // (Int adds wrap like Java's: the scan's 32-bit adds are the same)
-      const int32_t ipc = wave_scan_dpp(spc), iis = wave_scan_dpp(sis), ibd = wave_scan_dpp(sbd);
-      if (lane == 63) { ws_a[wave] = ipc; ws_b[wave] = iis; ws_c[wave] = ibd; }
+    if constexpr (NARROW) {
+      const int32_t ncx = s_ncx <= PL_WIN_WALKS ? (int32_t)s_ncx : 0;
+      const int32_t nwk = ncx + (int32_t)R.n_outlier;
+      if (nwk > 0) {
+        for (int32_t k = wave; k < nwk; k += NW)
+          walk_read(R, J, cf, uniform64(k < ncx ? win.plo + s_cx[k] : R.outliers[k - ncx]), L0, L1, lane, 64, sk, k >= ncx);
+        __syncthreads();
+      }
+    }
+    if (NARROW && (s_nrec > RECS || many_clips || s_ncx > PL_WIN_WALKS || reads_in + s_extra > PL_NARROW_MAX)) {
+      // beyond the narrow counters: nothing of the window has left the
+      // workgroup, the wide form piles it again
+      if (tid == 0) to_wide();
       __syncthreads();
-      int32_t cpc = j_sub(ipc, spc), cis = j_sub(iis, sis), cbd = j_sub(ibd, sbd);
-      for (int w2 = 0; w2 < wave; w2++) {
-        cpc = j_add(cpc, ws_a[w2]); cis = j_add(cis, ws_b[w2]); cbd = j_add(cbd, ws_c[w2]);
-      }
-      for (int i = 0; i < per; i++) {
-        if (b0 + i >= W) break;
-        cpc = j_add(cpc, pcA[b0 + i]);
-        cis = j_add(cis, isA[b0 + i]);
-        cbd = j_add(cbd, bdA[b0 + i]);
-        pcA[b0 + i] = cpc;
-        isA[b0 + i] = cis;
-        badA[b0 + i] += (uint32_t)cbd;
-      }
+      continue;
     }
-    __syncthreads();
 
-    // the window's evidence records, in one segment of the batch's: one
-    // atomic, coalesced 32-byte stores (room for the spilled ones at its end)
+    // Each wave finishes one span of the window's 64-position tiles.  The
+    // physCov, insertSize and badPair differences are summed a span (Int adds
+    // wrap like Java's: 32-bit adds do the same), and scanned in registers
+    // tile by tile.  What has a memory latency of its own, the segment of the
+    // window's evidence records and the first tile's reference bases, is
+    // asked for before the sums.
+    const int span = 64 * (((W >> 6) + NW - 1) / NW), q_lo = span * wave, q_hi = q_lo + span < W ? q_lo + span : W;
+    const uint32_t nt = s_nrec;
+    uint32_t recb = 0;
+    if (tid == 0 && nt) recb = atomicAdd(A.rec_n, nt);
+    const uint8_t* __restrict__ gref = R.ref + (L0 - 1);
+    uint8_t refN = q_lo + lane < nW ? gref[q_lo + lane] : (uint8_t)0;
     {
-      const uint32_t nt = s_nrec, nl = nt < RECS ? nt : RECS;
+      int32_t spc = 0, sis = 0, sbd = 0;
+      for (int p = q_lo + lane; p < q_hi; p += 64) {
+        spc = j_add(spc, pcA[p]); sis = j_add(sis, isA[p]); sbd = j_add(sbd, sk.bad_diff(p));
+      }
+      spc = wave_total_dpp(spc); sis = wave_total_dpp(sis); sbd = wave_total_dpp(sbd);
+      if (lane == 0) { ws_a[wave] = spc; ws_b[wave] = sis; ws_c[wave] = sbd; }
+    }
+    if (tid == 0) s_recbase = recb;
+    __syncthreads();
+    int32_t cpc = 0, cis = 0, cbd = 0;
+    for (int w2 = 0; w2 < wave; w2++) {
+      cpc = j_add(cpc, ws_a[w2]); cis = j_add(cis, ws_b[w2]); cbd = j_add(cbd, ws_c[w2]);
+    }
+    // the window's evidence records, in one segment of the batch's:
+    // coalesced 32-byte stores (room for the spilled ones at its end)
+    {
+      const uint32_t base = s_recbase, nl = nt < RECS ? nt : RECS;
       if (tid == 0) {
-        const uint32_t base = nt ? atomicAdd(A.rec_n, nt) : 0u;
-        s_recbase = base;
         A.win_rec[2 * wi] = base;
         A.win_rec[2 * wi + 1] = nt;
         if (nt && base + nt > A.rec_cap) *A.overflow = 1;
       }
-      __syncthreads();
       for (uint32_t t = tid; t < nl; t += BLOCK) {
-        const uint32_t k = s_recbase + t;
+        const uint32_t k = base + t;
         if (k < A.rec_cap) A.rec[k] = s_rec[t];
       }
     }
     const int64_t G = A.G;
-    uint32_t wmask = 0;   // bit i: position tid + i*BLOCK is wide
-    for (int q0 = 64 * wave, it = 0; q0 < W; q0 += BLOCK, it++) {
+    uint32_t wmask = 0;   // bit i: position q_lo + 64*i + lane is wide
+    for (int q0 = q_lo, it = 0; q0 < q_hi; q0 += 64, it++) {
       const int p = q0 + lane;
       const bool act = p < nW;
+      const uint8_t refb = refN;
+      if (q0 + 64 < q_hi) refN = p + 64 < nW ? gref[p + 64] : (uint8_t)0;
+      const int32_t ipc = j_add(cpc, wave_scan_dpp(pcA[p])), iis = j_add(cis, wave_scan_dpp(isA[p])),
+                    ibd = j_add(cbd, wave_scan_dpp(sk.bad_diff(p)));
+      cpc = lane63(ipc); cis = lane63(iis); cbd = lane63(ibd);
       bool is_cand = false, defer = false;
       if (act) {
-        const uint64_t b4[4] = {bs[p], bs[W + p], bs[2 * W + p], bs[3 * W + p]};
         PosOut o;
-        finalize_position(b4, mqq[p], insA[p], delA[p], badA[p], clpA[p], pcA[p], isA[p], R.ref[L0 + p - 1], cf, o);
+        sk.finish(p, refb, cf, ipc, iis, ibd, o);
         const int64_t g = J.out + win.p0 + p;
 #pragma unroll
         for (int f = 0; f < PL_NFIELDS; f++) A.pile[(int64_t)f * G + g] = o.f[f];
@@ -1154,7 +1362,7 @@ __global__ void __launch_bounds__(BLOCK, PL_WIN_WAVES_EU) k_window(EngineArgs A,
     }
     // wide columns (a qualSum beyond int32): the window's entries, in one
     // segment of the batch's list, with their exact sums from the LDS words
-    if (__syncthreads_or(wmask != 0)) {
+    if (!NARROW && __syncthreads_or(wmask != 0)) {
       const uint32_t mine = (uint32_t)__popc(wmask);
       const uint32_t inc = wave_scan_dpp(mine);
       if (lane == 63) ws_a[wave] = (int32_t)inc;
@@ -1168,13 +1376,13 @@ __global__ void __launch_bounds__(BLOCK, PL_WIN_WAVES_EU) k_window(EngineArgs A,
       }
       __syncthreads();
       for (uint32_t m = wmask; m; m &= m - 1) {
-        const int p = tid + (__ffs(m) - 1) * BLOCK;
+        const int p = q_lo + 64 * (__ffs(m) - 1) + lane;
         const uint32_t k = s_recbase + pre++;
         if (k < A.wide_cap) {
           WideCol wc;
           wc.gpos = (uint32_t)(J.out + win.p0 + p);
           wc.pad = 0;
-          for (int b = 0; b < 4; b++) { uint32_t n; unpack_base(bs[b * W + p], &wc.qs[b], &n); }
+          if constexpr (!NARROW) for (int b = 0; b < 4; b++) { uint32_t n; unpack_base(sk.bs[b * W + p], &wc.qs[b], &n); }
           A.wide[k] = wc;
         } else {
           *A.overflow = 1;
@@ -1203,12 +1411,15 @@ __global__ void __launch_bounds__(BLOCK, PL_WIN_WAVES_EU) k_window(EngineArgs A,
   }
 }
 
-template __global__ void k_window<256, false>(EngineArgs, int);
-template __global__ void k_window<512, false>(EngineArgs, int);
-template __global__ void k_window<1024, false>(EngineArgs, int);
-template __global__ void k_window<256, true>(EngineArgs, int);
-template __global__ void k_window<512, true>(EngineArgs, int);
-template __global__ void k_window<1024, true>(EngineArgs, int);
+template __global__ void k_window<256, false, true>(EngineArgs, int);
+template __global__ void k_window<512, false, true>(EngineArgs, int);
+template __global__ void k_window<1024, false, true>(EngineArgs, int);
+template __global__ void k_window<256, false, false>(EngineArgs, int);
+template __global__ void k_window<512, false, false>(EngineArgs, int);
+template __global__ void k_window<1024, false, false>(EngineArgs, int);
+template __global__ void k_window<256, true, false>(EngineArgs, int);
+template __global__ void k_window<512, true, false>(EngineArgs, int);
+template __global__ void k_window<1024, true, false>(EngineArgs, int);
 
 // ------------------------------------------------------------------ records
 // Spilled records into their windows' segments, each at the place it took
