@@ -27,6 +27,7 @@
 #define RI_SEG_MAX      31           // more segments: the read is walked instead
 #define RI_SEG_LONG     1            // of a long read: its segments follow a header segment
 #define PL_COST_BINS    256         // cost classes of the work queue's order
+#define PL_BIN_COPIES   8           // copies of their counts (k_plan)
 #define PL_LR_NANOPORE  1
 #define PL_LR_PACBIO    2
 
@@ -185,7 +186,7 @@ struct EngineArgs {
   int32_t W;                 // window size (positions)
   int32_t* queue;            // persistent work queue head
   uint8_t* cost;             // [n_wins] cost bin of each window (0 = most reads)
-  uint32_t* bins;            // [2 * PL_COST_BINS]: windows per cost bin, then queue slots taken per bin
+  uint32_t* bins;            // [PL_BIN_COPIES + 1][PL_COST_BINS]: windows per cost bin, then queue slots taken per bin
   const WinHead* heads;      // [n_wins] window heads in processing order
   int32_t* pile;             // [PL_NFIELDS][G]
   pl_call* calls;            // [G]

@@ -991,7 +991,7 @@ pl_status enqueue_batch(Lane* L, EngineArgs& A, const WindowLaunch& wl, int pers
   const bool ordered = persistent && n_wins > wl.grid;
   k_begin<<<dim3(1 + jb + (ordered ? 0 : pb)), dim3(256), 0, st>>>(A, kp, cnt, PL_COUNTERS, wins, ordered ? 0 : 1);
   if (ordered) {
-    k_plan<<<dim3(pb), dim3(256), 0, st>>>(A, wins);
+    k_plan<<<dim3((unsigned)(n_wins + 63) / 64), dim3(1024), 0, st>>>(A, wins);
     k_heads<<<dim3((unsigned)(n_wins + 255) / 256), dim3(256), 0, st>>>(A);
   }
   HIPCHK(hipGetLastError());
@@ -1100,7 +1100,7 @@ pl_status run_jobs(pl_ctx* c, Lane* L, const std::vector<JobReq>& reqs, int32_t 
   HIPCHK(L->heads.ensure(sizeof(WinHead) * (size_t)n_wins));
   HIPCHK(L->wheads.ensure(sizeof(WinHead) * (size_t)n_wins));
   HIPCHK(L->cost.ensure((size_t)n_wins));
-  HIPCHK(L->bins.ensure(8 * PL_COST_BINS));
+  HIPCHK(L->bins.ensure(4 * (PL_BIN_COPIES + 1) * PL_COST_BINS));
   HIPCHK(L->cmask.ensure(8 * (size_t)n_wins * (size_t)(W / 64)));
   HIPCHK(L->csums.ensure(4 * (((size_t)n_wins * (size_t)(W / 64) + PL_CAND_WORDS - 1) / PL_CAND_WORDS)));
   HIPCHK(L->prec.ensure(4 * (size_t)G));

@@ -335,6 +335,22 @@ __device__ __forceinline__ int64_t group_lower_pos(const int32_t* pos, int64_t l
   return lo + __popcll((__ballot(less) >> g0) & gm);
 }
 
+// the same for an answer expected near lo: one round of probes 16, 32, 64, ...
+// beyond it bounds the search (a window's reads end a few hundred on, and a
+// search of the whole set takes six rounds of scattered loads)
+template <int GL>
+__device__ __forceinline__ int64_t group_lower_pos_near(const int32_t* pos, int64_t lo, int64_t n, int64_t x) {
+  const int lane = threadIdx.x & 63, gl = lane & (GL - 1), g0 = lane & ~(GL - 1);
+  const uint64_t gm = GL == 64 ? ~0ull : (1ull << (GL & 63)) - 1ull;
+  const int64_t at = lo + (16ll << gl);
+  const bool less = at < n && (int64_t)pos[at] < x;
+  const int k = __popcll((__ballot(less) >> g0) & gm);
+  int64_t hi = n;
+  if (k < GL && lo + (16ll << k) < n) hi = lo + (16ll << k);
+  if (k > 0) lo += (16ll << (k - 1)) + 1;
+  return group_lower_pos<GL>(pos, lo, hi, x);
+}
+
 // cost bin of a window: 0 for the most work, four mantissa bits above 16
 // units (windows of one bin differ by at most 6%, what the queue's order is for)
 __device__ __forceinline__ uint32_t cost_bin(int64_t c) {
@@ -355,12 +371,12 @@ __device__ __forceinline__ void put_head(WinHead* heads, int32_t slot, int32_t w
   heads[slot] = h;
 }
 
-// The read ranges of 16 windows, one per group of 16 lanes of a 256-thread
-// block; returns this lane's window's cost bin (-1: past the last window).
+// The read ranges of the windows of a block, one per group of 16 lanes;
+// returns this lane's window's cost bin (-1: past the last window).
 // Windows are few and short, so the three searches are all latency: a lane
 // per window took 27 us for 47,000 windows and 14 us for 400.
 __device__ int plan_windows(const EngineArgs& A, int32_t blk, WinDev* wins, bool heads) {
-  const int32_t w0 = blk * 16 + (int32_t)(threadIdx.x >> 4);
+  const int32_t w0 = blk * (int32_t)(blockDim.x >> 4) + (int32_t)(threadIdx.x >> 4);
   const bool in = w0 < A.n_wins;
   const int32_t w = in ? w0 : A.n_wins - 1;                 // idle groups repeat the last window
   WinDev win = wins[w];
@@ -369,7 +385,7 @@ __device__ int plan_windows(const EngineArgs& A, int32_t blk, WinDev* wins, bool
   const int64_t L0 = (int64_t)J.start + win.p0, L1 = (int64_t)J.start + win.p1;
   const int32_t back = R.scal[0], lead = R.scal[1], fp = R.scal[6];
   win.lo = group_lower_pos<16>(R.pos, 0, R.n, L0 - back);
-  win.hi = group_lower_pos<16>(R.pos, win.lo, R.n, L1 + lead);
+  win.hi = group_lower_pos_near<16>(R.pos, win.lo, R.n, L1 + lead);
   // the end of the fragment-only reads: fragment_only_end with the group's search
   const bool all = fragment_all(J, (int32_t)L0, back, fp);
   const int64_t plo = group_lower_pos<16>(R.pos, win.lo, win.hi, L0 - fp);
@@ -469,7 +485,7 @@ __global__ void __launch_bounds__(256) k_begin(EngineArgs A, const uint32_t* con
   int32_t b = (int32_t)blockIdx.x;
   if (b == 0) {
     if ((int)threadIdx.x < n_counters) counters[threadIdx.x] = 0;
-    if (!plan) for (int k = threadIdx.x; k < 2 * PL_COST_BINS; k += 256) A.bins[k] = 0;
+    if (!plan) for (int k = threadIdx.x; k < (PL_BIN_COPIES + 1) * PL_COST_BINS; k += 256) A.bins[k] = 0;
     return;
   }
   b -= 1;
@@ -481,10 +497,20 @@ __global__ void __launch_bounds__(256) k_begin(EngineArgs A, const uint32_t* con
   if (plan) plan_windows(A, b - jb, wins, true);
 }
 
-// the windows' read ranges and cost bins (persistent form)
-__global__ void __launch_bounds__(256) k_plan(EngineArgs A, WinDev* wins) {
+// The windows' read ranges and cost bins (persistent form), 64 windows a
+// block.  Most windows of an even batch fall in a few bins, so what bounded
+// this kernel was atomics on a few addresses of one cache line: a block
+// counts in LDS, and its bins go to one of PL_BIN_COPIES copies, lines
+// apart.  38,062 windows: 224 us with an atomic a window, 41 us so.
+__global__ void __launch_bounds__(1024) k_plan(EngineArgs A, WinDev* wins) {
+  __shared__ uint32_t cnt[PL_COST_BINS];
+  if (threadIdx.x < PL_COST_BINS) cnt[threadIdx.x] = 0;
+  __syncthreads();
   const int bin = plan_windows(A, blockIdx.x, wins, false);
-  if (bin >= 0 && (threadIdx.x & 15) == 0) atomicAdd(&A.bins[bin], 1u);
+  if (bin >= 0 && (threadIdx.x & 15) == 0) atomicAdd(&cnt[bin], 1u);
+  __syncthreads();
+  if (threadIdx.x < PL_COST_BINS && cnt[threadIdx.x])
+    atomicAdd(&A.bins[(blockIdx.x % PL_BIN_COPIES) * PL_COST_BINS + threadIdx.x], cnt[threadIdx.x]);
 }
 
 // The window heads in cost order, most work first: a window's queue slot is
@@ -496,7 +522,9 @@ __global__ void __launch_bounds__(256) k_heads(EngineArgs A) {
   __shared__ uint32_t start[PL_COST_BINS], cnt[PL_COST_BINS];
   __shared__ uint32_t ws[4];
   const int tid = threadIdx.x;
-  const uint32_t v = A.bins[tid];
+  uint32_t v = 0;
+#pragma unroll
+  for (int k = 0; k < PL_BIN_COPIES; k++) v += A.bins[k * PL_COST_BINS + tid];
   const uint32_t inc = wave_scan_dpp(v);
   if ((tid & 63) == 63) ws[tid >> 6] = inc;
   cnt[tid] = 0;
@@ -508,7 +536,7 @@ __global__ void __launch_bounds__(256) k_heads(EngineArgs A) {
   uint32_t bin = 0, rank = 0;
   if (w < A.n_wins) { bin = A.cost[w]; rank = atomicAdd(&cnt[bin], 1u); }
   __syncthreads();
-  if (cnt[tid]) start[tid] += atomicAdd(&A.bins[PL_COST_BINS + tid], cnt[tid]);
+  if (cnt[tid]) start[tid] += atomicAdd(&A.bins[PL_BIN_COPIES * PL_COST_BINS + tid], cnt[tid]);
   __syncthreads();
   if (w < A.n_wins) put_head((WinHead*)A.heads, (int32_t)(start[bin] + rank), w, A.wins[w], A.jobs[A.wins[w].job], A.wins[w].m0);
 }
