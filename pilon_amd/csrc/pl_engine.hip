@@ -388,18 +388,26 @@ struct SortRecs { uint32_t *lo, *hi, *v; };
 
 // Stable LSD radix sort of n records by the low `bits` bits of their keys;
 // a is where they are, b room for as many; a holds the result.
-pl_status radix_sort(Lane* L, SortRecs& a, SortRecs& b, uint32_t n, int bits) {
-  const int32_t nb = (int32_t)std::max<int64_t>(1, ((int64_t)n + RS_TILE - 1) / RS_TILE);
+template <int ITEMS, bool FUSED>
+pl_status radix_passes(Lane* L, SortRecs& a, SortRecs& b, uint32_t n, int bits) {
+  const int32_t nb = (int32_t)std::max<int64_t>(1, ((int64_t)n + 256 * ITEMS - 1) / (256 * ITEMS));
   HIPCHK(L->hist.ensure(sizeof(uint32_t) * ((size_t)256 * nb + 1)));
   uint32_t* h = L->hist.as<uint32_t>();
   for (int shift = 0; shift < bits; shift += 8) {
-    k_rs_hist<<<dim3(nb), dim3(256), 0, L->stream>>>(a.lo, a.hi, n, shift, h, nb);
-    if (pl_status s = scan_u32(L, h, h, (int64_t)256 * nb)) return s;
-    k_rs_scatter<<<dim3(nb), dim3(256), 0, L->stream>>>(a.lo, a.hi, a.v, b.lo, b.hi, b.v, n, shift, h, nb);
+    k_rs_hist<ITEMS, FUSED><<<dim3(nb), dim3(256), 0, L->stream>>>(a.lo, a.hi, n, shift, h, nb);
+    if constexpr (!FUSED) {
+      if (pl_status s = scan_u32(L, h, h, (int64_t)256 * nb)) return s;
+    }
+    k_rs_scatter<ITEMS, FUSED><<<dim3(nb), dim3(256), 0, L->stream>>>(a.lo, a.hi, a.v, b.lo, b.hi, b.v, n, shift, h, nb);
     HIPCHK(hipGetLastError());
     std::swap(a, b);
   }
   return PL_OK;
+}
+pl_status radix_sort(Lane* L, SortRecs& a, SortRecs& b, uint32_t n, int bits) {
+  if (n <= 1024u * RS_FUSED_TILES) return radix_passes<4, true>(L, a, b, n, bits);
+  if (n <= 4096u * RS_FUSED_TILES) return radix_passes<16, true>(L, a, b, n, bits);
+  return radix_passes<16, false>(L, a, b, n, bits);
 }
 
 void to_kconf(const pl_config& p, KConf& k) {

@@ -1468,41 +1468,50 @@ __global__ void __launch_bounds__(256) k_spill_place(EngineArgs A) {
 __device__ __forceinline__ uint32_t rs_digit(const uint32_t* lo, const uint32_t* hi, uint32_t i, int shift) {
   return (shift < 32 ? lo[i] >> shift : hi[i] >> (shift - 32)) & 255u;
 }
+// Few tiles (FUSED): counts are kept tile by tile, and every block of the
+// scatter adds up the tiles before it itself, one coalesced load a tile, in
+// place of three scan kernels of 15 us together.  75 tiles: scatter 13 -> 16
+// us, so a pass 34 -> 22 us; the line is at RS_FUSED_TILES = 128 tiles, where
+// the loads cost half of what the scans do.  A sort that tiles of 1,024
+// records cut in no more tiles than that takes those: shorter blocks.
+template <int ITEMS, bool FUSED>
 __global__ void __launch_bounds__(256) k_rs_hist(const uint32_t* lo, const uint32_t* hi, uint32_t n, int shift,
                                                  uint32_t* hist, int32_t nblocks) {
   __shared__ uint32_t h[256];
   h[threadIdx.x] = 0;
   __syncthreads();
-  const uint32_t base = blockIdx.x * RS_TILE;
+  const uint32_t base = blockIdx.x * (256 * ITEMS);
 #pragma unroll
-  for (int i = 0; i < RS_ITEMS; i++) {
+  for (int i = 0; i < ITEMS; i++) {
     const uint32_t idx = base + i * 256 + threadIdx.x;
     if (idx < n) atomicAdd(&h[rs_digit(lo, hi, idx, shift)], 1u);
   }
   __syncthreads();
-  hist[(int64_t)threadIdx.x * nblocks + blockIdx.x] = h[threadIdx.x];
+  hist[FUSED ? (int64_t)blockIdx.x * 256 + threadIdx.x : (int64_t)threadIdx.x * nblocks + blockIdx.x] = h[threadIdx.x];
 }
 
 // A tile's records are ranked wave by wave (each wave a quarter of the tile,
 // 64 records a round, no workgroup barrier between rounds), put in digit
 // order in LDS and stored from there, so that consecutive lanes store
-// consecutive records of a digit.  12 M records, 12 bytes each, 8 bits: see
-// kmer_graph for what the pass takes.
+// consecutive records of a digit.  12.4 M records of 12 bytes: 100 us a
+// pass, 3.0 TB/s read and written (its stores come in runs of ~16 records).  off: the scanned counts, or the tiles' own (FUSED).
+template <int ITEMS, bool FUSED>
 __global__ void __launch_bounds__(256) k_rs_scatter(const uint32_t* lo, const uint32_t* hi, const uint32_t* v,
                                                     uint32_t* lo2, uint32_t* hi2, uint32_t* v2, uint32_t n, int shift,
                                                     const uint32_t* off, int32_t nblocks) {
+  constexpr uint32_t TILE = 256 * ITEMS;
   __shared__ uint32_t cnt[4][256];
   __shared__ uint32_t dst[256];                              // a digit's place in the output, less its place in the tile
-  __shared__ uint32_t ws[4];
-  __shared__ uint32_t slo[RS_TILE], shi[RS_TILE], sv[RS_TILE];
+  __shared__ uint32_t ws[4], wd[4];
+  __shared__ uint32_t slo[TILE], shi[TILE], sv[TILE];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   for (int w = 0; w < 4; w++) cnt[w][tid] = 0;
   __syncthreads();
-  const uint32_t base = blockIdx.x * RS_TILE, wbase = base + (uint32_t)wave * (RS_TILE / 4);
-  const uint32_t have = n - base < RS_TILE ? n - base : RS_TILE;
-  uint32_t kl[RS_ITEMS], kh[RS_ITEMS], kv[RS_ITEMS], at[RS_ITEMS];
+  const uint32_t base = blockIdx.x * TILE, wbase = base + (uint32_t)wave * (TILE / 4);
+  const uint32_t have = n - base < TILE ? n - base : TILE;
+  uint32_t kl[ITEMS], kh[ITEMS], kv[ITEMS], at[ITEMS];
 #pragma unroll
-  for (int r = 0; r < RS_ITEMS; r++) {
+  for (int r = 0; r < ITEMS; r++) {
     const uint32_t i = wbase + 64 * r + lane;
     const bool in = i < n;
     kl[r] = in ? lo[i] : 0u;
@@ -1510,7 +1519,7 @@ __global__ void __launch_bounds__(256) k_rs_scatter(const uint32_t* lo, const ui
     kv[r] = in ? v[i] : 0u;
   }
 #pragma unroll
-  for (int r = 0; r < RS_ITEMS; r++) {
+  for (int r = 0; r < ITEMS; r++) {
     const bool in = wbase + 64 * r + lane < n;
     const uint32_t d = (shift < 32 ? kl[r] >> shift : kh[r] >> (shift - 32)) & 255u;
     uint64_t m = __ballot(in);
@@ -1533,16 +1542,34 @@ __global__ void __launch_bounds__(256) k_rs_scatter(const uint32_t* lo, const ui
     uint32_t c[4], t = 0;
     for (int w = 0; w < 4; w++) { c[w] = cnt[w][tid]; t += c[w]; }
     const uint32_t inc = wave_scan_dpp(t);
+    uint32_t before = 0, all = 0, incd = 0;
+    if constexpr (FUSED) {
+      const int32_t me = (int32_t)blockIdx.x;
+#pragma unroll 8
+      for (int32_t k = 0; k < nblocks; k++) {
+        const uint32_t x = off[256 * k + tid];
+        all += x;
+        before += k < me ? x : 0u;
+      }
+      incd = wave_scan_dpp(all);
+      if (lane == 63) wd[wave] = incd;
+    } else {
+      before = off[(int64_t)tid * nblocks + blockIdx.x];
+    }
     if (lane == 63) ws[wave] = inc;
     __syncthreads();
     uint32_t s = inc - t;
     for (int w = 0; w < wave; w++) s += ws[w];
-    dst[tid] = off[(int64_t)tid * nblocks + blockIdx.x] - s;
+    if constexpr (FUSED) {
+      before += incd - all;
+      for (int w = 0; w < wave; w++) before += wd[w];
+    }
+    dst[tid] = before - s;
     for (int w = 0; w < 4; w++) { cnt[w][tid] = s; s += c[w]; }
   }
   __syncthreads();
 #pragma unroll
-  for (int r = 0; r < RS_ITEMS; r++) {
+  for (int r = 0; r < ITEMS; r++) {
     if (wbase + 64 * r + lane < n) {
       const uint32_t d = (shift < 32 ? kl[r] >> shift : kh[r] >> (shift - 32)) & 255u;
       const uint32_t p = cnt[wave][d] + at[r];
@@ -1553,7 +1580,7 @@ __global__ void __launch_bounds__(256) k_rs_scatter(const uint32_t* lo, const ui
   }
   __syncthreads();
 #pragma unroll
-  for (int r = 0; r < RS_ITEMS; r++) {
+  for (int r = 0; r < ITEMS; r++) {
     const uint32_t p = 256 * r + tid;
     if (p < have) {
       const uint32_t a = slo[p], b = shi[p];
@@ -1564,6 +1591,10 @@ __global__ void __launch_bounds__(256) k_rs_scatter(const uint32_t* lo, const ui
     }
   }
 }
+
+template __global__ void k_rs_hist<4, true>(const uint32_t*, const uint32_t*, uint32_t, int, uint32_t*, int32_t);
+template __global__ void k_rs_hist<16, true>(const uint32_t*, const uint32_t*, uint32_t, int, uint32_t*, int32_t);
+template __global__ void k_rs_hist<16, false>(const uint32_t*, const uint32_t*, uint32_t, int, uint32_t*, int32_t);
 
 // ------------------------------------------------------------------ indel pass
 namespace {

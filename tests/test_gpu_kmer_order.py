@@ -51,3 +51,26 @@ def test_kmer_byte_order(kind, n, K):
             assert got == ref
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("occ", [1, 1024, 1025, 131_072, 131_073, 524_288, 524_289])
+def test_kmer_sort_sizes(occ):
+    """Occurrences, all of different K-mers, that just fill the tiles of each
+    form of the radix sort, and one more."""
+    from oracle import oracle as O
+    from pilon_amd.engine import Context
+    print(f"case: kmer sort of {occ} occurrences", flush=True)
+    K, per = 24, 256
+    rng = np.random.default_rng(occ)
+    lens = [per] * (occ // per) + ([occ % per] if occ % per else [])
+    b = pack_reads([dict(pos=1, cigar=f"{n + K}M", seq="".join(np.array(list("ACGT"))[rng.integers(0, 4, n + K)]),
+                         qual=[30] * (n + K), mapq=40) for n in lens], sort=False)
+    cfg = default_config()
+    ctx = Context(cfg, device=0)
+    try:
+        got, _ = ctx.kmer_graph(b, K=K, min_depth=1)
+    finally:
+        ctx.close()
+    st, ref = O.kmer_graph(cfg, b, K=K, min_depth=1)
+    assert st == 0 and len(ref) > occ // 2
+    assert got == ref
