@@ -635,7 +635,7 @@ struct NarrowLds : SinkBase {
   uint32_t* cell;        // [4][W]
   int32_t *qc, *mc, *qs; // [4][W], [W], [W]
   uint32_t *in_, *de_;
-  uint32_t* cb;          // clips << 16, plus the badPair difference (signed); then badPair
+  uint32_t* cb;          // clips << 16, plus the badPair difference (signed)
   uint32_t* extra;       // slid bases and indels of the window
   __device__ uint32_t* init(unsigned long long* lds, int w) {
     W = w;
@@ -790,7 +790,6 @@ __global__ void __launch_bounds__(BLOCK, NARROW ? PL_NARROW_WAVES_EU : PL_WIN_WA
   int32_t* queue = mode == 2 ? A.wqueue : A.queue;
   const int32_t n_heads = mode == 2 ? (int32_t)*A.wide_wins : A.n_wins;
   __shared__ RunL s_run[NW * (2 * 64 + 1)];
-  __shared__ int32_t s_w;
   __shared__ int32_t ws_a[NW], ws_b[NW], ws_c[NW];
   __shared__ unsigned long long red[2][NW];
   __shared__ int32_t s_ovf;
@@ -807,7 +806,6 @@ __global__ void __launch_bounds__(BLOCK, NARROW ? PL_NARROW_WAVES_EU : PL_WIN_WA
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int lds_words = ((NARROW ? PL_NARROW_LDS_PER_POS : PL_WIN_LDS_PER_POS) * W) / 8 + 256 / 2;
   const KConf& cf = A.cf;
-  (void)s_w;
 
   if (tid == 0) {
     const int32_t q = persistent ? atomicAdd(queue, 1) : (int32_t)blockIdx.x;
