@@ -82,8 +82,10 @@ pl_status kmer_graph(pl_ctx* c, const pl_read_soa* R, int32_t K, int32_t min_dep
   // Hash bits the order is by: twice those of N, so that of N distinct
   // K-mers two share them in about half the calls at worst and, of the third
   // or less that are distinct in reads with errors, in a few of a hundred.
-  const int bits = std::min(64, (2 * bits_of(N) + 7) / 8 * 8);
-  A.hmask = bits >= 64 ? ~0u : bits > 32 ? (1u << (bits - 32)) - 1u : 0u;
+  // At least 32: the low word is compared whole, so a shorter order would cut
+  // the run of a K-mer wherever another shares its bits.
+  const int bits = std::min(64, std::max(32, (2 * bits_of(N) + 7) / 8 * 8));
+  A.hmask = bits >= 64 ? ~0u : (1u << (bits - 32)) - 1u;
   A.cap = (uint32_t)(N / std::max(min_depth, 1)) + 1;
   SortRecs a, b;
   uint32_t* counts;                                          // list_n, out_n, flags[2]
