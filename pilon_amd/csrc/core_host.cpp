@@ -114,6 +114,7 @@ void* ch_run(const pl_config* pc, const uint8_t* ref, int64_t ref_len, const cha
   }
   // ---- jobs and windows
   int64_t G = 0;
+  int32_t n_wins = 0;
   std::vector<JobDev> jobs((size_t)n_jobs);
   std::vector<JobStat> st((size_t)n_jobs);
   std::vector<uint32_t> hist((size_t)n_jobs * PL_HIST, 0);
@@ -125,6 +126,9 @@ void* ch_run(const pl_config* pc, const uint8_t* ref, int64_t ref_len, const cha
     J.qe = (int32_t)std::min<int64_t>((int64_t)J.stop + 10000, ref_len);
     J.size = J.stop - J.start + 1;
     J.out = G;
+    J.win0 = n_wins;
+    J.nwin = (J.size + W - 1) / W;
+    n_wins += J.nwin;
     G += J.size;
     std::memset(&st[j], 0, sizeof(JobStat));
     st[j].err_read_edge = INT64_MAX;
@@ -133,6 +137,7 @@ void* ch_run(const pl_config* pc, const uint8_t* ref, int64_t ref_len, const cha
   int32_t* pile = pile_out;
   pl_call* calls = calls_out;
   std::vector<IndelRec> recs;
+  std::vector<uint32_t> win_rec;                     // each window's first record and their count
   std::vector<uint32_t> defer;
   std::map<uint32_t, std::array<int64_t, 4>> wide;   // exact qualSums of wide columns
   auto patch = [&](Col& c, uint32_t g) {
@@ -165,6 +170,7 @@ void* ch_run(const pl_config* pc, const uint8_t* ref, int64_t ref_len, const cha
       std::fill(badA.begin(), badA.end(), 0); std::fill(clpA.begin(), clpA.end(), 0);
       std::fill(pcA.begin(), pcA.end(), 0); std::fill(isA.begin(), isA.end(), 0);
       HostSink sk;
+      const size_t rec0 = recs.size();
       sk.W = W; sk.bs = bs.data(); sk.mqq = mqq.data(); sk.ins_ = insA.data(); sk.del_ = delA.data();
       sk.bad_ = badA.data(); sk.clp_ = clpA.data(); sk.pc = pcA.data(); sk.is = isA.data(); sk.recs = &recs;
       const int64_t lo = lower_pos(R.pos, n, (int64_t)L0 - max_back);
@@ -225,6 +231,8 @@ void* ch_run(const pl_config* pc, const uint8_t* ref, int64_t ref_len, const cha
         }
       for (int64_t r : cplx) walk_read(R, J, cf, r, L0, L1, 0, 1, sk, false);
       for (int64_t r : outliers) walk_read(R, J, cf, r, L0, L1, 0, 1, sk, true);
+      win_rec.push_back((uint32_t)rec0);
+      win_rec.push_back((uint32_t)(recs.size() - rec0));
       if (sk.edge_read >= 0 && sk.edge_read < S.err_read_edge) S.err_read_edge = sk.edge_read;
       S.base_count += sk.bcount;
       S.aligned += sk.aligned_n;
@@ -287,11 +295,7 @@ void* ch_run(const pl_config* pc, const uint8_t* ref, int64_t ref_len, const cha
       }
     }
   }
-  // ---- sort records by key (stable), indel pass on deferred columns
-  std::vector<uint32_t> rkey(recs.size()), rval(recs.size());
-  for (size_t i = 0; i < recs.size(); i++) rval[i] = (uint32_t)i;
-  std::stable_sort(rval.begin(), rval.end(), [&](uint32_t a, uint32_t b) { return recs[a].key < recs[b].key; });
-  for (size_t i = 0; i < recs.size(); i++) rkey[i] = recs[rval[i]].key;
+  // ---- indel pass on deferred columns
   auto job_of = [&](int64_t g) {
     int32_t j = 0;
     while (j + 1 < n_jobs && jobs[j + 1].out <= g) j++;
@@ -304,8 +308,8 @@ void* ch_run(const pl_config* pc, const uint8_t* ref, int64_t ref_len, const cha
     patch(c, g);
     int32_t ilen;
     int64_t wrec;
-    pl_call cl = full_call(&R, J, c, ref[J.start + (g - J.out) - 1], recs.data(), rkey.data(), rval.data(),
-                           (int64_t)recs.size(), g, cf, &ilen, &wrec);
+    pl_call cl = full_call(R, c, ref[J.start + (g - J.out) - 1], recs.data(), (uint32_t)recs.size(), win_rec.data(),
+                           J.win0 + (int32_t)((g - J.out) / W), g, cf, &ilen, &wrec);
     cl.flags |= calls[g].flags & PL_CF_WIDE;
     calls[g] = cl;
     const int d = call_disp(cl);
@@ -332,8 +336,8 @@ void* ch_run(const pl_config* pc, const uint8_t* ref, int64_t ref_len, const cha
       patch(c, g);
       int32_t ilen;
       int64_t wrec;
-      pl_call cl = full_call(&R, J, c, ref[J.start + (g - J.out) - 1], recs.data(), rkey.data(), rval.data(),
-                             (int64_t)recs.size(), g, cf, &ilen, &wrec);
+      pl_call cl = full_call(R, c, ref[J.start + (g - J.out) - 1], recs.data(), (uint32_t)recs.size(), win_rec.data(),
+                             J.win0 + (int32_t)((g - J.out) / W), g, cf, &ilen, &wrec);
       cl.flags |= calls[g].flags & PL_CF_WIDE;
       calls[g].base = cl.base; calls[g].alt = cl.alt; calls[g].q = cl.q;
       calls[g].flags = (uint16_t)((cl.flags & ~PL_CF_DISP_MASK) | (calls[g].flags & PL_CF_DISP_MASK) | PL_CF_DELETED);
@@ -398,5 +402,45 @@ int64_t ch_text(void* h, int32_t j, int32_t which, const char** p) {
 }
 
 void ch_free(void* h) { delete (Handle*)h; }
+
+// The evidence buffers of n_wins windows of n_recs[w] records each, as the
+// window kernel and k_spill_place fill them (lds_cap records of a window
+// first, the rest through the spill list), over memory that held other
+// records: how many slots a column's scan then meets that this batch did not
+// write.  seen[w] takes the records of window w it meets.
+int64_t ch_evidence(int32_t n_wins, const int32_t* n_recs, int32_t lds_cap, uint32_t rec_cap, uint32_t spill_cap,
+                    int32_t* seen) {
+  constexpr uint32_t KEY = 7;
+  IndelRec stale, e;
+  std::memset(&stale, 0, sizeof stale);
+  stale.key = KEY;
+  stale.src = -1;
+  e = stale;
+  e.src = 1;
+  std::vector<IndelRec> rec(rec_cap, stale), spill(spill_cap, stale);
+  std::vector<std::array<uint32_t, 2>> at(spill_cap);
+  std::vector<uint32_t> win_rec(2 * (size_t)n_wins);
+  uint32_t rec_n = 0, spill_n = 0;
+  for (int32_t w = 0; w < n_wins; w++) {
+    win_rec[2 * w] = rec_n;
+    win_rec[2 * w + 1] = (uint32_t)n_recs[w];
+    for (uint32_t j = 0; j < (uint32_t)n_recs[w]; j++) {
+      if (j < (uint32_t)lds_cap) { if (rec_n + j < rec_cap) rec[rec_n + j] = e; }
+      else if (spill_n++ < spill_cap) { spill[spill_n - 1] = e; at[spill_n - 1] = {(uint32_t)w, j}; }
+    }
+    rec_n += (uint32_t)n_recs[w];
+  }
+  for (uint32_t i = 0; i < std::min(spill_n, spill_cap); i++) {
+    const uint32_t k = win_rec[2 * at[i][0]] + at[i][1];
+    if (k < rec_cap) rec[k] = spill[i];
+  }
+  int64_t unwritten = 0;
+  for (int32_t w = 0; w < n_wins; w++) {
+    const ColRecs C = col_recs(rec.data(), rec_cap, win_rec.data(), w, spill_n, spill_cap, KEY);
+    seen[w] = (int32_t)std::max<int64_t>(C.b - C.a, 0);
+    for (int64_t i = C.a; i < C.b; i++) unwritten += rec[(size_t)i].src < 0;
+  }
+  return unwritten;
+}
 
 }  // extern "C"

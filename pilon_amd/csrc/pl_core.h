@@ -968,36 +968,49 @@ PL_HD bool rec_same(const RSDev& R, const IndelRec& x, const IndelRec& y) {
   return true;
 }
 
-// Exact strict-majority test over one (position, kind) group of records:
-// a string with count > n/2 exists iff the Boyer-Moore candidate has it, so
-// the outcome is that of map.toSeq.sortBy(_._2).last with the strict-majority
-// test of hetIndelCall, independent of order.
-struct Majority { int32_t n, win; int64_t rec; };
-PL_HD Majority group_majority(const RSDev& R, const IndelRec* recs, const uint32_t* idx, int64_t a, int64_t b) {
-  Majority m;
-  m.n = (int32_t)(b - a);
-  m.win = 0;
-  m.rec = -1;
-  if (b <= a) return m;
-  int64_t cand = idx[a];
-  int32_t cnt = 0;
-  for (int64_t i = a; i < b; i++) {
-    const IndelRec& e = recs[idx[i]];
-    if (cnt == 0) { cand = idx[i]; cnt = 1; }
-    else if (rec_same(R, e, recs[cand])) cnt++;
-    else cnt--;
-  }
-  int32_t c = 0;
-  for (int64_t i = a; i < b; i++) if (rec_same(R, recs[idx[i]], recs[cand])) c++;
-  m.win = c;
-  m.rec = cand;
-  return m;
+// A column's evidence: the records of its key, (position << 1) | kind, among
+// its window's, which lie together in the batch's (win_rec: each window's
+// first record and their count).  A record beyond a window's LDS buffer is
+// put in its place from the spill list; with more of those than the list
+// holds, a window counts records that nobody wrote, so no window has any (the
+// batch runs again with room for them).
+struct ColRecs {
+  const IndelRec* recs;
+  int64_t a, b;
+  uint32_t key;
+};
+PL_HD ColRecs col_recs(const IndelRec* recs, uint32_t rec_cap, const uint32_t* win_rec, int32_t w, uint32_t spill_n,
+                       uint32_t spill_cap, uint32_t key) {
+  ColRecs C;
+  C.recs = recs;
+  C.key = key;
+  C.a = win_rec[2 * w];
+  C.b = C.a + win_rec[2 * w + 1];
+  if (C.b > (int64_t)rec_cap) C.b = rec_cap;               // an overfull buffer: the batch runs again
+  if (spill_n > spill_cap) C.b = C.a;
+  return C;
 }
 
-PL_HD int64_t lower_bound_u32(const uint32_t* k, int64_t n, uint32_t x) {
-  int64_t lo = 0, hi = n;
-  while (lo < hi) { int64_t m = (lo + hi) >> 1; if (k[m] < x) lo = m + 1; else hi = m; }
-  return lo;
+// Exact strict-majority test over a column's records: a string with count >
+// n/2 exists iff the Boyer-Moore candidate has it, so the outcome is that of
+// map.toSeq.sortBy(_._2).last with the strict-majority test of hetIndelCall,
+// independent of order.
+struct Majority { int32_t n, win; int64_t rec; };
+PL_HD Majority col_majority(const RSDev& R, const ColRecs& C) {
+  Majority m;
+  m.n = m.win = 0;
+  m.rec = -1;
+  int32_t cnt = 0;
+  for (int64_t i = C.a; i < C.b; i++) {
+    if (C.recs[i].key != C.key) continue;
+    m.n++;
+    if (cnt == 0) { m.rec = i; cnt = 1; }
+    else if (rec_same(R, C.recs[i], C.recs[m.rec])) cnt++;
+    else cnt--;
+  }
+  for (int64_t i = C.a; i < C.b; i++)
+    if (C.recs[i].key == C.key && rec_same(R, C.recs[i], C.recs[m.rec])) m.win++;
+  return m;
 }
 
 // ------------------------------------------------------------ window flush
@@ -1194,23 +1207,20 @@ PL_HD void finalize_narrow(const NarrowCol& N, uint8_t refb, const KConf& cf, Po
   o.call = make_call(f, 0, true, refb, cf);
 }
 
-// The full BaseCall of one position from the pileup and its sorted evidence
+// The full BaseCall of one position from the pileup and its window's evidence
 // records (indel pass and recomputation after Pass-1 mutations).
-PL_HD pl_call full_call(const RSDev* rsets, const JobDev& J, const Col& c, uint8_t refb,
-                        const IndelRec* recs, const uint32_t* rkey, const uint32_t* rval, int64_t nrec,
-                        uint32_t gpos, const KConf& cf, int32_t* indel_len, int64_t* win_rec) {
+PL_HD pl_call full_call(const RSDev& R, const Col& c, uint8_t refb, const IndelRec* recs, uint32_t n_recs,
+                        const uint32_t* win_rec, int32_t w, uint32_t gpos, const KConf& cf, int32_t* indel_len,
+                        int64_t* win_rec_out) {
   BaseFacts bf = base_facts(c);
   int32_t pct = 0;
   int need = indel_kind_needed(c, cf, &pct);
   int indel = 0;
   bool homo = true;
   *indel_len = 0;
-  *win_rec = -1;
+  *win_rec_out = -1;
   if (need) {
-    const uint32_t key = (gpos << 1) | (uint32_t)(need - 1);
-    const int64_t a = lower_bound_u32(rkey, nrec, key);
-    const int64_t b = lower_bound_u32(rkey, nrec, key + 1);
-    Majority m = group_majority(rsets[J.rs], recs, rval, a, b);
+    const Majority m = col_majority(R, col_recs(recs, n_recs, win_rec, w, 0, 0, (gpos << 1) | (uint32_t)(need - 1)));
     if (m.rec >= 0) {
       const IndelRec& e = recs[m.rec];
       int d = het_indel_decide(m.n, m.win, e.len, (e.flags & 2u) != 0, pct, cf);
@@ -1218,7 +1228,7 @@ PL_HD pl_call full_call(const RSDev* rsets, const JobDev& J, const Col& c, uint8
         indel = need;
         homo = d == 2;
         *indel_len = e.len;
-        *win_rec = m.rec;
+        *win_rec_out = m.rec;
       }
     }
   }

@@ -1608,32 +1608,6 @@ __device__ __forceinline__ int32_t job_of(const JobDev* jobs, int32_t n_jobs, in
 
 namespace {
 
-// a column's records among its window's
-struct ColRecs {
-  const IndelRec* recs;
-  int64_t a, b;              // the window's segment
-  uint32_t key;              // (gpos << 1) | kind
-};
-
-// the strict majority of a column's records by one lane in record order:
-// the exact form group_majority, over the records of one key
-__device__ Majority col_majority_serial(const RSDev& R, const ColRecs& C) {
-  Majority m;
-  m.n = m.win = 0;
-  m.rec = -1;
-  int32_t cnt = 0;
-  for (int64_t i = C.a; i < C.b; i++) {
-    if (C.recs[i].key != C.key) continue;
-    m.n++;
-    if (cnt == 0) { m.rec = i; cnt = 1; }
-    else if (rec_same(R, C.recs[i], C.recs[m.rec])) cnt++;
-    else cnt--;
-  }
-  for (int64_t i = C.a; i < C.b; i++)
-    if (C.recs[i].key == C.key && rec_same(R, C.recs[i], C.recs[m.rec])) m.win++;
-  return m;
-}
-
 // The strict majority over a column's records, by the whole wave.  The
 // window's records are not sorted: a window holds a handful, and the wave
 // tests 64 keys at a time, which costs less than sorting every record of
@@ -1643,7 +1617,7 @@ __device__ Majority col_majority_serial(const RSDev& R, const ColRecs& C) {
 // (a merge keeps a majority class if there is one), and the winning class's
 // string is counted exactly.  A class with a strict majority whose
 // representative string falls short (a hash collision) is resolved by the
-// serial scan.  Same result as group_majority.
+// serial scan.  Same result as col_majority.
 __device__ Majority wave_majority(const RSDev& R, const ColRecs& C, int lane) {
   Majority m;
   m.n = m.win = 0;
@@ -1683,7 +1657,7 @@ __device__ Majority wave_majority(const RSDev& R, const ColRecs& C, int lane) {
   cls = wave_sum(cls);
   same = wave_sum(same);
   if (2 * same > m.n) { m.win = same; m.rec = cr; return m; }
-  if (2 * cls > m.n) return col_majority_serial(R, C);             // collision inside the majority class
+  if (2 * cls > m.n) return col_majority(R, C);                    // collision inside the majority class
   m.win = same;                                                     // no strict majority
   return m;
 }
@@ -1732,12 +1706,7 @@ __device__ void indel_columns(const EngineArgs& A, const uint32_t* list, uint32_
     bool homo = true;
     int64_t wrec = -1;
     if (need) {
-      ColRecs C;
-      C.recs = A.rec;
-      C.key = (g << 1) | (uint32_t)(need - 1);
-      C.a = A.win_rec[2 * w];
-      C.b = C.a + A.win_rec[2 * w + 1];
-      if (C.b > (int64_t)A.rec_cap) C.b = A.rec_cap;              // an overfull buffer: the batch runs again
+      const ColRecs C = col_recs(A.rec, A.rec_cap, A.win_rec, w, *A.spill_n, A.spill_cap, (g << 1) | (uint32_t)(need - 1));
       const Majority mj = wave_majority(R, C, lane);
       if (mj.rec >= 0) {
         const IndelRec& e = A.rec[mj.rec];

@@ -22,6 +22,8 @@ def lib():
         L.ch_text.restype = C.c_int64
         L.ch_text.argtypes = [C.c_void_p, C.c_int32, C.c_int32, C.POINTER(C.c_char_p)]
         L.ch_free.argtypes = [C.c_void_p]
+        L.ch_evidence.restype = C.c_int64
+        L.ch_evidence.argtypes = [C.c_int32, C.c_void_p, C.c_int32, C.c_uint32, C.c_uint32, C.c_void_p]
         _lib = L
     return _lib
 
@@ -58,3 +60,11 @@ def run(cfg, contig, batch, regions, W=1024, name="ctg", lrt=None, set_kinds=1):
         off += n
     L.ch_free(h)
     return out
+
+
+def evidence(n_recs, lds_cap, rec_cap, spill_cap):
+    """(slots a column's scan meets that the batch did not write, records met per window)."""
+    n = np.array(n_recs, np.int32)
+    seen = np.zeros(len(n), np.int32)
+    bad = lib().ch_evidence(len(n), n.ctypes.data, lds_cap, rec_cap, spill_cap, seen.ctypes.data)
+    return bad, seen

@@ -123,3 +123,16 @@ def test_long_reads_by_segments_core_host(read_len, lr, W):
             assert_same_region(g["pile"], g["calls"], ref, f"{lr} {s}-{e}")
             assert_same_stats(g["stats"], ref["stats"])
             assert g["changes"] == ref["changes"] and g["bases"] == ref["bases"]
+
+
+@pytest.mark.parametrize("n_recs,rec_cap,spill_cap,whole", [
+    ([0, 128, 129, 5], 1000, 1, True), ([300, 300, 2], 1000, 344, True),       # the list just holds the spilled ones
+    ([300, 300, 2], 1000, 343, False), ([128, 400, 10, 200], 4000, 16, False),  # ... and does not
+    ([300, 300, 2], 500, 344, False), ([300, 300, 2], 500, 10, False),          # an overfull record buffer
+])
+def test_no_unwritten_record_is_read(n_recs, rec_cap, spill_cap, whole):
+    """A column's scan of its window's records meets every one of them, or,
+    where they did not all find room, none that the batch did not write."""
+    bad, seen = CH.evidence(n_recs, 128, rec_cap, spill_cap)
+    assert bad == 0
+    assert (list(seen) == n_recs) == whole

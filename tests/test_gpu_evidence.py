@@ -1,7 +1,8 @@
 """Indel evidence and candidate order of a batch against the oracle: windows
 whose records just fit their LDS buffer (128) and spill beyond it, at one
 column and over many, with the windows taken in their own order and, when
-more than the launch holds at once, in cost order."""
+more than the launch holds at once, in cost order; more spilled records than
+their list holds at first, on a context that held another set's records."""
 import numpy as np
 import pytest
 
@@ -57,6 +58,35 @@ def test_window_record_buffer(n, window, persistent):
     assert_same_stats(stats[0], want["stats"], f"{n} records")
     assert changes == want["changes"]
     assert text == want["vcf"]
+
+
+def test_more_spilled_than_the_list_holds():
+    """16,720 spilled records (the list starts at 16,384) at the columns where
+    an earlier batch of another read set left its own, then that set again."""
+    from oracle import oracle as O
+    from pilon_amd.engine import Context
+    print("case: spill list overflow over an earlier batch's records", flush=True)
+    rng = np.random.default_rng(5)
+    ref = "".join("ACGT"[x] for x in rng.integers(0, 4, 20_000))
+    few = pack_reads(indel_reads(ref, [(64 * w + 41, "I", 4, 110) for w in range(1, 300)], 1))
+    out = indel_reads(ref, [(64 * w + 41, "I", 3, 1800) for w in range(150, 160)], 2)
+    for r in out:                                  # an N: walked, so the read set's segments do not tell
+        r["seq"] = r["seq"][:3] + "N" + r["seq"][4:]
+    many = pack_reads(out)
+    cfg = default_config()
+    want = [O.run_region(cfg, ref.encode(), 1, len(ref), [b], name="ctg") for b in (few, many)]
+    ctx = Context(cfg, device=0)
+    try:
+        ctx.ref_upload(0, "ctg", ref)
+        ids = [ctx.readset_upload(0, b) for b in (few, many)]
+        for k in (0, 1, 0):
+            pile, calls, stats = ctx.batch_run([(0, 1, len(ref), ids[k])], window=64, block=256, persistent=1)
+            changes, _ = ctx.batch_fix()
+            assert_same_region(pile, calls, want[k], f"set {k}")
+            assert_same_stats(stats[0], want[k]["stats"], f"set {k}")
+            assert changes == want[k]["changes"]
+    finally:
+        ctx.close()
 
 
 def test_candidates_over_many_blocks():
