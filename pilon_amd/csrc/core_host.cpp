@@ -144,6 +144,7 @@ void* ch_run(const pl_config* pc, const uint8_t* ref, int64_t ref_len, const cha
     auto it = wide.find(g);
     if (it != wide.end()) for (int b = 0; b < 4; b++) c.qs[b] = it->second[b];
   };
+  bool forms_differ = false;
   std::vector<Cand> cands;
   std::vector<uint64_t> bs(4 * (size_t)W), mqq(W), insA(W), delA(W);
   std::vector<uint32_t> badA(W), clpA(W);
@@ -244,7 +245,8 @@ void* ch_run(const pl_config* pc, const uint8_t* ref, int64_t ref_len, const cha
         const int64_t g = J.out + p0 + p;
         PosOut o;
         finalize_position(b4, mqq[p], insA[p], delA[p], badA[p], clpA[p], apc, ais, ref[L0 + p - 1], cf, o);
-        // the same column through the narrow counters, when it fits them
+        // the same column through the narrow counters, when it fits them,
+        // must come out the same
         if (cf.min_qual >= 0 && o.f[PL_F_INSERTIONS] <= PL_NARROW_MAX && o.f[PL_F_DELETIONS] <= PL_NARROW_MAX) {
           NarrowCol N;
           N.m0 = 1 + (int32_t)(g % 61);
@@ -265,9 +267,10 @@ void* ch_run(const pl_config* pc, const uint8_t* ref, int64_t ref_len, const cha
           N.del = ((uint32_t)o.f[PL_F_DELETIONS] << PL_NARROW_SHIFT) | (uint32_t)o.f[PL_F_DELQUAL];
           N.clips = clpA[p]; N.bad = badA[p]; N.pc = apc; N.is = ais;
           if (fits && depth + o.f[PL_F_INSERTIONS] + o.f[PL_F_DELETIONS] <= PL_NARROW_MAX) {
-            PosOut w = o;
-            finalize_narrow(N, ref[L0 + p - 1], cf, o);
-            std::memcpy(o.qs, w.qs, sizeof o.qs);
+            PosOut w;
+            finalize_narrow(N, ref[L0 + p - 1], cf, w);
+            forms_differ = forms_differ || std::memcmp(w.f, o.f, sizeof o.f) != 0 ||
+                           std::memcmp(&w.call, &o.call, sizeof o.call) != 0 || w.defer != o.defer;
           }
         }
         if (o.overflow) S.overflow = 1;
@@ -387,7 +390,8 @@ void* ch_run(const pl_config* pc, const uint8_t* ref, int64_t ref_len, const cha
     o.dels = fr.dels; o.del_bases = fr.del_bases;
     o.n_unknown_ops = (int32_t)st[j].unknown_ops;
     o.aligned_bases = st[j].aligned;
-    errs[j] = st[j].err_read_inval < st[j].err_read_edge ? PL_E_INVAL
+    errs[j] = forms_differ ? PL_E_DEVICE
+              : st[j].err_read_inval < st[j].err_read_edge ? PL_E_INVAL
               : st[j].err_read_edge != INT64_MAX ? PL_E_EDGE : st[j].overflow ? PL_E_OVERFLOW : PL_OK;
   }
   (void)ovf;
