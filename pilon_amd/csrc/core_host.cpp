@@ -407,6 +407,8 @@ int64_t ch_text(void* h, int32_t j, int32_t which, const char** p) {
 
 void ch_free(void* h) { delete (Handle*)h; }
 
+uint32_t ch_cost_bin(int64_t c) { return cost_bin(c); }
+
 // The evidence buffers of n_wins windows of n_recs[w] records each, as the
 // window kernel and k_spill_place fill them (lds_cap records of a window
 // first, the rest through the spill list), over memory that held other

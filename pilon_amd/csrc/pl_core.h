@@ -247,6 +247,16 @@ PL_HD PrepOut prep_read(const RSDev& R, int64_t r, const KConf& cf) {
   return o;
 }
 
+// Cost bin of a window: 0 for the most work, four mantissa bits above 16
+// units (windows of one bin differ by at most 6%, what the queue's order is
+// for).  Costs above 65,535 share a bin: 208 of the PL_COST_BINS are in use.
+PL_HD uint32_t cost_bin(int64_t c) {
+  const uint32_t v = (uint32_t)(c > 65535 ? 65535 : c);
+  const uint32_t lg = 31u - (uint32_t)__builtin_clz(v | 1u);
+  const uint32_t b = v < 16u ? v : (lg - 3u) * 16u + ((v >> (lg - 4u)) & 15u);
+  return PL_COST_BINS - 1u - b;
+}
+
 // ------------------------------------------------------------ the read walk
 // addRead's homoRun(i0) >= 4 (PileUpRegion.scala:120-126): the contig byte
 // at 0-based index i0 (0 <= i0 < ref_len) and the three after it are equal.

@@ -351,15 +351,6 @@ __device__ __forceinline__ int64_t group_lower_pos_near(const int32_t* pos, int6
   return group_lower_pos<GL>(pos, lo, hi, x);
 }
 
-// cost bin of a window: 0 for the most work, four mantissa bits above 16
-// units (windows of one bin differ by at most 6%, what the queue's order is for)
-__device__ __forceinline__ uint32_t cost_bin(int64_t c) {
-  const uint32_t v = (uint32_t)(c > 0xffffll ? 0xffffll : c);
-  const uint32_t lg = 31u - (uint32_t)__clz((int)(v | 1u));
-  const uint32_t b = v < 16u ? v : (lg - 3u) * 16u + ((v >> (lg - 4u)) & 15u);
-  return PL_COST_BINS - 1u - b;
-}
-
 __device__ __forceinline__ void put_head(WinHead* heads, int32_t slot, int32_t wi, const WinDev& w, const JobDev& J,
                                          int32_t m0) {
   WinHead h;

@@ -22,6 +22,8 @@ def lib():
         L.ch_text.restype = C.c_int64
         L.ch_text.argtypes = [C.c_void_p, C.c_int32, C.c_int32, C.POINTER(C.c_char_p)]
         L.ch_free.argtypes = [C.c_void_p]
+        L.ch_cost_bin.restype = C.c_uint32
+        L.ch_cost_bin.argtypes = [C.c_int64]
         L.ch_evidence.restype = C.c_int64
         L.ch_evidence.argtypes = [C.c_int32, C.c_void_p, C.c_int32, C.c_uint32, C.c_uint32, C.c_void_p]
         _lib = L

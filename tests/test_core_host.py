@@ -136,3 +136,26 @@ def test_no_unwritten_record_is_read(n_recs, rec_cap, spill_cap, whole):
     bad, seen = CH.evidence(n_recs, 128, rec_cap, spill_cap)
     assert bad == 0
     assert (list(seen) == n_recs) == whole
+
+
+def test_cost_bins_order_every_window():
+    """Any cost falls in a bin of the table, more work never in a later one,
+    and windows placed by their bins fill the queue's slots once each."""
+    bin_of = CH.lib().ch_cost_bin
+    costs = [0, 1, 15, 16, 17, 31, 32, 255, 256, 4095, 4096, 65_534, 65_535, 65_536, 2 ** 19 - 1, 2 ** 19, 557_056,
+             2 ** 20, 2 ** 24 - 1, 2 ** 31 - 1, 2 ** 31, 2 ** 40]
+    bins = [bin_of(c) for c in costs]
+    assert all(0 <= b < 256 for b in bins) and bins == sorted(bins, reverse=True)
+    assert all(bin_of(c) >= bin_of(c + 1) for c in range(70_000))
+    rng = np.random.default_rng(3)
+    cost = np.concatenate([np.full(2000, 300), rng.integers(0, 2 ** 24, 500), [6, 6, 6, 2 ** 20, 2 ** 31]])
+    b = np.array([bin_of(int(c)) for c in cost])
+    start = np.concatenate([[0], np.cumsum(np.bincount(b, minlength=256))[:-1]])
+    taken = np.zeros(256, int)
+    slot = []
+    for x in b:                                    # k_plan's counts, k_heads' slots
+        slot.append(start[x] + taken[x])
+        taken[x] += 1
+    assert sorted(slot) == list(range(len(cost)))
+    c = np.minimum(cost, 65_535)[np.argsort(slot)]
+    assert np.all(c[1:] <= 1.0625 * c[:-1] + 1)
