@@ -151,100 +151,127 @@ PL_HD uint32_t del_hash(const uint8_t* ref, int64_t off, int32_t len, uint32_t* 
 // (PileUpRegion.scala:107,139-141), the span of positions the read can touch
 // (M bases, soft clips, slid indels) and its physical-coverage fragment
 // (physCovIncr, PileUpRegion.scala:62-73).
+// The pieces are per CIGAR op, so that a wave can take a long read's ops side
+// by side; prep_read takes them in order.
 struct PrepOut { RMeta m; int32_t events; bool clips; };   // clips: more than two S ops
 
-PL_HD PrepOut prep_read(const RSDev& R, int64_t r, const KConf& cf) {
-  PrepOut o;
+struct ReadSums {            // of a read's ops
+  int32_t refLen = 0, readLen = 0, clipped = 0, nP = 0, nS = 0;
+  bool bad = false;
+};
+PL_HD void add_op(ReadSums& s, uint32_t w) {
+  const int op = (int)(w & 15);
+  const int32_t ln = (int32_t)(w >> 4);
+  if (op > 8) s.bad = true;
+  if (consumes_ref(op)) s.refLen += ln;
+  if (consumes_read(op)) s.readLen += ln;
+  if (op == 4) s.clipped = j_add(s.clipped, ln);
+  s.nS += op == 4 ? 1 : 0;
+  s.nP += op == 6 ? 1 : 0;
+}
+
+PL_HD uint32_t read_info(const RSDev& R, int64_t r, const ReadSums& s, const KConf& cf, int32_t* aend) {
   const uint16_t flag = R.flag[r];
   const int32_t mq = R.mapq[r];
-  const int32_t pos = R.pos[r];
-  const int32_t tlen = R.tlen[r];
   const int64_t c0 = R.cigar_off[r], c1 = R.cigar_off[r + 1];
   const int32_t L = (int32_t)(R.seq_off[r + 1] - R.seq_off[r]);
+  const bool bad = s.bad || (L > 0 && s.readLen != L);
   uint32_t info = 0;
-  int32_t refLen = 0, readLen = 0, clipped = 0, nP = 0, nS = 0;
-  bool bad = false, hasS = false;
-  for (int64_t k = c0; k < c1; k++) {
-    uint32_t w = R.cigar[k];
-    int op = (int)(w & 15);
-    int32_t ln = (int32_t)(w >> 4);
-    if (op > 8) bad = true;
-    if (consumes_ref(op)) refLen += ln;
-    if (consumes_read(op)) readLen += ln;
-    if (op == 4) { clipped = j_add(clipped, ln); hasS = true; nS++; }
-    if (op == 6) nP++;
-  }
-  if (L > 0 && readLen != L) bad = true;
-  const int32_t aend = (flag & 0x4) ? 0 : pos + refLen - 1;
+  *aend = (flag & 0x4) ? 0 : R.pos[r] + s.refLen - 1;
   const bool keep = (cf.nonpf || !(flag & 0x200)) && (cf.duplicates || !(flag & 0x400)) && !(flag & 0x100);
   const bool paired = (flag & 0x1) != 0;
   const bool valid = (mq >= cf.min_mq) && (!paired || (((flag & 0x2) != 0) && ((flag & PL_RF_MATE_SAME_REF) != 0)));
-  const int32_t adjMq = round_div_i(j_mul(mq, j_sub(L, clipped)), L);
+  const int32_t adjMq = round_div_i(j_mul(mq, j_sub(L, s.clipped)), L);
   info |= (uint32_t)adjMq & RI_ADJMQ_MASK;
   if (valid) info |= RI_VALID;
   if (keep) info |= RI_KEEP;
   if (flag & PL_RF_EXOTIC) info |= RI_EXOTIC;
   if (flag & PL_RF_NO_QUAL) info |= RI_NOQUAL;
   if (bad) info |= RI_BAD;
-  if (L == 0 && hasS) info |= RI_EDGE_CLIP;
-  info |= (uint32_t)(nP > 255 ? 255 : nP) << RI_UNK_SHIFT;
-  // a long read is always walked (its bases and indels depend on the
-  // reference around them): never simple, and too many segments
+  if (L == 0 && s.nS > 0) info |= RI_EDGE_CLIP;
+  info |= (uint32_t)(s.nP > 255 ? 255 : s.nP) << RI_UNK_SHIFT;
+  // a long read is never simple (its bases and indels depend on the
+  // reference around them), and walked until it has its segments
   const uint32_t lr = R.lrt ? (uint32_t)R.lrt[r] : 0u;
   if (lr) info |= (lr << RI_LR_SHIFT) | ((uint32_t)RI_SEG_MAX << RI_SEG_SHIFT);
-  const uint32_t op0 = c1 > c0 ? R.cigar[c0] : 0u;
   if (c1 - c0 == 1 && L > 0 && !bad && !(flag & PL_RF_EXOTIC) && !lr) {
-    const int op = (int)(op0 & 15);
+    const int op = (int)(R.cigar[c0] & 15);
     if (op == 0 || op == 7 || op == 8) info |= RI_SIMPLE;
   }
+  return info;
+}
 
-  int32_t lo = INT_MAX, hi = INT_MIN, events = 0;
-  if (!bad) {
-    ReadAcc a = read_acc(R, r, info, cf.default_qual);
-    const int32_t flank = cf.flank;
-    int32_t readOffset = 0, refOffset = 0;
-    for (int64_t k = c0; k < c1; k++) {
-      uint32_t w = R.cigar[k];
-      int op = (int)(w & 15);
-      int32_t len = (int32_t)(w >> 4);
-      int32_t locus = pos + refOffset;
-      bool tr = readOffset >= flank && j_sub(L, flank) > readOffset;
-      if ((op == 0 || op == 7 || op == 8) && len > 0) {
-        lo = locus < lo ? locus : lo;
-        hi = locus + len - 1 > hi ? locus + len - 1 : hi;
-      } else if (op == 4 && len > 0) {
-        int32_t cs = readOffset == 0 ? locus - len : locus;
-        lo = cs < lo ? cs : lo;
-        hi = cs + len - 1 > hi ? cs + len - 1 : hi;
-      } else if (op == 1 && len > 0 && valid && tr && locus <= R.ref_len) {
-        int32_t rot;
-        int32_t il = slide_insertion(R.ref, a, readOffset, len, locus, &rot);
-        lo = il < lo ? il : lo;
-        hi = locus > hi ? locus : hi;
-        events++;
-      } else if (op == 2 && len > 0 && valid && tr && (int64_t)locus + len - 1 <= R.ref_len) {
-        int32_t dl = locus, rl = readOffset;
-        while (dl > 1 && rl > 0 && R.ref[dl - 2] == R.ref[dl + len - 2]) { dl--; rl--; }
-        lo = dl < lo ? dl : lo;
-        hi = locus + len - 1 > hi ? locus + len - 1 : hi;
-        events++;
-      }
-      if (consumes_read(op)) readOffset += len;
-      if (consumes_ref(op)) refOffset += len;
-    }
+struct OpSpan { int32_t lo = INT_MAX, hi = INT_MIN, events = 0; };   // positions touched, indel events
+PL_HD OpSpan op_span(const RSDev& R, const ReadAcc& a, uint32_t info, const KConf& cf, uint32_t w, int32_t locus,
+                   int32_t readOffset, int32_t L, OpSpan s) {
+  const int op = (int)(w & 15);
+  const int32_t len = (int32_t)(w >> 4);
+  const bool valid = (info & RI_VALID) != 0;
+  const bool tr = readOffset >= cf.flank && j_sub(L, cf.flank) > readOffset;
+  int32_t lo, hi;
+  if ((op == 0 || op == 7 || op == 8) && len > 0) {
+    lo = locus;
+    hi = locus + len - 1;
+  } else if (op == 4 && len > 0) {
+    lo = readOffset == 0 ? locus - len : locus;
+    hi = lo + len - 1;
+  } else if (op == 1 && len > 0 && valid && tr && locus <= R.ref_len) {
+    int32_t rot;
+    lo = slide_insertion(R.ref, a, readOffset, len, locus, &rot);
+    hi = locus;
+    s.events++;
+  } else if (op == 2 && len > 0 && valid && tr && (int64_t)locus + len - 1 <= R.ref_len) {
+    int32_t dl = locus, rl = readOffset;
+    while (dl > 1 && rl > 0 && R.ref[dl - 2] == R.ref[dl + len - 2]) { dl--; rl--; }
+    lo = dl;
+    hi = locus + len - 1;
+    s.events++;
+  } else {
+    return s;
   }
-  if (events) info |= RI_EVENTS;
+  s.lo = lo < s.lo ? lo : s.lo;
+  s.hi = hi > s.hi ? hi : s.hi;
+  return s;
+}
+
+PL_HD PrepOut prep_result(const RSDev& R, int64_t r, uint32_t info, int32_t aend, const ReadSums& sums, const OpSpan& s) {
+  PrepOut o;
+  const int32_t pos = R.pos[r], tlen = R.tlen[r];
+  const bool paired = (R.flag[r] & 0x1) != 0;
+  const int64_t c0 = R.cigar_off[r], c1 = R.cigar_off[r + 1];
+  if (s.events) info |= RI_EVENTS;
   // physCovIncr fragment (only valid reads, and not the right mate of a pair)
   int32_t flo = 0, fhi = 0;
-  if (valid && keep && !(paired && tlen <= 0)) {
+  if ((info & RI_VALID) && (info & RI_KEEP) && !(paired && tlen <= 0)) {
     if (!paired) { flo = pos < aend ? pos : aend; fhi = pos > aend ? pos : aend; }
     else { flo = pos; fhi = j_add(pos, tlen); }
   }
-  o.m.pos = pos; o.m.info = info; o.m.fp_lo = lo; o.m.fp_hi = hi;
-  o.m.fr_lo = flo; o.m.fr_hi = fhi; o.m.aend = aend; o.m.op0 = op0;
-  o.events = events;
-  o.clips = nS > 2;
+  o.m.pos = pos; o.m.info = info; o.m.fp_lo = s.lo; o.m.fp_hi = s.hi;
+  o.m.fr_lo = flo; o.m.fr_hi = fhi; o.m.aend = aend; o.m.op0 = c1 > c0 ? R.cigar[c0] : 0u;
+  o.events = s.events;
+  o.clips = sums.nS > 2;
   return o;
+}
+
+PL_HD PrepOut prep_read(const RSDev& R, int64_t r, const KConf& cf) {
+  const int64_t c0 = R.cigar_off[r], c1 = R.cigar_off[r + 1];
+  ReadSums sums;
+  for (int64_t k = c0; k < c1; k++) add_op(sums, R.cigar[k]);
+  int32_t aend;
+  const uint32_t info = read_info(R, r, sums, cf, &aend);
+  OpSpan s;
+  if (!(info & RI_BAD)) {
+    const int32_t L = (int32_t)(R.seq_off[r + 1] - R.seq_off[r]);
+    const ReadAcc a = read_acc(R, r, info, cf.default_qual);
+    int32_t readOffset = 0, locus = R.pos[r];
+    for (int64_t k = c0; k < c1; k++) {
+      const uint32_t w = R.cigar[k];
+      s = op_span(R, a, info, cf, w, locus, readOffset, L, s);
+      if (consumes_read((int)(w & 15))) readOffset += (int32_t)(w >> 4);
+      if (consumes_ref((int)(w & 15))) locus += (int32_t)(w >> 4);
+    }
+  }
+  return prep_result(R, r, info, aend, sums, s);
 }
 
 // Cost bin of a window: 0 for the most work, four mantissa bits above 16
@@ -559,90 +586,93 @@ PL_HD int32_t seg_end(const Seg& g) {
 }
 
 // Whether a long read's segments may be cut to a window's: clips only at its
-// ends (one between other ops would break the order of seg_end).
-PL_HD bool long_segs_ok(const RSDev& R, int64_t r) {
-  const int64_t c0 = R.cigar_off[r], c1 = R.cigar_off[r + 1];
-  int32_t done = 0;                                        // read bases before the op
-  bool last = false;
-  const int32_t L = (int32_t)(R.seq_off[r + 1] - R.seq_off[r]);
-  for (int64_t k = c0; k < c1; k++) {
-    const int op = (int)(R.cigar[k] & 15);
-    const int32_t len = (int32_t)(R.cigar[k] >> 4);
-    if (last && (consumes_read(op) || consumes_ref(op)) && len > 0) return false;
-    if (op == 4 && len > 0 && done > 0) last = true;
-    if (consumes_read(op)) done += len;
-    else if (consumes_ref(op) && len > 0 && done == 0) return false;   // a deletion before the first base
+// ends (one between other ops would break the order of seg_end) and no
+// deletion before its first base.  Facts of its ops, in any order; k is the
+// op's index and readOffset the read bases before it.
+struct LongOps { int32_t clip = INT_MAX, last = -1; bool lead = false; };   // first clip after a base, last op that consumes
+PL_HD LongOps add_long_op(LongOps s, uint32_t w, int32_t k, int32_t readOffset) {
+  const int op = (int)(w & 15);
+  if ((int32_t)(w >> 4) <= 0) return s;
+  if (op == 4 && readOffset > 0 && k < s.clip) s.clip = k;
+  if ((consumes_read(op) || consumes_ref(op)) && k > s.last) s.last = k;
+  if (!consumes_read(op) && consumes_ref(op) && readOffset == 0) s.lead = true;
+  return s;
+}
+PL_HD bool long_segs_ok(const LongOps& s, int32_t L) { return L > 0 && !s.lead && s.last <= s.clip; }
+
+// Writes the segments of one op into out (if non-null); returns their count.
+// The insertions a long read drops have no segment.
+PL_HD int op_segs(const RSDev& R, const ReadAcc& a, uint32_t info, const KConf& cf, uint32_t w, int32_t locus,
+                  int32_t readOffset, int32_t L, Seg* out) {
+  const int op = (int)(w & 15);
+  const int32_t len = (int32_t)(w >> 4);
+  const int32_t flank = cf.flank;
+  const bool valid = (info & RI_VALID) != 0, lr = (info & RI_LR_MASK) != 0;
+  const bool tr = readOffset >= flank && j_sub(L, flank) > readOffset;
+  if (len <= 0) return 0;
+  if (op == 0 || op == 7 || op == 8) {
+    if (out) { Seg& g = out[0]; g.kq = SEG_M; g.locus = locus; g.roff = readOffset; g.len = len; g.fin = 0; g.hash = 0; g.rotn = 0; g.pad = 0; }
+    return 1;
   }
-  return L > 0;
+  if (op == 4) {
+    if (out) {
+      Seg& g = out[0];
+      g.kq = SEG_S; g.locus = readOffset == 0 ? locus - len : locus; g.roff = readOffset; g.len = len;
+      g.fin = 0; g.hash = 0; g.rotn = 0; g.pad = 0;
+    }
+    return 1;
+  }
+  if (op == 1 && valid && tr && locus <= R.ref_len) {
+    int32_t rot = 0, il = 0;
+    if (out || lr) il = slide_insertion(R.ref, a, readOffset, len, locus, &rot);
+    if (lr && il < R.ref_len && homo_run4(R, il)) return 0;   // dropped (PileUpRegion.scala:160)
+    if (out) {
+      uint32_t hasN;
+      const uint32_t h = ins_hash(a, readOffset, len, rot, &hasN);
+      Seg& g = out[0];
+      g.kq = SEG_I | (a.qual(readOffset) << 8); g.locus = locus; g.roff = readOffset; g.len = len;
+      g.fin = il; g.hash = h; g.rotn = rot | (int32_t)(hasN << 30); g.pad = 0;
+    }
+    return 1;
+  }
+  if (op == 2 && valid && tr && (int64_t)locus + len - 1 <= R.ref_len) {
+    int32_t dl = locus, rl = readOffset;
+    int n = 1;
+    while (dl > 1 && rl > 0 && R.ref[dl - 2] == R.ref[dl + len - 2]) {
+      dl--; rl--;
+      if (rl >= flank && j_sub(L, flank) > rl) {
+        if (out) {
+          Seg& g = out[n];
+          g.kq = SEG_A | (a.qual(rl) << 8); g.locus = dl; g.roff = rl; g.len = len;
+          g.fin = a.bi(rl); g.hash = 0; g.rotn = 0; g.pad = locus;   // pad: the deletion's own locus (its gate)
+        }
+        n++;
+      }
+    }
+    if (out) {
+      uint32_t hasN;
+      const uint32_t h = del_hash(R.ref, (int64_t)dl - 1, len, &hasN);
+      Seg& g = out[0];
+      g.kq = SEG_D | (a.qual(readOffset) << 8); g.locus = locus; g.roff = readOffset; g.len = len;
+      g.fin = dl; g.hash = h; g.rotn = (int32_t)(hasN << 30); g.pad = 0;
+    }
+    return n;
+  }
+  return 0;
 }
 
 // Writes the segments of read r into out (if non-null); returns their count.
-// lr: longReadType of the read (the insertions it drops have no segment).
 PL_HD int build_segs(const RSDev& R, int64_t r, uint32_t info, const KConf& cf, Seg* out) {
-  const uint32_t lr = (info & RI_LR_MASK) >> RI_LR_SHIFT;
   const int64_t c0 = R.cigar_off[r], c1 = R.cigar_off[r + 1];
   const int32_t L = (int32_t)(R.seq_off[r + 1] - R.seq_off[r]);
-  const int32_t pos = R.pos[r];
-  const bool valid = (info & RI_VALID) != 0;
-  const int32_t flank = cf.flank;
   const ReadAcc a = read_acc(R, r, info, cf.default_qual);
   int n = 0;
-  int32_t readOffset = 0, refOffset = 0;
+  int32_t readOffset = 0, locus = R.pos[r];
   for (int64_t k = c0; k < c1; k++) {
     const uint32_t w = R.cigar[k];
-    const int op = (int)(w & 15);
-    const int32_t len = (int32_t)(w >> 4);
-    const int32_t locus = pos + refOffset;
-    const bool tr = readOffset >= flank && j_sub(L, flank) > readOffset;
-    if ((op == 0 || op == 7 || op == 8) && len > 0) {
-      if (out) { Seg& g = out[n]; g.kq = SEG_M; g.locus = locus; g.roff = readOffset; g.len = len; g.fin = 0; g.hash = 0; g.rotn = 0; g.pad = 0; }
-      n++;
-    } else if (op == 4 && len > 0) {
-      if (out) {
-        Seg& g = out[n];
-        g.kq = SEG_S; g.locus = readOffset == 0 ? locus - len : locus; g.roff = readOffset; g.len = len;
-        g.fin = 0; g.hash = 0; g.rotn = 0; g.pad = 0;
-      }
-      n++;
-    } else if (op == 1 && len > 0 && valid && tr && locus <= R.ref_len) {
-      int32_t rot = 0, il = 0;
-      if (out || lr) il = slide_insertion(R.ref, a, readOffset, len, locus, &rot);
-      if (lr && il < R.ref_len && homo_run4(R, il)) {      // dropped (PileUpRegion.scala:160)
-        readOffset += len;
-        continue;
-      }
-      if (out) {
-        uint32_t hasN;
-        const uint32_t h = ins_hash(a, readOffset, len, rot, &hasN);
-        Seg& g = out[n];
-        g.kq = SEG_I | (a.qual(readOffset) << 8); g.locus = locus; g.roff = readOffset; g.len = len;
-        g.fin = il; g.hash = h; g.rotn = rot | (int32_t)(hasN << 30); g.pad = 0;
-      }
-      n++;
-    } else if (op == 2 && len > 0 && valid && tr && (int64_t)locus + len - 1 <= R.ref_len) {
-      int32_t dl = locus, rl = readOffset;
-      const int d_at = n++;
-      while (dl > 1 && rl > 0 && R.ref[dl - 2] == R.ref[dl + len - 2]) {
-        dl--; rl--;
-        if (rl >= flank && j_sub(L, flank) > rl) {
-          if (out) {
-            Seg& g = out[n];
-            g.kq = SEG_A | (a.qual(rl) << 8); g.locus = dl; g.roff = rl; g.len = len;
-            g.fin = a.bi(rl); g.hash = 0; g.rotn = 0; g.pad = locus;   // pad: the deletion's own locus (its gate)
-          }
-          n++;
-        }
-      }
-      if (out) {
-        uint32_t hasN;
-        const uint32_t h = del_hash(R.ref, (int64_t)dl - 1, len, &hasN);
-        Seg& g = out[d_at];
-        g.kq = SEG_D | (a.qual(readOffset) << 8); g.locus = locus; g.roff = readOffset; g.len = len;
-        g.fin = dl; g.hash = h; g.rotn = (int32_t)(hasN << 30); g.pad = 0;
-      }
-    }
-    if (consumes_read(op)) readOffset += len;
-    if (consumes_ref(op)) refOffset += len;
+    n += op_segs(R, a, info, cf, w, locus, readOffset, L, out ? out + n : nullptr);
+    if (consumes_read((int)(w & 15))) readOffset += (int32_t)(w >> 4);
+    if (consumes_ref((int)(w & 15))) locus += (int32_t)(w >> 4);
   }
   return n;
 }
@@ -654,35 +684,47 @@ PL_HD bool wants_segs(uint32_t info) {
 // Table entries of read r: its segments, a header before a long read's.  0
 // for none and for a long read that is walked (odd clips, or deletions that
 // slide so far that the table would outgrow the CIGAR).
+PL_HD uint32_t long_seg_slots(const LongOps& lo, int32_t L, int64_t n, int64_t n_ops) {
+  return long_segs_ok(lo, L) && n > 0 && n <= 4 * n_ops + 64 ? (uint32_t)n + 1u : 0u;
+}
 PL_HD uint32_t seg_slots(const RSDev& R, int64_t r, uint32_t info, const KConf& cf) {
   if (!wants_segs(info)) return 0u;
-  const bool lr = (info & RI_LR_MASK) != 0;
-  if (lr && !long_segs_ok(R, r)) return 0u;
-  const int64_t n = build_segs(R, r, info, cf, nullptr);
-  if (!lr) return (uint32_t)n;
-  return n > 0 && n <= 4 * (R.cigar_off[r + 1] - R.cigar_off[r]) + 64 ? (uint32_t)n + 1u : 0u;
+  const int64_t n = build_segs(R, r, info, cf, nullptr), c0 = R.cigar_off[r], c1 = R.cigar_off[r + 1];
+  if (!(info & RI_LR_MASK)) return (uint32_t)n;
+  LongOps lo;
+  int32_t readOffset = 0;
+  for (int64_t k = c0; k < c1; k++) {
+    lo = add_long_op(lo, R.cigar[k], (int32_t)(k - c0), readOffset);
+    if (consumes_read((int)(R.cigar[k] & 15))) readOffset += (int32_t)(R.cigar[k] >> 4);
+  }
+  return long_seg_slots(lo, (int32_t)(R.seq_off[r + 1] - R.seq_off[r]), n, c1 - c0);
+}
+// how far left of its op's locus a segment touches
+PL_HD int32_t seg_reach(const Seg& g) {
+  const int kd = seg_kind(g);
+  return seg_key(g) - (kd == SEG_I || kd == SEG_D ? g.fin : kd == SEG_A ? g.locus + g.len : g.locus);
+}
+// The header of a long read's c entries, and the info word of a read whose
+// table entries number c (RMeta.op0 is the first).
+PL_HD void put_seg_header(Seg& h, int32_t pos, uint32_t c, int32_t reach) {
+  h.kq = SEG_H; h.locus = pos; h.roff = 0; h.len = (int32_t)c - 1; h.fin = reach; h.hash = 0; h.rotn = 0; h.pad = 0;
+}
+PL_HD uint32_t seg_info(uint32_t info, uint32_t c) {
+  uint32_t n = c < RI_SEG_MAX ? c : (uint32_t)RI_SEG_MAX;
+  if (info & RI_LR_MASK) n = c ? (uint32_t)RI_SEG_LONG : (uint32_t)RI_SEG_MAX;
+  return (info & ~RI_SEG_MASK) | (n << RI_SEG_SHIFT);
 }
 // Fills read r's c entries from segs[o]; returns its info word (RMeta.op0 becomes o).
 PL_HD uint32_t seg_fill(const RSDev& R, int64_t r, uint32_t info, const KConf& cf, Seg* segs, uint32_t o, uint32_t c) {
-  uint32_t n = c < RI_SEG_MAX ? c : (uint32_t)RI_SEG_MAX;
-  if (!(info & RI_LR_MASK)) {
-    if (c) build_segs(R, r, info, cf, segs + o);
-  } else if (c == 0) {
-    n = RI_SEG_MAX;
-  } else {
-    n = RI_SEG_LONG;
+  if (c && (info & RI_LR_MASK)) {
     build_segs(R, r, info, cf, segs + o + 1);
-    int32_t reach = 0;                                     // how far left of its op's locus a segment touches
-    for (uint32_t i = o + 1; i < o + c; i++) {
-      const Seg& g = segs[i];
-      const int kd = seg_kind(g);
-      const int32_t first = kd == SEG_I || kd == SEG_D ? g.fin : kd == SEG_A ? g.locus + g.len : g.locus;
-      reach = seg_key(g) - first > reach ? seg_key(g) - first : reach;
-    }
-    Seg& h = segs[o];
-    h.kq = SEG_H; h.locus = R.pos[r]; h.roff = 0; h.len = (int32_t)c - 1; h.fin = reach; h.hash = 0; h.rotn = 0; h.pad = 0;
+    int32_t reach = 0;
+    for (uint32_t i = o + 1; i < o + c; i++) reach = seg_reach(segs[i]) > reach ? seg_reach(segs[i]) : reach;
+    put_seg_header(segs[o], R.pos[r], c, reach);
+  } else if (c) {
+    build_segs(R, r, info, cf, segs + o);
   }
-  return (info & ~RI_SEG_MASK) | (n << RI_SEG_SHIFT);
+  return seg_info(info, c);
 }
 
 // One segment of a multi-op read at window time, applied on its own: every

@@ -426,6 +426,18 @@ int64_t nib_bytes(const pl_read_soa* s) {
   return (mx + 1) / 2 + 1;
 }
 
+// blocks of 256 threads for n reads, a thread or (lng) a wave each
+unsigned prep_blocks(int64_t n, bool lng) {
+  const int64_t per = lng ? 4 : 256;
+  return (unsigned)std::min<int64_t>(std::max<int64_t>(1, (n + per - 1) / per), 8192);
+}
+// k_prep over set d: its short reads by threads, its long ones by waves
+void launch_prep(const RSDev& d, const KConf& cf, uint32_t* keep, uint32_t* segc, int64_t* outl, int64_t ocap,
+                 hipStream_t st) {
+  if (!d.all_long) k_prep<<<dim3(prep_blocks(d.n, false)), dim3(256), 0, st>>>(d, cf, keep, segc, d.scal, outl, ocap);
+  if (d.lrt) k_prep_long<<<dim3(prep_blocks(d.n, true)), dim3(256), 0, st>>>(d, cf, keep, segc, d.scal, outl, ocap);
+}
+
 // lrt: each read's longReadType (null: none); kinds: RS_FRAGS | RS_NANO
 #define RS_FRAGS 1
 #define RS_NANO 2
@@ -500,8 +512,7 @@ pl_status readset_upload(pl_ctx* c, int32_t contig_id, const pl_read_soa* s, int
   if (pl_status e = B.get(&segoff, 4 * (size_t)(n + 1))) return e;
   for (int attempt = 0; attempt < 2; attempt++) {
     HIPCHK(hipMemsetAsync(d.scal, 0, 64, st));
-    const int64_t blocks = std::min<int64_t>(std::max<int64_t>(1, (n + 255) / 256), 8192);
-    k_prep<<<dim3((unsigned)blocks), dim3(256), 0, st>>>(d, c->cf, keepflag, segcount, d.scal, outl, ocap);
+    launch_prep(d, c->cf, keepflag, segcount, outl, ocap, st);
     HIPCHK(hipGetLastError());
     HIPCHK(hipMemcpyAsync(rs->scal, d.scal, 32, hipMemcpyDeviceToHost, st));
     HIPCHK(hipStreamSynchronize(st));
@@ -519,11 +530,9 @@ pl_status readset_upload(pl_ctx* c, int32_t contig_id, const pl_read_soa* s, int
   HIPCHK(hipStreamSynchronize(st));
   HIPCHK(hipMalloc(&p, sizeof(Seg) * ((size_t)nseg + 1))); rs->mem.push_back(p);
   d.segs = (const Seg*)p;
-  {
-    const int64_t blocks = std::min<int64_t>(std::max<int64_t>(1, (n + 255) / 256), 8192);
-    k_segfill<<<dim3((unsigned)blocks), dim3(256), 0, st>>>(d, c->cf, segoff, (Seg*)p);
-    HIPCHK(hipGetLastError());
-  }
+  if (!d.all_long) k_segfill<<<dim3(prep_blocks(n, false)), dim3(256), 0, st>>>(d, c->cf, segoff, (Seg*)p);
+  if (d.lrt) k_segfill_long<<<dim3(prep_blocks(n, true)), dim3(256), 0, st>>>(d, c->cf, segoff, (Seg*)p);
+  HIPCHK(hipGetLastError());
   rs->nseg = nseg;
   const int64_t no = rs->scal[3];
   if (no > 0) {
@@ -626,6 +635,7 @@ pl_status prep_sets(pl_ctx* c, std::vector<std::unique_ptr<ReadSet>>& rs, const 
   std::vector<RSDev> views((size_t)std::max(n_sets, 1));
   std::vector<int64_t> blk((size_t)n_sets + 1, 0), ocaps((size_t)std::max(n_sets, 1));
   std::vector<int64_t*> outls((size_t)std::max(n_sets, 1));
+  bool any_short = false, any_long = false;                // (a set's reads are all long or none)
   for (int32_t i = 0; i < n_sets; i++) {
     Tab& t = T[(size_t)i];
     ReadSet& R = *rs[(size_t)i];
@@ -639,7 +649,9 @@ pl_status prep_sets(pl_ctx* c, std::vector<std::unique_ptr<ReadSet>>& rs, const 
     d.ftail = (FragTail*)(D + t.ftail);
     R.kp = KP + OBv[(size_t)i];
     views[(size_t)i] = d;
-    blk[(size_t)i + 1] = blk[(size_t)i] + std::min<int64_t>(std::max<int64_t>(1, (R.n + 255) / 256), 8192);
+    blk[(size_t)i + 1] = blk[(size_t)i] + prep_blocks(R.n, d.lrt != nullptr);
+    any_short = any_short || !d.lrt;
+    any_long = any_long || d.lrt;
     ocaps[(size_t)i] = t.ocap;
     outls[(size_t)i] = (int64_t*)(D + t.outl);
   }
@@ -649,9 +661,15 @@ pl_status prep_sets(pl_ctx* c, std::vector<std::unique_ptr<ReadSet>>& rs, const 
     HIPCHK(hipMemcpyAsync(X + blk_at, blk.data(), 8 * blk.size(), hipMemcpyHostToDevice, st));
     HIPCHK(hipMemcpyAsync(X + oc_at, ocaps.data(), 8 * ocaps.size(), hipMemcpyHostToDevice, st));
     HIPCHK(hipMemcpyAsync(X + ol_at, outls.data(), sizeof(int64_t*) * outls.size(), hipMemcpyHostToDevice, st));
-    k_prep_sets<<<dim3((unsigned)blk[(size_t)n_sets]), dim3(256), 0, st>>>(
-        (const RSDev*)(X + v_at), (const int64_t*)(X + blk_at), n_sets, c->cf, KEEP, SEGC, (const int64_t*)(X + b_at),
-        (int64_t* const*)(X + ol_at), (const int64_t*)(X + oc_at));
+    const dim3 grid((unsigned)blk[(size_t)n_sets]);
+    if (any_short)
+      k_prep_sets<<<grid, dim3(256), 0, st>>>((const RSDev*)(X + v_at), (const int64_t*)(X + blk_at), n_sets, c->cf, KEEP,
+                                              SEGC, (const int64_t*)(X + b_at), (int64_t* const*)(X + ol_at),
+                                              (const int64_t*)(X + oc_at));
+    if (any_long)
+      k_prep_long_sets<<<grid, dim3(256), 0, st>>>((const RSDev*)(X + v_at), (const int64_t*)(X + blk_at), n_sets, c->cf,
+                                                   KEEP, SEGC, (const int64_t*)(X + b_at), (int64_t* const*)(X + ol_at),
+                                                   (const int64_t*)(X + oc_at));
     HIPCHK(hipGetLastError());
   }
   std::vector<int32_t> scal(16 * (size_t)std::max(n_sets, 1));
@@ -669,9 +687,7 @@ pl_status prep_sets(pl_ctx* c, std::vector<std::unique_ptr<ReadSet>>& rs, const 
       R.mem.push_back(p);
       outl[(size_t)i] = (int64_t*)p;
       HIPCHK(hipMemsetAsync(R.d.scal, 0, 64, st));
-      const int64_t blocks = std::min<int64_t>(std::max<int64_t>(1, (R.n + 255) / 256), 8192);
-      k_prep<<<dim3((unsigned)blocks), dim3(256), 0, st>>>(R.d, c->cf, KEEP + Bv[(size_t)i], SEGC + Bv[(size_t)i],
-                                                           R.d.scal, (int64_t*)p, cnt);
+      launch_prep(R.d, c->cf, KEEP + Bv[(size_t)i], SEGC + Bv[(size_t)i], (int64_t*)p, cnt, st);
       HIPCHK(hipGetLastError());
       HIPCHK(hipMemcpyAsync(&scal[16 * (size_t)i], R.d.scal, 64, hipMemcpyDeviceToHost, st));
     }
@@ -707,9 +723,13 @@ pl_status prep_sets(pl_ctx* c, std::vector<std::unique_ptr<ReadSet>>& rs, const 
   }
   if (n_sets > 0) {                                        // k_segfill over all sets in one launch
     HIPCHK(hipMemcpyAsync(X + sg_at, segp.data(), sizeof(Seg*) * segp.size(), hipMemcpyHostToDevice, st));
-    k_segfill_sets<<<dim3((unsigned)blk[(size_t)n_sets]), dim3(256), 0, st>>>(
-        (const RSDev*)(X + v_at), (const int64_t*)(X + blk_at), n_sets, c->cf, SEGO, (const int64_t*)(X + ob_at),
-        (Seg* const*)(X + sg_at));
+    const dim3 grid((unsigned)blk[(size_t)n_sets]);
+    if (any_short)
+      k_segfill_sets<<<grid, dim3(256), 0, st>>>((const RSDev*)(X + v_at), (const int64_t*)(X + blk_at), n_sets, c->cf, SEGO,
+                                                 (const int64_t*)(X + ob_at), (Seg* const*)(X + sg_at));
+    if (any_long)
+      k_segfill_long_sets<<<grid, dim3(256), 0, st>>>((const RSDev*)(X + v_at), (const int64_t*)(X + blk_at), n_sets, c->cf,
+                                                      SEGO, (const int64_t*)(X + ob_at), (Seg* const*)(X + sg_at));
     HIPCHK(hipGetLastError());
   }
   // the outlier lists in order: every list to one pinned buffer, sorted

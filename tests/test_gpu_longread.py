@@ -136,3 +136,57 @@ def test_long_reads_by_segments(read_len, lr, window, block):
                 off += n
     finally:
         ctx.close()
+
+
+def read_of_ops(ref, pos, ops, rng):
+    """A read at 0-based pos with these (op, length) pairs: the reference's
+    bases where it matches, random ones where it inserts or is clipped."""
+    seq, at = "", pos
+    for op, n in ops:
+        if op in "IS":
+            seq += "".join("ACGT"[x] for x in rng.integers(0, 4, n))
+        else:
+            seq += ref[at:at + n] if op == "M" else ""
+            at += n
+    return dict(pos=pos + 1, cigar="".join(f"{n}{op}" for op, n in ops), seq=seq, mapq=int(rng.integers(5, 61)),
+                qual=[int(x) for x in rng.integers(3, 41, len(seq))])
+
+
+@pytest.mark.parametrize("n_ops", [1, 2, 63, 64, 65, 127, 128, 129, 300])
+@pytest.mark.parametrize("ends", ["plain", "clipped", "inner_clip", "lead_del", "lead_ins"])
+def test_long_reads_of_any_op_count(n_ops, ends):
+    """Reads whose ops just fill the rounds of 64 a wave takes of them, with
+    clips at their ends (or, walked, between ops) and indels first."""
+    from oracle import oracle as O
+    from pilon_amd.engine import Context
+    from pilon_amd.reads import pack_reads
+    print(f"case: long reads of {n_ops} ops, {ends}", flush=True)
+    rng = np.random.default_rng(n_ops)
+    ref = "".join("ACGT"[x] for x in rng.integers(0, 4, 6000))
+    ref = ref[:900] + "A" * 40 + "CAG" * 30 + ref[1030:2000] + "CCAGG" * 30 + ref[2150:]
+    reads = []
+    for k in range(24):
+        ops = [("M", int(rng.integers(3, 14))) if i % 2 == 0 else ("ID"[int(rng.integers(0, 2))], int(rng.integers(1, 4)))
+               for i in range(n_ops)]
+        if ends == "clipped":
+            ops = [("S", 7)] + ops + [("S", 9)]
+        elif ends == "inner_clip" and k % 2:
+            ops.insert(len(ops) // 2, ("S", 5))
+        elif ends == "lead_del":
+            ops = [("D", 2)] + ops
+        elif ends == "lead_ins":
+            ops = [("I", 3)] + ops
+        reads.append(read_of_ops(ref, int(rng.integers(600, 1400)), ops, rng))
+    b = pack_reads(reads)
+    cfg = default_config(longread=1, flank=0)
+    want = O.run_region(cfg, ref.encode(), 1, len(ref), [b], name="ctg", set_types=[BAM_TYPES["nanopore"]])
+    assert want["status"] == 0
+    ctx = Context(cfg, device=0)
+    try:
+        ctx.ref_upload(0, "ctg", ref)
+        for rid in (ctx.readset_upload(0, b, bam_type="nanopore"), ctx.readset_upload_many([(0, b, "nanopore")])[0]):
+            pile, calls, stats = ctx.batch_run([(0, 1, len(ref), rid)], window=256, block=256, persistent=1)
+            assert_same_region(pile, calls, want, f"{n_ops} ops, {ends}")
+            assert_same_stats(stats[0], want["stats"], f"{n_ops} ops, {ends}")
+    finally:
+        ctx.close()
