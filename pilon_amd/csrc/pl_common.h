@@ -111,11 +111,9 @@ struct JobDev {              // one region of a batch
 struct WinDev {
   int32_t job;
   int32_t p0, p1;            // region-relative [p0, p1)
-  int32_t order;             // position in the work queue
+  int32_t m0;                // adjMq + 1 of most of a sample of the reads in [plo, hi)
   int64_t lo, hi;            // reads whose pos is in [locus(p0)-back, locus(p1)+lead)
   int64_t plo;               // reads in [lo, plo) reach the window only through their fragments
-  int32_t m0;                // adjMq + 1 of most of a sample of the reads in [plo, hi)
-  int32_t pad_;
 };
 
 // What the window kernel needs about one window and its region, in the
@@ -153,9 +151,11 @@ struct IndelRec {
   uint16_t mq1;              // indelMq + 1
   uint32_t hash;             // FNV-1a of the (rotated) string
   int32_t rot;               // insertion: right rotations applied
-  uint32_t flags;            // bit0: source is nib stream; bit1: contains 'N'
+  uint32_t flags;            // bit0: source is nib stream; bit1: contains 'N'; PL_REC_WINS
   int64_t src;               // insertion: first base (2-bit or nibble index); deletion: contig offset
 };
+
+#define PL_REC_WINS 4u        // the winning record of a column the deletion pass changed
 
 #define PL_CAND_INS 32
 // a change candidate (a column whose disposition before Pass 1 is a change)
@@ -198,13 +198,15 @@ struct EngineArgs {
   // records beyond a window's LDS buffer, with their window and their place among its records
   IndelRec* spill; uint2* spill_at; uint32_t* spill_n; uint32_t spill_cap;
   uint64_t* cmask;           // [n_wins][W / 64] candidate columns of each window, a bit per position
-  int32_t* prec;             // [G] winning record of the columns the indel pass called (-1: none)
+  // the deferred columns: a bit per position as in cmask, the place in defer
+  // of each word's first, and the winning record of each (-1: none)
+  uint64_t* dmask; uint32_t* dbase; int32_t* drec;
   Cand* cand; uint32_t* cand_n; uint32_t cand_cap;   // candidates in position order
   uint32_t* defer; uint32_t* defer_n; uint32_t defer_cap;
   uint32_t* mutated; uint32_t* mutated_n; uint32_t mutated_cap;
   int32_t* overflow;                // capacity overflow flag
   struct WideCol* wide; uint32_t* wide_n; uint32_t wide_cap;   // exact sums of wide columns
   int32_t* win_wide;                // [2 * n_wins]: each window's first wide entry and count
-  WinHead* wheads; uint32_t* wide_wins; int32_t* wqueue;   // windows beyond the narrow counters, and their queue
+  int32_t* wide_heads; uint32_t* wide_wins; int32_t* wqueue;   // heads of the windows beyond the narrow counters, and their queue
   uint32_t* deep;                   // set when some region's minDepth is above the confirmed histogram
 };

@@ -5,8 +5,9 @@
 //   pile   int32 [PL_NFIELDS][G]   field-major PileUp counters
 //   calls  pl_call [G]             BaseCall + disposition, 8 B
 //   rec    IndelRec [cap]          insertion/deletion evidence, 32 B each
-//   prec   int32 [G]               winning evidence record (called columns)
 //   cmask  bit [G]                 candidate columns, per window
+//   dmask  bit [G]                 columns the indel pass calls; their winning
+//                                  records (drec) in defer's order
 //   cand   Cand [cap]              change candidates (sparse), in order
 // Resident per contig: the raw reference bytes; per read set: the packed
 // reads plus 24 B/read of derived facts (span, alignment end, info word) and
@@ -192,8 +193,8 @@ enum { PL_N_REC = 0, PL_N_CAND, PL_N_DEFER, PL_N_MUTATED, PL_N_OVERFLOW, PL_N_QU
 struct Lane {
   hipStream_t stream = nullptr;
   hipEvent_t ev[4] = {};
-  DBuf rsarr, kparr, jobs, wins, cost, bins, pile, calls, prec, cmask, csums, res, dhist, rec, winrec, spill,
-      spillat, defer, mutated, strpool, stridx, stroff, wide, winwide, heads, wheads;
+  DBuf rsarr, kparr, jobs, wins, cost, bins, pile, calls, cmask, dmask, dbase, drec, csums, res, dhist, rec, winrec, spill,
+      spillat, defer, mutated, strpool, stridx, stroff, wide, winwide, heads, wideheads;
   DBuf hist, tiles;                // sort and scan scratch (uploads, K-mers)
   // res holds what the host needs of a batch, one copy's worth: the counters,
   // the regions' JobStat, the candidates
@@ -247,9 +248,9 @@ struct Lane {
   bool has_jdepth = false;
 
   template <class F> void for_each_buffer(F&& f) {
-    DBuf* b[] = {&rsarr, &kparr, &jobs, &wins, &cost, &bins, &pile, &calls, &prec, &cmask, &csums, &res, &dhist, &rec,
+    DBuf* b[] = {&rsarr, &kparr, &jobs, &wins, &cost, &bins, &pile, &calls, &cmask, &dmask, &dbase, &drec, &csums, &res, &dhist, &rec,
                  &winrec, &spill, &spillat, &defer, &mutated, &strpool, &stridx, &stroff,
-                 &wide, &winwide, &heads, &wheads, &hist, &tiles, &jdepth};
+                 &wide, &winwide, &heads, &wideheads, &hist, &tiles, &jdepth};
     for (DBuf* x : b) f(*x);
   }
   size_t device_bytes() {
@@ -1126,12 +1127,13 @@ pl_status run_jobs(pl_ctx* c, Lane* L, const std::vector<JobReq>& reqs, int32_t 
   HIPCHK(L->winwide.ensure(8 * (size_t)n_wins));
   HIPCHK(L->winrec.ensure(8 * (size_t)n_wins));
   HIPCHK(L->heads.ensure(sizeof(WinHead) * (size_t)n_wins));
-  HIPCHK(L->wheads.ensure(sizeof(WinHead) * (size_t)n_wins));
+  HIPCHK(L->wideheads.ensure(4 * (size_t)n_wins));
   HIPCHK(L->cost.ensure((size_t)n_wins));
   HIPCHK(L->bins.ensure(4 * (PL_BIN_COPIES + 1) * PL_COST_BINS));
   HIPCHK(L->cmask.ensure(8 * (size_t)n_wins * (size_t)(W / 64)));
   HIPCHK(L->csums.ensure(4 * (((size_t)n_wins * (size_t)(W / 64) + PL_CAND_WORDS - 1) / PL_CAND_WORDS)));
-  HIPCHK(L->prec.ensure(4 * (size_t)G));
+  HIPCHK(L->dmask.ensure(8 * (size_t)n_wins * (size_t)(W / 64)));
+  HIPCHK(L->dbase.ensure(4 * (size_t)n_wins * (size_t)(W / 64)));
   HIPCHK(L->dhist.ensure(4 * (size_t)PL_HIST * (size_t)n_jobs));
   HIPCHK(L->pile.ensure(4 * (size_t)PL_NFIELDS * G));
   HIPCHK(L->calls.ensure(sizeof(pl_call) * (size_t)G));
@@ -1170,6 +1172,7 @@ pl_status run_jobs(pl_ctx* c, Lane* L, const std::vector<JobReq>& reqs, int32_t 
     HIPCHK(L->spillat.ensure(8 * (size_t)L->spill_cap));
     HIPCHK(L->res.ensure(Lane::cand_at((size_t)n_jobs) + sizeof(Cand) * (size_t)L->cand_cap));
     HIPCHK(L->defer.ensure(4 * (size_t)L->defer_cap));
+    HIPCHK(L->drec.ensure(4 * (size_t)L->defer_cap));
     HIPCHK(L->mutated.ensure(4 * (size_t)L->mut_cap));
     HIPCHK(L->wide.ensure(sizeof(WideCol) * (size_t)L->wide_cap));
     uint32_t* cnt = L->counters();
@@ -1184,7 +1187,7 @@ pl_status run_jobs(pl_ctx* c, Lane* L, const std::vector<JobReq>& reqs, int32_t 
     A.W = W;
     A.queue = (int32_t*)(cnt + PL_N_QUEUE);
     A.deep = cnt + PL_N_DEEP;
-    A.wheads = L->wheads.as<WinHead>();
+    A.wide_heads = L->wideheads.as<int32_t>();
     A.wide_wins = cnt + PL_N_WIDE_WINS;
     A.wqueue = (int32_t*)(cnt + PL_N_WIDE_QUEUE);
     A.cost = L->cost.as<uint8_t>();
@@ -1200,7 +1203,9 @@ pl_status run_jobs(pl_ctx* c, Lane* L, const std::vector<JobReq>& reqs, int32_t 
     A.spill = L->spill.as<IndelRec>(); A.spill_at = L->spillat.as<uint2>();
     A.spill_n = cnt + PL_N_SPILL; A.spill_cap = L->spill_cap;
     A.cmask = L->cmask.as<uint64_t>();
-    A.prec = L->prec.as<int32_t>();
+    A.dmask = L->dmask.as<uint64_t>();
+    A.dbase = L->dbase.as<uint32_t>();
+    A.drec = L->drec.as<int32_t>();
     A.cand = L->cands((size_t)n_jobs); A.cand_n = cnt + PL_N_CAND; A.cand_cap = L->cand_cap;
     A.defer = L->defer.as<uint32_t>(); A.defer_n = cnt + PL_N_DEFER; A.defer_cap = L->defer_cap;
     A.mutated = L->mutated.as<uint32_t>(); A.mutated_n = cnt + PL_N_MUTATED; A.mutated_cap = L->mut_cap;

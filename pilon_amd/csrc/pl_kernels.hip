@@ -544,6 +544,8 @@ __device__ int plan_windows(const EngineArgs& A, int32_t blk, WinDev* wins, bool
     A.cost[w] = (uint8_t)bin;
     if (heads) put_head((WinHead*)A.heads, w, w, win, J, win.m0);
   }
+  if (in)
+    for (int q = threadIdx.x & 15; q < A.W >> 6; q += 16) A.dmask[(int64_t)w * (A.W >> 6) + q] = 0;   // for the indel pass
   return in ? bin : -1;
 }
 
@@ -905,9 +907,9 @@ static_assert(PL_CHUNK % 2 == 1 && PL_CHUNK <= 31, "an odd chunk of at most 31 b
 // LONG: the batch's read sets hold long reads (their segments and the
 // nanopore base rule cost the other batches' kernel seven spilled registers).
 // NARROW: the window's counters are 32-bit words (NarrowLds); a window they
-// do not hold is added to A.wheads, and a wide launch of mode 2 piles those.
+// do not hold is added to A.wide_heads, and a wide launch of mode 2 piles those.
 // mode: 0 a window per workgroup, 1 windows from the queue, 2 the windows of
-// A.wheads from their queue.
+// A.wide_heads from their queue.
 template <int BLOCK, bool LONG, bool NARROW>
 __global__ void __launch_bounds__(BLOCK, NARROW ? PL_NARROW_WAVES_EU : PL_WIN_WAVES_EU) k_window(EngineArgs A, int mode) {
   static_assert(!(LONG && NARROW), "long reads have an event every few bases");
@@ -918,7 +920,7 @@ __global__ void __launch_bounds__(BLOCK, NARROW ? PL_NARROW_WAVES_EU : PL_WIN_WA
   __shared__ uint32_t s_extra, s_ncx;
   __shared__ uint16_t s_cx[NARROW ? PL_WIN_WALKS : 1];   // reads to walk, from win.plo
   const bool persistent = mode != 0;
-  const WinHead* heads = mode == 2 ? A.wheads : A.heads;
+  auto head_of = [&](int32_t q) { return A.heads[mode == 2 ? A.wide_heads[q] : q]; };
   int32_t* queue = mode == 2 ? A.wqueue : A.queue;
   const int32_t n_heads = mode == 2 ? (int32_t)*A.wide_wins : A.n_wins;
   __shared__ RunL s_run[NW * (2 * 64 + 1)];
@@ -942,7 +944,7 @@ __global__ void __launch_bounds__(BLOCK, NARROW ? PL_NARROW_WAVES_EU : PL_WIN_WA
   if (tid == 0) {
     const int32_t q = persistent ? atomicAdd(queue, 1) : (int32_t)blockIdx.x;
     s_slot[0] = q;
-    if (q < n_heads) s_head[0] = heads[q];
+    if (q < n_heads) s_head[0] = head_of(q);
   }
   __syncthreads();
   for (int iter = 0;; iter++) {
@@ -968,9 +970,9 @@ __global__ void __launch_bounds__(BLOCK, NARROW ? PL_NARROW_WAVES_EU : PL_WIN_WA
     const int32_t L0 = J.start + win.p0, L1 = J.start + win.p1, nW = win.p1 - win.p0;
     auto next_window = [&]() {                 // by thread 0
       s_slot[cur ^ 1] = persistent ? next_slot : n_heads;
-      if (persistent && next_slot < n_heads) s_head[cur ^ 1] = heads[next_slot];
+      if (persistent && next_slot < n_heads) s_head[cur ^ 1] = head_of(next_slot);
     };
-    auto to_wide = [&]() { A.wheads[atomicAdd(A.wide_wins, 1u)] = s_head[cur]; };
+    auto to_wide = [&]() { A.wide_heads[atomicAdd(A.wide_wins, 1u)] = s_slot[cur]; };
     const int64_t reads_in = win.hi - win.plo + R.n_outlier;
     if (NARROW && reads_in > PL_NARROW_MAX) {
       if (tid == 0) { to_wide(); next_window(); }
@@ -1509,7 +1511,8 @@ __global__ void __launch_bounds__(BLOCK, NARROW ? PL_NARROW_WAVES_EU : PL_WIN_WA
         }
       }
       // the candidates as a bit per position, in order without a sort; the
-      // deferred columns as a list (their order is of no consequence)
+      // deferred columns as a list, those of 64 positions together in order
+      // (indel_columns finds its way back by that)
       const uint64_t cm = __ballot(is_cand);
       if (lane == 0) A.cmask[(int64_t)wi * (W >> 6) + (q0 >> 6)] = cm;
       const uint32_t kd = wave_append(A.defer_n, defer);
@@ -1813,11 +1816,47 @@ __device__ int32_t wave_job_of(const JobDev* jobs, int32_t n_jobs, int64_t g, in
 
 }  // namespace
 
+namespace {
+
+// Place in the defer list of column g, or -1 when the window kernel did not
+// defer it: a bit per position and the place of each 64 positions' first take
+// 0.2 bytes a position where an index of its own would take four.
+__device__ __forceinline__ int64_t defer_place(const EngineArgs& A, const JobDev& J, int64_t g) {
+  const int32_t w = J.win0 + (int32_t)((g - J.out) / A.W), p = (int32_t)((g - J.out) % A.W);
+  const int64_t word = (int64_t)w * (A.W >> 6) + (p >> 6);
+  const uint64_t m = A.dmask[word], bit = 1ull << (p & 63);
+  if (!(m & bit)) return -1;
+  const uint32_t k = A.dbase[word] + (uint32_t)__popcll(m & (bit - 1ull));
+  return k < A.defer_cap ? (int64_t)k : -1;
+}
+
+// The winning record of a column the deletion pass changed: in the deferred
+// column's place, or else a mark on the record.
+__device__ __forceinline__ void put_record(const EngineArgs& A, const JobDev& J, int64_t g, int64_t rec) {
+  const int64_t k = defer_place(A, J, g);
+  if (k >= 0) A.drec[k] = (int32_t)rec;
+  else if (rec >= 0) A.rec[rec].flags |= PL_REC_WINS;
+}
+
+// The winning record of column g, called with an insertion or a deletion (key
+// kind 0 or 1); -1: none.
+__device__ __forceinline__ int64_t col_record(const EngineArgs& A, const JobDev& J, int64_t g, uint32_t kind) {
+  const int64_t k = defer_place(A, J, g);
+  if (k >= 0) return A.drec[k];
+  const int32_t w = J.win0 + (int32_t)((g - J.out) / A.W);
+  const ColRecs C = col_recs(A.rec, A.rec_cap, A.win_rec, w, *A.spill_n, A.spill_cap, ((uint32_t)g << 1) | kind);
+  for (int64_t i = C.a; i < C.b; i++)
+    if (C.recs[i].key == C.key && (C.recs[i].flags & PL_REC_WINS)) return i;
+  return -1;
+}
+
+}  // namespace
+
 // One wave per listed column: the full BaseCall with the column's evidence
 // records (hetIndelCall), lane 0 writing the results.
 // mode 0: deferred columns (writes call, marks candidates, counts confirmed)
 // mode 1: columns changed by the deletion pass (keeps disposition bits)
-// Both leave the column's winning record in A.prec.
+// Both leave the column's winning record where col_record finds it.
 __device__ void indel_columns(const EngineArgs& A, const uint32_t* list, uint32_t n, int mode, uint32_t first,
                               uint32_t nw) {
   const int lane = threadIdx.x & 63;
@@ -1849,17 +1888,19 @@ __device__ void indel_columns(const EngineArgs& A, const uint32_t* list, uint32_
     if (lane != 0) continue;
     pl_call cl = make_call(bf, indel, homo, refb, A.cf);
     cl.flags |= wflag;
-    A.prec[g] = (int32_t)wrec;
     if (mode == 0) {
+      A.drec[i] = (int32_t)wrec;
+      const int32_t p = (int32_t)((g - J.out) % A.W);
+      const int64_t word = (int64_t)w * (A.W >> 6) + (p >> 6);
+      atomicOr((unsigned long long*)&A.dmask[word], 1ull << (p & 63));
+      if (i == 0 || list[i - 1] >= g || list[i - 1] < g - (uint32_t)(p & 63)) A.dbase[word] = i;   // its word's first
       A.calls[g] = cl;
       const int d = call_disp(cl);
       const int64_t dep = c.depth();
       if (d == PL_D_CONFIRMED) atomicAdd(&A.hist[(int64_t)j * PL_HIST + (dep > 255 ? 255 : (dep < 0 ? 0 : dep))], 1u);
-      else if (d != PL_D_NONE) {
-        const int32_t p = (int32_t)((g - J.out) % A.W);
-        atomicOr((unsigned long long*)&A.cmask[(int64_t)w * (A.W >> 6) + (p >> 6)], 1ull << (p & 63));
-      }
+      else if (d != PL_D_NONE) atomicOr((unsigned long long*)&A.cmask[word], 1ull << (p & 63));
     } else {
+      put_record(A, J, g, wrec);
       pl_call& o = A.calls[g];
       o.base = cl.base; o.alt = cl.alt; o.q = cl.q;
       o.flags = (uint16_t)((cl.flags & ~PL_CF_DISP_MASK) | (o.flags & PL_CF_DISP_MASK) | PL_CF_DELETED);
@@ -1928,6 +1969,8 @@ __global__ void __launch_bounds__(256) k_cand_list(EngineArgs A, int64_t n_words
     const WinDev win = A.wins[wi];
     const JobDev& J = A.jobs[win.job];
     if (word == 0 && win.p0 == 0) A.st[win.job].cand_lo = (int32_t)at;
+    const uint64_t dm = m[k] ? A.dmask[x] : 0ull;              // an insertion or deletion was deferred
+    const uint32_t db = dm ? A.dbase[x] : 0u;
     for (uint64_t b = m[k]; b; b &= b - 1) {
       const int64_t g = J.out + win.p0 + 64 * word + (__ffsll((unsigned long long)b) - 1);
       if (at < A.cand_cap) {
@@ -1941,7 +1984,10 @@ __global__ void __launch_bounds__(256) k_cand_list(EngineArgs A, int64_t n_words
         c.kind = call_disp(cl);
         c.len = 0;
         c.rec = -1;
-        if (c.kind == PL_D_INS || c.kind == PL_D_DEL) { c.rec = A.prec[g]; c.len = A.rec[c.rec].len; }
+        if (c.kind == PL_D_INS || c.kind == PL_D_DEL) {
+          c.rec = A.drec[db + (uint32_t)__popcll(dm & ((b & (0ull - b)) - 1ull))];
+          c.len = A.rec[c.rec].len;
+        }
         c.base = cl.base;
         c.alt = cl.alt;
         c.pad = 0;

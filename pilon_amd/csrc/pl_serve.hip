@@ -42,18 +42,17 @@ struct ServeDone {
   std::vector<plh::Change> changes;
 };
 
-// Device bytes one region of G positions can need inside a lane, as admission
-// counts them: pileup and calls (80 B/position), window tables, and its share
-// of the evidence buffers at their growth rates, plus a fixed floor for the
-// smallest buffer sizes.  (A lane holds about 86 B/position for large
-// regions: 4 of them the called columns' record indices.  The weights stay,
-// so a budget admits the requests it always has.)
+// Device bytes one region of G positions can need inside a lane: pileup and
+// calls (80 B/position), window tables, and its share of the evidence buffers
+// at their growth rates, plus a fixed floor for the smallest buffer sizes.
+// At windows of 512 that is 83.4 B/position; the lane's buffers
+// (Lane::for_each_buffer) come to 82.9.  The weights are admission's contract,
+// the same whatever the buffers become below them: a budget admits the
+// requests it always has.
 int64_t estimate_bytes(int64_t G, int32_t W) {
   const int64_t per_pos = 4 * PL_NFIELDS + (int64_t)sizeof(pl_call);        // pileup + calls
   const int64_t wins = (G + W - 1) / W;
-  const int64_t rec = G / 16 * ((int64_t)sizeof(IndelRec) + 16);            // records, their columns' indices
-  const int64_t cand = G / 256 * (3 * (int64_t)sizeof(Cand));               // candidates, defer, mutated
-  return G * per_pos + wins * ((int64_t)sizeof(WinDev) + 20) + rec + cand + ((int64_t)8 << 20);
+  return G * per_pos + wins * 68 + G / 16 * 48 + G / 256 * 72 + ((int64_t)8 << 20);
 }
 
 }  // namespace

@@ -232,7 +232,7 @@ __device__ __forceinline__ uint32_t vcf_locus(char* out, const VcfArgs& V, const
   if (f & PL_CF_WIDE) wide_patch(v.c, V.A.wide, V.A.wide_cap, V.A.win_wide, J, V.A.W, g);
   const bool deleted = (f & PL_CF_DELETED) != 0 || (V.embed && V.embed[g]);
   int64_t rec = -1;
-  if (i > 0 && (f & (PL_CF_INSERTION | PL_CF_DELETION))) rec = V.A.prec[g];
+  if (i > 0 && (f & (PL_CF_INSERTION | PL_CF_DELETION))) rec = col_record(V.A, J, g, f & PL_CF_DELETION ? 1u : 0u);
   vcf_record<WRITE>(o, V, J, R, name, name_len, minDepth, v, f, rec, i, deleted, true);
   if (i > 0 && (f & PL_CF_INDEL) && !deleted)
     vcf_record<WRITE>(o, V, J, R, name, name_len, minDepth, v, f, rec, i,

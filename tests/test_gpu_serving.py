@@ -129,6 +129,48 @@ def test_admission_budget_and_limits(resident):
         srv.close()
 
 
+def test_large_request_fits_its_estimate():
+    """A lane's device memory after a request of 60 Mb stays within the bytes
+    that admission counted (5.0 GB; an allocation's rounding, some 2 MiB for
+    each of 30 buffers, is inside its fixed 8 MiB and what a lane holds less a
+    position)."""
+    import ctypes as C
+    from pilon_amd.engine import Context, Server, lib
+    from pilon_amd.reads import pack_reads
+
+    def free_bytes():
+        free, total = C.c_size_t(), C.c_size_t()
+        assert lib().hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+        return free.value
+
+    print("case: device bytes of a 60 Mb request", flush=True)
+    n = 60_000_000
+    ref = np.frombuffer(b"ACGT", np.uint8)[np.random.default_rng(1).integers(0, 4, n, dtype=np.uint8)].tobytes()
+    reads = [dict(pos=k + 1, cigar="60M", seq=ref[k:k + 60].decode(), qual=[30] * 60) for k in range(0, 6000, 20)]
+    ctx = Context(default_config(), device=0)
+    try:
+        ctx.ref_upload(0, "big", ref)
+        rid = ctx.readset_upload(0, pack_reads(reads))
+        srv = Server(ctx, lanes=1)                 # the kernels' own stacks, before the measurement
+        srv.submit(0, 1, 20_000, rid)
+        _wait_all(srv, 1)
+        srv.close()
+        srv = Server(ctx, lanes=1, mem_budget=8 << 30)
+        try:
+            ctx.synchronize()
+            free = free_bytes()
+            srv.submit(0, 1, n, rid)
+            res = _wait_all(srv, 1)[0]
+            assert res["status"] == 0
+            used = free - free_bytes()
+            print(f"used {used}, estimate {res['est_bytes']}", flush=True)
+            assert 72 * n < used <= res["est_bytes"]
+        finally:
+            srv.close()
+    finally:
+        ctx.close()
+
+
 def test_uploads_refused_while_serving(resident):
     from pilon_amd.engine import PilonError, Server
     d, ctx, rids = resident
