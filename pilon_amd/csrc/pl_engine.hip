@@ -1122,6 +1122,20 @@ pl_status run_jobs(pl_ctx* c, Lane* L, const std::vector<JobReq>& reqs, int32_t 
   L->cand_cap = std::max<uint32_t>(L->cand_cap, (uint32_t)std::min<int64_t>(G / 256 + 16384, 1ll << 30));
   L->defer_cap = std::max<uint32_t>(L->defer_cap, (uint32_t)std::min<int64_t>(G / 256 + 16384, 1ll << 30));
   L->mut_cap = std::max<uint32_t>(L->mut_cap, (uint32_t)std::min<int64_t>(G / 256 + 16384, 1ll << 30));
+  // the segments of the batch's reads bound its records; where that is more
+  // than half of what the windows hold in LDS, as many may spill as there is
+  // room for records (a first pass that found the list short ran again: long
+  // reads given as unpaired, 200 kb at 40x, 26.5 ms for 10.1).  Serving lanes
+  // and the scratch array keep to their sizes.
+  if (L == &c->main || L == &c->aux) {
+    double segs = 0;
+    for (const JobReq& q : reqs) {
+      const ReadSet* rs = c->rsets[q.rs].get();
+      if (rs) segs += (double)rs->nseg * (double)(q.stop - q.start + 1) / (double)rs->d.ref_len;
+    }
+    if (segs > (double)(PL_WIN_RECS / 2) * n_wins)
+      L->spill_cap = std::max<uint32_t>(L->spill_cap, (uint32_t)std::min<double>(segs, (double)L->rec_cap));
+  }
   HIPCHK(L->jobs.ensure(sizeof(JobDev) * n_jobs));
   HIPCHK(L->wins.ensure(sizeof(WinDev) * n_wins));
   HIPCHK(L->winwide.ensure(8 * (size_t)n_wins));
