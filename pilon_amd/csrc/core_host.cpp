@@ -15,6 +15,7 @@
 
 #include "pl_core.h"
 #include "pl_host.h"
+#include "pl_scratch.h"
 
 namespace {
 
@@ -44,6 +45,26 @@ struct HostSink {
   }
   void edge(int64_t r) { if (edge_read < 0 || r < edge_read) edge_read = r; }
 };
+
+// memory of so many bytes for the scratch tests
+struct FewBytes {
+  static size_t cap, live;
+  static std::map<void*, size_t> sizes;
+  static bool alloc(void** p, size_t n) {
+    if (live + n > cap) return false;
+    *p = std::malloc(1);
+    sizes[*p] = n;
+    live += n;
+    return true;
+  }
+  static void free(void* p) {
+    live -= sizes.at(p);
+    sizes.erase(p);
+    std::free(p);
+  }
+};
+size_t FewBytes::cap = 0, FewBytes::live = 0;
+std::map<void*, size_t> FewBytes::sizes;
 
 struct Handle {
   std::vector<std::string> changes, bases;
@@ -406,6 +427,46 @@ int64_t ch_text(void* h, int32_t j, int32_t which, const char** p) {
 }
 
 void ch_free(void* h) { delete (Handle*)h; }
+
+// Two lanes' scratch in a memory of 100 MB: the number of the first thing
+// that goes wrong, 0 if nothing does.
+int32_t ch_scratch() {
+  constexpr size_t MB = (size_t)1 << 20;
+  using Call = ScratchCall<FewBytes>;
+  FewBytes::cap = 100 * MB;
+  void* p;
+  {
+    Scratch<FewBytes> x, y;
+    { Call c(x); if (!c.take(30 * MB, &p) || !c.take(20 * MB, &p)) return 1; }
+    if (FewBytes::live != 50 * MB) return 2;                       // kept
+    { Call c(x); if (!c.take(30 * MB, &p) || !c.take(20 * MB, &p) || FewBytes::live != 50 * MB) return 3; }   // and used again
+    { Call c(y); if (!c.take(60 * MB, &p) || FewBytes::live != 60 * MB) return 4; }   // an idle lane's given back
+    if (!alloc_or_give_back<FewBytes>(&p, 80 * MB) || FewBytes::live != 80 * MB) return 5;   // ... for any allocation
+    FewBytes::free(p);
+    {
+      Call c(x);
+      if (!c.take(50 * MB, &p)) return 6;
+      Call d(y);
+      if (d.take(60 * MB, &p) || FewBytes::live != 50 * MB) return 7;   // not a lane's in use
+      if (!d.take(40 * MB, &p)) return 8;
+    }
+    { Call c(x); if (!c.take(70 * MB, &p)) return 9; }              // its own too small block, and the other lane's
+    {
+      Call c(x);
+      if (!c.take(5 * MB, &p)) return 10;
+      { Call d(x); if (!d.take(20 * MB, &p) || !c.take(10 * MB, &p)) return 11; }   // the outer call's, on its own
+      if (FewBytes::live != 80 * MB) return 12;
+    }
+    if (FewBytes::live != 70 * MB) return 13;
+    FewBytes::cap = (size_t)5 << 30;
+    { Call c(x); if (!c.take((size_t)3 << 30, &p)) return 14; }     // more than a lane keeps
+    if (FewBytes::live != 0) return 15;
+    { Call c(y); for (int k = 0; k < 20; k++) if (!c.take(2 * MB, &p)) return 16; }
+    if (FewBytes::live != 0) return 17;                            // many blocks: one the next time
+    { Call c(y); if (!c.take(2 * MB, &p) || FewBytes::live < 40 * MB) return 18; }
+  }
+  return FewBytes::live ? 19 : 0;
+}
 
 uint32_t ch_cost_bin(int64_t c) { return cost_bin(c); }
 

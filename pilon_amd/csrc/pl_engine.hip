@@ -33,6 +33,7 @@
 
 #include "pl_kernels.hip"
 #include "pl_host.h"
+#include "pl_scratch.h"
 
 namespace {
 
@@ -53,6 +54,19 @@ pl_status fail(pl_status s, const char* fmt, ...) {
     hipError_t e_ = (x);                                                              \
     if (e_ != hipSuccess) return fail(PL_E_DEVICE, "%s: %s", #x, hipGetErrorString(e_)); \
   } while (0)
+
+struct DevMem {
+  static bool alloc(void** p, size_t n) {
+    if (hipMalloc(p, n) == hipSuccess) return true;
+    (void)hipGetLastError();
+    return false;
+  }
+  static void free(void* p) { (void)hipFree(p); }
+};
+// hipMalloc that has idle lanes give their scratch back before it fails
+hipError_t dev_malloc(void** p, size_t n) {
+  return alloc_or_give_back<DevMem>(p, n) ? hipSuccess : hipErrorOutOfMemory;
+}
 
 // Device memory handed out by bumping an offset in a block the library
 // holds for the process (the no-allocation entry point's scratch array).
@@ -80,54 +94,12 @@ struct DBuf {
     if (p) { hipError_t e = hipFree(p); if (e != hipSuccess) return e; }
     p = nullptr;
     cap = 0;
-    hipError_t e = hipMalloc(&p, bytes);
+    hipError_t e = dev_malloc(&p, bytes);
     if (e == hipSuccess) cap = bytes;
     return e;
   }
   void release() { if (p && !arena) (void)hipFree(p); p = nullptr; cap = 0; }
   template <class T> T* as() const { return (T*)p; }
-};
-
-// Device memory of passes that need scratch for one call (VCF, tracks,
-// K-mers): blocks handed out by bumping an offset and taken back when the
-// call ends (ScratchBufs), kept for the lane's next call up to
-// PL_SCRATCH_KEEP.  A call's hipMalloc and hipFree of its dozen buffers took
-// longer than its kernels on small batches.
-#define PL_SCRATCH_KEEP ((size_t)2 << 30)
-struct Scratch {
-  struct Block { uint8_t* p; size_t n; };
-  std::vector<Block> blocks;
-  size_t at = 0, used = 0;         // the block in use and how much of it
-  size_t want = 0;                 // size of the next first block
-  void* top = nullptr;             // the innermost ScratchBufs alive
-  hipError_t get(size_t bytes, void** out) {
-    bytes = (std::max<size_t>(bytes, 1) + 255) & ~(size_t)255;
-    while (at < blocks.size() && bytes > blocks[at].n - used) { at++; used = 0; }
-    if (at == blocks.size()) {
-      Block b{nullptr, std::max(bytes, blocks.empty() && want ? want : (size_t)1 << 20)};
-      const hipError_t e = hipMalloc((void**)&b.p, b.n);
-      if (e != hipSuccess) return e;
-      blocks.push_back(b);
-      used = 0;
-    }
-    *out = blocks[at].p + used;
-    used += bytes;
-    return hipSuccess;
-  }
-  void release() {
-    for (Block& b : blocks) (void)hipFree(b.p);
-    blocks.clear();
-    at = used = 0;
-  }
-  // nothing in use any more: many blocks become one next time, and none is
-  // kept above the bound
-  void settle() {
-    size_t t = 0;
-    for (const Block& b : blocks) t += b.n;
-    at = used = 0;
-    if (t > PL_SCRATCH_KEEP) { want = 0; release(); }
-    else if (blocks.size() > 16) { want = t; release(); }
-  }
 };
 
 struct Contig {
@@ -241,7 +213,7 @@ struct Lane {
   hipEvent_t stage_ev[2] = {nullptr, nullptr};
   // pinned slots for the counters of repeated passes (pl_batch_repeat)
   uint32_t* rep_hc = nullptr;
-  Scratch scratch;
+  Scratch<DevMem> scratch;
   // depth of the batch's "jumps" reads before Pass 1, per position, which
   // fragment coverage leaves out (valid for the last batch when set)
   DBuf jdepth;
@@ -344,34 +316,15 @@ pl_status region_jump_depth(pl_region* r);   // pl_track.hip
 
 namespace {
 
-// Device buffers of one call, given back on every exit: to the lane's
-// scratch (calls nest, so the last one begun is the first to end), or freed
-// when they were allocated while a call begun later was still using it.
-struct ScratchBufs {
-  explicit ScratchBufs(Lane* lane) : s(lane->scratch), at(s.at), used(s.used), outer(s.top) { s.top = this; }
-  ~ScratchBufs() {
-    for (void* x : own) (void)hipFree(x);
-    s.top = outer;
-    s.at = at;
-    s.used = used;
-    if (!outer) s.settle();
-  }
-  ScratchBufs(const ScratchBufs&) = delete;
-  ScratchBufs& operator=(const ScratchBufs&) = delete;
+// A call's buffers in its lane's scratch.
+struct ScratchBufs : ScratchCall<DevMem> {
+  explicit ScratchBufs(Lane* lane) : ScratchCall<DevMem>(lane->scratch) {}
   template <class T> pl_status get(T** out, size_t n) {
     void* q = nullptr;
-    const hipError_t e = s.top == this ? s.get(n, &q) : hipMalloc(&q, n ? n : 1);
-    if (e != hipSuccess) return fail(PL_E_OOM, "device allocation of %zu bytes failed", n);
-    if (s.top != this) own.push_back(q);
+    if (!take(n, &q)) return fail(PL_E_OOM, "device allocation of %zu bytes failed", n);
     *out = (T*)q;
     return PL_OK;
   }
-
- private:
-  Scratch& s;
-  size_t at, used;
-  void* outer;
-  std::vector<void*> own;
 };
 
 pl_status scan_u32(Lane* L, const uint32_t* in, uint32_t* out, int64_t n) {
@@ -483,7 +436,7 @@ pl_status readset_upload(pl_ctx* c, int32_t contig_id, const pl_read_soa* s, int
   const Part meta = part(nullptr, (int64_t)sizeof(RMeta) * (n + 1), 0), ftail = part(nullptr, (int64_t)sizeof(FragTail) * (n + 1), 0),
              kp = part(nullptr, 4 * (n + 1), 0), scal = part(nullptr, 64, 0), outs = part(nullptr, 8 * ocap, 0);
   void* p;
-  HIPCHK(hipMalloc(&p, size));
+  HIPCHK(dev_malloc(&p, size));
   rs->mem.push_back(p);
   uint8_t* D = (uint8_t*)p;
   HIPCHK(hipMemsetAsync(D, 0, copied, st));
@@ -519,7 +472,7 @@ pl_status readset_upload(pl_ctx* c, int32_t contig_id, const pl_read_soa* s, int
     HIPCHK(hipStreamSynchronize(st));
     if (rs->scal[3] <= ocap) break;
     ocap = rs->scal[3];
-    HIPCHK(hipMalloc(&p, 8 * (size_t)ocap)); rs->mem.push_back(p); outl = (int64_t*)p;
+    HIPCHK(dev_malloc(&p, 8 * (size_t)ocap)); rs->mem.push_back(p); outl = (int64_t*)p;
   }
   pl_status ss = scan_u32(L, keepflag, rs->kp, n);
   if (ss) return ss;
@@ -529,7 +482,7 @@ pl_status readset_upload(pl_ctx* c, int32_t contig_id, const pl_read_soa* s, int
   uint32_t nseg = 0;
   HIPCHK(hipMemcpyAsync(&nseg, segoff + n, 4, hipMemcpyDeviceToHost, st));
   HIPCHK(hipStreamSynchronize(st));
-  HIPCHK(hipMalloc(&p, sizeof(Seg) * ((size_t)nseg + 1))); rs->mem.push_back(p);
+  HIPCHK(dev_malloc(&p, sizeof(Seg) * ((size_t)nseg + 1))); rs->mem.push_back(p);
   d.segs = (const Seg*)p;
   if (!d.all_long) k_segfill<<<dim3(prep_blocks(n, false)), dim3(256), 0, st>>>(d, c->cf, segoff, (Seg*)p);
   if (d.lrt) k_segfill_long<<<dim3(prep_blocks(n, true)), dim3(256), 0, st>>>(d, c->cf, segoff, (Seg*)p);
@@ -619,9 +572,9 @@ pl_status prep_sets(pl_ctx* c, std::vector<std::unique_ptr<ReadSet>>& rs, const 
                sg_at = take(sizeof(Seg*) * (size_t)std::max(n_sets, 1));
   auto dfree = [](void* p) { (void)hipFree(p); };
   void* p = nullptr;
-  HIPCHK(hipMalloc(&p, dev));
+  HIPCHK(dev_malloc(&p, dev));
   std::shared_ptr<void> dev_arena(p, dfree);
-  HIPCHK(hipMalloc(&p, std::max<size_t>(tmp, 256)));
+  HIPCHK(dev_malloc(&p, std::max<size_t>(tmp, 256)));
   std::unique_ptr<void, decltype(dfree)> tmp_arena(p, dfree);
   uint8_t* D = (uint8_t*)dev_arena.get();
   uint8_t* X = (uint8_t*)tmp_arena.get();
@@ -684,7 +637,7 @@ pl_status prep_sets(pl_ctx* c, std::vector<std::unique_ptr<ReadSet>>& rs, const 
     outl[(size_t)i] = (int64_t*)(D + t.outl);
     const int32_t cnt = scal[16 * (size_t)i + 3];
     if (cnt > t.ocap) {
-      HIPCHK(hipMalloc(&p, 8 * (size_t)cnt));
+      HIPCHK(dev_malloc(&p, 8 * (size_t)cnt));
       R.mem.push_back(p);
       outl[(size_t)i] = (int64_t*)p;
       HIPCHK(hipMemsetAsync(R.d.scal, 0, 64, st));
@@ -711,7 +664,7 @@ pl_status prep_sets(pl_ctx* c, std::vector<std::unique_ptr<ReadSet>>& rs, const 
   size_t segsz = 0;
   std::vector<size_t> segat((size_t)std::max(n_sets, 1));
   for (int32_t i = 0; i < n_sets; i++) { segat[(size_t)i] = segsz; segsz = align(segsz + sizeof(Seg) * ((size_t)nseg[(size_t)i] + 1)); }
-  HIPCHK(hipMalloc(&p, std::max<size_t>(segsz, 256)));
+  HIPCHK(dev_malloc(&p, std::max<size_t>(segsz, 256)));
   std::shared_ptr<void> seg_arena(p, dfree);
   std::vector<Seg*> segp((size_t)std::max(n_sets, 1));
   for (int32_t i = 0; i < n_sets; i++) {
@@ -842,7 +795,7 @@ pl_status readsets_upload_many(pl_ctx* c, int32_t n_sets, const int32_t* contig_
   HIPCHK(hipSetDevice(c->device));
   auto dfree = [](void* p) { (void)hipFree(p); };
   void* p = nullptr;
-  HIPCHK(hipMalloc(&p, std::max<size_t>(up, 256)));
+  HIPCHK(dev_malloc(&p, std::max<size_t>(up, 256)));
   std::shared_ptr<void> up_arena(p, dfree);
   uint8_t* U = (uint8_t*)up_arena.get();
   // the host arrays through two pinned staging buffers, packed by host
@@ -963,7 +916,7 @@ void lane_destroy(Lane* L) {
   if (L->stream) (void)hipStreamSynchronize(L->stream);
   drop_graph(L);
   L->free_buffers();
-  L->scratch.release();
+  L->scratch.drop();
   for (int k = 0; k < 2; k++) {
     if (L->stage_ev[k]) (void)hipEventDestroy(L->stage_ev[k]);
     if (L->stage[k]) (void)hipHostFree(L->stage[k]);
@@ -1653,7 +1606,7 @@ pl_status pl_ref_upload(pl_ctx* c, int32_t contig_id, const char* name, const ui
   ct.name = name ? name : "";
   ct.host.assign(ascii, ascii + len);
   ct.len = len;
-  HIPCHK(hipMalloc((void**)&ct.dev, (size_t)len + 64));
+  HIPCHK(dev_malloc((void**)&ct.dev, (size_t)len + 64));
   HIPCHK(hipMemcpyAsync(ct.dev, ascii, (size_t)len, hipMemcpyHostToDevice, L->stream));
   HIPCHK(hipMemsetAsync(ct.dev + len, 0, 64, L->stream));
   HIPCHK(hipStreamSynchronize(L->stream));

@@ -404,7 +404,7 @@ pl_status loader_finish(pl_loader* ld, int32_t nref, const int32_t* contig_ids, 
                o_lrt = lr ? take((size_t)P) : 0;
   HIPCHK(hipSetDevice(c->device));
   void* p = nullptr;
-  HIPCHK(hipMalloc(&p, std::max<size_t>(at, 256)));
+  HIPCHK(dev_malloc(&p, std::max<size_t>(at, 256)));
   std::shared_ptr<void> arena(p, [](void* q) { (void)hipFree(q); });
   uint8_t* U = (uint8_t*)p;
   HIPCHK(hipMemsetAsync(U, 0, std::max<size_t>(at, 256), st));
@@ -489,8 +489,8 @@ pl_status pl_loader_open(pl_ctx* c, int64_t record_bytes, int64_t slice_bytes, p
   }
   ld->bytes_cap = record_bytes + 64;
   ld->offs_cap = record_bytes / 36 + 1;
-  HIPCHK(hipMalloc((void**)&ld->bytes, (size_t)ld->bytes_cap + 64));
-  HIPCHK(hipMalloc((void**)&ld->offs, 8 * (size_t)ld->offs_cap));
+  HIPCHK(dev_malloc((void**)&ld->bytes, (size_t)ld->bytes_cap + 64));
+  HIPCHK(dev_malloc((void**)&ld->offs, 8 * (size_t)ld->offs_cap));
   *out = ld.release();
   return PL_OK;
 }

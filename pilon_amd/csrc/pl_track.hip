@@ -39,7 +39,7 @@ pl_status build_gcv(pl_ctx* c, const std::vector<int32_t>& ids, Lane* L) {
     jobs.push_back(g);
   }
   uint8_t* block = nullptr;
-  if (hipMalloc((void**)&block, bytes) != hipSuccess)
+  if (dev_malloc((void**)&block, bytes) != hipSuccess)
     return fail(PL_E_OOM, "device allocation of %zu bytes failed", bytes);
   std::shared_ptr<uint8_t> mem(block, [](uint8_t* p) { (void)hipFree(p); });
   for (size_t i = 0; i < jobs.size(); i++) jobs[i].gcv = block + off[i];

@@ -138,6 +138,12 @@ def test_no_unwritten_record_is_read(n_recs, rec_cap, spill_cap, whole):
     assert (list(seen) == n_recs) == whole
 
 
+def test_kept_scratch_makes_no_call_fail():
+    """A lane's scratch stays for its next call, up to a bound, and goes back
+    when any allocation finds no memory, unless a call is using it."""
+    assert CH.lib().ch_scratch() == 0
+
+
 def test_cost_bins_order_every_window():
     """Any cost falls in a bin of the table, more work never in a later one,
     and windows placed by their bins fill the queue's slots once each."""
