@@ -635,7 +635,8 @@ __global__ void __launch_bounds__(256) k_begin(EngineArgs A, const uint32_t* con
 // block.  Most windows of an even batch fall in a few bins, so what bounded
 // this kernel was atomics on a few addresses of one cache line: a block
 // counts in LDS, and its bins go to one of PL_BIN_COPIES copies, lines
-// apart.  38,062 windows: 224 us with an atomic a window, 41 us so.
+// apart.  38,062 windows: 265 us with an atomic a window and the whole set
+// searched for each window's last read, 41 us so.
 __global__ void __launch_bounds__(1024) k_plan(EngineArgs A, WinDev* wins) {
   __shared__ uint32_t cnt[PL_COST_BINS];
   if (threadIdx.x < PL_COST_BINS) cnt[threadIdx.x] = 0;
@@ -760,7 +761,7 @@ struct WideLds : SinkBase {
 // than the LDS buffer holds, or of a set with reads of many clips is left to
 // the wide form (k_window): its quals and counts could leave their 20 and 12
 // bits.  512 positions, narrow for wide: 24 Mb at 60x 2.05 -> 1.80 ms, 2 Mb
-// at 250x 0.45 -> 0.30 ms (at 60x the window's own phases, not the bases,
+// at 100x 0.45 -> 0.30 ms (at 60x the window's own phases, not the bases,
 // take two thirds of the time).
 struct NarrowLds : SinkBase {
   static constexpr bool narrow = true;
@@ -896,10 +897,9 @@ __device__ __forceinline__ int32_t long_seg_range(const Seg* sg, uint32_t n, int
 // (a third of the time) and a dozen dependent phases (head, read facts,
 // segments, sums, columns, statistics) at 3 waves a SIMD; VALU issue is
 // half used, LDS a fifth, HBM 40%.  Measured on 24 Mb, 512 positions: the
-// facts of the first chunk asked for before the counters are cleared, the
-// segment of the evidence records and the reference before the sums, sums
-// scanned in registers, simple runs in their table before the segments are
-// applied (161 VGPRs for 168 and 2 spilled): 1.87 -> 1.80 ms.  Tried and
+// segment of the evidence records and the reference asked for before the
+// sums, sums scanned in registers, simple runs in their table before the
+// segments are applied (161 VGPRs for 168 and 2 spilled): 1.87 -> 1.80 ms.  Tried and
 // slower: 4 waves a SIMD (16 spills, 1.99), loads two batches ahead (13
 // spills, 2.09), 512 threads a window (3.86).
 static_assert(PL_CHUNK % 2 == 1 && PL_CHUNK <= 31, "an odd chunk of at most 31 bases (two 16-base words)");
@@ -1000,8 +1000,6 @@ __global__ void __launch_bounds__(BLOCK, NARROW ? PL_NARROW_WAVES_EU : PL_WIN_WA
       CR = ch <= NW || 4 * even <= 5 * ch ? (n > even ? (n + even - 1) / even : 1) : 64;
     }
     const bool stager = lane < CR;
-    // the next chunk's read facts are loaded while the current one is piled,
-    // the first one's while the counters are cleared
     int64_t t0 = win.plo + CR * wave;
     {
       uint4* l4 = (uint4*)lds;   // 16-byte stores: lds is 16-byte aligned
@@ -1604,9 +1602,12 @@ __device__ __forceinline__ uint32_t rs_digit(const uint32_t* lo, const uint32_t*
 // Few tiles (FUSED): counts are kept tile by tile, and every block of the
 // scatter adds up the tiles before it itself, one coalesced load a tile, in
 // place of three scan kernels of 15 us together.  75 tiles: scatter 13 -> 16
-// us, so a pass 34 -> 22 us; the line is at RS_FUSED_TILES = 128 tiles, where
-// the loads cost half of what the scans do.  A sort that tiles of 1,024
-// records cut in no more tiles than that takes those: shorter blocks.
+// us, so a pass 34 -> 22 us.  A sort that tiles of 1,024 records cut in no
+// more tiles than RS_FUSED_TILES takes those: shorter blocks.  K-mer graphs
+// of 130,000 / 200,000 / 520,000 / 700,000 / 2,000,000 occurrences with the
+// line at 64 tiles: 202 / 210 / 276 / 279 / 361 us, at 128: 187 / 211 / 240 /
+// 279 / 360, at 256: 184 / 197 / 238 / 244 / 361, at 512: 189 / 201 / 294 /
+// 250 / 403 (the loads are as long as the scans were).
 template <int ITEMS, bool FUSED>
 __global__ void __launch_bounds__(256) k_rs_hist(const uint32_t* lo, const uint32_t* hi, uint32_t n, int shift,
                                                  uint32_t* hist, int32_t nblocks) {

@@ -2,7 +2,8 @@
 whose records just fit their LDS buffer (128) and spill beyond it, at one
 column and over many, with the windows taken in their own order and, when
 more than the launch holds at once, in cost order; more spilled records than
-their list holds at first, on a context that held another set's records."""
+their list holds at first, on a context that held another set's records; a
+window of more reads than the cost order tells apart among them."""
 import numpy as np
 import pytest
 
@@ -126,3 +127,32 @@ def test_candidates_over_many_blocks():
         want_c += w["changes"]
     assert changes == want_c
     assert changes.count("\n") > 2000
+
+
+def test_very_deep_window_in_cost_order():
+    """A window of 70,000 reads (costs are told apart up to 65,535), one of
+    66,000 and a contig's last, of a position, among more windows than the
+    launch holds at once: every window is piled."""
+    from oracle import oracle as O
+    from pilon_amd.engine import Context
+    print("case: very deep windows in cost order", flush=True)
+    rng = np.random.default_rng(11)
+    n = 64 * 2600 + 1
+    ref = "".join("ACGT"[x] for x in rng.integers(0, 4, n))
+    starts = np.concatenate([np.full(70_000, 64 * 900 + 20), np.full(66_000, 64 * 2100 + 20),
+                             rng.integers(0, n - 30, 20_000)])
+    b = pack_reads([dict(pos=int(a) + 1, cigar="30M", seq=ref[a:a + 30], qual=[30] * 30, mapq=40 + int(a) % 3)
+                    for a in np.sort(starts)])
+    cfg = default_config()
+    want = O.run_region(cfg, ref.encode(), 1, n, [b], name="ctg")
+    assert want["status"] == 0
+    ctx = Context(cfg, device=0)
+    try:
+        ctx.ref_upload(0, "ctg", ref)
+        rid = ctx.readset_upload(0, b)
+        for window in (64, 512):
+            pile, calls, stats = ctx.batch_run([(0, 1, n, rid)], window=window, block=256, persistent=1)
+            assert_same_region(pile, calls, want, f"window {window}")
+            assert_same_stats(stats[0], want["stats"], f"window {window}")
+    finally:
+        ctx.close()
