@@ -155,6 +155,19 @@ PL_HD uint32_t del_hash(const uint8_t* ref, int64_t off, int32_t len, uint32_t* 
 // by side; prep_read takes them in order.
 struct PrepOut { RMeta m; int32_t events; bool clips; };   // clips: more than two S ops
 
+struct ReadHead {            // a read's header, loaded at once
+  int64_t c0, c1;            // its CIGAR
+  int32_t pos, tlen, L, mapq;
+  uint32_t flag;
+};
+PL_HD ReadHead read_head(const RSDev& R, int64_t r) {
+  ReadHead h;
+  h.flag = R.flag[r]; h.mapq = R.mapq[r]; h.pos = R.pos[r]; h.tlen = R.tlen[r];
+  h.c0 = R.cigar_off[r]; h.c1 = R.cigar_off[r + 1];
+  h.L = (int32_t)(R.seq_off[r + 1] - R.seq_off[r]);
+  return h;
+}
+
 struct ReadSums {            // of a read's ops
   int32_t refLen = 0, readLen = 0, clipped = 0, nP = 0, nS = 0;
   bool bad = false;
@@ -170,14 +183,13 @@ PL_HD void add_op(ReadSums& s, uint32_t w) {
   s.nP += op == 6 ? 1 : 0;
 }
 
-PL_HD uint32_t read_info(const RSDev& R, int64_t r, const ReadSums& s, const KConf& cf, int32_t* aend) {
-  const uint16_t flag = R.flag[r];
-  const int32_t mq = R.mapq[r];
-  const int64_t c0 = R.cigar_off[r], c1 = R.cigar_off[r + 1];
-  const int32_t L = (int32_t)(R.seq_off[r + 1] - R.seq_off[r]);
+PL_HD uint32_t read_info(const RSDev& R, int64_t r, const ReadHead& h, const ReadSums& s, uint32_t op0, const KConf& cf,
+                         int32_t* aend) {
+  const uint32_t flag = h.flag;
+  const int32_t mq = h.mapq, L = h.L;
   const bool bad = s.bad || (L > 0 && s.readLen != L);
   uint32_t info = 0;
-  *aend = (flag & 0x4) ? 0 : R.pos[r] + s.refLen - 1;
+  *aend = (flag & 0x4) ? 0 : h.pos + s.refLen - 1;
   const bool keep = (cf.nonpf || !(flag & 0x200)) && (cf.duplicates || !(flag & 0x400)) && !(flag & 0x100);
   const bool paired = (flag & 0x1) != 0;
   const bool valid = (mq >= cf.min_mq) && (!paired || (((flag & 0x2) != 0) && ((flag & PL_RF_MATE_SAME_REF) != 0)));
@@ -194,8 +206,8 @@ PL_HD uint32_t read_info(const RSDev& R, int64_t r, const ReadSums& s, const KCo
   // reference around them), and walked until it has its segments
   const uint32_t lr = R.lrt ? (uint32_t)R.lrt[r] : 0u;
   if (lr) info |= (lr << RI_LR_SHIFT) | ((uint32_t)RI_SEG_MAX << RI_SEG_SHIFT);
-  if (c1 - c0 == 1 && L > 0 && !bad && !(flag & PL_RF_EXOTIC) && !lr) {
-    const int op = (int)(R.cigar[c0] & 15);
+  if (h.c1 - h.c0 == 1 && L > 0 && !bad && !(flag & PL_RF_EXOTIC) && !lr) {
+    const int op = (int)(op0 & 15);
     if (op == 0 || op == 7 || op == 8) info |= RI_SIMPLE;
   }
   return info;
@@ -234,11 +246,11 @@ PL_HD OpSpan op_span(const RSDev& R, const ReadAcc& a, uint32_t info, const KCon
   return s;
 }
 
-PL_HD PrepOut prep_result(const RSDev& R, int64_t r, uint32_t info, int32_t aend, const ReadSums& sums, const OpSpan& s) {
+PL_HD PrepOut prep_result(const ReadHead& h, uint32_t op0, uint32_t info, int32_t aend, const ReadSums& sums,
+                          const OpSpan& s) {
   PrepOut o;
-  const int32_t pos = R.pos[r], tlen = R.tlen[r];
-  const bool paired = (R.flag[r] & 0x1) != 0;
-  const int64_t c0 = R.cigar_off[r], c1 = R.cigar_off[r + 1];
+  const int32_t pos = h.pos, tlen = h.tlen;
+  const bool paired = (h.flag & 0x1) != 0;
   if (s.events) info |= RI_EVENTS;
   // physCovIncr fragment (only valid reads, and not the right mate of a pair)
   int32_t flo = 0, fhi = 0;
@@ -247,31 +259,31 @@ PL_HD PrepOut prep_result(const RSDev& R, int64_t r, uint32_t info, int32_t aend
     else { flo = pos; fhi = j_add(pos, tlen); }
   }
   o.m.pos = pos; o.m.info = info; o.m.fp_lo = s.lo; o.m.fp_hi = s.hi;
-  o.m.fr_lo = flo; o.m.fr_hi = fhi; o.m.aend = aend; o.m.op0 = c1 > c0 ? R.cigar[c0] : 0u;
+  o.m.fr_lo = flo; o.m.fr_hi = fhi; o.m.aend = aend; o.m.op0 = op0;
   o.events = s.events;
   o.clips = sums.nS > 2;
   return o;
 }
 
 PL_HD PrepOut prep_read(const RSDev& R, int64_t r, const KConf& cf) {
-  const int64_t c0 = R.cigar_off[r], c1 = R.cigar_off[r + 1];
+  const ReadHead h = read_head(R, r);
   ReadSums sums;
-  for (int64_t k = c0; k < c1; k++) add_op(sums, R.cigar[k]);
+  for (int64_t k = h.c0; k < h.c1; k++) add_op(sums, R.cigar[k]);
+  const uint32_t op0 = h.c1 > h.c0 ? R.cigar[h.c0] : 0u;
   int32_t aend;
-  const uint32_t info = read_info(R, r, sums, cf, &aend);
+  const uint32_t info = read_info(R, r, h, sums, op0, cf, &aend);
   OpSpan s;
   if (!(info & RI_BAD)) {
-    const int32_t L = (int32_t)(R.seq_off[r + 1] - R.seq_off[r]);
     const ReadAcc a = read_acc(R, r, info, cf.default_qual);
-    int32_t readOffset = 0, locus = R.pos[r];
-    for (int64_t k = c0; k < c1; k++) {
+    int32_t readOffset = 0, locus = h.pos;
+    for (int64_t k = h.c0; k < h.c1; k++) {
       const uint32_t w = R.cigar[k];
-      s = op_span(R, a, info, cf, w, locus, readOffset, L, s);
+      s = op_span(R, a, info, cf, w, locus, readOffset, h.L, s);
       if (consumes_read((int)(w & 15))) readOffset += (int32_t)(w >> 4);
       if (consumes_ref((int)(w & 15))) locus += (int32_t)(w >> 4);
     }
   }
-  return prep_result(R, r, info, aend, sums, s);
+  return prep_result(h, op0, info, aend, sums, s);
 }
 
 // Cost bin of a window: 0 for the most work, four mantissa bits above 16

@@ -222,18 +222,19 @@ __device__ __forceinline__ void prep_long(const RSDev& R, int64_t r, const KConf
                                           uint32_t* segcount, int32_t* scal, int64_t* outliers, int64_t out_cap,
                                           PrepAcc& acc) {
   const int lane = threadIdx.x & 63;
-  const int32_t L = (int32_t)(R.seq_off[r + 1] - R.seq_off[r]);
-  const int64_t n_ops = R.cigar_off[r + 1] - R.cigar_off[r];
+  const ReadHead h = read_head(R, r);
+  const int32_t L = h.L;
   ReadSums sums;
-  for (int64_t k = R.cigar_off[r] + lane; k < R.cigar_off[r + 1]; k += 64) add_op(sums, R.cigar[k]);
+  for (int64_t k = h.c0 + lane; k < h.c1; k += 64) add_op(sums, R.cigar[k]);
   sums.refLen = wave_sum(sums.refLen);
   sums.readLen = wave_sum(sums.readLen);
   sums.clipped = (int32_t)wave_sum((uint32_t)sums.clipped);          // (Int sums wrap)
   sums.nP = wave_sum(sums.nP);
   sums.nS = wave_sum(sums.nS);
   sums.bad = __ballot(sums.bad) != 0;
+  const uint32_t op0 = h.c1 > h.c0 ? R.cigar[h.c0] : 0u;
   int32_t aend;
-  const uint32_t info = read_info(R, r, sums, cf, &aend);
+  const uint32_t info = read_info(R, r, h, sums, op0, cf, &aend);
   OpSpan span;
   LongOps lo;
   int64_t n = 0;
@@ -258,7 +259,7 @@ __device__ __forceinline__ void prep_long(const RSDev& R, int64_t r, const KConf
   }
   if (info & RI_NOQUAL) fill_quals(R, r, cf, lane, 64);
   if (lane == 0)
-    prep_put(R, r, prep_result(R, r, info, aend, sums, span), wants_segs(info) ? long_seg_slots(lo, L, n, n_ops) : 0u,
+    prep_put(R, r, prep_result(h, op0, info, aend, sums, span), wants_segs(info) ? long_seg_slots(lo, L, n, h.c1 - h.c0) : 0u,
              keepflag, segcount, scal, outliers, out_cap, acc);
 }
 
