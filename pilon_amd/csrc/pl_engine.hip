@@ -165,7 +165,7 @@ enum { PL_N_REC = 0, PL_N_CAND, PL_N_DEFER, PL_N_MUTATED, PL_N_OVERFLOW, PL_N_QU
 struct Lane {
   hipStream_t stream = nullptr;
   hipEvent_t ev[4] = {};
-  DBuf rsarr, kparr, jobs, wins, cost, bins, pile, calls, cmask, dmask, dbase, drec, csums, res, dhist, rec, winrec, spill,
+  DBuf rsarr, kparr, jobs, wins, cost, bins, pile, calls, cmask, dwords, csums, res, dhist, rec, winrec, spill,
       spillat, defer, mutated, strpool, stridx, stroff, wide, winwide, heads, wideheads;
   DBuf hist, tiles;                // sort and scan scratch (uploads, K-mers)
   // res holds what the host needs of a batch, one copy's worth: the counters,
@@ -220,7 +220,7 @@ struct Lane {
   bool has_jdepth = false;
 
   template <class F> void for_each_buffer(F&& f) {
-    DBuf* b[] = {&rsarr, &kparr, &jobs, &wins, &cost, &bins, &pile, &calls, &cmask, &dmask, &dbase, &drec, &csums, &res, &dhist, &rec,
+    DBuf* b[] = {&rsarr, &kparr, &jobs, &wins, &cost, &bins, &pile, &calls, &cmask, &dwords, &csums, &res, &dhist, &rec,
                  &winrec, &spill, &spillat, &defer, &mutated, &strpool, &stridx, &stroff,
                  &wide, &winwide, &heads, &wideheads, &hist, &tiles, &jdepth};
     for (DBuf* x : b) f(*x);
@@ -1068,18 +1068,19 @@ pl_status run_jobs(pl_ctx* c, Lane* L, const std::vector<JobReq>& reqs, int32_t 
     L->rs_seen = c->rs_version;
   }
   // ---- capacities (grown and re-run on overflow)
-  if (!L->rec_cap) { L->rec_cap = 1u << 18; L->cand_cap = 1u << 16; L->defer_cap = 1u << 16; L->mut_cap = 1u << 16; }
+  if (!L->cand_cap) { L->cand_cap = 1u << 16; L->defer_cap = 1u << 16; L->mut_cap = 1u << 16; }
   if (!L->spill_cap) L->spill_cap = 1u << 14;
   if (!L->wide_cap) L->wide_cap = 1u << 12;
-  L->rec_cap = std::max<uint32_t>(L->rec_cap, (uint32_t)std::min<int64_t>(G / 16 + 65536, 1ll << 30));
+  const uint32_t room = std::max<uint32_t>(1u << 18, (uint32_t)std::min<int64_t>(G / 16 + 65536, 1ll << 30));
+  L->rec_cap = std::max(L->rec_cap, room);
   L->cand_cap = std::max<uint32_t>(L->cand_cap, (uint32_t)std::min<int64_t>(G / 256 + 16384, 1ll << 30));
   L->defer_cap = std::max<uint32_t>(L->defer_cap, (uint32_t)std::min<int64_t>(G / 256 + 16384, 1ll << 30));
   L->mut_cap = std::max<uint32_t>(L->mut_cap, (uint32_t)std::min<int64_t>(G / 256 + 16384, 1ll << 30));
   // the segments of the batch's reads bound its records; where that is more
   // than half of what the windows hold in LDS, as many may spill as there is
-  // room for records (a first pass that found the list short ran again: long
-  // reads given as unpaired, 200 kb at 40x, 26.5 ms for 10.1).  Serving lanes
-  // and the scratch array keep to their sizes.
+  // room for records at first (a first pass that found the list short ran
+  // again: long reads given as unpaired, 200 kb at 40x, 26.5 ms for 10.1).
+  // Serving lanes and the scratch array keep to their sizes.
   if (L == &c->main || L == &c->aux) {
     double segs = 0;
     for (const JobReq& q : reqs) {
@@ -1087,7 +1088,7 @@ pl_status run_jobs(pl_ctx* c, Lane* L, const std::vector<JobReq>& reqs, int32_t 
       if (rs) segs += (double)rs->nseg * (double)(q.stop - q.start + 1) / (double)rs->d.ref_len;
     }
     if (segs > (double)(PL_WIN_RECS / 2) * n_wins)
-      L->spill_cap = std::max<uint32_t>(L->spill_cap, (uint32_t)std::min<double>(segs, (double)L->rec_cap));
+      L->spill_cap = std::max<uint32_t>(L->spill_cap, (uint32_t)std::min<double>(segs, (double)room));
   }
   HIPCHK(L->jobs.ensure(sizeof(JobDev) * n_jobs));
   HIPCHK(L->wins.ensure(sizeof(WinDev) * n_wins));
@@ -1097,10 +1098,10 @@ pl_status run_jobs(pl_ctx* c, Lane* L, const std::vector<JobReq>& reqs, int32_t 
   HIPCHK(L->wideheads.ensure(4 * (size_t)n_wins));
   HIPCHK(L->cost.ensure((size_t)n_wins));
   HIPCHK(L->bins.ensure(4 * (PL_BIN_COPIES + 1) * PL_COST_BINS));
-  HIPCHK(L->cmask.ensure(8 * (size_t)n_wins * (size_t)(W / 64)));
-  HIPCHK(L->csums.ensure(4 * (((size_t)n_wins * (size_t)(W / 64) + PL_CAND_WORDS - 1) / PL_CAND_WORDS)));
-  HIPCHK(L->dmask.ensure(8 * (size_t)n_wins * (size_t)(W / 64)));
-  HIPCHK(L->dbase.ensure(4 * (size_t)n_wins * (size_t)(W / 64)));
+  const size_t n_words = (size_t)n_wins * (size_t)(W / 64);
+  HIPCHK(L->cmask.ensure(8 * n_words));
+  HIPCHK(L->csums.ensure(4 * ((n_words + PL_CAND_WORDS - 1) / PL_CAND_WORDS)));
+  HIPCHK(L->dwords.ensure(12 * n_words));            // dmask, then dbase
   HIPCHK(L->dhist.ensure(4 * (size_t)PL_HIST * (size_t)n_jobs));
   HIPCHK(L->pile.ensure(4 * (size_t)PL_NFIELDS * G));
   HIPCHK(L->calls.ensure(sizeof(pl_call) * (size_t)G));
@@ -1138,8 +1139,7 @@ pl_status run_jobs(pl_ctx* c, Lane* L, const std::vector<JobReq>& reqs, int32_t 
     HIPCHK(L->spill.ensure(sizeof(IndelRec) * (size_t)L->spill_cap));
     HIPCHK(L->spillat.ensure(8 * (size_t)L->spill_cap));
     HIPCHK(L->res.ensure(Lane::cand_at((size_t)n_jobs) + sizeof(Cand) * (size_t)L->cand_cap));
-    HIPCHK(L->defer.ensure(4 * (size_t)L->defer_cap));
-    HIPCHK(L->drec.ensure(4 * (size_t)L->defer_cap));
+    HIPCHK(L->defer.ensure(8 * (size_t)L->defer_cap));   // defer, then drec
     HIPCHK(L->mutated.ensure(4 * (size_t)L->mut_cap));
     HIPCHK(L->wide.ensure(sizeof(WideCol) * (size_t)L->wide_cap));
     uint32_t* cnt = L->counters();
@@ -1170,9 +1170,9 @@ pl_status run_jobs(pl_ctx* c, Lane* L, const std::vector<JobReq>& reqs, int32_t 
     A.spill = L->spill.as<IndelRec>(); A.spill_at = L->spillat.as<uint2>();
     A.spill_n = cnt + PL_N_SPILL; A.spill_cap = L->spill_cap;
     A.cmask = L->cmask.as<uint64_t>();
-    A.dmask = L->dmask.as<uint64_t>();
-    A.dbase = L->dbase.as<uint32_t>();
-    A.drec = L->drec.as<int32_t>();
+    A.dmask = L->dwords.as<uint64_t>();
+    A.dbase = (uint32_t*)(A.dmask + n_words);
+    A.drec = L->defer.as<int32_t>() + L->defer_cap;
     A.cand = L->cands((size_t)n_jobs); A.cand_n = cnt + PL_N_CAND; A.cand_cap = L->cand_cap;
     A.defer = L->defer.as<uint32_t>(); A.defer_n = cnt + PL_N_DEFER; A.defer_cap = L->defer_cap;
     A.mutated = L->mutated.as<uint32_t>(); A.mutated_n = cnt + PL_N_MUTATED; A.mutated_cap = L->mut_cap;
