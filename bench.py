@@ -388,7 +388,7 @@ def main():
                "stream_wall_ms": swall, "stream_GB_per_s": nbytes / (swall / 1000.0) / 1e9,
                "records_per_s": lines / (vms / 1000.0), "text_GB_per_s": nbytes / (vms / 1000.0) / 1e9,
                "note": "Vcf.writeRecord lines of every locus (GenomeRegion.writeVcf) formatted on the device; "
-                       "device_ms covers the mark, indel, length, scan and write passes; wall_ms is pl_batch_vcf "
+                       "device_ms covers the length, scan and write passes; wall_ms is pl_batch_vcf "
                        "with the text copied into one host buffer it allocates; stream_wall_ms is "
                        "pl_batch_vcf_stream handing the same text to a consumer in 32 MB pieces"}
         log(f"bench: VCF: {lines} records, {nbytes / 1e9:.2f} GB in {vms:.1f} ms on the device "

@@ -896,8 +896,9 @@ __device__ __forceinline__ int32_t long_seg_range(const Seg* sg, uint32_t n, int
 //
 // What bounds it: latency.  At 60x a window is ~9 batches of pieces a wave
 // (a third of the time) and a dozen dependent phases (head, read facts,
-// segments, sums, columns, statistics) at 3 waves a SIMD; VALU issue is
-// half used, LDS a fifth, HBM 40%.  Measured on 24 Mb, 512 positions: the
+// segments, sums, columns, statistics) at 3 waves a SIMD; on 60 Mb at 60x
+// VALU issue is half used, LDS a third, HBM 35% of 8 TB/s, and waves wait 65%
+// of their cycles.  Measured on 24 Mb, 512 positions: the
 // segment of the evidence records and the reference asked for before the
 // sums, sums scanned in registers, simple runs in their table before the
 // segments are applied (161 VGPRs for 168 and 2 spilled): 1.87 -> 1.80 ms.  Tried and
