@@ -2,6 +2,7 @@
 oracle's, byte for byte: the known-answer cases (region API), synthetic
 batches of many regions (clips, improper pairs, MAPQ-0 repeats, indels, N,
 diploid hotspots), and the --diploid / --vcfqe variants."""
+import numpy as np
 import pytest
 
 from pilon_amd.abi import default_config
@@ -173,3 +174,46 @@ def test_vcf_stream_equals_text(engine):
     with pytest.raises(PilonError) as e:
         engine.batch_vcf_stream(lambda b: False)
     assert e.value.status == 1
+
+
+@pytest.mark.parametrize("n_own,op,ln,at", [(2, "D", 2, (3, 6)), (2, "D", 2, (3,)), (2, "I", 3, (3, 6)), (3, "D", 1, (4,)),
+                                            (9, "I", 2, (3, 6)), (9, "D", 3, (3, 6))])
+def test_vcf_columns_under_a_deletion(n_own, op, ln, at):
+    """Columns under a called deletion that have indel records of their own:
+    called again with the deletion's count, so that two records win a column
+    the window kernel left alone (whose call type tells, where no read has a
+    base there); the batch and its repeated passes."""
+    from oracle import oracle as O
+    from pilon_amd.engine import Context
+    from pilon_amd.reads import pack_reads
+    print(f"case: {n_own} own {op} records under a deletion", flush=True)
+    rng = np.random.default_rng(7 + n_own)
+    ref = "".join("ACGT"[x] for x in rng.integers(0, 4, 1500))
+    reads = []
+
+    def read(p, dels, ins):
+        cut = p + 40 + dels
+        seq = ref[p:p + 40] + "GATC"[:ins] + ref[cut:cut + 40]
+        reads.append(dict(pos=p + 1, cigar=f"40M{dels}D40M" if dels else f"40M{ins}I40M", seq=seq,
+                          qual=[int(x) for x in rng.integers(20, 41, len(seq))], mapq=60))
+
+    for site in range(200, 1300, 130):
+        for _ in range(20):
+            read(site - 40, 9, 0)
+        for k in at:
+            for _ in range(n_own):
+                read(site - 40 + k, ln if op == "D" else 0, ln if op == "I" else 0)
+    b = pack_reads(reads)
+    cfg = default_config()
+    want = O.run_region(cfg, ref.encode(), 1, len(ref), [b], name="ctg", vcf=O.VCF_ON)
+    assert want["status"] == 0
+    ctx = Context(cfg, device=0)
+    try:
+        ctx.ref_upload(0, "ctg", ref)
+        rid = ctx.readset_upload(0, b)
+        ctx.batch_run([(0, 1, len(ref), rid)], window=64, block=256, persistent=1, copy_out=False, use_graph=True)
+        assert ctx.batch_vcf()[0] == want["vcf"]
+        ctx.batch_repeat(2)
+        assert ctx.batch_vcf()[0] == want["vcf"]
+    finally:
+        ctx.close()
